@@ -220,3 +220,30 @@ def test_runtime_quant_zero_extents_and_rejections(device):
     with pytest.raises(capi.VecopsHipError) as e:
         capi.quantize_rows(torch.zeros((4, 8), device=device), one, 3, torch.zeros((4, 9), dtype=torch.uint8, device=device))
     assert e.value.code == 1
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 1, 1), (3, 7, 15), (17, 33, 127), (24, 250, 129), (5, 40, 2047), (300, 257, 2049),
+                                   (130, 64, 4100)])
+def test_runtime_quant_packed_edges_equal_the_unpacked_call(device, m, n, k):
+    """Packed weights at the edges of the quantisation's 2048-element pieces, of the K padding of the quantised rows and
+    of the row sums' eight-row workgroups, in a workspace full of garbage: the unpacked call's bits (integer sums)."""
+    import torch
+    from vecops_amd import capi
+    a = dev((synth.uniform_pm1(1, (m, k)) * np.float32(60.0)).astype(np.float32), device)
+    b = dev(synth.int8_sym(2, (n, k)), device)
+    mult = dev((np.float32(3.0) + synth.uniform_pm1(3, (m,))).astype(np.float32), device)
+    rs, cs = dev(synth.scales(4, m), device), dev(synth.scales(5, n), device)
+    packed, corr = capi.pack_b(b, a_zero_point=128)
+    sums = b.cpu().numpy().astype(np.int64).sum(axis=1)
+    assert np.array_equal(corr.cpu().numpy(), (-128 * sums).astype(np.int32))
+    q = torch.empty((m, k), dtype=torch.uint8, device=device)
+    capi.quantize_rows(a, mult, 128, q)
+    acc = q.cpu().numpy().astype(np.int64) @ b.cpu().numpy().astype(np.int64).T - 128 * sums
+    want = (acc.astype(np.int32).astype(np.float32) * rs.cpu().numpy()[:, None]) * cs.cpu().numpy()[None, :]
+    ws = torch.full((1 << 24,), 0xA5, dtype=torch.uint8, device=device)
+    for packed_call in (True, False):
+        c = torch.full((m, n), float("nan"), device=device)
+        call, weights = (capi.matmul_runtime_quant_packed_b, packed) if packed_call else (capi.matmul_runtime_quant, b)
+        call(a, mult, 128, weights, rs, cs, c, correction=corr, workspace=ws)
+        torch.cuda.synchronize()
+        assert np.array_equal(c.cpu().numpy().view(np.uint32), want.view(np.uint32)), packed_call

@@ -9,6 +9,7 @@
 #include <cstring>
 
 #include "gemm_f64.h"
+#include "packed_row_sums.h"
 #include "skinny_dense.h"
 #include "skinny_w8a16.h"
 #include "tile_gemm_launch.h"
@@ -890,7 +891,7 @@ int32_t unsigned_side_terms(const Problem& pr, TileGemmParams* params, int32_t* 
     p.row_term = row_term;
   }
   if (pr.a_unsigned && pr.packed_b) {  // the same term from the packed rows, one copy per batch
-    e = launch_packed_row_sums(pr.b.data, p.n, p.k, p.batch, 128u, nullptr, col_term, stream);
+    e = launch_packed_row_sums({pr.b.data, p.n, p.k, p.batch, 128u, nullptr, 0, col_term}, stream);
     if (e != hipSuccess) return fail(ST_EXEC, "row-sum kernel launch: %s", hipGetErrorString(e));
     p.col_term = col_term;
   } else if (pr.a_unsigned) {  // + 128 * sum_k b'[n,k] per column
@@ -1417,12 +1418,15 @@ namespace {
 // goes into the correction rows.  Workspace: the quantised activations (one [M,K] matrix per batch, or a single
 // one when every batch shares activations and multipliers), the correction rows (N int32 per batch, or a single
 // row when every batch shares weights and correction) - both rounded up to 256 bytes - then the product's own
-// scratch.
+// scratch.  The matrix's rows are padded to whole 16-byte chunks, so that the loads that write LDS can fetch them; against
+// packed weights, whose k past K are zeros up to a whole K tile, to whole K tiles, and the product runs over the padded
+// K without a partial tile (what the padding holds is multiplied by zeros).
 struct RuntimeQuant {
   VecopsHipOperand a3, b3, c3, q, c_acc;
   Problem pr{};
   VecopsHipPlan plan;
   int64_t batch, m, n, k;
+  int64_t q_pitch;                 // elements from row to row of the quantised activations
   int64_t q_batches, row_batches;  // distinct quantised matrices / correction rows
   int64_t scale_bs, correction_bs;
   uint64_t q_bytes, row_bytes;
@@ -1477,7 +1481,9 @@ int32_t describe_runtime_quant(const VecopsHipOperand* a_given, const VecopsHipO
   const bool shared_b = packed != nullptr || d->b3.strides[0] == 0 || d->batch <= 1;
   d->q_batches = (d->batch > 1 && (d->a3.strides[0] != 0 || scale_bs != 0)) ? d->batch : 1;
   d->row_batches = (d->batch > 1 && (!shared_b || correction_bs != 0)) ? d->batch : 1;
-  d->q_bytes = (static_cast<uint64_t>(d->q_batches) * d->m * d->k + 255u) & ~uint64_t{255};
+  const int64_t q_step = packed != nullptr ? k_tile_elements(SRC_I8) : 16;
+  d->q_pitch = (d->k + q_step - 1) / q_step * q_step;
+  d->q_bytes = (static_cast<uint64_t>(d->q_batches) * d->m * d->q_pitch + 255u) & ~uint64_t{255};
   d->row_bytes = (static_cast<uint64_t>(d->row_batches) * d->n * 4u + 255u) & ~uint64_t{255};
   // the quantised activations: dense [batch, M, K], every batch the same matrix when there is only one
   memset(&d->q, 0, sizeof(d->q));
@@ -1485,9 +1491,9 @@ int32_t describe_runtime_quant(const VecopsHipOperand* a_given, const VecopsHipO
   d->q.dtype = DT_I8;
   d->q.rank = a_given->rank;
   const int base = a_given->rank == 3 ? 1 : 0;
-  if (base) { d->q.sizes[0] = d->batch; d->q.strides[0] = d->q_batches > 1 ? d->m * d->k : 0; }
-  d->q.sizes[base] = d->m; d->q.strides[base] = d->k;
-  d->q.sizes[base + 1] = d->k; d->q.strides[base + 1] = 1;
+  if (base) { d->q.sizes[0] = d->batch; d->q.strides[0] = d->q_batches > 1 ? d->m * d->q_pitch : 0; }
+  d->q.sizes[base] = d->m; d->q.strides[base] = d->q_pitch;
+  d->q.sizes[base + 1] = packed != nullptr ? d->q_pitch : d->k; d->q.strides[base + 1] = 1;
   d->c_acc = *c_given;
   d->c_acc.dtype = DT_I32;  // accumulator class; the epilogue writes fp32
   // Batches fold into rows ([batch * M, K] x the one B) only when the scales run on with the rows and one
@@ -1532,36 +1538,36 @@ int32_t run_runtime_quant(const VecopsHipOperand* a, const float* multipliers, i
   normalise(&d.a3, &vx);
   // correction[batch][n] + 128 * sum_k b[batch][n,k]
   int32_t* rows = reinterpret_cast<int32_t*>(static_cast<char*>(workspace) + d.q_bytes);
-  if (packed == nullptr && d.q_batches * d.m * d.k > 0 && d.row_batches * d.n > 0) {
-    // the activations' quantisation and the weight rows' sums in one launch: neither needs the other
-    View vb;
-    normalise(&d.b3, &vb);
-    hipError_t both = launch_quantize_and_row_sums(
-        static_cast<const float*>(vx.data), static_cast<int32_t>(d.q_batches), static_cast<int32_t>(d.m), static_cast<int32_t>(d.k),
-        vx.bs, vx.rs, vx.cs, multipliers, d.scale_bs, zero_point, 0x80u, static_cast<uint8_t*>(workspace), d.m * d.k, d.k, 1,
-        vb.data, static_cast<int32_t>(d.row_batches), static_cast<int32_t>(d.n), vb.bs, vb.rs, vb.cs, 0u, 128u, correction,
-        d.correction_bs, rows, s);
-    if (both != hipSuccess) return fail(ST_EXEC, "quantize and row-sum kernel launch: %s", hipGetErrorString(both));
-    return run_problem(d.pr, d.plan, row_scales, column_scales, rows, static_cast<char*>(workspace) + d.q_bytes + d.row_bytes,
-                       workspace_size - d.q_bytes - d.row_bytes, s);
-  }
-  hipError_t e = launch_quantize_rows(static_cast<const float*>(vx.data), static_cast<int32_t>(d.q_batches),
-                                      static_cast<int32_t>(d.m), static_cast<int32_t>(d.k), vx.bs, vx.rs, vx.cs,
-                                      multipliers, d.scale_bs, zero_point, 0x80u, static_cast<uint8_t*>(workspace),
-                                      d.m * d.k, d.k, 1, s);
-  if (e != hipSuccess) return fail(ST_EXEC, "quantize kernel launch: %s", hipGetErrorString(e));
+  // one launch quantises the activations and sums the weight rows (neither needs the other) unless one of the two has
+  // nothing to do
+  hipError_t e = hipSuccess;
+  const int32_t q_batches = static_cast<int32_t>(d.q_batches), m = static_cast<int32_t>(d.m), k = static_cast<int32_t>(d.k);
+  const bool quantizes = d.q_batches * d.m * d.k > 0, sums = d.row_batches * d.n > 0;
+  uint8_t* q = static_cast<uint8_t*>(workspace);
   if (packed != nullptr) {
     // one packed operand: the same sums for every batch, the caller's correction per batch
-    for (int64_t bi = 0; bi < d.row_batches && e == hipSuccess; ++bi)
-      e = launch_packed_row_sums(packed, static_cast<int32_t>(d.n), static_cast<int32_t>(d.k), 1, 128u,
-                                 correction ? correction + bi * d.correction_bs : nullptr, rows + bi * d.n, s);
+    const PackedRowSums packed_sums{packed, static_cast<int32_t>(d.n), k, static_cast<int32_t>(d.row_batches), 128u, correction,
+                                    d.correction_bs, rows};
+    if (quantizes && sums) {
+      e = launch_quantize_and_packed_row_sums(static_cast<const float*>(vx.data), q_batches, m, k, vx.bs, vx.rs, vx.cs, multipliers,
+                                              d.scale_bs, zero_point, 0x80u, q, d.m * d.q_pitch, d.q_pitch, 1, packed_sums, s);
+    } else if (sums) {
+      e = launch_packed_row_sums(packed_sums, s);
+    }
   } else {
     View vb;
     normalise(&d.b3, &vb);
-    e = launch_byte_row_sums(vb.data, static_cast<int32_t>(d.row_batches), static_cast<int32_t>(d.n),
-                             static_cast<int32_t>(d.k), vb.bs, vb.rs, vb.cs, 0u, 128u, correction, d.correction_bs, rows, s);
+    if (quantizes && sums) {
+      e = launch_quantize_and_row_sums(static_cast<const float*>(vx.data), q_batches, m, k, vx.bs, vx.rs, vx.cs, multipliers,
+                                       d.scale_bs, zero_point, 0x80u, q, d.m * d.q_pitch, d.q_pitch, 1, vb.data,
+                                       static_cast<int32_t>(d.row_batches), static_cast<int32_t>(d.n), vb.bs, vb.rs, vb.cs, 0u, 128u,
+                                       correction, d.correction_bs, rows, s);
+    } else if (sums) {
+      e = launch_byte_row_sums(vb.data, static_cast<int32_t>(d.row_batches), static_cast<int32_t>(d.n), k, vb.bs, vb.rs, vb.cs, 0u,
+                               128u, correction, d.correction_bs, rows, s);
+    }
   }
-  if (e != hipSuccess) return fail(ST_EXEC, "row-sum kernel launch: %s", hipGetErrorString(e));
+  if (e != hipSuccess) return fail(ST_EXEC, "quantize and row-sum kernel launch: %s", hipGetErrorString(e));
   return run_problem(d.pr, d.plan, row_scales, column_scales, rows, static_cast<char*>(workspace) + d.q_bytes + d.row_bytes,
                      workspace_size - d.q_bytes - d.row_bytes, s);
 }

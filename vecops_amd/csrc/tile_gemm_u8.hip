@@ -1,5 +1,6 @@
 // Tile GEMM instances for 8-bit integer operands with an unsigned side, and the
 // row-sum kernel that produces their epilogue terms.
+#include "packed_row_sums.h"
 #include "tile_gemm_launch.h"
 namespace vecops_hip {
 hipError_t launch_tile_gemm_i8_flip(const TileGemmParams& p, int tile_m, int tile_n, int mode, hipStream_t stream) {
@@ -58,8 +59,10 @@ __global__ __launch_bounds__(256) void byte_row_sums_kernel(const ByteRowSums a)
 // RuntimePerRowAsymmetricQuantizeTransform (matmul/Quantization.h:91-146) and the conversion of its fp32
 // result to the uint8 compute type - a multiply and an add, each rounded (the file is compiled without
 // contraction), truncation toward zero, NaN and values outside int32 to INT32_MIN, saturation to 0..255.
-// One thread per four consecutive k: one 16-byte load when x is K-contiguous and the quad is aligned, one
-// 4-byte store when q is.  flip (0 or 0x80) is xored into every byte.
+// Rows contiguous on both sides (quantize_contiguous_rows): a workgroup takes kQuantizePiece elements of one row, two
+// quads a lane, each one 16-byte load and one 4-byte store at whatever alignment.  Bound by the bytes: no division per
+// lane, and enough workgroups (a 2048-element piece each) that their loads overlap.  Other strides: one thread per four
+// consecutive k, element by element where a quad cannot be taken whole.  flip (0 or 0x80) is xored into every byte.
 struct QuantizeRows {
   const float* x;
   int32_t batch, rows, k;
@@ -72,6 +75,48 @@ struct QuantizeRows {
   int64_t qbs, qrs, qks;
 };
 
+constexpr int kQuantizePiece = 2048;
+
+struct __attribute__((packed, aligned(4))) FloatQuad { float v[4]; };
+struct __attribute__((packed, aligned(1))) ByteQuad { uint32_t v; };
+
+// (block: the workgroup's number among those that quantise; xks == qks == 1)
+__device__ __forceinline__ void quantize_contiguous_rows(const QuantizeRows& a, uint32_t block) {
+  const uint32_t pieces = (static_cast<uint32_t>(a.k) + kQuantizePiece - 1) / kQuantizePiece;
+  const uint32_t row = block / pieces, piece = block - row * pieces;
+  const uint32_t b = row / static_cast<uint32_t>(a.rows), r = row - b * static_cast<uint32_t>(a.rows);
+  const float* src = a.x + b * a.xbs + r * a.xrs;
+  uint8_t* dst = a.q + b * a.qbs + r * a.qrs;
+  const float mult = a.multipliers[b * a.mult_bs + r];
+  constexpr int kQuads = kQuantizePiece / 1024;
+  const int k0 = static_cast<int>(piece) * kQuantizePiece + static_cast<int>(threadIdx.x) * 4;
+  FloatQuad quad[kQuads];
+#pragma unroll
+  for (int i = 0; i < kQuads; ++i) {
+    const int k = k0 + i * 1024;
+    if (k + 4 <= a.k) {
+      quad[i] = *reinterpret_cast<const FloatQuad*>(src + k);
+    } else {
+      for (int e = 0; e < 4; ++e) quad[i].v[e] = k + e < a.k ? src[k + e] : 0.0f;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < kQuads; ++i) {
+    const int k = k0 + i * 1024;
+    uint32_t word = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float scaled = quad[i].v[e] * mult;
+      word |= (narrow_to_byte(scaled + a.zero_point, false) ^ a.flip) << (8 * e);  // flip 0x80: the byte as q - 128 in int8
+    }
+    if (k + 4 <= a.k) {
+      reinterpret_cast<ByteQuad*>(dst + k)->v = word;
+    } else {
+      for (int e = 0; k + e < a.k; ++e) dst[k + e] = static_cast<uint8_t>(word >> (8 * e));
+    }
+  }
+}
+
 // (block of blocks: the workgroup's number among those that quantise, and how many they are)
 __device__ __forceinline__ void quantize_rows(const QuantizeRows& a, int64_t block, int64_t blocks) {
   const float* x = a.x;
@@ -81,6 +126,10 @@ __device__ __forceinline__ void quantize_rows(const QuantizeRows& a, int64_t blo
   const float zero_point = a.zero_point;
   const uint32_t flip = a.flip;
   uint8_t* q = a.q;
+  if (xks == 1 && qks == 1) {
+    quantize_contiguous_rows(a, static_cast<uint32_t>(block));
+    return;
+  }
   const int64_t quads_per_row = (static_cast<int64_t>(k) + 3) / 4;
   const int64_t total = static_cast<int64_t>(batch) * rows * quads_per_row;
   for (int64_t idx = block * 256ll + threadIdx.x; idx < total; idx += blocks * 256ll) {
@@ -92,22 +141,10 @@ __device__ __forceinline__ void quantize_rows(const QuantizeRows& a, int64_t blo
     const float mult = multipliers[b * mult_bs + r];
     const int left = min(4, k - k0);
     float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (left == 4 && xks == 1 && (reinterpret_cast<uintptr_t>(src) & 15u) == 0) {
-      const f32x4 quad = *reinterpret_cast<const f32x4*>(src);
-      v[0] = quad[0]; v[1] = quad[1]; v[2] = quad[2]; v[3] = quad[3];
-    } else {
-      for (int e = 0; e < left; ++e) v[e] = src[e * xks];
-    }
-    uint32_t bytes[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
+    for (int e = 0; e < left; ++e) v[e] = src[e * xks];
+    for (int e = 0; e < left; ++e) {
       const float scaled = v[e] * mult;
-      bytes[e] = narrow_to_byte(scaled + zero_point, false) ^ flip;  // flip 0x80: the byte as q - 128 in int8
-    }
-    if (left == 4 && qks == 1 && (reinterpret_cast<uintptr_t>(dst) & 3u) == 0) {
-      *reinterpret_cast<uint32_t*>(dst) = bytes[0] | (bytes[1] << 8) | (bytes[2] << 16) | (bytes[3] << 24);
-    } else {
-      for (int e = 0; e < left; ++e) dst[e * qks] = static_cast<uint8_t>(bytes[e]);
+      dst[e * qks] = static_cast<uint8_t>(narrow_to_byte(scaled + zero_point, false) ^ flip);
     }
   }
 }
@@ -122,9 +159,19 @@ __global__ __launch_bounds__(256) void quantize_and_row_sums_kernel(const Quanti
   else byte_row_sums(sa, blockIdx.x - quantize_blocks);
 }
 
+// The same with the weights packed.
+__global__ __launch_bounds__(256) void quantize_and_packed_row_sums_kernel(const QuantizeRows qa, const PackedRowSums sa, uint32_t quantize_blocks) {
+  if (blockIdx.x < quantize_blocks) quantize_rows(qa, blockIdx.x, quantize_blocks);
+  else packed_row_sums(sa, blockIdx.x - quantize_blocks);
+}
+
 namespace {
-int64_t quantize_blocks_for(int64_t total_quads) {
-  int64_t blocks = (total_quads + 255) / 256;
+// Workgroups of quantize_rows; 0 when there is nothing to quantise, more than INT32_MAX when they cannot be launched.
+int64_t quantize_blocks_for(const QuantizeRows& a) {
+  const int64_t rows = static_cast<int64_t>(a.batch) * a.rows;
+  if (rows <= 0 || a.k <= 0) return 0;
+  if (a.xks == 1 && a.qks == 1) return rows * ((static_cast<int64_t>(a.k) + kQuantizePiece - 1) / kQuantizePiece);
+  const int64_t blocks = (rows * ((static_cast<int64_t>(a.k) + 3) / 4) + 255) / 256;
   return blocks > 256 * 32 ? 256 * 32 : blocks;
 }
 }  // namespace
@@ -132,10 +179,11 @@ int64_t quantize_blocks_for(int64_t total_quads) {
 hipError_t launch_quantize_rows(const float* x, int32_t batch, int32_t rows, int32_t k, int64_t xbs, int64_t xrs,
                                 int64_t xks, const float* multipliers, int64_t mult_bs, int32_t zero_point, uint32_t flip,
                                 uint8_t* q, int64_t qbs, int64_t qrs, int64_t qks, hipStream_t stream) {
-  const int64_t total = static_cast<int64_t>(batch) * rows * ((static_cast<int64_t>(k) + 3) / 4);
-  if (total <= 0) return hipSuccess;
   const QuantizeRows a{x, batch, rows, k, xbs, xrs, xks, multipliers, mult_bs, static_cast<float>(zero_point), flip & 0xffu, q, qbs, qrs, qks};
-  hipLaunchKernelGGL(quantize_rows_kernel, dim3(static_cast<unsigned>(quantize_blocks_for(total))), dim3(256), 0, stream, a);
+  const int64_t blocks = quantize_blocks_for(a);
+  if (blocks == 0) return hipSuccess;
+  if (blocks > INT32_MAX) return hipErrorInvalidConfiguration;
+  hipLaunchKernelGGL(quantize_rows_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, a);
   return hipGetLastError();
 }
 
@@ -157,14 +205,27 @@ hipError_t launch_quantize_and_row_sums(const float* x, int32_t batch, int32_t r
                                         uint8_t* q, int64_t qbs, int64_t qrs, int64_t qks, const void* w, int32_t w_batch,
                                         int32_t w_rows, int64_t w_bs, int64_t w_rs, int64_t w_ks, uint32_t w_flip, uint32_t scale,
                                         const int32_t* add, int64_t add_bs, int32_t* out, hipStream_t stream) {
-  const int64_t total = static_cast<int64_t>(batch) * rows * ((static_cast<int64_t>(k) + 3) / 4);
-  const int64_t sums = static_cast<int64_t>(w_batch) * w_rows;
-  if (total <= 0 || sums <= 0) return hipErrorInvalidValue;
-  const int64_t q_blocks = quantize_blocks_for(total), s_blocks = (sums + 3) / 4;
-  if (q_blocks + s_blocks > INT32_MAX) return hipErrorInvalidConfiguration;
   const QuantizeRows qa{x, batch, rows, k, xbs, xrs, xks, multipliers, mult_bs, static_cast<float>(zero_point), flip & 0xffu, q, qbs, qrs, qks};
+  const int64_t sums = static_cast<int64_t>(w_batch) * w_rows;
+  const int64_t q_blocks = quantize_blocks_for(qa), s_blocks = (sums + 3) / 4;
+  if (q_blocks <= 0 || sums <= 0) return hipErrorInvalidValue;
+  if (q_blocks + s_blocks > INT32_MAX) return hipErrorInvalidConfiguration;
   const ByteRowSums sa{static_cast<const uint8_t*>(w), w_batch, w_rows, k, w_bs, w_rs, w_ks, w_flip, scale, add, add_bs, out};
   hipLaunchKernelGGL(quantize_and_row_sums_kernel, dim3(static_cast<unsigned>(q_blocks + s_blocks)), dim3(256), 0, stream, qa, sa,
+                     static_cast<uint32_t>(q_blocks));
+  return hipGetLastError();
+}
+
+// launch_quantize_rows and launch_packed_row_sums as one launch (both must have work).
+hipError_t launch_quantize_and_packed_row_sums(const float* x, int32_t batch, int32_t rows, int32_t k, int64_t xbs, int64_t xrs,
+                                               int64_t xks, const float* multipliers, int64_t mult_bs, int32_t zero_point,
+                                               uint32_t flip, uint8_t* q, int64_t qbs, int64_t qrs, int64_t qks,
+                                               const PackedRowSums& sums, hipStream_t stream) {
+  const QuantizeRows qa{x, batch, rows, k, xbs, xrs, xks, multipliers, mult_bs, static_cast<float>(zero_point), flip & 0xffu, q, qbs, qrs, qks};
+  const int64_t q_blocks = quantize_blocks_for(qa), s_blocks = packed_row_sums_blocks(sums);
+  if (q_blocks <= 0 || s_blocks <= 0) return hipErrorInvalidValue;
+  if (q_blocks + s_blocks > INT32_MAX) return hipErrorInvalidConfiguration;
+  hipLaunchKernelGGL(quantize_and_packed_row_sums_kernel, dim3(static_cast<unsigned>(q_blocks + s_blocks)), dim3(256), 0, stream, qa, sums,
                      static_cast<uint32_t>(q_blocks));
   return hipGetLastError();
 }
