@@ -245,3 +245,43 @@ def test_wide_tile_c_input_and_fused_transform(device, kind, out):
         assert float((c.double() - want).abs().max()) <= 1.0      # truncation next to an integer boundary
     else:
         assert rel_err(c.double().cpu().numpy(), want.cpu().numpy()) <= 1e-4 + (2.0 ** -8 if out == "bf16" else 0.0)
+
+
+@pytest.mark.parametrize("kind,out,bias_type", [("bf16", "own", "own"), ("bf16", "f32", "f32"), ("f16", "own", "f32"), ("f16", "f32", "own"),
+                                                ("bf16", "own", None)])
+@pytest.mark.parametrize("steps", ["none", "relu", "clamp", "sigmoid", "silu", "column scales, silu", "row scales", "scale, shift, clamp"])
+def test_wide_tile_bias_row_equals_the_same_bias_as_a_full_c_input(device, kind, out, bias_type, steps):
+    """A bias row and the scales come from LDS, each combination with only the steps it has; the same bias written out as
+    a whole C input goes through the general finishing step on the same tile: the results are equal bit for bit, NaN and
+    infinities in the bias among them, on edge tiles in both directions."""
+    import torch
+    from vecops_amd import capi
+    m, n, k = 1500, 11000, 512
+    gen = torch.Generator().manual_seed(5)
+    own = {"bf16": torch.bfloat16, "f16": torch.float16}[kind]
+    a = (torch.rand((m, k), generator=gen) * 2 - 1).to(own).to(device)
+    b = (torch.rand((n, k), generator=gen) * 2 - 1).to(own).to(device)
+    rs = (torch.rand(m, generator=gen) * 0.5 + 0.75).to(device)
+    cs = (torch.rand(n, generator=gen) * 0.5 + 0.75).to(device)
+    bias = (torch.rand((1, n), generator=gen) * 8 - 4).to(own if bias_type == "own" else torch.float32).to(device)
+    bias[0, [0, 17, n - 1]] = float("nan")
+    bias[0, [1, 352, n - 2]] = float("inf")
+    bias[0, [2, 353, n - 3]] = float("-inf")
+    if bias_type is None:
+        bias = torch.full((1, n), -0.0, device=device)    # adding it changes nothing
+    activation = next((s for s in ("relu", "clamp", "sigmoid", "silu") if s in steps), "none")
+    ep = capi.epilogue(activation=activation, clamp=(-1.5, 2.0), scale=0.75 if "scale, shift" in steps else None,
+                       shift=0.25 if "shift" in steps else None, row_scales=rs if "row scales" in steps else None,
+                       column_scales=cs if "column scales" in steps else None)
+    out_dtype = own if out == "own" else torch.float32
+    got, want = torch.zeros((m, n), dtype=out_dtype, device=device), torch.zeros((m, n), dtype=out_dtype, device=device)
+    row = None if bias_type is None else bias.expand(m, n)
+    full = bias.expand(m, n).contiguous()
+    for c_in, c in ((row, got), (full, want)):
+        assert capi.FAMILY_NAMES[capi.plan_matmul_fused(a, b, c, ep, c_in=c_in).family] == "tile_256x352"
+        capi.matmul_fused(a, b, c, ep, c_in=c_in)
+    torch.cuda.synchronize()
+    bits = torch.int32 if out == "f32" else torch.int16
+    if out == "own" and kind == "bf16" and bias_type is not None and "clamp" not in steps and "relu" not in steps:
+        assert bool((got.view(bits)[:, 0] == 0x7fc0).all())
+    assert torch.equal(got.view(bits), want.view(bits))
