@@ -1,6 +1,7 @@
 // Tile GEMM instances for 8-bit integer operands with an unsigned side, and the
 // row-sum kernel that produces their epilogue terms.
 #include "packed_row_sums.h"
+#include "row_work_split.h"
 #include "tile_gemm_launch.h"
 namespace vecops_hip {
 hipError_t launch_tile_gemm_i8_flip(const TileGemmParams& p, int tile_m, int tile_n, int mode, hipStream_t stream) {
@@ -75,41 +76,37 @@ struct QuantizeRows {
   int64_t qbs, qrs, qks;
 };
 
-constexpr int kQuantizePiece = 2048;
-
 struct __attribute__((packed, aligned(4))) FloatQuad { float v[4]; };
 struct __attribute__((packed, aligned(1))) ByteQuad { uint32_t v; };
 
 // (block: the workgroup's number among those that quantise; xks == qks == 1)
 __device__ __forceinline__ void quantize_contiguous_rows(const QuantizeRows& a, uint32_t block) {
-  const uint32_t pieces = (static_cast<uint32_t>(a.k) + kQuantizePiece - 1) / kQuantizePiece;
+  const uint32_t pieces = static_cast<uint32_t>(quantize_pieces(a.k));
   const uint32_t row = block / pieces, piece = block - row * pieces;
   const uint32_t b = row / static_cast<uint32_t>(a.rows), r = row - b * static_cast<uint32_t>(a.rows);
   const float* src = a.x + b * a.xbs + r * a.xrs;
   uint8_t* dst = a.q + b * a.qbs + r * a.qrs;
   const float mult = a.multipliers[b * a.mult_bs + r];
-  constexpr int kQuads = kQuantizePiece / 1024;
-  const int k0 = static_cast<int>(piece) * kQuantizePiece + static_cast<int>(threadIdx.x) * 4;
-  FloatQuad quad[kQuads];
+  FloatQuad quad[kQuantizeQuads];
 #pragma unroll
-  for (int i = 0; i < kQuads; ++i) {
-    const int k = k0 + i * 1024;
-    if (k + 4 <= a.k) {
+  for (int i = 0; i < kQuantizeQuads; ++i) {
+    const int64_t k = quantize_quad(piece, threadIdx.x, i);
+    if (quantize_quad_is_whole(k, a.k)) {
       quad[i] = *reinterpret_cast<const FloatQuad*>(src + k);
     } else {
       for (int e = 0; e < 4; ++e) quad[i].v[e] = k + e < a.k ? src[k + e] : 0.0f;
     }
   }
 #pragma unroll
-  for (int i = 0; i < kQuads; ++i) {
-    const int k = k0 + i * 1024;
+  for (int i = 0; i < kQuantizeQuads; ++i) {
+    const int64_t k = quantize_quad(piece, threadIdx.x, i);
     uint32_t word = 0;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const float scaled = quad[i].v[e] * mult;
       word |= (narrow_to_byte(scaled + a.zero_point, false) ^ a.flip) << (8 * e);  // flip 0x80: the byte as q - 128 in int8
     }
-    if (k + 4 <= a.k) {
+    if (quantize_quad_is_whole(k, a.k)) {
       reinterpret_cast<ByteQuad*>(dst + k)->v = word;
     } else {
       for (int e = 0; k + e < a.k; ++e) dst[k + e] = static_cast<uint8_t>(word >> (8 * e));
@@ -170,7 +167,7 @@ namespace {
 int64_t quantize_blocks_for(const QuantizeRows& a) {
   const int64_t rows = static_cast<int64_t>(a.batch) * a.rows;
   if (rows <= 0 || a.k <= 0) return 0;
-  if (a.xks == 1 && a.qks == 1) return rows * ((static_cast<int64_t>(a.k) + kQuantizePiece - 1) / kQuantizePiece);
+  if (a.xks == 1 && a.qks == 1) return rows * quantize_pieces(a.k);
   const int64_t blocks = (rows * ((static_cast<int64_t>(a.k) + 3) / 4) + 255) / 256;
   return blocks > 256 * 32 ? 256 * 32 : blocks;
 }
