@@ -247,3 +247,41 @@ def test_runtime_quant_packed_edges_equal_the_unpacked_call(device, m, n, k):
         call(a, mult, 128, weights, rs, cs, c, correction=corr, workspace=ws)
         torch.cuda.synchronize()
         assert np.array_equal(c.cpu().numpy().view(np.uint32), want.view(np.uint32)), packed_call
+
+
+def _quantized(a, mult, zero_point):
+    """The same multiply, add and truncation element by element (values far from the ends of int32)."""
+    import torch
+    return (a * mult[:, None] + float(zero_point)).to(torch.int32).clamp(0, 255).to(torch.uint8)
+
+
+@pytest.mark.parametrize("m,k", [((1 << 24) + 3, 5), (70001, 1030), (33001, 2049)])
+def test_quantize_more_rows_than_workgroups(device, m, k):
+    """Contiguous rows by the million: a workgroup each would be more than a launch takes, so the workgroups stride over
+    them; and several ten thousand pieces, a workgroup each."""
+    import torch
+    from vecops_amd import capi
+    a = torch.randn((m, k), generator=torch.Generator(device).manual_seed(1), device=device)
+    mult = torch.linspace(20.0, 60.0, m, device=device)
+    q = torch.full((m, k), 99, dtype=torch.uint8, device=device)
+    capi.quantize_rows(a, mult, 100, q)
+    assert torch.equal(q, _quantized(a, mult, 100))
+
+
+@pytest.mark.parametrize("packed", [False, True])
+def test_runtime_quant_more_rows_than_a_launch_has_workgroups(device, packed):
+    import torch
+    from vecops_amd import capi
+    m, n, k = (1 << 24) + 3, 9, 16
+    gen = torch.Generator(device).manual_seed(2)
+    a = torch.randn((m, k), generator=gen, device=device)
+    b = torch.randint(-127, 128, (n, k), generator=gen, device=device, dtype=torch.int8)
+    mult, rs, cs = torch.linspace(20.0, 60.0, m, device=device), torch.linspace(0.5, 2.0, m, device=device), torch.rand(n, device=device)
+    c = torch.full((m, n), float("nan"), device=device)
+    if packed:
+        capi.matmul_runtime_quant_packed_b(a, mult, 100, capi.pack_b(b), rs, cs, c)
+    else:
+        capi.matmul_runtime_quant(a, mult, 100, b, rs, cs, c)
+    # sixteen products of at most 255 * 127: every partial sum is a whole number that fp32 holds
+    want = (_quantized(a, mult, 100).float() @ b.float().t()) * rs[:, None] * cs[None, :]
+    assert torch.equal(c, want)

@@ -1,19 +1,59 @@
 // How the byte preparations of a product are dealt to workgroups of 256 lanes: arithmetic on whole numbers only, compiled
-// into the kernels and into the CPU test of the positions.
+// into the kernels, their launches and the CPU test of both.
 #pragma once
 #include <cstdint>
 
 namespace vecops_hip {
 
-// Quantisation of contiguous rows: a workgroup takes one piece of a row, a lane two quads of it, 1024 elements apart.
+// A launch has fewer than 2^32 lanes.
+constexpr int64_t kMostBlocks = (int64_t{1} << 24) - 1;
+
+// Quantisation of contiguous rows, by pieces: a workgroup takes one piece of a row, a lane two quads of it, 1024 elements
+// apart.  By quads: the quads of all rows are one sequence, a lane takes one and then the one a launch's lanes further on.
+// What has more pieces than a launch may have workgroups goes by quads (65536 x 4096 fp32: 230 us by pieces, 277 by quads).
 constexpr int kQuantizePiece = 2048;
 constexpr int kQuantizeQuads = kQuantizePiece / 1024;
+constexpr int64_t kMostPieces = 1 << 23;
+constexpr int64_t kMostQuadBlocks = 8192;
 
 constexpr int64_t quantize_pieces(int64_t k) { return (k + kQuantizePiece - 1) / kQuantizePiece; }
+constexpr bool quantize_by_pieces(int64_t rows, int64_t k) { return rows * quantize_pieces(k) <= kMostPieces; }
+constexpr int64_t quantize_blocks(int64_t rows, int64_t k) {
+  if (quantize_by_pieces(rows, k)) return rows * quantize_pieces(k);
+  const int64_t blocks = (rows * ((k + 3) / 4) + 255) / 256;
+  return blocks < kMostQuadBlocks ? blocks : kMostQuadBlocks;
+}
 
-// First element of a lane's i-th quad, and whether all four of them lie in a row of k.  64 bits: a row may have INT32_MAX
-// elements, and the last quad of its last piece ends past what 32 bits hold.
-constexpr int64_t quantize_quad(int64_t piece, int lane, int i) { return piece * kQuantizePiece + i * 1024 + lane * 4; }
-constexpr bool quantize_quad_is_whole(int64_t quad, int64_t k) { return quad + 4 <= k; }
+// By pieces.  Elements of a row of k that lie in its piece, where the piece begins, and where in the piece a lane's i-th quad
+// does.  (The beginning in 64 bits, what is compared lane by lane below 4096: a row may have INT32_MAX elements.)
+constexpr int64_t quantize_piece_begin(uint32_t piece) { return static_cast<int64_t>(piece) * kQuantizePiece; }
+constexpr int quantize_piece_length(uint32_t piece, int64_t k) {
+  return k - quantize_piece_begin(piece) < kQuantizePiece ? static_cast<int>(k - quantize_piece_begin(piece)) : kQuantizePiece;
+}
+constexpr int quantize_quad(int lane, int i) { return i * 1024 + lane * 4; }
+
+// By quads.  The way of a lane over the quads of all rows: its first one, and the next, a launch's lanes further on.  That
+// step is divided into whole rows and quads once, for the launch; the first quad's number fits 32 bits, all quads together
+// need not.
+struct QuantizeWalk {
+  uint32_t quads;  // of a row
+  uint32_t step_rows, step_quads;
+};
+constexpr QuantizeWalk quantize_walk(int64_t k, uint32_t blocks) {
+  const uint32_t quads = static_cast<uint32_t>((k + 3) / 4);
+  return {quads, blocks * 256 / quads, blocks * 256 % quads};
+}
+struct QuantizeQuad {
+  int64_t row;
+  uint32_t quad;
+};
+constexpr QuantizeQuad quantize_first(const QuantizeWalk& w, uint32_t lane) { return {lane / w.quads, lane % w.quads}; }
+constexpr QuantizeQuad quantize_next(const QuantizeWalk& w, const QuantizeQuad& at) {
+  const uint32_t quad = at.quad + w.step_quads;
+  return quad < w.quads ? QuantizeQuad{at.row + w.step_rows, quad} : QuantizeQuad{at.row + w.step_rows + 1, quad - w.quads};
+}
+
+// Elements of a quad that begins at `begin` in a piece or row of `length`: 0 to 4.
+constexpr int quantize_quad_length(int begin, int length) { return length - begin >= 4 ? 4 : length > begin ? length - begin : 0; }
 
 }  // namespace vecops_hip

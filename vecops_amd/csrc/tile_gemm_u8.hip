@@ -60,10 +60,11 @@ __global__ __launch_bounds__(256) void byte_row_sums_kernel(const ByteRowSums a)
 // RuntimePerRowAsymmetricQuantizeTransform (matmul/Quantization.h:91-146) and the conversion of its fp32
 // result to the uint8 compute type - a multiply and an add, each rounded (the file is compiled without
 // contraction), truncation toward zero, NaN and values outside int32 to INT32_MIN, saturation to 0..255.
-// Rows contiguous on both sides (quantize_contiguous_rows): a workgroup takes kQuantizePiece elements of one row, two
-// quads a lane, each one 16-byte load and one 4-byte store at whatever alignment.  Bound by the bytes: no division per
-// lane, and enough workgroups (a 2048-element piece each) that their loads overlap.  Other strides: one thread per four
-// consecutive k, element by element where a quad cannot be taken whole.  flip (0 or 0x80) is xored into every byte.
+// Rows contiguous on both sides: by pieces of kQuantizePiece elements, a workgroup each (two quads a lane, each one 16-byte
+// load and one 4-byte store at whatever alignment; no division per lane, and workgroups enough that their loads overlap), or
+// by quads over all rows; row_work_split.h says which.  Bound by the bytes.
+// Other strides: one thread per four consecutive k, element by element.  flip (0 or 0x80) is
+// xored into every byte.
 struct QuantizeRows {
   const float* x;
   int32_t batch, rows, k;
@@ -74,43 +75,71 @@ struct QuantizeRows {
   uint32_t flip;
   uint8_t* q;
   int64_t qbs, qrs, qks;
+  QuantizeWalk walk;  // rows contiguous on both sides: quads 0 goes by pieces
 };
 
-struct __attribute__((packed, aligned(4))) FloatQuad { float v[4]; };
-struct __attribute__((packed, aligned(1))) ByteQuad { uint32_t v; };
+typedef float f32x4_align4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32_align1 __attribute__((aligned(1)));
 
-// (block: the workgroup's number among those that quantise; xks == qks == 1)
-__device__ __forceinline__ void quantize_contiguous_rows(const QuantizeRows& a, uint32_t block) {
+// Four consecutive elements of a contiguous row, or the first `length` of them, at any element's address.
+__device__ __forceinline__ f32x4 load_quad(const float* src, int length) {
+  f32x4 quad = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (length == 4) {
+    quad = *reinterpret_cast<const f32x4_align4*>(src);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 3; ++e)
+      if (e < length) quad[e] = src[e];
+  }
+  return quad;
+}
+
+__device__ __forceinline__ void quantize_quad_out(const QuantizeRows& a, const f32x4& quad, float mult, uint8_t* dst, int length) {
+  uint32_t word = 0;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float scaled = quad[e] * mult;
+    word |= (narrow_to_byte(scaled + a.zero_point, false) ^ a.flip) << (8 * e);  // flip 0x80: the byte as q - 128 in int8
+  }
+  if (length == 4) {
+    *reinterpret_cast<u32_align1*>(dst) = word;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 3; ++e)
+      if (e < length) dst[e] = static_cast<uint8_t>(word >> (8 * e));
+  }
+}
+
+// (block: the workgroup's number among those that quantise; xks == qks == 1; batch * rows is at most INT32_MAX)
+__device__ __forceinline__ void quantize_by_pieces(const QuantizeRows& a, uint32_t block) {
   const uint32_t pieces = static_cast<uint32_t>(quantize_pieces(a.k));
   const uint32_t row = block / pieces, piece = block - row * pieces;
   const uint32_t b = row / static_cast<uint32_t>(a.rows), r = row - b * static_cast<uint32_t>(a.rows);
-  const float* src = a.x + b * a.xbs + r * a.xrs;
-  uint8_t* dst = a.q + b * a.qbs + r * a.qrs;
+  const float* src = a.x + b * a.xbs + r * a.xrs + quantize_piece_begin(piece);
+  uint8_t* dst = a.q + b * a.qbs + r * a.qrs + quantize_piece_begin(piece);
+  const int length = quantize_piece_length(piece, a.k);
   const float mult = a.multipliers[b * a.mult_bs + r];
-  FloatQuad quad[kQuantizeQuads];
+  f32x4 quad[kQuantizeQuads];
 #pragma unroll
   for (int i = 0; i < kQuantizeQuads; ++i) {
-    const int64_t k = quantize_quad(piece, threadIdx.x, i);
-    if (quantize_quad_is_whole(k, a.k)) {
-      quad[i] = *reinterpret_cast<const FloatQuad*>(src + k);
-    } else {
-      for (int e = 0; e < 4; ++e) quad[i].v[e] = k + e < a.k ? src[k + e] : 0.0f;
-    }
+    const int k = quantize_quad(threadIdx.x, i);
+    quad[i] = load_quad(src + k, quantize_quad_length(k, length));
   }
 #pragma unroll
   for (int i = 0; i < kQuantizeQuads; ++i) {
-    const int64_t k = quantize_quad(piece, threadIdx.x, i);
-    uint32_t word = 0;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const float scaled = quad[i].v[e] * mult;
-      word |= (narrow_to_byte(scaled + a.zero_point, false) ^ a.flip) << (8 * e);  // flip 0x80: the byte as q - 128 in int8
-    }
-    if (quantize_quad_is_whole(k, a.k)) {
-      reinterpret_cast<ByteQuad*>(dst + k)->v = word;
-    } else {
-      for (int e = 0; k + e < a.k; ++e) dst[k + e] = static_cast<uint8_t>(word >> (8 * e));
-    }
+    const int k = quantize_quad(threadIdx.x, i);
+    quantize_quad_out(a, quad[i], mult, dst + k, quantize_quad_length(k, length));
+  }
+}
+
+__device__ __forceinline__ void quantize_by_quads(const QuantizeRows& a, uint32_t block) {
+  const int64_t rows = static_cast<int64_t>(a.batch) * a.rows;
+  for (QuantizeQuad at = quantize_first(a.walk, block * 256 + threadIdx.x); at.row < rows; at = quantize_next(a.walk, at)) {
+    const uint32_t row = static_cast<uint32_t>(at.row);
+    const uint32_t b = a.batch == 1 ? 0 : row / static_cast<uint32_t>(a.rows), r = row - b * static_cast<uint32_t>(a.rows);
+    const int k = static_cast<int>(at.quad) * 4, length = quantize_quad_length(k, a.k);
+    const f32x4 quad = load_quad(a.x + b * a.xbs + r * a.xrs + k, length);
+    quantize_quad_out(a, quad, a.multipliers[b * a.mult_bs + r], a.q + b * a.qbs + r * a.qrs + k, length);
   }
 }
 
@@ -124,7 +153,8 @@ __device__ __forceinline__ void quantize_rows(const QuantizeRows& a, int64_t blo
   const uint32_t flip = a.flip;
   uint8_t* q = a.q;
   if (xks == 1 && qks == 1) {
-    quantize_contiguous_rows(a, static_cast<uint32_t>(block));
+    if (a.walk.quads == 0) quantize_by_pieces(a, static_cast<uint32_t>(block));
+    else quantize_by_quads(a, static_cast<uint32_t>(block));
     return;
   }
   const int64_t quads_per_row = (static_cast<int64_t>(k) + 3) / 4;
@@ -163,11 +193,15 @@ __global__ __launch_bounds__(256) void quantize_and_packed_row_sums_kernel(const
 }
 
 namespace {
-// Workgroups of quantize_rows; 0 when there is nothing to quantise, more than INT32_MAX when they cannot be launched.
-int64_t quantize_blocks_for(const QuantizeRows& a) {
+// Workgroups of quantize_rows, 0 when there is nothing to quantise; fills in the walk.
+int64_t quantize_blocks_for(QuantizeRows& a) {
   const int64_t rows = static_cast<int64_t>(a.batch) * a.rows;
   if (rows <= 0 || a.k <= 0) return 0;
-  if (a.xks == 1 && a.qks == 1) return rows * quantize_pieces(a.k);
+  if (a.xks == 1 && a.qks == 1) {
+    const int64_t blocks = quantize_blocks(rows, a.k);
+    if (!quantize_by_pieces(rows, a.k)) a.walk = quantize_walk(a.k, static_cast<uint32_t>(blocks));
+    return blocks;
+  }
   const int64_t blocks = (rows * ((static_cast<int64_t>(a.k) + 3) / 4) + 255) / 256;
   return blocks > 256 * 32 ? 256 * 32 : blocks;
 }
@@ -176,10 +210,9 @@ int64_t quantize_blocks_for(const QuantizeRows& a) {
 hipError_t launch_quantize_rows(const float* x, int32_t batch, int32_t rows, int32_t k, int64_t xbs, int64_t xrs,
                                 int64_t xks, const float* multipliers, int64_t mult_bs, int32_t zero_point, uint32_t flip,
                                 uint8_t* q, int64_t qbs, int64_t qrs, int64_t qks, hipStream_t stream) {
-  const QuantizeRows a{x, batch, rows, k, xbs, xrs, xks, multipliers, mult_bs, static_cast<float>(zero_point), flip & 0xffu, q, qbs, qrs, qks};
+  QuantizeRows a{x, batch, rows, k, xbs, xrs, xks, multipliers, mult_bs, static_cast<float>(zero_point), flip & 0xffu, q, qbs, qrs, qks, {}};
   const int64_t blocks = quantize_blocks_for(a);
   if (blocks == 0) return hipSuccess;
-  if (blocks > INT32_MAX) return hipErrorInvalidConfiguration;
   hipLaunchKernelGGL(quantize_rows_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, a);
   return hipGetLastError();
 }
@@ -190,7 +223,7 @@ hipError_t launch_byte_row_sums(const void* x, int32_t batch, int32_t rows, int3
   const int64_t total = static_cast<int64_t>(batch) * rows;
   if (total <= 0) return hipSuccess;
   const int64_t blocks = (total + 3) / 4;
-  if (blocks > INT32_MAX) return hipErrorInvalidConfiguration;
+  if (blocks > kMostBlocks) return hipErrorInvalidConfiguration;
   const ByteRowSums a{static_cast<const uint8_t*>(x), batch, rows, k, bs, rs, ks, flip, scale, add, add_bs, out};
   hipLaunchKernelGGL(byte_row_sums_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, a);
   return hipGetLastError();
@@ -202,11 +235,11 @@ hipError_t launch_quantize_and_row_sums(const float* x, int32_t batch, int32_t r
                                         uint8_t* q, int64_t qbs, int64_t qrs, int64_t qks, const void* w, int32_t w_batch,
                                         int32_t w_rows, int64_t w_bs, int64_t w_rs, int64_t w_ks, uint32_t w_flip, uint32_t scale,
                                         const int32_t* add, int64_t add_bs, int32_t* out, hipStream_t stream) {
-  const QuantizeRows qa{x, batch, rows, k, xbs, xrs, xks, multipliers, mult_bs, static_cast<float>(zero_point), flip & 0xffu, q, qbs, qrs, qks};
+  QuantizeRows qa{x, batch, rows, k, xbs, xrs, xks, multipliers, mult_bs, static_cast<float>(zero_point), flip & 0xffu, q, qbs, qrs, qks, {}};
   const int64_t sums = static_cast<int64_t>(w_batch) * w_rows;
   const int64_t q_blocks = quantize_blocks_for(qa), s_blocks = (sums + 3) / 4;
   if (q_blocks <= 0 || sums <= 0) return hipErrorInvalidValue;
-  if (q_blocks + s_blocks > INT32_MAX) return hipErrorInvalidConfiguration;
+  if (q_blocks + s_blocks > kMostBlocks) return hipErrorInvalidConfiguration;
   const ByteRowSums sa{static_cast<const uint8_t*>(w), w_batch, w_rows, k, w_bs, w_rs, w_ks, w_flip, scale, add, add_bs, out};
   hipLaunchKernelGGL(quantize_and_row_sums_kernel, dim3(static_cast<unsigned>(q_blocks + s_blocks)), dim3(256), 0, stream, qa, sa,
                      static_cast<uint32_t>(q_blocks));
@@ -218,10 +251,10 @@ hipError_t launch_quantize_and_packed_row_sums(const float* x, int32_t batch, in
                                                int64_t xks, const float* multipliers, int64_t mult_bs, int32_t zero_point,
                                                uint32_t flip, uint8_t* q, int64_t qbs, int64_t qrs, int64_t qks,
                                                const PackedRowSums& sums, hipStream_t stream) {
-  const QuantizeRows qa{x, batch, rows, k, xbs, xrs, xks, multipliers, mult_bs, static_cast<float>(zero_point), flip & 0xffu, q, qbs, qrs, qks};
+  QuantizeRows qa{x, batch, rows, k, xbs, xrs, xks, multipliers, mult_bs, static_cast<float>(zero_point), flip & 0xffu, q, qbs, qrs, qks, {}};
   const int64_t q_blocks = quantize_blocks_for(qa), s_blocks = packed_row_sums_blocks(sums);
   if (q_blocks <= 0 || s_blocks <= 0) return hipErrorInvalidValue;
-  if (q_blocks + s_blocks > INT32_MAX) return hipErrorInvalidConfiguration;
+  if (q_blocks + s_blocks > kMostBlocks) return hipErrorInvalidConfiguration;
   hipLaunchKernelGGL(quantize_and_packed_row_sums_kernel, dim3(static_cast<unsigned>(q_blocks + s_blocks)), dim3(256), 0, stream, qa, sums,
                      static_cast<uint32_t>(q_blocks));
   return hipGetLastError();
