@@ -105,3 +105,12 @@ def test_every_element_of_every_row_once(split, rows, k, blocks):
 def test_launches_stay_within_what_the_device_takes(split, rows, k):
     assert 1 <= split.blocks(rows, k) * 256 < 2 ** 32      # work items of a launch's dimension
     assert split.by_pieces(rows, k) == 0 or split.blocks(rows, k) == rows * ((k + 2047) // 2048)
+
+
+def test_short_rows_leave_no_lane_idle(split):
+    """Up to 1024 elements a row goes by quads: a workgroup's lanes take neighbouring quads across rows."""
+    for k in (1, 3, 17, 64, 100, 512, 1000, 1024):
+        rows = 1 << 16
+        assert split.by_pieces(rows, k) == 0
+        assert _taken(split, False, rows, k, 0, split.blocks(rows, k))[0].size == 256
+    assert split.by_pieces(1 << 16, 1025) == 1

@@ -10,14 +10,17 @@ constexpr int64_t kMostBlocks = (int64_t{1} << 24) - 1;
 
 // Quantisation of contiguous rows, by pieces: a workgroup takes one piece of a row, a lane two quads of it, 1024 elements
 // apart.  By quads: the quads of all rows are one sequence, a lane takes one and then the one a launch's lanes further on.
-// What has more pieces than a launch may have workgroups goes by quads (65536 x 4096 fp32: 230 us by pieces, 277 by quads).
+// Short rows go by quads, because the lanes past a row's end would idle (1048576 x 64 fp32: 937 us by pieces, 61 by quads,
+// 131072 x 512 119 and 59, 65536 x 1000 67 and 58; 65536 x 4096 230 and 277), and so does what has more pieces than a
+// launch may have workgroups.
 constexpr int kQuantizePiece = 2048;
 constexpr int kQuantizeQuads = kQuantizePiece / 1024;
+constexpr int kQuantizeShortRow = 1024;
 constexpr int64_t kMostPieces = 1 << 23;
 constexpr int64_t kMostQuadBlocks = 8192;
 
 constexpr int64_t quantize_pieces(int64_t k) { return (k + kQuantizePiece - 1) / kQuantizePiece; }
-constexpr bool quantize_by_pieces(int64_t rows, int64_t k) { return rows * quantize_pieces(k) <= kMostPieces; }
+constexpr bool quantize_by_pieces(int64_t rows, int64_t k) { return k > kQuantizeShortRow && rows * quantize_pieces(k) <= kMostPieces; }
 constexpr int64_t quantize_blocks(int64_t rows, int64_t k) {
   if (quantize_by_pieces(rows, k)) return rows * quantize_pieces(k);
   const int64_t blocks = (rows * ((k + 3) / 4) + 255) / 256;
