@@ -285,3 +285,25 @@ def test_runtime_quant_more_rows_than_a_launch_has_workgroups(device, packed):
     # sixteen products of at most 255 * 127: every partial sum is a whole number that fp32 holds
     want = (_quantized(a, mult, 100).float() @ b.float().t()) * rs[:, None] * cs[None, :]
     assert torch.equal(c, want)
+
+
+@pytest.mark.parametrize("m,k", [(1, 1), (3, 5), (65, 130), (300, 2049), (64, 1024)])
+@pytest.mark.parametrize("x_contiguous,q_contiguous", [(True, False), (False, True), (False, False)])
+def test_quantize_rows_contiguous_on_one_side(device, x_contiguous, q_contiguous, m, k):
+    """One side stored [M,K] with rows at odd addresses, the other [K,M]: a quad is taken whole where its side allows it,
+    and nothing outside the rows is written."""
+    import torch
+    from vecops_amd import capi
+    x = torch.randn((m, k), generator=torch.Generator(device).manual_seed(3), device=device)
+    mult = torch.linspace(20.0, 60.0, m, device=device)
+
+    def stored(contiguous, fill, dtype):
+        store = torch.full((m, k + 3) if contiguous else (k, m + 3), fill, dtype=dtype, device=device)
+        return store, store[:, 1:k + 1] if contiguous else store[:, 1:m + 1].t()
+
+    _, xv = stored(x_contiguous, float("nan"), torch.float32)
+    xv.copy_(x)
+    qstore, qv = stored(q_contiguous, 77, torch.uint8)
+    capi.quantize_rows(xv, mult, 100, qv)
+    assert torch.equal(qv, _quantized(x, mult, 100))
+    assert (qstore[:, 0] == 77).all() and (qstore[:, -2:] == 77).all()

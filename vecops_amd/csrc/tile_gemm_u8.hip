@@ -63,7 +63,7 @@ __global__ __launch_bounds__(256) void byte_row_sums_kernel(const ByteRowSums a)
 // Rows contiguous on both sides: by pieces of kQuantizePiece elements, a workgroup each (two quads a lane, each one 16-byte
 // load and one 4-byte store at whatever alignment; no division per lane, and workgroups enough that their loads overlap), or
 // by quads over all rows; row_work_split.h says which.  Bound by the bytes.
-// Other strides: one thread per four consecutive k, element by element.  flip (0 or 0x80) is
+// Other strides: one thread per four consecutive k, a quad at a time on the side that is contiguous.  flip (0 or 0x80) is
 // xored into every byte.
 struct QuantizeRows {
   const float* x;
@@ -167,11 +167,19 @@ __device__ __forceinline__ void quantize_rows(const QuantizeRows& a, int64_t blo
     uint8_t* dst = q + b * qbs + r * qrs + k0 * qks;
     const float mult = multipliers[b * mult_bs + r];
     const int left = min(4, k - k0);
-    float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int e = 0; e < left; ++e) v[e] = src[e * xks];
-    for (int e = 0; e < left; ++e) {
-      const float scaled = v[e] * mult;
-      dst[e * qks] = static_cast<uint8_t>(narrow_to_byte(scaled + zero_point, false) ^ flip);
+    f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (xks == 1) {
+      v = load_quad(src, left);
+    } else {
+      for (int e = 0; e < left; ++e) v[e] = src[e * xks];
+    }
+    if (qks == 1) {
+      quantize_quad_out(a, v, mult, dst, left);
+    } else {
+      for (int e = 0; e < left; ++e) {
+        const float scaled = v[e] * mult;
+        dst[e * qks] = static_cast<uint8_t>(narrow_to_byte(scaled + zero_point, false) ^ flip);
+      }
     }
   }
 }
