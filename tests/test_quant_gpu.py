@@ -307,3 +307,26 @@ def test_quantize_rows_contiguous_on_one_side(device, x_contiguous, q_contiguous
     capi.quantize_rows(xv, mult, 100, qv)
     assert torch.equal(qv, _quantized(x, mult, 100))
     assert (qstore[:, 0] == 77).all() and (qstore[:, -2:] == 77).all()
+
+
+@pytest.mark.parametrize("n,k", [(65504, 33), (65505, 1), (65505, 200), (65536, 128), (65545, 512), (65545, 513), (100000, 500)])
+def test_packed_row_sums_of_many_panels(device, n, k):
+    """Weights of about 2048 panels of 32 rows, where the sums of short rows change from a workgroup for eight rows to a wavefront a
+    panel: as the correction of unsigned activations and of runtime-quantised ones.  (Up to 513 products of at most
+    255 * 127: every partial sum is a whole number that fp32 holds.)"""
+    import torch
+    from vecops_amd import capi
+    gen = torch.Generator(device).manual_seed(4)
+    m = 17
+    b = torch.randint(-127, 128, (n, k), generator=gen, device=device, dtype=torch.int8)
+    packed, corr = capi.pack_b(b, a_zero_point=100)
+    a8 = torch.randint(0, 256, (m, k), generator=gen, device=device, dtype=torch.uint8)
+    c = torch.full((m, n), -7, dtype=torch.int32, device=device)
+    capi.matmul_packed_b(a8, packed, c)
+    assert torch.equal(c, (a8.float() @ b.float().t()).to(torch.int32))
+    a = torch.randn((m, k), generator=gen, device=device)
+    mult, rs, cs = torch.linspace(20.0, 60.0, m, device=device), torch.linspace(0.5, 2.0, m, device=device), torch.rand(n, device=device)
+    out = torch.full((m, n), float("nan"), device=device)
+    capi.matmul_runtime_quant_packed_b(a, mult, 100, packed, rs, cs, out, correction=corr)
+    want = ((_quantized(a, mult, 100).float() - 100.0) @ b.float().t()) * rs[:, None] * cs[None, :]
+    assert torch.equal(out, want)

@@ -17,6 +17,7 @@ using namespace vecops_hip;
 extern "C" {
 int32_t by_pieces(int64_t rows, int64_t k) { return quantize_by_pieces(rows, k); }
 int64_t blocks(int64_t rows, int64_t k) { return quantize_blocks(rows, k); }
+int64_t sum_blocks(int64_t n, int64_t k) { return packed_sums_blocks(n, k); }
 // What a workgroup takes: row, first element, elements (0: none).  By pieces [lane][i], 512 entries; by quads the first
 // `most` of each lane, [lane][step], rows past the end among them.
 void by_pieces_of(int64_t k, uint32_t block, int64_t* row, int64_t* first, int32_t* length) {
@@ -52,8 +53,8 @@ def split(tmp_path_factory):
     subprocess.run(["g++", "-std=c++17", "-O1", "-fsanitize=undefined", "-fno-sanitize-recover=all", "-shared", "-fPIC", "-Wall",
                     "-Werror", "-I", CSRC, "-o", str(out), str(source)], check=True)
     lib = C.CDLL(str(out))
-    lib.blocks.restype = C.c_int64
-    lib.blocks.argtypes = lib.by_pieces.argtypes = [C.c_int64, C.c_int64]
+    lib.blocks.restype = lib.sum_blocks.restype = C.c_int64
+    lib.blocks.argtypes = lib.sum_blocks.argtypes = lib.by_pieces.argtypes = [C.c_int64, C.c_int64]
     lib.by_pieces_of.argtypes = [C.c_int64, C.c_uint32] + [C.c_void_p] * 3
     lib.by_quads_of.argtypes = [C.c_int64, C.c_uint32, C.c_uint32, C.c_int64] + [C.c_void_p] * 3
     return lib
@@ -98,6 +99,12 @@ def test_every_element_of_every_row_once(split, rows, k, blocks):
         for e in range(4):
             np.add.at(taken, (row[length > e], first[length > e] + e), 1)
     assert (taken == 1).all()
+
+
+@pytest.mark.parametrize("n", [1, 8, 65504, 65505, 2 ** 23 - 32, 2 ** 23, 2 ** 27, 2 ** 27 + 8, 2 ** 30])
+@pytest.mark.parametrize("k", [1, 512, 513, 8192])
+def test_packed_row_sums_launches_stay_within_what_the_device_takes(split, n, k):
+    assert 1 <= split.sum_blocks(n, k) * 256 < 2 ** 32
 
 
 @pytest.mark.parametrize("rows,k", [(2 ** 24, 16), (2 ** 24 + 1, 1), (17_000_000, 64), (2 ** 23, 2048), (2 ** 23, 2049), (2 ** 25, 2049),

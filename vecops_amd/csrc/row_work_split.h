@@ -59,4 +59,14 @@ constexpr QuantizeQuad quantize_next(const QuantizeWalk& w, const QuantizeQuad& 
 // Elements of a quad that begins at `begin` in a piece or row of `length`: 0 to 4.
 constexpr int quantize_quad_length(int begin, int length) { return length - begin >= 4 ? 4 : length > begin ? length - begin : 0; }
 
+// Sums over the rows of a packed operand (panels of 32 rows): a panel is a wavefront's, or its quarters of eight rows are a
+// workgroup's each (packed_row_sums.h).  By panel where the panels are many and K is short, because the lanes of a workgroup
+// past a quarter's K would idle (the unsigned 17 x 262144 x 64 product 34 us by quarter, 26 by panel, 131072 x 256 29 and 27;
+// 131072 x 512 level; 256 x 11008 x 4096 57 and 88), and where the quarters are more than a launch should have workgroups.
+constexpr int64_t kShortKPanels = 2048, kPanelShortK = 512, kLongKPanels = 1 << 18;
+constexpr bool packed_sums_by_panel(int64_t n, int64_t k) { return (n + 31) / 32 >= (k <= kPanelShortK ? kShortKPanels : kLongKPanels); }
+constexpr int64_t packed_sums_blocks(int64_t n, int64_t k) {
+  return packed_sums_by_panel(n, k) ? ((n + 31) / 32 + 3) / 4 : (n + 7) / 8;
+}
+
 }  // namespace vecops_hip
