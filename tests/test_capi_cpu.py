@@ -309,3 +309,18 @@ def test_family_request_known_answers():
     # no request = automatic
     assert capi.lib().vecops_hip_plan_matmul_family(C.byref(big[0]), C.byref(big[1]), None, C.byref(big[2]), 0, None,
                                                     C.byref(plan)) == 0 and capi.FAMILY_NAMES[plan.family] == "tile_256"
+
+
+def test_grouped_refuses_more_workgroups_than_a_launch_takes():
+    """A launch has fewer than 2^32 lanes, 2^24 workgroups of 256: more are refused before anything is launched (the
+    group table numbers them in 32 bits)."""
+    batch, k = 65535 * 16, 8            # single elements of C, a workgroup each
+    for count, refused in ((16, False), (17, True)):
+        a = (capi.Operand * count)(*[_operand(capi.BF16, (batch, 1, k)) for _ in range(count)])
+        b = (capi.Operand * count)(*[_operand(capi.BF16, (batch, 1, k)) for _ in range(count)])
+        c = (capi.Operand * count)(*[_operand(capi.BF16, (batch, 1, 1)) for _ in range(count)])
+        need = capi.lib().vecops_hip_matmul_grouped_workspace(count, a, b, None, c, 0)
+        assert (need == 0) == refused, count
+        if refused:
+            rc = capi.lib().vecops_hip_matmul_grouped(count, a, b, None, c, 0, None, 0, None)
+            assert rc == 1 and b"too many workgroups" in capi.lib().vecops_hip_last_error()

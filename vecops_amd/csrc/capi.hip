@@ -1755,7 +1755,8 @@ int32_t describe_grouped(uint32_t count, const VecopsHipOperand* a, const Vecops
     g->first.push_back(static_cast<int32_t>(next));
     const int64_t wgs = ((pr.m + g->tile - 1) / g->tile) * ((pr.n + g->tile - 1) / g->tile) * pr.batch;
     next += (wgs + 7) & ~int64_t{7};  // a multiple of eight: the XCD renumbering then works per group
-    if (next > INT32_MAX) return fail(ST_INVALID, "matmul_grouped: too many workgroups");
+    // (a launch of more is refused; checked before the table is written, whose entries are numbered in 32 bits)
+    if (next > kMostBlocks) return fail(ST_INVALID, "matmul_grouped: too many workgroups");
   }
   g->first.push_back(static_cast<int32_t>(next));
   g->first_bytes = round_up_256(g->first.size() * 4u);
