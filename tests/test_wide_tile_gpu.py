@@ -285,3 +285,28 @@ def test_wide_tile_bias_row_equals_the_same_bias_as_a_full_c_input(device, kind,
     if out == "own" and kind == "bf16" and bias_type is not None and "clamp" not in steps and "relu" not in steps:
         assert bool((got.view(bits)[:, 0] == 0x7fc0).all())
     assert torch.equal(got.view(bits), want.view(bits))
+
+
+@pytest.mark.parametrize("kind,out,bias_type", [("bf16", "own", "own"), ("bf16", "f32", "f32"), ("f16", "own", "f32"), ("f16", "f32", "own")])
+def test_wide_tile_bias_row_with_prepacked_weights(device, kind, out, bias_type):
+    """The bias row from LDS on the prepacked operand's column order (a wavefront's blocks alternate there): the bits of
+    the same bias written out as a whole C input, on edge tiles in both directions."""
+    import torch
+    from vecops_amd import capi
+    m, n, k = 1500, 11000, 512
+    gen = torch.Generator().manual_seed(6)
+    own = {"bf16": torch.bfloat16, "f16": torch.float16}[kind]
+    a = (torch.rand((m, k), generator=gen) * 2 - 1).to(own).to(device)
+    packed = capi.pack_b((torch.rand((n, k), generator=gen) * 2 - 1).to(own).to(device))
+    bias = (torch.rand((1, n), generator=gen) * 8 - 4).to(own if bias_type == "own" else torch.float32).to(device)
+    bias[0, [0, 17, n - 1]] = float("nan")
+    bias[0, [1, 352, n - 2]] = float("inf")
+    out_dtype = own if out == "own" else torch.float32
+    got, want = torch.zeros((m, n), dtype=out_dtype, device=device), torch.zeros((m, n), dtype=out_dtype, device=device)
+    for c_in, c in ((bias.expand(m, n), got), (bias.expand(m, n).contiguous(), want)):
+        assert capi.FAMILY_NAMES[capi.plan_matmul_packed_b(a, packed, c, c_in).family] == "tile_256x352"
+        capi.matmul_packed_b(a, packed, c, c_in=c_in)
+    torch.cuda.synchronize()
+    bits = torch.int32 if out == "f32" else torch.int16
+    assert torch.equal(got.view(bits), want.view(bits))
+    assert not torch.equal(got[:, 2:16].float(), torch.zeros_like(got[:, 2:16].float()))
