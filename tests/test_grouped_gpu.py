@@ -325,18 +325,23 @@ def test_prepared_grouped_call_repeats_the_plain_one(device):
 
 
 def test_grouped_long_and_short_runs_across_table_chunks(device):
-    """Runs of several hundred workgroups (their map entries are written by more than one workgroup of the table's launch)
-    beside single tiles, at the beginning and the end of the table's chunks of twelve groups; a second call through the
-    same workspace with the groups in the other order writes the whole table anew."""
+    """Runs of more than 256 workgroups (their map entries are written by more than one workgroup of the table's launch)
+    beside single tiles, at the beginning, in the middle and at the end of the table's chunks of twelve groups; a second
+    call through the same workspace, full of garbage before each, with the groups in the other order."""
     import torch
     from vecops_amd import capi
-    shapes = [(2200, 4200, 72) if i in (0, 11, 12, 24) else (1 + 3 * i, 8 + 8 * i, 72) for i in range(25)]
+    # 4400 x 4400: 18 x 18 tiles of 256 x 256, the tile that these groups take together, in two shares; of any smaller
+    # tile there are more
+    shapes = [(4400, 4400, 72) if i in (0, 5, 11, 12, 24) else (1 + 3 * i, 8 + 8 * i, 72) for i in range(25)]
     gen = torch.Generator().manual_seed(3)
     a = [(torch.rand((m, k), generator=gen) * 2 - 1).to(torch.bfloat16).to(device) for m, _, k in shapes]
     b = [(torch.rand((n, k), generator=gen) * 2 - 1).to(torch.bfloat16).to(device) for _, n, k in shapes]
+    workspace = torch.empty(1 << 20, dtype=torch.uint8, device=device)
     for order in (1, -1):
         c = [torch.full((m, n), float("nan"), device=device) for m, n, _ in shapes]
-        capi.matmul_grouped(a[::order], b[::order], c[::order])
+        workspace.fill_(0xA5)
+        capi.matmul_grouped(a[::order], b[::order], c[::order], workspace=workspace)
+        assert not bool((workspace[:256] == 0xA5).all())              # the table lies in the given workspace
         for x, y, z in zip(a, b, c):
             # 72 products of magnitude up to 1, summed in fp32
             assert float((z.double() - x.double() @ y.double().t()).abs().max()) <= 72 * 72 * 2.0 ** -24
