@@ -324,3 +324,15 @@ def test_grouped_refuses_more_workgroups_than_a_launch_takes():
         if refused:
             rc = capi.lib().vecops_hip_matmul_grouped(count, a, b, None, c, 0, None, 0, None)
             assert rc == 1 and b"too many workgroups" in capi.lib().vecops_hip_last_error()
+
+
+def test_runtime_quant_workspace_of_narrow_products():
+    """Narrow N and short K: the quantised activations take their M x K bytes and no padding; else rows of whole 16-byte
+    chunks, against packed weights of whole K tiles (the rest: N correction sums, both rounded up to 256 bytes)."""
+    L = capi.lib()
+    m = 1 << 20
+    for n, k, packed_row, plain_row in ((9, 1, 1, 1), (9, 72, 72, 72), (128, 1001, 1001, 1001), (129, 72, 128, 80), (9, 1025, 1152, 1040)):
+        a, b, c = _operand(capi.F32, (m, k)), _operand(capi.I8, (n, k)), _operand(capi.F32, (m, n))
+        rows = (4 * n + 255) // 256 * 256
+        assert L.vecops_hip_matmul_runtime_quant_packed_b_workspace(C.byref(a), n, C.byref(c)) == m * packed_row + rows
+        assert L.vecops_hip_matmul_runtime_quant_workspace(C.byref(a), C.byref(b), C.byref(c)) == m * plain_row + rows

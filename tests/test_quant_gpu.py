@@ -223,9 +223,9 @@ def test_runtime_quant_zero_extents_and_rejections(device):
 
 
 @pytest.mark.parametrize("m,n,k", [(1, 1, 1), (3, 7, 15), (17, 33, 127), (24, 250, 129), (5, 40, 2047), (300, 257, 2049),
-                                   (130, 64, 4100)])
+                                   (130, 64, 4100), (70, 128, 1024), (70, 128, 1025), (70, 129, 1000), (65, 9, 72)])
 def test_runtime_quant_packed_edges_equal_the_unpacked_call(device, m, n, k):
-    """Packed weights at the edges of the quantisation's 2048-element pieces, of the K padding of the quantised rows and
+    """Packed weights at the edges of the quantisation's 2048-element pieces, of the K padding of the quantised rows (none where N is narrow and K short) and
     of the row sums' eight-row workgroups, in a workspace full of garbage: the unpacked call's bits (integer sums)."""
     import torch
     from vecops_amd import capi

@@ -1421,7 +1421,11 @@ namespace {
 // row when every batch shares weights and correction) - both rounded up to 256 bytes - then the product's own
 // scratch.  The matrix's rows are padded to whole 16-byte chunks, so that the loads that write LDS can fetch them; against
 // packed weights, whose k past K are zeros up to a whole K tile, to whole K tiles, and the product runs over the padded
-// K without a partial tile (what the padding holds is multiplied by zeros).
+// K without a partial tile (what the padding holds is multiplied by zeros).  Not padded where N is narrow and K short: there
+// the matrix's bytes are what the call takes, and rows with gaps are written in parts of lines (packed weights, us unpadded /
+// to whole tiles: 2097152 x 9 x 72 405 / 494, x 32 x 200 667 / 785, 524288 x 64 x 200 174 / 203, 131072 x 128 x 520 101 / 108;
+// 131072 x 128 x 4090 640 / 618, 32768 x 512 x 1030 79 / 73, 2048 x 4096 x 1000 28 / 25).
+constexpr int64_t kNarrowN = 128, kNarrowK = 1024;
 struct RuntimeQuant {
   VecopsHipOperand a3, b3, c3, q, c_acc;
   Problem pr{};
@@ -1482,7 +1486,9 @@ int32_t describe_runtime_quant(const VecopsHipOperand* a_given, const VecopsHipO
   const bool shared_b = packed != nullptr || d->b3.strides[0] == 0 || d->batch <= 1;
   d->q_batches = (d->batch > 1 && (d->a3.strides[0] != 0 || scale_bs != 0)) ? d->batch : 1;
   d->row_batches = (d->batch > 1 && (!shared_b || correction_bs != 0)) ? d->batch : 1;
-  const int64_t q_step = packed != nullptr ? k_tile_elements(SRC_I8) : 16;
+  const bool pads = d->n > kNarrowN || d->k > kNarrowK;
+  const bool whole_k_tiles = pads && packed != nullptr;
+  const int64_t q_step = whole_k_tiles ? k_tile_elements(SRC_I8) : pads ? 16 : 1;
   d->q_pitch = (d->k + q_step - 1) / q_step * q_step;
   d->q_bytes = (static_cast<uint64_t>(d->q_batches) * d->m * d->q_pitch + 255u) & ~uint64_t{255};
   d->row_bytes = (static_cast<uint64_t>(d->row_batches) * d->n * 4u + 255u) & ~uint64_t{255};
@@ -1494,7 +1500,7 @@ int32_t describe_runtime_quant(const VecopsHipOperand* a_given, const VecopsHipO
   const int base = a_given->rank == 3 ? 1 : 0;
   if (base) { d->q.sizes[0] = d->batch; d->q.strides[0] = d->q_batches > 1 ? d->m * d->q_pitch : 0; }
   d->q.sizes[base] = d->m; d->q.strides[base] = d->q_pitch;
-  d->q.sizes[base + 1] = packed != nullptr ? d->q_pitch : d->k; d->q.strides[base + 1] = 1;
+  d->q.sizes[base + 1] = whole_k_tiles ? d->q_pitch : d->k; d->q.strides[base + 1] = 1;
   d->c_acc = *c_given;
   d->c_acc.dtype = DT_I32;  // accumulator class; the epilogue writes fp32
   // Batches fold into rows ([batch * M, K] x the one B) only when the scales run on with the rows and one
