@@ -14,6 +14,7 @@ INT32_MAX = 2 ** 31 - 1
 SOURCE = """
 #include "row_work_split.h"
 using namespace vecops_hip;
+static int elements(int left) { return left >= 4 ? 4 : left > 0 ? left : 0; }
 extern "C" {
 int32_t by_pieces(int64_t rows, int64_t k) { return quantize_by_pieces(rows, k); }
 int64_t blocks(int64_t rows, int64_t k) { return quantize_blocks(rows, k); }
@@ -25,8 +26,9 @@ void by_pieces_of(int64_t k, uint32_t block, int64_t* row, int64_t* first, int32
   for (int lane = 0; lane < 256; ++lane)
     for (int i = 0; i < kQuantizeQuads; ++i) {
       *row++ = block / pieces;
-      *first++ = quantize_piece_begin(piece) + quantize_quad(lane, i);
-      *length++ = quantize_quad_length(quantize_quad(lane, i), quantize_piece_length(piece, k));
+      const int begin = quantize_quad(piece, lane, i);
+      *first++ = begin;
+      *length++ = elements(static_cast<int>(k) - begin);
     }
 }
 void by_quads_of(int64_t k, uint32_t block, uint32_t blocks, int64_t most, int64_t* row, int64_t* first, int32_t* length) {
@@ -37,7 +39,7 @@ void by_quads_of(int64_t k, uint32_t block, uint32_t blocks, int64_t most, int64
       const int begin = static_cast<int>(at.quad) * 4;
       *row++ = at.row;
       *first++ = begin;
-      *length++ = quantize_quad_length(begin, static_cast<int>(k));
+      *length++ = elements(static_cast<int>(k) - begin);
     }
   }
 }

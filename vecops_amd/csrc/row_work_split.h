@@ -27,13 +27,9 @@ constexpr int64_t quantize_blocks(int64_t rows, int64_t k) {
   return blocks < kMostQuadBlocks ? blocks : kMostQuadBlocks;
 }
 
-// By pieces.  Elements of a row of k that lie in its piece, where the piece begins, and where in the piece a lane's i-th quad
-// does.  (The beginning in 64 bits, what is compared lane by lane below 4096: a row may have INT32_MAX elements.)
-constexpr int64_t quantize_piece_begin(uint32_t piece) { return static_cast<int64_t>(piece) * kQuantizePiece; }
-constexpr int quantize_piece_length(uint32_t piece, int64_t k) {
-  return k - quantize_piece_begin(piece) < kQuantizePiece ? static_cast<int>(k - quantize_piece_begin(piece)) : kQuantizePiece;
-}
-constexpr int quantize_quad(int lane, int i) { return i * 1024 + lane * 4; }
+// By pieces: where a lane's i-th quad begins.  It fits 32 bits in a row of INT32_MAX elements, up to 2047 past its end; where
+// the quad ends need not (what is left of the row is compared, which may be less than nothing).
+constexpr int quantize_quad(uint32_t piece, int lane, int i) { return static_cast<int>(piece) * kQuantizePiece + i * 1024 + lane * 4; }
 
 // By quads.  The way of a lane over the quads of all rows: its first one, and the next, a launch's lanes further on.  That
 // step is divided into whole rows and quads once, for the launch; the first quad's number fits 32 bits, all quads together
@@ -55,9 +51,6 @@ constexpr QuantizeQuad quantize_next(const QuantizeWalk& w, const QuantizeQuad& 
   const uint32_t quad = at.quad + w.step_quads;
   return quad < w.quads ? QuantizeQuad{at.row + w.step_rows, quad} : QuantizeQuad{at.row + w.step_rows + 1, quad - w.quads};
 }
-
-// Elements of a quad that begins at `begin` in a piece or row of `length`: 0 to 4.
-constexpr int quantize_quad_length(int begin, int length) { return length - begin >= 4 ? 4 : length > begin ? length - begin : 0; }
 
 // Sums over the rows of a packed operand (panels of 32 rows): a panel is a wavefront's, or its quarters of eight rows are a
 // workgroup's each (packed_row_sums.h).  By panel where the panels are many and K is short, because the lanes of a workgroup
