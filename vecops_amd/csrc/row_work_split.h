@@ -10,8 +10,8 @@ constexpr int64_t kMostBlocks = (int64_t{1} << 24) - 1;
 
 // Quantisation of contiguous rows, by pieces: a workgroup takes one piece of a row, a lane two quads of it, 1024 elements
 // apart.  By quads: the quads of all rows are one sequence, a lane takes one and then the one a launch's lanes further on.
-// Short rows go by quads, because the lanes past a row's end would idle (1048576 x 64 fp32: 937 us by pieces, 61 by quads,
-// 131072 x 512 119 and 59, 65536 x 1000 67 and 58; 65536 x 4096 230 and 277), and so does what has more pieces than a
+// Short rows go by quads, because the lanes past a row's end would idle (1048576 x 64 fp32: 937 us by pieces, 59 by quads,
+// 131072 x 512 119 and 58, 65536 x 1000 67 and 57; 65536 x 4096 230 and 277), and so does what has more pieces than a
 // launch may have workgroups.
 constexpr int kQuantizePiece = 2048;
 constexpr int kQuantizeQuads = kQuantizePiece / 1024;
