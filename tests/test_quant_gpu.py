@@ -35,7 +35,7 @@ def test_quantize_rows_edge_values_and_double_rounding(device):
     assert np.array_equal(q.cpu().numpy().astype(np.int32), GOLD["fma_bytes"])       # 1 everywhere; a fused rounding gives 0
 
 
-@pytest.mark.parametrize("batch,m,k", [(1, 19, 69), (1, 1, 1), (3, 37, 130), (1, 300, 4096), (2, 5, 3)])
+@pytest.mark.parametrize("batch,m,k", [(1, 19, 69), (1, 1, 1), (3, 37, 130), (1, 300, 4096), (2, 5, 3), (3, 20, 2049)])
 def test_quantize_rows_strided_and_batched(device, oracle, batch, m, k):
     """Rank 2 and 3, row strides wider than K on both sides, K not a multiple of four, a transposed source."""
     import torch
