@@ -1,0 +1,163 @@
+"""The slim tiles (tile_gemm_slim.hip): what the library runs in place of the rule table's own 64x64 or 128x128 tiles where
+few of them, or many K tiles for each, leave the chip waiting.  Each tile at the edges of its rows, columns and K - single
+elements past a tile, K shorter than a chunk, one K tile, a partial tile behind any number of whole ones, rings that wrap -
+with rows at any alignment, C inputs, output types, scales and transforms.  The forms are checked by their results, which
+differ in the last bits from the tile kernels' (K in four parts): a form that no longer takes a slim tile fails here."""
+import numpy as np
+import pytest
+
+from conftest import rel_err
+from test_matmul_gpu import fp32_tol
+
+pytestmark = pytest.mark.gpu
+
+# (m, n, k): by the estimates of slim_tile (capi.hip), with the tile each takes
+SHAPES = {
+    "32x16": [(17, 350, 960), (1, 21, 205), (33, 257, 1913), (1, 49, 447), (2, 20, 319), (20, 16, 520), (1, 37, 384)],
+    "32x32": [(64, 4096, 1024), (2, 6689, 454), (1, 5035, 385), (33, 2672, 448), (97, 1999, 2048)],
+    "32x48": [(33, 4285, 640), (32, 9231, 1216), (17, 11007, 1501), (1, 11713, 705)],
+    "32x64": [(31, 14336, 640), (17, 12743, 512), (2, 14529, 769)],
+    "64x48": [(33, 8209, 2560), (65, 5678, 1536), (129, 3338, 1344), (33, 8880, 2049), (100, 4224, 4672)],
+    "64x64": [(127, 8001, 1023), (64, 14336, 768), (65, 7553, 1472), (65, 7754, 1217)],
+    "128x48": [(128, 11008, 4096), (129, 6083, 512), (65, 11787, 641), (513, 2401, 960)],
+    "128x64": [(128, 14336, 2048), (129, 8170, 239), (257, 5377, 190), (65, 13433, 512)],
+}
+ALL = [s for shapes in SHAPES.values() for s in shapes]
+
+
+def _operands(device, dtype, m, n, k, seed=1, batch=(), pad=0):
+    import torch
+    g = torch.Generator(device=device).manual_seed(seed)
+    if dtype == torch.int8:
+        make = lambda shape: torch.randint(-128, 128, shape, generator=g, device=device, dtype=torch.int8)  # noqa: E731
+    else:
+        make = lambda shape: torch.randn(shape, generator=g, device=device).to(dtype)  # noqa: E731
+    return make((*batch, m, k + pad))[..., :k], make((*batch, n, k + pad))[..., :k]
+
+
+def _exact(a, b):
+    """The products of the operands as they are, in float64 (int8: exact below 2^53)."""
+    return np.matmul(a.double().cpu().numpy(), b.double().cpu().numpy().swapaxes(-1, -2))
+
+
+@pytest.mark.parametrize("m,n,k", ALL)
+@pytest.mark.parametrize("kind", ["bf16", "f16"])
+def test_against_float64(device, kind, m, n, k):
+    import torch
+    from vecops_amd import capi
+    dtype = torch.bfloat16 if kind == "bf16" else torch.float16
+    a, b = _operands(device, dtype, m, n, k)
+    c = torch.full((m, n), float("nan"), device=device)
+    capi.matmul(a, b, c)
+    prepared = torch.full((m, n), float("nan"), device=device)
+    capi.PreparedMatmul(a, b, prepared)()
+    rounded = torch.full((m, n), float("nan"), device=device, dtype=dtype)
+    capi.matmul(a, b, rounded)
+    torch.cuda.synchronize()
+    assert rel_err(c.cpu().numpy(), _exact(a, b)) <= fp32_tol(k)
+    assert torch.equal(c, prepared)
+    assert torch.equal(c.to(dtype), rounded)     # one rounding of the same sums
+
+
+@pytest.mark.parametrize("m,n,k,pad", [(17, 350, 960, 0), (33, 257, 1913, 0), (31, 300, 513, 2), (64, 2072, 1912, 8), (129, 999, 1000, 1),
+                                       (100, 700, 4099, 0), (128, 11008, 1024, 0), (40, 640, 447, 0)])
+def test_int8_exact(device, m, n, k, pad):
+    """Exact sums, rows at every byte alignment; and dequantised, two roundings a value, with a correction row."""
+    import torch
+    from vecops_amd import capi
+    a, b = _operands(device, torch.int8, m, n, k, pad=pad)
+    c = torch.full((m, n), -1, dtype=torch.int32, device=device)
+    capi.matmul(a, b, c)
+    rows, columns = torch.rand(m, device=device) + 0.5, torch.rand(n, device=device) + 0.5
+    correction = torch.randint(-1000, 1000, (n,), device=device, dtype=torch.int32)
+    f = torch.full((m, n), float("nan"), device=device)
+    capi.matmul_i8_dequant(a, b, rows, columns, f, correction=correction)
+    torch.cuda.synchronize()
+    want = torch.from_numpy(_exact(a, b).astype(np.int64)).to(torch.int32).to(device)
+    assert torch.equal(c, want)
+    assert torch.equal(f, ((want + correction).float() * rows[:, None]) * columns)
+
+
+@pytest.mark.parametrize("m,n,k", [(17, 350, 960), (129, 4225, 1025), (127, 801, 1023), (128, 4800, 1920)])
+@pytest.mark.parametrize("form", ["full", "bias", "strided", "transform", "transposed", "padded"])
+def test_epilogues(device, m, n, k, form):
+    """A C input's forms, the fused transform, C with strides that take the general store: all add to, or are made from, the
+    same sums, so the plain product's fp32 result gives the expected bits."""
+    import torch
+    from vecops_amd import capi
+    a, b = _operands(device, torch.bfloat16, m, n, k)
+    sums = torch.empty((m, n), device=device)
+    capi.matmul(a, b, sums)
+    g = torch.Generator(device=device).manual_seed(7)
+    cin = torch.randn((m, n), generator=g, device=device).bfloat16()
+    c = torch.full((m, n), float("nan"), device=device, dtype=torch.bfloat16)
+    if form == "bias":
+        cin = cin[:1].expand(m, n)
+    elif form == "strided":
+        wide = torch.randn((m, 2 * n), generator=g, device=device).bfloat16()
+        cin = wide[:, ::2]
+    elif form == "transposed":
+        c = torch.full((n, m), float("nan"), device=device, dtype=torch.bfloat16).t()
+    elif form == "padded":
+        c = torch.full((m, n + 3), float("nan"), device=device, dtype=torch.bfloat16)[:, :n]
+    if form == "transform":
+        scales = torch.rand(n, generator=g, device=device) + 0.5
+        capi.matmul_fused(a, b, c, capi.epilogue(activation="relu", column_scales=scales, scale=0.5, shift=0.25), c_in=cin)
+        want = torch.relu(((sums + cin.float()) * scales) * 0.5 + 0.25)
+    else:
+        capi.matmul(a, b, c, c_in=cin)
+        want = sums + cin.float()
+    torch.cuda.synchronize()
+    assert torch.equal(c, want.bfloat16())
+
+
+def test_batches(device):
+    import torch
+    from vecops_amd import capi
+    a, b = _operands(device, torch.float16, 33, 260, 1000, batch=(5,))
+    c = torch.full((5, 33, 260), float("nan"), device=device)
+    capi.matmul(a, b, c)
+    torch.cuda.synchronize()
+    assert rel_err(c.cpu().numpy(), _exact(a, b)) <= fp32_tol(1000)
+
+
+def test_whose_plan_it_is(device):
+    """The table's own plan runs on a slim tile wherever it comes from; a required family and split run as named."""
+    import torch
+    from vecops_amd import capi
+    a, b = _operands(device, torch.bfloat16, 64, 2048, 1408)
+    own, planned, automatic, required = (torch.empty((64, 2048), device=device) for _ in range(4))
+    plan = capi.plan_matmul(a, b, own)
+    assert capi.FAMILY_NAMES[plan.family] == "tile_64" and plan.split_k == 1
+    capi.matmul(a, b, own)
+    capi.matmul_planned(a, b, planned, plan)
+    capi.matmul_family(a, b, automatic, capi.family_request("tile_64", capi.SELECT_AUTOMATIC))
+    capi.matmul_family(a, b, required, capi.family_request("tile_64", capi.SELECT_REQUIRE, split_k=1))
+    torch.cuda.synchronize()
+    assert torch.equal(own, planned) and torch.equal(own, automatic)
+    assert not torch.equal(own, required)        # K in four parts here, front to back there
+    assert rel_err(own.cpu().numpy(), required.cpu().numpy()) <= fp32_tol(1408)
+
+
+def test_captured(device):
+    """Replayed several times with work of its own between the replays."""
+    import torch
+    from vecops_amd import capi
+    a, b = _operands(device, torch.bfloat16, 33, 1027, 1913)
+    want = torch.empty((33, 1027), device=device)
+    capi.matmul(a, b, want)
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        c = torch.empty_like(want)
+        call = capi.PreparedMatmul(a, b, c)
+        call()
+        stream.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            capi.PreparedMatmul(a, b, c)()
+    for _ in range(3):
+        c.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(c, want)

@@ -310,6 +310,17 @@ struct RuleConstants {
   //    batch 8 of 3000 x 3000 x 17 to fp32 54 us against 69, to bf16 42 against 53; 8192 x 8192 x 32 43 against 57; with
   //    a second step along K - its loads are not overlapped - the two-stage kernel is ahead, 65 against 71 us at K = 64)
   int64_t short_k_direct_max_k = 32;
+  // -- the slim tiles (tile_gemm_slim.hip) in place of the table's own plan of 64x64 or 128x128 tiles: both sides in ns, the
+  //    constants fitted to 617 products of 16-bit operands (17 <= M <= 1024, 256 <= N, K <= 14336, half of them with rows at
+  //    any alignment; the mean of weights in a cache and not), the slim side to have a margin of 5 %: of the 617 calls 320 take
+  //    a slim tile, on average 0.75 of the time they took, the worst 1.1 (`tests/test_slim_gpu.py` names the forms).
+  //    slim: a launch, and for every round of workgroups its start and end and (BM + BN) rows of K at slim_bytes_per_ns;
+  //    own: a launch, K tiles of a part at own_*_tile_ns or, with more workgroups, own_*_ns_per_wg of a unit's each (rows
+  //    that are not 16-byte aligned: times own_*_staged per mille), a K split's second launch and its partial sums' way.
+  int64_t slim_launch_ns = 2000, slim_round_ns = 2000, slim_row_ns = 10, slim_bytes_per_ns = 65, slim_bytes_per_ns_unaligned = 40;
+  int64_t slim_margin_num = 95, slim_margin_den = 100;
+  int64_t own_64_ns = 3640, own_64_tile_ns = 320, own_64_ns_per_wg = 415, own_64_staged = 1360, own_64_split_ns = 4430, own_64_ns_per_mb = 275;
+  int64_t own_128_ns = 5640, own_128_tile_ns = 515, own_128_ns_per_wg = 96, own_128_staged = 2120, own_128_split_ns = 3650, own_128_ns_per_mb = 585;
 };
 constexpr RuleConstants kRules{};
 
@@ -910,8 +921,45 @@ int32_t unsigned_side_terms(const Problem& pr, TileGemmParams* params, int32_t* 
   return ST_OK;
 }
 
+// Whether the rule table's own plan of 64x64 or 128x128 tiles is run by a slim tile instead, and by which (its result needs
+// no K split and no workspace).  A pure integer function of the problem and the plan; both sides' times are estimates in ns
+// (RuleConstants).  The result's type and a C input do not enter: a product's bf16 output stays its rounded fp32 output.
+bool slim_tile(const Problem& pr, const VecopsHipPlan& plan, const TileGemmParams& p, int mode, int* bm, int* bn) {
+  const bool small = plan.family == VECOPS_HIP_FAMILY_TILE_64;
+  if (!small && plan.family != VECOPS_HIP_FAMILY_TILE_128) return false;
+  if (pr.packed_b || (mode != MODE_KVEC && mode != MODE_KVEC_DMA) || !launch_tile_gemm_slim_serves(pr.src, p)) return false;
+  const bool aligned = mode == MODE_KVEC_DMA;
+  const int64_t ktile = k_tile_elements(pr.src), k_tiles = (pr.k + ktile - 1) / ktile;
+  const int64_t split = plan.split_k, tile = small ? 64 : 128;
+  const int64_t wgs = ((pr.m + tile - 1) / tile) * ((pr.n + tile - 1) / tile) * pr.batch * split;
+  int64_t tile_ns = std::max(small ? kRules.own_64_tile_ns : kRules.own_128_tile_ns,
+                             (small ? kRules.own_64_ns_per_wg : kRules.own_128_ns_per_wg) * wgs / kComputeUnits);
+  if (!aligned) tile_ns = tile_ns * (small ? kRules.own_64_staged : kRules.own_128_staged) / 1000;
+  int64_t own_ns = (small ? kRules.own_64_ns : kRules.own_128_ns) + (k_tiles + split - 1) / split * tile_ns;
+  if (split > 1)
+    own_ns += (small ? kRules.own_64_split_ns : kRules.own_128_split_ns) +
+              split * pr.batch * pr.m * pr.n * 4 / 1024 * (small ? kRules.own_64_ns_per_mb : kRules.own_128_ns_per_mb) / 1024;
+  static constexpr struct { int bm, bn; } tiles[] = {{32, 16}, {32, 32}, {32, 48}, {32, 64}, {64, 48}, {64, 64}, {128, 48}, {128, 64}};
+  int64_t best_ns = own_ns * kRules.slim_margin_num / kRules.slim_margin_den;
+  bool found = false;
+  for (const auto& t : tiles) {
+    const int64_t count = ((pr.m + t.bm - 1) / t.bm) * ((pr.n + t.bn - 1) / t.bn) * pr.batch;
+    const int64_t rounds = (count + kComputeUnits - 1) / kComputeUnits, rows = t.bm + t.bn;
+    const int64_t fetch_ns = rows * k_tiles * 128 / (aligned ? kRules.slim_bytes_per_ns : kRules.slim_bytes_per_ns_unaligned);
+    const int64_t ns = kRules.slim_launch_ns + rounds * (kRules.slim_round_ns + rows * kRules.slim_row_ns + fetch_ns);
+    if (ns < best_ns) {
+      best_ns = ns;
+      *bm = t.bm;
+      *bn = t.bn;
+      found = true;
+    }
+  }
+  return found;
+}
+
+// own_plan: the plan is the rule table's own (not a family or split that the caller requires).
 int32_t run_problem(const Problem& pr, const VecopsHipPlan& plan, const float* row_scales, const float* column_scales,
-                    const int32_t* correction, void* workspace, uint64_t workspace_size, hipStream_t stream) {
+                    const int32_t* correction, void* workspace, uint64_t workspace_size, hipStream_t stream, bool own_plan = true) {
   if (plan.family == VECOPS_HIP_FAMILY_NONE) return ST_OK;
   if (int32_t rc = check_device(); rc != ST_OK) return rc;
   if (pr.a.data == nullptr && pr.k > 0) return fail(ST_INVALID, "matmul: a has no storage");
@@ -1031,6 +1079,12 @@ int32_t run_problem(const Problem& pr, const VecopsHipPlan& plan, const float* r
   const int mode = fetch_mode(pr, plan);
 
   hipError_t e;
+  int slim_m = 0, slim_n = 0;
+  if (own_plan && slim_tile(pr, plan, p, mode, &slim_m, &slim_n)) {
+    e = launch_tile_gemm_slim(pr.src, p, slim_m, slim_n, stream);
+    if (e != hipSuccess) return fail(ST_EXEC, "slim tile kernel launch: %s", hipGetErrorString(e));
+    return ST_OK;
+  }
   if (pr.src == SRC_I8_FLIP) {
     // terms of the unsigned side(s), kept behind the split-K partials in the workspace
     const uint64_t partial_bytes = plan.split_k > 1 ? static_cast<uint64_t>(plan.split_k) * pr.batch * pr.m * pr.n * 4u : 0;
@@ -2031,9 +2085,12 @@ int32_t vecops_hip_matmul_family(const VecopsHipOperand* a, const VecopsHipOpera
   if (rc != ST_OK) return rc;
   VecopsHipPlan plan;
   choose(pr, &plan);
+  const VecopsHipPlan table = plan;
   rc = apply_request(pr, request, &plan);
   if (rc != ST_OK) return rc;
-  return run_problem(pr, plan, nullptr, nullptr, nullptr, workspace, workspace_size, static_cast<hipStream_t>(stream));
+  const bool own_plan = request == nullptr || request->selection == VECOPS_HIP_SELECT_AUTOMATIC ||
+                        (request->selection == VECOPS_HIP_SELECT_PREFER && memcmp(&plan, &table, sizeof(plan)) == 0);
+  return run_problem(pr, plan, nullptr, nullptr, nullptr, workspace, workspace_size, static_cast<hipStream_t>(stream), own_plan);
 }
 
 int32_t vecops_hip_matmul(const VecopsHipOperand* a, const VecopsHipOperand* b, const VecopsHipOperand* c_in,
@@ -2086,7 +2143,12 @@ int32_t vecops_hip_matmul_planned(const VecopsHipOperand* a, const VecopsHipOper
     if (checked.split_k != plan->split_k)
       return fail(ST_INVALID, "matmul_planned: the plan splits K %u ways, these operands allow %u", plan->split_k, checked.split_k);
   }
-  return run_problem(pr, checked, nullptr, nullptr, nullptr, workspace, workspace_size, static_cast<hipStream_t>(stream));
+  // (a plan that the rule table makes itself may run on a slim tile, as the unplanned call does; one for a required family
+  // or split runs that)
+  VecopsHipPlan table;
+  choose(pr, &table);
+  const bool own_plan = table.family == checked.family && table.split_k == checked.split_k && table.peeled_columns == checked.peeled_columns;
+  return run_problem(pr, checked, nullptr, nullptr, nullptr, workspace, workspace_size, static_cast<hipStream_t>(stream), own_plan);
 }
 
 uint64_t vecops_hip_matmul_i8_dequant_workspace(int64_t m, int64_t n, int64_t k) {

@@ -226,6 +226,10 @@ hipError_t launch_tile_gemm_deep128(int src, const TileGemmParams& p, int mode, 
 // per compute unit (tile_gemm_deep_f32.hip); b_as_kn: B handed over as [K,N].
 bool launch_tile_gemm_deep_f32_serves(const TileGemmParams& p, int tile, bool b_as_kn);
 hipError_t launch_tile_gemm_deep_f32(const TileGemmParams& p, int tile, bool b_as_kn, hipStream_t stream);
+// Tiles of bm = 32, 64 or 128 rows by bn = 16 to 64 columns over the whole K (tile_gemm_slim.hip): bf16, f16 or signed 8-bit
+// operands, both K-contiguous at any alignment; bm x bn one of 32 x {16, 32, 48, 64}, 64 x {48, 64}, 128 x {48, 64}.
+bool launch_tile_gemm_slim_serves(int src, const TileGemmParams& p);
+hipError_t launch_tile_gemm_slim(int src, const TileGemmParams& p, int bm, int bn, hipStream_t stream);
 // Very short K on 16-bit compute, operands K-contiguous: fragments loaded straight from memory, 64 x 128 of C a workgroup
 // (tile_gemm_short_k.hip).
 bool launch_tile_gemm_short_k_serves(int src, const TileGemmParams& p);
