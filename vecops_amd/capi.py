@@ -165,6 +165,28 @@ def lib() -> C.CDLL:
     return _lib
 
 
+CALLS_PATH = os.path.join(HERE, "lib", "vecops_torch_calls.so")
+_calls = None
+
+
+def native_calls():
+    """The per-call work of the functions below in native code (``host/torch/calls.cpp``): each of its functions answers
+    with the library's status, or with -1 for a call it leaves to the Python form (tensors that are not plain device
+    tensors, element types and ranks outside the table)."""
+    global _calls
+    if _calls is None:
+        import importlib.util
+        import torch  # noqa: F401  (the module links torch's libraries)
+        if not os.path.exists(CALLS_PATH):
+            raise RuntimeError(f"{CALLS_PATH} is missing: build it with vecops_amd.build.build_all()")
+        lib()
+        spec = importlib.util.spec_from_file_location("vecops_torch_calls", CALLS_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _calls = module
+    return _calls
+
+
 def _check(rc: int) -> None:
     if rc != 0:
         raise VecopsHipError(rc, lib().vecops_hip_last_error().decode())
@@ -212,6 +234,12 @@ def matmul(a, b, c, c_in=None, compute=COMPUTE_BF16, workspace=None, stream=None
     stream: pass ``stream`` only when it is that stream (the default), or pass a workspace of your own that outlives
     the work on the stream you name.
     """
+    if stream is None:
+        rc = (_calls or native_calls()).matmul(a, b, c, c_in, compute, workspace)
+        if rc == 0:
+            return c
+        if rc > 0:
+            _check(rc)
     import torch
     plan = plan_matmul(a, b, c, c_in, compute)
     if plan.workspace_bytes and (workspace is None or workspace.numel() * workspace.element_size()
@@ -347,6 +375,12 @@ def plan_matmul_fused(a, b, c, ep: Epilogue, c_in=None, compute=COMPUTE_BF16) ->
 def matmul_fused(a, b, c, ep: Epilogue, c_in=None, compute=COMPUTE_BF16, workspace=None, stream=None):
     """c = convert(transform(c_in + a . b^T)) with the output transform ``ep`` (see ``epilogue``) fused into the
     kernel's store; a bias is a ``c_in`` whose row stride is 0.  Mirrors ``tensor::output<Acc>(c, transform)``."""
+    if stream is None:
+        rc = (_calls or native_calls()).matmul_fused(a, b, c, c_in, compute, workspace, C.addressof(ep))
+        if rc == 0:
+            return c
+        if rc > 0:
+            _check(rc)
     import torch
     plan = plan_matmul_fused(a, b, c, ep, c_in, compute)
     if plan.workspace_bytes and (workspace is None or workspace.numel() * workspace.element_size()
@@ -362,6 +396,12 @@ def matmul_fused(a, b, c, ep: Epilogue, c_in=None, compute=COMPUTE_BF16, workspa
 
 
 def matmul_i8_dequant(a, b, row_scales, column_scales, c, correction=None, workspace=None, stream=None):
+    if stream is None:
+        rc = (_calls or native_calls()).matmul_i8_dequant(a, b, row_scales, column_scales, c, correction, workspace, -1)
+        if rc == 0:
+            return c
+        if rc > 0:
+            _check(rc)
     import torch
     m, k = a.shape
     n = b.shape[0]
@@ -389,6 +429,13 @@ def quantize_rows(x, multipliers, zero_point: int, q, stream=None):
 def matmul_runtime_quant(a, multipliers, zero_point: int, b, row_scales, column_scales, c, correction=None,
                          workspace=None, stream=None):
     """c = dequantise(quantise(a) . b^T + correction): fp32 a quantised on the way in, int8 b, fp32 c."""
+    if stream is None:
+        rc = (_calls or native_calls()).matmul_runtime_quant(a, multipliers, int(zero_point), b, row_scales, column_scales, c,
+                                                             correction, workspace, -1)
+        if rc == 0:
+            return c
+        if rc > 0:
+            _check(rc)
     import torch
     oa, ob, oc = operand(a), operand(b), operand(c)
     need = lib().vecops_hip_matmul_runtime_quant_workspace(C.byref(oa), C.byref(ob), C.byref(oc))
@@ -477,6 +524,13 @@ class PreparedGrouped:
 def matmul_runtime_quant_packed_b(a, multipliers, zero_point: int, packed, row_scales, column_scales, c, correction=None,
                                   workspace=None, stream=None):
     """``matmul_runtime_quant`` against weights packed once by ``pack_b`` (int8)."""
+    if stream is None:
+        rc = (_calls or native_calls()).matmul_runtime_quant(a, multipliers, int(zero_point), packed.storage, row_scales,
+                                                             column_scales, c, correction, workspace, packed.n)
+        if rc == 0:
+            return c
+        if rc > 0:
+            _check(rc)
     import torch
     oa, oc = operand(a), operand(c)
     need = lib().vecops_hip_matmul_runtime_quant_packed_b_workspace(C.byref(oa), packed.n, C.byref(oc))
@@ -492,6 +546,12 @@ def matmul_runtime_quant_packed_b(a, multipliers, zero_point: int, packed, row_s
 
 
 def matmul_w8a16_group(x, w, scales, y, group: int, stream=None):
+    if stream is None:
+        rc = (_calls or native_calls()).matmul_w8a16_group(x, w, scales, y, group)
+        if rc == 0:
+            return y
+        if rc > 0:
+            _check(rc)
     m, k = x.shape
     n = w.shape[0]
     assert x.stride(1) == 1 and w.stride(1) == 1 and y.stride(1) == 1 and scales.is_contiguous()
@@ -586,6 +646,12 @@ def plan_matmul_packed_b(a, packed: PackedB, c, c_in=None) -> Plan:
 
 def matmul_packed_b(a, packed: PackedB, c, c_in=None, workspace=None, stream=None):
     """c[..,M,N] = c_in + a[..,M,K] . B^T with B packed by ``pack_b``; returns c."""
+    if stream is None:
+        rc = (_calls or native_calls()).matmul_packed_b(a, packed.storage, c, c_in, packed.dtype, workspace, packed.n)
+        if rc == 0:
+            return c
+        if rc > 0:
+            _check(rc)
     import torch
     plan = plan_matmul_packed_b(a, packed, c, c_in)
     if plan.workspace_bytes and (workspace is None or workspace.numel() * workspace.element_size()
@@ -603,6 +669,13 @@ def matmul_packed_b(a, packed: PackedB, c, c_in=None, workspace=None, stream=Non
 
 def matmul_i8_dequant_packed_b(a, packed: PackedB, row_scales, column_scales, c, correction=None, workspace=None,
                                stream=None):
+    if stream is None and packed.dtype == I8 and packed.k == a.shape[-1]:
+        rc = (_calls or native_calls()).matmul_i8_dequant(a, packed.storage, row_scales, column_scales, c, correction, workspace,
+                                                          packed.n)
+        if rc == 0:
+            return c
+        if rc > 0:
+            _check(rc)
     import torch
     m, k = a.shape
     n = packed.n

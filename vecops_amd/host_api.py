@@ -215,6 +215,13 @@ class HostOperator:
         except Exception:
             pass
 
+    def native_entries(self) -> tuple[int, int, int]:
+        """For native callers: the operator in its host library's C interface, and the addresses of that library's bridge
+        entry and workspace query."""
+        lib = self._lib.lib
+        return (self._h, C.cast(lib.vecops_operator_bridge_invoke_v1, C.c_void_p).value,
+                C.cast(lib.vecops_hip_host_operator_workspace, C.c_void_p).value)
+
     def bridge_handle(self) -> int:
         """Registers the operator with the process-local bridge (once) and returns its handle."""
         if not getattr(self, "_bridge", 0):

@@ -22,6 +22,7 @@ from __future__ import annotations
 import threading
 from types import SimpleNamespace
 
+from . import capi
 from . import host_api as H
 
 # Positional parameters of the operators this package ships (name, kind); kind is
@@ -165,11 +166,16 @@ class _Registration:
         def meta(*args, **kwargs):
             return tuple(args[i] for i in outputs) if return_outputs else None
 
-        lib.impl(self.name, self.invoke, "CUDA")
+        # device tensors: native code from the dispatcher to the bridge entry, which hands calls it does not serve (host
+        # tensors among them, types outside the table) to ``invoke``
+        capi.native_calls().register_device_kernel(
+            self.library, self.name, self.operator.bridge_handle(), *self.operator.native_entries(),
+            [kind for _, kind in self.params], list(self.specs.items()), return_outputs, self.invoke, H.HostError)
         lib.impl(self.name, self.invoke, "CPU")
         lib.impl(self.name, meta, "Meta")
         self._library = lib                                         # keeps the definitions alive
-        self.torch_op = getattr(getattr(torch.ops, self.library), self.name)
+        # (the one overload: the packet would look for it on each call)
+        self.torch_op = getattr(getattr(torch.ops, self.library), self.name).default
 
     # -- the public callable --------------------------------------------------------------
     def public(self, *args, **kwargs):
