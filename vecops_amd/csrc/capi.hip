@@ -16,6 +16,7 @@
 #include "tile_gemm_launch.h"
 #include "tile_gemm_packed.h"
 #include "vecops_hip.h"
+#include "w8a16_ring.h"
 
 namespace {
 
@@ -2192,6 +2193,37 @@ int32_t vecops_hip_matmul_i8_dequant(const int8_t* a, int64_t lda, const int8_t*
                      static_cast<hipStream_t>(stream));
 }
 
+}  // extern "C"
+
+namespace {
+// How many weight rows a workgroup of the ring kernel (w8a16_ring.hip) takes for a weight-only product, 0 where the other
+// kernels of the skinny family are ahead.  By estimated ns, `rounds * (start and end + what a workgroup fetches)`: the fewest
+// rows that fit one round, mostly - 16 x 8352 x 6272 in groups of 128 16.5 us on 48 rows (26.4 on 16, 25.3 on 32, 19.9 on 64;
+// 33.3 before), 14 x 1848 x 5376 7.5 on 16 (13.0), 16 x 4096 x 4096 8.5 on 16 (10.5), 16 x 8192 x 4096 11.9 on 32 (14.5).
+//   * From five rows of activations on; with three or four (the other kernels' share of activation loads is smaller) from K =
+//     2048 on: 4 x 15616 x 3840 14.7 against 19.6, 4 x 5760 x 2048 6.4 against 6.5, 4 x 6400 x 1664 6.1 against 6.0.
+//   * At K = 4096 with more than 8192 weight rows the kernel whose activations are resident is level or ahead (16 x 14336 in
+//     a cache 13.1 against 13.9, not in one 17.0 both).
+int ring_weight_rows(const SkinnyW8A16Params& p) {
+  if (p.m < 3 || (p.m < 5 && p.k < 2048)) return 0;
+  if (p.k == 4096 && p.n > 8192 && (p.group == 128 || p.group == 256) && p.ldx < (int64_t{1} << 26)) return 0;
+  int best = 0;
+  int64_t best_ns = INT64_MAX;
+  for (const int rows : {16, 32, 48, 64}) {
+    if (!launch_w8a16_ring_serves(p, rows)) continue;
+    const int64_t rounds = ((p.n + rows - 1) / rows + kComputeUnits - 1) / kComputeUnits;
+    const int64_t ns = rounds * (2000 + static_cast<int64_t>(32 + rows) * p.k / 36);
+    if (ns < best_ns) {
+      best_ns = ns;
+      best = rows;
+    }
+  }
+  return best;
+}
+}  // namespace
+
+extern "C" {
+
 int32_t vecops_hip_matmul_w8a16_group(const void* x, int64_t ldx, const int8_t* w, int64_t ldw, const float* scales,
                                       void* y, int64_t ldy, int64_t m, int64_t n, int64_t k, int64_t group,
                                       void* stream) {
@@ -2220,9 +2252,16 @@ int32_t vecops_hip_matmul_w8a16_group(const void* x, int64_t ldx, const int8_t* 
   p.groups = static_cast<int32_t>(k / group);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (int32_t rc = check_device(); rc != ST_OK) return rc;
+  hipError_t e;
   // GPU rule table of the skinny family: matrix cores once the widening of a weight
   // byte can be shared by three or more activation rows
   const bool mfma_ok = group % 64 == 0 && (group == 64 || group == 128 || group == 256);
+  const int ring_rows = ring_weight_rows(p);
+  if (ring_rows > 0) {
+    e = launch_w8a16_ring(p, ring_rows, s);
+    if (e != hipSuccess) return fail(ST_EXEC, "weight-only ring kernel launch: %s", hipGetErrorString(e));
+    return ST_OK;
+  }
   if (m == 2 && k == 4096 && n >= 4096) {
     // two rows of activations: the streaming walk of M = 1 with both rows resident (13.9 us at N = 14336 where
     // the matrix-core kernel takes 17.0)
@@ -2249,7 +2288,7 @@ int32_t vecops_hip_matmul_w8a16_group(const void* x, int64_t ldx, const int8_t* 
   else if (m <= 4) launch_skinny<4, 2, 1>(p, s);
   else if (m <= 8) launch_skinny<8, 2, 1>(p, s);
   else launch_skinny<16, 1, 1>(p, s);
-  hipError_t e = hipGetLastError();
+  e = hipGetLastError();
   if (e != hipSuccess) return fail(ST_EXEC, "skinny kernel launch: %s", hipGetErrorString(e));
   return ST_OK;
 }
