@@ -1123,6 +1123,9 @@ int32_t run_problem(const Problem& pr, const VecopsHipPlan& plan, const float* r
              launch_tile_gemm_deep_f32_serves(p, tile_m, mode == MODE_NVEC_B)) {
     // fp32 compute, at most one workgroup per compute unit: the ring of LDS stages (tile_gemm_deep_f32.hip)
     e = launch_tile_gemm_deep_f32(p, tile_m, mode == MODE_NVEC_B, stream);
+  } else if (plan.family == VECOPS_HIP_FAMILY_TILE_128X256 && mode == MODE_KVEC && launch_tile_gemm_rows_serves(pr.src, p)) {
+    // rows at any alignment on the 128x256 tile: three stages by loads that write LDS (tile_gemm_rows.hip)
+    e = launch_tile_gemm_rows(pr.src, p, stream);
   } else switch (pr.src) {
     case SRC_I8_FLIP: e = launch_tile_gemm_i8_flip(p, tile_m, tile_n, mode, stream); break;
     case SRC_BF16: e = launch_tile_gemm_bf16(p, tile_m, tile_n, mode, stream); break;

@@ -230,6 +230,9 @@ hipError_t launch_tile_gemm_deep_f32(const TileGemmParams& p, int tile, bool b_a
 // operands, both K-contiguous at any alignment; bm x bn one of 32 x {16, 32, 48, 64}, 64 x {48, 64}, 128 x {48, 64}.
 bool launch_tile_gemm_slim_serves(int src, const TileGemmParams& p);
 hipError_t launch_tile_gemm_slim(int src, const TileGemmParams& p, int bm, int bn, hipStream_t stream);
+// The 128 x 256 tile for K-contiguous bf16, f16 or signed 8-bit operands with rows at any alignment (tile_gemm_rows.hip).
+bool launch_tile_gemm_rows_serves(int src, const TileGemmParams& p);
+hipError_t launch_tile_gemm_rows(int src, const TileGemmParams& p, hipStream_t stream);
 // Very short K on 16-bit compute, operands K-contiguous: fragments loaded straight from memory, 64 x 128 of C a workgroup
 // (tile_gemm_short_k.hip).
 bool launch_tile_gemm_short_k_serves(int src, const TileGemmParams& p);
