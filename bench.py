@@ -266,6 +266,8 @@ def bench_batched(dev, steps, warmup, m, n, k):
     label = _kernel_label(plan, "bf16")
     if capi.FAMILY_NAMES[plan.family] == "tile_128" and 8 <= k <= 32:
         label = "tile_gemm_short_k_kernel<bf16>"   # what run_problem launches for such a plan
+    if capi.FAMILY_NAMES[plan.family] == "tile_128x256" and k % 8 != 0:
+        label = label.replace("tile_gemm_kernel<bf16>", "tile_gemm_rows_kernel<bf16>")   # likewise, rows not 16-byte aligned
     roof.update(kernel=label, algorithmic_flops_per_launch=flops, algorithmic_bytes_per_launch=nbytes,
                 **_traffic(f"batched_{m}x{n}x{k}"), **_timing_fields(t))
     return {"metric": f"bf16_batched_{m}x{n}x{k}_tflops", "workload": f"batch 8 x bf16 ({m},{n},{k}), A[8,M,K] and "
