@@ -85,7 +85,12 @@ typedef struct VecopsHipPlan {
   uint32_t split_k;    /* >= 1; > 1 needs workspace */
   uint32_t vector_a;   /* 1 = 16-byte loads along K usable for A */
   uint32_t vector_b;   /* 1 = 16-byte loads usable for B */
-  uint32_t b_layout;   /* 0 = K contiguous, 1 = N contiguous, 2 = generic */
+  uint16_t b_layout;   /* 0 = K contiguous, 1 = N contiguous, 2 = generic */
+  uint16_t slim_tile;  /* 0: the family's own tiles, K split as split_k says.  Else 256 * rows + columns of the slim tile
+                          (32x16 to 128x64) that runs in their place, in one launch over the whole K: in the
+                          library's own plans, where tile_64 or tile_128 would leave the chip short of work.  family,
+                          split_k and workspace_bytes are then what runs with slim_tile set to 0, and a requested
+                          family always runs as named */
   uint32_t peeled_columns; /* > 0: the last so many columns of c are a second product with a plan of its own (few
                               tiles, K split), cut off so that the rest fills whole rounds of workgroups */
   uint64_t workspace_bytes;
@@ -137,9 +142,11 @@ VECOPS_HIP_EXPORT int32_t vecops_hip_matmul(const VecopsHipOperand* a, const Vec
  * vecops_hip_matmul with the plan made beforehand - the prepared invocation of vecops (ops::Matmul<Config>::prepare /
  * Prepared / PatternPrepared, ops/Matmul.h:183-500; the prepared-call cache of docs/Runtime.md:196-206): `plan` is what
  * vecops_hip_plan_matmul or vecops_hip_plan_matmul_family returned for operands of the same metadata (extents, strides,
- * dtypes, alignment); the rule table is not consulted again.  The plan is checked against the operands - a family
- * that cannot serve them, a K split beyond the K tiles or columns peeled where the table peels none is status 1
- * (invalid argument), nothing is launched - and its workspace need is recomputed, never trusted.
+ * dtypes, alignment); the rule table is consulted again only for a plan that peels columns, so the call runs what the
+ * plan names: its slim tile, or its family and K split - the same kernels as the call that the plan was made for.  The
+ * plan is checked against the operands - a family or slim tile that cannot serve them, a K split beyond the K tiles or
+ * columns peeled where the table peels none is status 1 (invalid argument), nothing is launched - and its workspace need
+ * is recomputed, never trusted.
  */
 VECOPS_HIP_EXPORT int32_t vecops_hip_matmul_planned(const VecopsHipOperand* a, const VecopsHipOperand* b,
                                                     const VecopsHipOperand* c_in, const VecopsHipOperand* c,
@@ -214,8 +221,9 @@ VECOPS_HIP_EXPORT int32_t vecops_hip_matmul_static_workspace(const VecopsHipOper
  * unsigned side count as a mix), groups with K = 0 and groups whose K vecops_hip_matmul would split (few output tiles,
  * long K: they run that call's plan, partial sums behind the table) run as launches of their own on the same stream.
  * Results
- * are those of vecops_hip_matmul on each group (bit-equal when that call runs the same tile shape without splitting K -
- * except 16-bit products with K <= 256 on 128 x 128 tiles, where the single call takes the other MFMA shape; otherwise equal up to the order of the fp32 sums - integer results are always the same bits).  workspace: vecops_hip_matmul_grouped_workspace bytes, 16-byte aligned.
+ * are those of vecops_hip_matmul on each group (bit-equal when that call runs the same tile shape without splitting K and
+ * its plan names no slim tile - except 16-bit products with K <= 256 on 128 x 128 tiles, where the single call takes the
+ * other MFMA shape; otherwise equal up to the order of the fp32 sums - integer results are always the same bits).  workspace: vecops_hip_matmul_grouped_workspace bytes, 16-byte aligned.
  */
 VECOPS_HIP_EXPORT uint64_t vecops_hip_matmul_grouped_workspace(uint32_t count, const VecopsHipOperand* a,
                                                                const VecopsHipOperand* b, const VecopsHipOperand* c_in,
@@ -464,8 +472,8 @@ VECOPS_HIP_EXPORT int32_t vecops_hip_matmul_packed_b(const VecopsHipOperand* a, 
  * packed A (tests/ops/MatmulMixedPackingTest.cpp:24-28).  C = C_in + A . B^T with A[M,K] prepacked runs as
  * C^T = C_in^T + B . A^T on the packed-operand kernels: b is then the operand that travels through LDS and the
  * packed a the one fetched straight into registers; c and c_in are written and read through their transposed views
- * (any strides are legal, the stores of a row-major c are element-wise).  Same sums in the same order as the plain
- * product.  b rank 2 or 3 (the one packed a serves every batch), dtypes as for vecops_hip_matmul_packed_b with the
+ * (any strides are legal, the stores of a row-major c are element-wise).  The sums are taken in the
+ * order of vecops_hip_matmul_packed_b, and so equal the plain product's bits where that entry's do.  b rank 2 or 3 (the one packed a serves every batch), dtypes as for vecops_hip_matmul_packed_b with the
  * sides exchanged.
  */
 VECOPS_HIP_EXPORT int32_t vecops_hip_pack_a(const VecopsHipOperand* a, void* packed, uint64_t packed_size, void* stream);

@@ -11,7 +11,7 @@ from test_matmul_gpu import fp32_tol
 
 pytestmark = pytest.mark.gpu
 
-# (m, n, k): by the estimates of slim_tile (capi.hip), with the tile each takes
+# (m, n, k): by the estimates of take_slim_tile (capi.hip), with the tile each takes
 SHAPES = {
     "32x16": [(17, 350, 960), (1, 21, 205), (33, 257, 1913), (1, 49, 447), (2, 20, 319), (20, 16, 520), (1, 37, 384)],
     "32x32": [(64, 4096, 1024), (2, 6689, 454), (1, 5035, 385), (33, 2672, 448), (97, 1999, 2048)],
@@ -161,3 +161,39 @@ def test_captured(device):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(c, want)
+
+
+def test_planned_calls_run_what_the_plan_names(device):
+    """A plan made for a required or preferred family gives that family's bits in the planned call too, where the table's own
+    plan has the same family and split; a slim tile in a plan is checked like the rest of it."""
+    import torch
+    from vecops_amd import capi
+    a, b = _operands(device, torch.bfloat16, 64, 2048, 1408)
+    make = lambda: torch.full((64, 2048), 7.0, device=device)  # noqa: E731
+    own = capi.matmul(a, b, make())
+    for selection in (capi.SELECT_REQUIRE, capi.SELECT_PREFER):
+        for split in (0, 1):
+            request = capi.family_request("tile_64", selection, split_k=split)
+            plan = capi.plan_matmul_family(a, b, make(), request)
+            table = capi.plan_matmul(a, b, make())
+            assert (plan.family, plan.split_k, plan.slim_tile) == (table.family, table.split_k, 0) and table.slim_tile != 0
+            named, planned = capi.matmul_family(a, b, make(), request), capi.matmul_planned(a, b, make(), plan)
+            assert torch.equal(named, planned) and not torch.equal(named, own)
+    plan = capi.plan_matmul(a, b, make())
+    for bm, bn in ((32, 16), (32, 32), (32, 48), (32, 64), (64, 48), (64, 64), (128, 48), (128, 64)):   # any of them may be asked for
+        plan.slim_tile = 256 * bm + bn
+        assert torch.equal(capi.matmul_planned(a, b, make(), plan), own)   # K in the same four parts
+    c = make()
+    for code in (1, 256 * 48 + 48, 256 * 64 + 32, 0xffff):
+        plan.slim_tile = code
+        with pytest.raises(capi.VecopsHipError) as e:
+            capi.matmul_planned(a, b, c, plan)
+        assert e.value.code == 1
+    plan.slim_tile = 256 * 32 + 16
+    with pytest.raises(capi.VecopsHipError):      # operands that slim tiles do not serve
+        capi.matmul_planned(a, torch.empty((1408, 2048), device=device, dtype=torch.bfloat16).t(), c, plan)
+    plan.family = capi.FAMILY_CODES["tile_256"]   # and tiles that they do not stand in for
+    with pytest.raises(capi.VecopsHipError):
+        capi.matmul_planned(a, b, c, plan)
+    torch.cuda.synchronize()
+    assert float(c.min()) == 7.0 and float(c.max()) == 7.0

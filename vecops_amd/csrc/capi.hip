@@ -462,8 +462,10 @@ bool tile_192_serves(const Problem& pr, const VecopsHipPlan& plan) {
 // data, a lightly loaded round clocks higher, and narrower tiles (256x192 was
 // measured) cost more LDS and L2 traffic per flop than the better balance saves.
 // (scratch_limit: partial sums the caller can hold - the mid-band K split below is skipped where it needs more)
-// (peel_allowed: false for the product of a peel itself)
-void choose(const Problem& pr, VecopsHipPlan* plan, uint64_t scratch_limit = UINT64_MAX, bool peel_allowed = true) {
+// (peel_allowed: false for the product of a peel itself, which is chosen as a call of its own is, by `choose`)
+void choose(const Problem& pr, VecopsHipPlan* plan, uint64_t scratch_limit = UINT64_MAX, bool peel_allowed = true);
+
+void choose_table(const Problem& pr, VecopsHipPlan* plan, uint64_t scratch_limit = UINT64_MAX, bool peel_allowed = true) {
   memset(plan, 0, sizeof(*plan));
   plan->split_k = 1;
   if (pr.batch == 0 || pr.m == 0 || pr.n == 0) {
@@ -764,8 +766,10 @@ const char* family_name(uint32_t family) {
 // and is an error when required (family_selection::Require turns an inapplicable family into a hard error,
 // tests/ops/MatmulTest.cpp:514-536).  The tile families serve every non-empty product; the skinny family only its
 // own shapes; none / zero_k only the degenerate problems they name.
-int32_t apply_request(const Problem& pr, const VecopsHipFamilyRequest* request, VecopsHipPlan* plan) {
-  if (request == nullptr || request->selection == VECOPS_HIP_SELECT_AUTOMATIC) return ST_OK;
+// table_choice: set where the plan stays the rule table's own - nothing was asked for, or a preferred family cannot serve.
+int32_t apply_request(const Problem& pr, const VecopsHipFamilyRequest* request, VecopsHipPlan* plan, bool* table_choice) {
+  *table_choice = request == nullptr || request->selection == VECOPS_HIP_SELECT_AUTOMATIC;
+  if (*table_choice) return ST_OK;
   if (request->struct_size < sizeof(VecopsHipFamilyRequest)) return fail(ST_INVALID, "matmul: family request record too short");
   if (request->selection != VECOPS_HIP_SELECT_PREFER && request->selection != VECOPS_HIP_SELECT_REQUIRE)
     return fail(ST_INVALID, "matmul: unknown family selection %u", request->selection);
@@ -789,7 +793,10 @@ int32_t apply_request(const Problem& pr, const VecopsHipFamilyRequest* request, 
                                                                : true;
   }
   if (!serves) {
-    if (request->selection == VECOPS_HIP_SELECT_PREFER) return ST_OK;  // the rule table's choice stands
+    if (request->selection == VECOPS_HIP_SELECT_PREFER) {
+      *table_choice = true;
+      return ST_OK;
+    }
     return fail(ST_NOT_APPLICABLE, "matmul: the required family %s cannot serve this call (the rule table chooses %s)",
                 family_name(request->family), family_name(plan->family));
   }
@@ -922,14 +929,27 @@ int32_t unsigned_side_terms(const Problem& pr, TileGemmParams* params, int32_t* 
   return ST_OK;
 }
 
-// Whether the rule table's own plan of 64x64 or 128x128 tiles is run by a slim tile instead, and by which (its result needs
-// no K split and no workspace).  A pure integer function of the problem and the plan; both sides' times are estimates in ns
-// (RuleConstants).  The result's type and a C input do not enter: a product's bf16 output stays its rounded fp32 output.
-bool slim_tile(const Problem& pr, const VecopsHipPlan& plan, const TileGemmParams& p, int mode, int* bm, int* bn) {
+// The slim tiles (tile_gemm_slim.hip), and a plan's `slim_tile` for each.
+constexpr struct { int bm, bn; } kSlimTiles[] = {{32, 16}, {32, 32}, {32, 48}, {32, 64}, {64, 48}, {64, 64}, {128, 48}, {128, 64}};
+uint16_t slim_code(int bm, int bn) { return static_cast<uint16_t>(bm << 8 | bn); }
+
+// Whether slim tiles can run a problem, as far as its operands go.
+bool slim_serves(const Problem& pr, const VecopsHipPlan& plan) {
+  if (pr.packed_b || pr.src == kSrcF64) return false;
+  const int mode = fetch_mode(pr, plan);
+  return (mode == MODE_KVEC || mode == MODE_KVEC_DMA) &&
+         launch_tile_gemm_slim_serves(pr.src, base_params(pr, nullptr, nullptr, nullptr, nullptr));
+}
+
+// Hands the rule table's own plan of 64x64 or 128x128 tiles to a slim tile where that is ahead: the plan then names it
+// (slim_tile) beside the table's family, split and workspace, none of which the call uses.  A pure integer function of the
+// problem and the plan; both sides' times are estimates in ns (RuleConstants).  The result's type and a C input do not enter:
+// a product's bf16 output stays its rounded fp32 output.  (A plan that peels columns keeps its tiles, which are whole rounds.)
+void take_slim_tile(const Problem& pr, VecopsHipPlan* chosen) {
+  const VecopsHipPlan& plan = *chosen;
   const bool small = plan.family == VECOPS_HIP_FAMILY_TILE_64;
-  if (!small && plan.family != VECOPS_HIP_FAMILY_TILE_128) return false;
-  if (pr.packed_b || (mode != MODE_KVEC && mode != MODE_KVEC_DMA) || !launch_tile_gemm_slim_serves(pr.src, p)) return false;
-  const bool aligned = mode == MODE_KVEC_DMA;
+  if ((!small && plan.family != VECOPS_HIP_FAMILY_TILE_128) || plan.peeled_columns > 0 || !slim_serves(pr, plan)) return;
+  const bool aligned = fetch_mode(pr, plan) == MODE_KVEC_DMA;
   const int64_t ktile = k_tile_elements(pr.src), k_tiles = (pr.k + ktile - 1) / ktile;
   const int64_t split = plan.split_k, tile = small ? 64 : 128;
   const int64_t wgs = ((pr.m + tile - 1) / tile) * ((pr.n + tile - 1) / tile) * pr.batch * split;
@@ -940,27 +960,39 @@ bool slim_tile(const Problem& pr, const VecopsHipPlan& plan, const TileGemmParam
   if (split > 1)
     own_ns += (small ? kRules.own_64_split_ns : kRules.own_128_split_ns) +
               split * pr.batch * pr.m * pr.n * 4 / 1024 * (small ? kRules.own_64_ns_per_mb : kRules.own_128_ns_per_mb) / 1024;
-  static constexpr struct { int bm, bn; } tiles[] = {{32, 16}, {32, 32}, {32, 48}, {32, 64}, {64, 48}, {64, 64}, {128, 48}, {128, 64}};
   int64_t best_ns = own_ns * kRules.slim_margin_num / kRules.slim_margin_den;
-  bool found = false;
-  for (const auto& t : tiles) {
+  uint16_t found = 0;
+  for (const auto& t : kSlimTiles) {
     const int64_t count = ((pr.m + t.bm - 1) / t.bm) * ((pr.n + t.bn - 1) / t.bn) * pr.batch;
     const int64_t rounds = (count + kComputeUnits - 1) / kComputeUnits, rows = t.bm + t.bn;
     const int64_t fetch_ns = rows * k_tiles * 128 / (aligned ? kRules.slim_bytes_per_ns : kRules.slim_bytes_per_ns_unaligned);
     const int64_t ns = kRules.slim_launch_ns + rounds * (kRules.slim_round_ns + rows * kRules.slim_row_ns + fetch_ns);
     if (ns < best_ns) {
       best_ns = ns;
-      *bm = t.bm;
-      *bn = t.bn;
-      found = true;
+      found = slim_code(t.bm, t.bn);
     }
   }
-  return found;
+  chosen->slim_tile = found;
 }
 
-// own_plan: the plan is the rule table's own (not a family or split that the caller requires).
+// The library's own plan: the rule table's, or a slim tile in its place.
+void choose(const Problem& pr, VecopsHipPlan* plan, uint64_t scratch_limit, bool peel_allowed) {
+  choose_table(pr, plan, scratch_limit, peel_allowed);
+  take_slim_tile(pr, plan);
+}
+
+// The plan under a family request: the library's own where nothing is asked for or a preferred family cannot serve, else the
+// family and split that the request names.
+int32_t choose_requested(const Problem& pr, const VecopsHipFamilyRequest* request, VecopsHipPlan* plan) {
+  choose_table(pr, plan);
+  bool table_choice = false;
+  const int32_t rc = apply_request(pr, request, plan, &table_choice);
+  if (rc == ST_OK && table_choice) take_slim_tile(pr, plan);
+  return rc;
+}
+
 int32_t run_problem(const Problem& pr, const VecopsHipPlan& plan, const float* row_scales, const float* column_scales,
-                    const int32_t* correction, void* workspace, uint64_t workspace_size, hipStream_t stream, bool own_plan = true) {
+                    const int32_t* correction, void* workspace, uint64_t workspace_size, hipStream_t stream) {
   if (plan.family == VECOPS_HIP_FAMILY_NONE) return ST_OK;
   if (int32_t rc = check_device(); rc != ST_OK) return rc;
   if (pr.a.data == nullptr && pr.k > 0) return fail(ST_INVALID, "matmul: a has no storage");
@@ -1080,9 +1112,8 @@ int32_t run_problem(const Problem& pr, const VecopsHipPlan& plan, const float* r
   const int mode = fetch_mode(pr, plan);
 
   hipError_t e;
-  int slim_m = 0, slim_n = 0;
-  if (own_plan && slim_tile(pr, plan, p, mode, &slim_m, &slim_n)) {
-    e = launch_tile_gemm_slim(pr.src, p, slim_m, slim_n, stream);
+  if (plan.slim_tile != 0) {
+    e = launch_tile_gemm_slim(pr.src, p, plan.slim_tile >> 8, plan.slim_tile & 255, stream);
     if (e != hipSuccess) return fail(ST_EXEC, "slim tile kernel launch: %s", hipGetErrorString(e));
     return ST_OK;
   }
@@ -2055,8 +2086,12 @@ int32_t vecops_hip_matmul_static_workspace(const VecopsHipOperand* a, const Veco
   // beyond the row sums of an unsigned operand): the call is then slower than with a caller's workspace, not refused.
   int tile_m = 0, tile_n = 0;
   tile_of_family(plan.family, &tile_m, &tile_n);
-  while (tile_m != 0 && plan.peeled_columns == 0 && plan.split_k > 1 && plan.workspace_bytes > VECOPS_HIP_STATIC_WORKSPACE_BYTES)
+  while (plan.slim_tile == 0 && tile_m != 0 && plan.peeled_columns == 0 && plan.split_k > 1 &&
+         plan.workspace_bytes > VECOPS_HIP_STATIC_WORKSPACE_BYTES) {
     finish_tile_plan(pr, &plan, plan.split_k / 2);
+    take_slim_tile(pr, &plan);  // (ahead of fewer parts, perhaps)
+  }
+  if (plan.slim_tile != 0) plan.workspace_bytes = 0;  // (it uses none)
   if (plan.workspace_bytes > VECOPS_HIP_STATIC_WORKSPACE_BYTES)
     return fail(ST_NOT_APPLICABLE, "matmul_static_workspace: the call needs %llu bytes of scratch, the library holds %llu",
                 (unsigned long long)plan.workspace_bytes, (unsigned long long)VECOPS_HIP_STATIC_WORKSPACE_BYTES);
@@ -2077,8 +2112,7 @@ int32_t vecops_hip_plan_matmul_family(const VecopsHipOperand* a, const VecopsHip
   Problem pr{};
   int32_t rc = describe(a, b, c_in, c, compute, &pr);
   if (rc != ST_OK) return rc;
-  choose(pr, plan);
-  return apply_request(pr, request, plan);
+  return choose_requested(pr, request, plan);
 }
 
 int32_t vecops_hip_matmul_family(const VecopsHipOperand* a, const VecopsHipOperand* b, const VecopsHipOperand* c_in,
@@ -2088,13 +2122,9 @@ int32_t vecops_hip_matmul_family(const VecopsHipOperand* a, const VecopsHipOpera
   int32_t rc = describe(a, b, c_in, c, compute, &pr);
   if (rc != ST_OK) return rc;
   VecopsHipPlan plan;
-  choose(pr, &plan);
-  const VecopsHipPlan table = plan;
-  rc = apply_request(pr, request, &plan);
+  rc = choose_requested(pr, request, &plan);
   if (rc != ST_OK) return rc;
-  const bool own_plan = request == nullptr || request->selection == VECOPS_HIP_SELECT_AUTOMATIC ||
-                        (request->selection == VECOPS_HIP_SELECT_PREFER && memcmp(&plan, &table, sizeof(plan)) == 0);
-  return run_problem(pr, plan, nullptr, nullptr, nullptr, workspace, workspace_size, static_cast<hipStream_t>(stream), own_plan);
+  return run_problem(pr, plan, nullptr, nullptr, nullptr, workspace, workspace_size, static_cast<hipStream_t>(stream));
 }
 
 int32_t vecops_hip_matmul(const VecopsHipOperand* a, const VecopsHipOperand* b, const VecopsHipOperand* c_in,
@@ -2141,18 +2171,24 @@ int32_t vecops_hip_matmul_planned(const VecopsHipOperand* a, const VecopsHipOper
     request.selection = VECOPS_HIP_SELECT_REQUIRE;
     request.family = plan->family;
     request.split_k = plan->split_k;
-    if (apply_request(pr, &request, &checked) != ST_OK)
+    bool table_choice = false;
+    if (apply_request(pr, &request, &checked, &table_choice) != ST_OK)
       return fail(ST_INVALID, "matmul_planned: the plan's family %s cannot serve these operands", family_name(plan->family));
     checked.family = plan->family;
     if (checked.split_k != plan->split_k)
       return fail(ST_INVALID, "matmul_planned: the plan splits K %u ways, these operands allow %u", plan->split_k, checked.split_k);
   }
-  // (a plan that the rule table makes itself may run on a slim tile, as the unplanned call does; one for a required family
-  // or split runs that)
-  VecopsHipPlan table;
-  choose(pr, &table);
-  const bool own_plan = table.family == checked.family && table.split_k == checked.split_k && table.peeled_columns == checked.peeled_columns;
-  return run_problem(pr, checked, nullptr, nullptr, nullptr, workspace, workspace_size, static_cast<hipStream_t>(stream), own_plan);
+  // a slim tile: one that there is, for operands it serves, in place of tiles that it may replace
+  if (plan->slim_tile != 0) {
+    const bool listed = std::any_of(std::begin(kSlimTiles), std::end(kSlimTiles),
+                                    [&](const auto& t) { return slim_code(t.bm, t.bn) == plan->slim_tile; });
+    if (!listed || (checked.family != VECOPS_HIP_FAMILY_TILE_64 && checked.family != VECOPS_HIP_FAMILY_TILE_128) ||
+        checked.peeled_columns != 0 || !slim_serves(pr, checked))
+      return fail(ST_INVALID, "matmul_planned: the plan's slim tile (%u x %u) cannot serve these operands", plan->slim_tile >> 8,
+                  plan->slim_tile & 255u);
+    checked.slim_tile = plan->slim_tile;
+  }
+  return run_problem(pr, checked, nullptr, nullptr, nullptr, workspace, workspace_size, static_cast<hipStream_t>(stream));
 }
 
 uint64_t vecops_hip_matmul_i8_dequant_workspace(int64_t m, int64_t n, int64_t k) {

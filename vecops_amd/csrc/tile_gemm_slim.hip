@@ -3,8 +3,8 @@
 //
 // What bounds it: the loads' way into LDS, (BM + BN) rows of K - a compute unit takes 137 bytes a ns of whole lines by
 // itself and 100 where all do, 70 of 16-byte aligned rows that start inside a line and 50 of others - and for weights that
-// no cache holds their way from memory.  So a tile is chosen by how many bytes the fullest unit fetches (slim_tile in
-// capi.hip).
+// no cache holds their way from memory.  So a tile is chosen by how many bytes the fullest unit fetches (take_slim_tile
+// in capi.hip).
 //   * Eight wavefronts split a stage's K in four and the tile's rows in two: a tile this narrow has too few fragments for
 //     eight wavefronts side by side, and a product of one K part needs no partial sums in memory and no second launch.
 //     The four sums meet in LDS at the end.
