@@ -87,10 +87,10 @@ typedef struct VecopsHipPlan {
   uint32_t vector_b;   /* 1 = 16-byte loads usable for B */
   uint16_t b_layout;   /* 0 = K contiguous, 1 = N contiguous, 2 = generic */
   uint16_t slim_tile;  /* 0: the family's own tiles, K split as split_k says.  Else 256 * rows + columns of the slim tile
-                          (32x16 to 128x64) that runs in their place, in one launch over the whole K: in the
-                          library's own plans, where tile_64 or tile_128 would leave the chip short of work.  family,
-                          split_k and workspace_bytes are then what runs with slim_tile set to 0, and a requested
-                          family always runs as named */
+                          (32x16 to 128x64) that runs in their place, in one launch over the whole K that uses no
+                          workspace (a call may bring none): in the library's own plans, where tile_64 or tile_128
+                          would leave the chip short of work.  family, split_k and workspace_bytes are then what runs
+                          with slim_tile set to 0, and a requested family always runs as named */
   uint32_t peeled_columns; /* > 0: the last so many columns of c are a second product with a plan of its own (few
                               tiles, K split), cut off so that the rest fills whole rounds of workgroups */
   uint64_t workspace_bytes;
@@ -132,7 +132,7 @@ VECOPS_HIP_EXPORT int32_t vecops_hip_plan_matmul(const VecopsHipOperand* a, cons
  * bf16, i32 or f64) and may alias c element for element.  K == 0 writes zeros or
  * C_in; zero M, N or batch writes nothing (ops/Matmul.h:41-43).  Operand
  * metadata is validated as planning/families/ArchitectureFamily.h:1590-1652
- * does.  `workspace` must hold vecops_hip_plan_matmul(...).workspace_bytes.
+ * does.  `workspace` must hold vecops_hip_plan_matmul(...).workspace_bytes (nothing where that plan names a slim tile).
  */
 VECOPS_HIP_EXPORT int32_t vecops_hip_matmul(const VecopsHipOperand* a, const VecopsHipOperand* b,
                                             const VecopsHipOperand* c_in, const VecopsHipOperand* c, uint32_t compute,

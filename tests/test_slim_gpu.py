@@ -197,3 +197,39 @@ def test_planned_calls_run_what_the_plan_names(device):
         capi.matmul_planned(a, b, c, plan)
     torch.cuda.synchronize()
     assert float(c.min()) == 7.0 and float(c.max()) == 7.0
+
+
+def test_no_workspace(device):
+    """128 x 11008 x 4096: the table's tiles would split K, the slim tile takes nothing - no workspace has to be handed in, and
+    the entry points allocate and hold none."""
+    import ctypes as C
+    import torch
+    from vecops_amd import capi
+    a, b = _operands(device, torch.bfloat16, 128, 11008, 4096)
+    c = torch.empty((128, 11008), device=device)
+    plan = capi.plan_matmul(a, b, c)
+    assert plan.split_k > 1 and plan.workspace_bytes == plan.split_k * 128 * 11008 * 4 and plan.slim_tile and plan.scratch_bytes == 0
+    want = capi.matmul(a, b, c).clone()
+    operands = [C.byref(o) if o is not None else None for o in (capi.operand(a), capi.operand(b), None, capi.operand(c))]
+    lib = capi.lib()
+    for call in (lambda: lib.vecops_hip_matmul(*operands, 0, None, 0, capi._stream_handle(None)),
+                 lambda: lib.vecops_hip_matmul_planned(*operands, 0, C.byref(plan), None, 0, capi._stream_handle(None)),
+                 lambda: lib.vecops_hip_matmul_static_workspace(*operands, 0, capi._stream_handle(None))):
+        c.fill_(float("nan"))
+        capi._check(call())
+        assert torch.equal(c, want)
+    plan.slim_tile = 0                   # the table's own tiles need theirs
+    assert lib.vecops_hip_matmul_planned(*operands, 0, C.byref(plan), None, 0, None) == 1
+    stream = torch.cuda.current_stream()
+    prepared = capi.PreparedMatmul(a, b, c)
+    ep = capi.epilogue(activation="relu")
+    for call in (lambda: capi.matmul(a, b, c), lambda: capi.matmul(a, b, c, stream=stream), prepared,
+                 lambda: capi.matmul_fused(a, b, c, ep), lambda: capi.matmul_fused(a, b, c, ep, stream=stream),
+                 lambda: capi.matmul_planned(a, b, c, capi.plan_matmul(a, b, c))):
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        call()
+        torch.cuda.synchronize()
+        assert torch.cuda.max_memory_allocated() == before
+    assert prepared._keep[4] is None

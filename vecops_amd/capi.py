@@ -53,6 +53,11 @@ class Plan(C.Structure):
                 ("b_layout", C.c_uint16), ("slim_tile", C.c_uint16), ("peeled_columns", C.c_uint32),
                 ("workspace_bytes", C.c_uint64)]
 
+    @property
+    def scratch_bytes(self) -> int:
+        """What a call by this plan uses of a workspace: ``workspace_bytes``, nothing where a slim tile runs."""
+        return 0 if self.slim_tile else int(self.workspace_bytes)
+
 
 class Epilogue(C.Structure):
     _fields_ = [("struct_size", C.c_uint32), ("activation", C.c_uint32), ("flags", C.c_uint32), ("scale", C.c_float),
@@ -243,9 +248,8 @@ def matmul(a, b, c, c_in=None, compute=COMPUTE_BF16, workspace=None, stream=None
             _check(rc)
     import torch
     plan = plan_matmul(a, b, c, c_in, compute)
-    if plan.workspace_bytes and (workspace is None or workspace.numel() * workspace.element_size()
-                                 < plan.workspace_bytes):
-        workspace = torch.empty(plan.workspace_bytes, dtype=torch.uint8, device=c.device)
+    if plan.scratch_bytes and (workspace is None or workspace.numel() * workspace.element_size() < plan.scratch_bytes):
+        workspace = torch.empty(plan.scratch_bytes, dtype=torch.uint8, device=c.device)
     oa, ob, oc = operand(a), operand(b), operand(c)
     oi = operand(c_in) if c_in is not None else None
     ws_ptr = workspace.data_ptr() if workspace is not None else None
@@ -259,8 +263,8 @@ def matmul_planned(a, b, c, plan: Plan, c_in=None, compute=COMPUTE_BF16, workspa
     """``matmul`` with a plan made beforehand (``plan_matmul`` / ``plan_matmul_family`` on operands of the same
     metadata): ``vecops_hip_matmul_planned``."""
     import torch
-    if plan.workspace_bytes and (workspace is None or workspace.numel() * workspace.element_size() < plan.workspace_bytes):
-        workspace = torch.empty(plan.workspace_bytes, dtype=torch.uint8, device=c.device)
+    if plan.scratch_bytes and (workspace is None or workspace.numel() * workspace.element_size() < plan.scratch_bytes):
+        workspace = torch.empty(plan.scratch_bytes, dtype=torch.uint8, device=c.device)
     oa, ob, oc = operand(a), operand(b), operand(c)
     oi = operand(c_in) if c_in is not None else None
     ws_ptr = workspace.data_ptr() if workspace is not None else None
@@ -279,7 +283,7 @@ class PreparedMatmul:
     def __init__(self, a, b, c, c_in=None, compute=COMPUTE_BF16, workspace=None, stream=None):
         import torch
         self.plan = plan_matmul(a, b, c, c_in, compute)
-        need = int(self.plan.workspace_bytes)
+        need = self.plan.scratch_bytes
         if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
             workspace = torch.empty(need, dtype=torch.uint8, device=c.device)
         self._keep = (a, b, c, c_in, workspace)
@@ -311,9 +315,8 @@ def matmul_family(a, b, c, request: FamilyRequest, c_in=None, compute=COMPUTE_BF
     """``matmul`` on the kernel family the caller prefers or requires (``family_request``)."""
     import torch
     plan = plan_matmul_family(a, b, c, request, c_in, compute)
-    if plan.workspace_bytes and (workspace is None or workspace.numel() * workspace.element_size()
-                                 < plan.workspace_bytes):
-        workspace = torch.empty(plan.workspace_bytes, dtype=torch.uint8, device=c.device)
+    if plan.scratch_bytes and (workspace is None or workspace.numel() * workspace.element_size() < plan.scratch_bytes):
+        workspace = torch.empty(plan.scratch_bytes, dtype=torch.uint8, device=c.device)
     oa, ob, oc = operand(a), operand(b), operand(c)
     oi = operand(c_in) if c_in is not None else None
     ws_ptr = workspace.data_ptr() if workspace is not None else None
@@ -384,9 +387,8 @@ def matmul_fused(a, b, c, ep: Epilogue, c_in=None, compute=COMPUTE_BF16, workspa
             _check(rc)
     import torch
     plan = plan_matmul_fused(a, b, c, ep, c_in, compute)
-    if plan.workspace_bytes and (workspace is None or workspace.numel() * workspace.element_size()
-                                 < plan.workspace_bytes):
-        workspace = torch.empty(plan.workspace_bytes, dtype=torch.uint8, device=c.device)
+    if plan.scratch_bytes and (workspace is None or workspace.numel() * workspace.element_size() < plan.scratch_bytes):
+        workspace = torch.empty(plan.scratch_bytes, dtype=torch.uint8, device=c.device)
     oa, ob, oc = operand(a), operand(b), operand(c)
     oi = operand(c_in) if c_in is not None else None
     ws_ptr = workspace.data_ptr() if workspace is not None else None
@@ -607,8 +609,8 @@ def matmul_packed_a(packed: PackedB, b, c, c_in=None, workspace=None, stream=Non
     oi = operand(c_in) if c_in is not None else None
     oi_ref = C.byref(oi) if oi is not None else None
     _check(lib().vecops_hip_plan_matmul_packed_a(packed.dtype, packed.n, C.byref(ob), oi_ref, C.byref(oc), C.byref(plan)))
-    if plan.workspace_bytes and (workspace is None or workspace.numel() * workspace.element_size() < plan.workspace_bytes):
-        workspace = torch.empty(plan.workspace_bytes, dtype=torch.uint8, device=c.device)
+    if plan.scratch_bytes and (workspace is None or workspace.numel() * workspace.element_size() < plan.scratch_bytes):
+        workspace = torch.empty(plan.scratch_bytes, dtype=torch.uint8, device=c.device)
     ws_ptr = workspace.data_ptr() if workspace is not None else None
     ws_size = workspace.numel() * workspace.element_size() if workspace is not None else 0
     _check(lib().vecops_hip_matmul_packed_a(packed.storage.data_ptr(), packed.dtype, packed.n, C.byref(ob), oi_ref,
@@ -655,9 +657,8 @@ def matmul_packed_b(a, packed: PackedB, c, c_in=None, workspace=None, stream=Non
             _check(rc)
     import torch
     plan = plan_matmul_packed_b(a, packed, c, c_in)
-    if plan.workspace_bytes and (workspace is None or workspace.numel() * workspace.element_size()
-                                 < plan.workspace_bytes):
-        workspace = torch.empty(plan.workspace_bytes, dtype=torch.uint8, device=c.device)
+    if plan.scratch_bytes and (workspace is None or workspace.numel() * workspace.element_size() < plan.scratch_bytes):
+        workspace = torch.empty(plan.scratch_bytes, dtype=torch.uint8, device=c.device)
     oa, oc = operand(a), operand(c)
     oi = operand(c_in) if c_in is not None else None
     ws_ptr = workspace.data_ptr() if workspace is not None else None

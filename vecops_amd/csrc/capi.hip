@@ -999,7 +999,7 @@ int32_t run_problem(const Problem& pr, const VecopsHipPlan& plan, const float* r
   if (pr.b.data == nullptr && pr.k > 0) return fail(ST_INVALID, "matmul: b has no storage");
   if (pr.packed_b && plan.family == VECOPS_HIP_FAMILY_SKINNY) return fail(ST_INVALID, "matmul: plan does not fit a packed b");
   if (pr.c.data == nullptr) return fail(ST_INVALID, "matmul: c has no storage");
-  if (plan.workspace_bytes > workspace_size || (plan.workspace_bytes > 0 && workspace == nullptr))
+  if (plan.slim_tile == 0 && (plan.workspace_bytes > workspace_size || (plan.workspace_bytes > 0 && workspace == nullptr)))
     return fail(ST_INVALID, "matmul: workspace of %llu bytes required, %llu supplied",
                 (unsigned long long)plan.workspace_bytes, (unsigned long long)workspace_size);
 
@@ -2091,7 +2091,7 @@ int32_t vecops_hip_matmul_static_workspace(const VecopsHipOperand* a, const Veco
     finish_tile_plan(pr, &plan, plan.split_k / 2);
     take_slim_tile(pr, &plan);  // (ahead of fewer parts, perhaps)
   }
-  if (plan.slim_tile != 0) plan.workspace_bytes = 0;  // (it uses none)
+  if (plan.slim_tile != 0) plan.workspace_bytes = 0;
   if (plan.workspace_bytes > VECOPS_HIP_STATIC_WORKSPACE_BYTES)
     return fail(ST_NOT_APPLICABLE, "matmul_static_workspace: the call needs %llu bytes of scratch, the library holds %llu",
                 (unsigned long long)plan.workspace_bytes, (unsigned long long)VECOPS_HIP_STATIC_WORKSPACE_BYTES);

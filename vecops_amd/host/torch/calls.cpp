@@ -130,7 +130,7 @@ int product(PyObject* const* args, uint64_t epilogue_address) {
   VecopsHipPlan plan;
   int32_t rc = epilogue ? vecops_hip_plan_matmul_fused(&a, &b, ci, &c, how, epilogue, &plan) : vecops_hip_plan_matmul(&a, &b, ci, &c, how, &plan);
   if (rc != 0) return rc;
-  const Workspace workspace(args[5], plan.workspace_bytes, *out);
+  const Workspace workspace(args[5], plan.slim_tile != 0 ? 0 : plan.workspace_bytes, *out);
   if (!workspace.usable) return kNotPlain;
   return epilogue ? vecops_hip_matmul_fused(&a, &b, ci, &c, how, epilogue, workspace.data, workspace.size, current_stream())
                   : vecops_hip_matmul(&a, &b, ci, &c, how, workspace.data, workspace.size, current_stream());
