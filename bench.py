@@ -100,7 +100,16 @@ def _kernel_label(plan, operands):
     split = f", split-K {plan.split_k}" if plan.split_k > 1 else ""
     wide = "tile_gemm_wide_i8_kernel" if operands.startswith("int8") else f"tile_gemm_wide_16_kernel<{operands}>"
     kernel = wide if family == "tile_256x352" else f"tile_gemm_kernel<{operands}>"
+    if plan.slim_tile:      # runs in place of the family's tiles, K whole
+        return f"vecops_hip tile_gemm_slim_kernel<{operands}, {plan.slim_tile >> 8}, {plan.slim_tile & 255}>, {loads}, {b}"
     return f"vecops_hip {kernel} family {family}, {loads}, {b}{split}"
+
+
+def _plan_label(plan):
+    from vecops_amd import capi
+    if plan.slim_tile:
+        return f"slim_{plan.slim_tile >> 8}x{plan.slim_tile & 255}"
+    return capi.FAMILY_NAMES.get(plan.family, str(plan.family)) + f"/{max(plan.split_k, 1)}"
 
 
 def _roofline(bound, achieved, peak, unit, **extra):
@@ -579,8 +588,7 @@ def bench_rule_check(dev, steps, warmup):
                     continue   # the family cannot serve this problem
                 tried[f"{family}/{split}"] = round(t["event_ms"] * 1e3, 2)
         best = min(tried, key=tried.get)
-        pick = capi.FAMILY_NAMES.get(plan.family, str(plan.family)) + f"/{max(plan.split_k, 1)}" + (
-            f" (+{plan.peeled_columns} peeled columns)" if plan.peeled_columns else "")
+        pick = _plan_label(plan) + (f" (+{plan.peeled_columns} peeled columns)" if plan.peeled_columns else "")
         rows.append({"shape": f"{kind} {m}x{n}x{k}", "pick": pick, "pick_us": round(auto, 2), "best": best,
                      "best_us": tried[best], "regret_us": round(auto - tried[best], 2), "tried_us": tried})
     worst = max(rows, key=lambda r: r["regret_us"])
@@ -633,16 +641,14 @@ def bench_vendor_grid(dev, steps, warmup):
             run = capi.PreparedMatmul(a, ours_b, c, workspace=ws)
             row[f"bf16_{layout}"] = {"ours_us": time_us(lambda: run(), hint),
                                      "vendor_us": time_us(lambda: torch.matmul(a, theirs_b, out=c), hint),
-                                     "plan": capi.FAMILY_NAMES.get(plan.family, str(plan.family)) + f"/{max(plan.split_k, 1)}" +
-                                             ("+peel" if plan.peeled_columns else "")}
+                                     "plan": _plan_label(plan) + ("+peel" if plan.peeled_columns else "")}
         ai = torch.from_numpy(synth.int8_sym(1, (m, k))).to(dev)
         bi = torch.from_numpy(synth.int8_sym(2, (n, k))).to(dev)
         ci = torch.empty((m, n), dtype=torch.int32, device=dev)
         plan = capi.plan_matmul(ai, bi, ci)
         run = capi.PreparedMatmul(ai, bi, ci, workspace=ws)
         entry = {"ours_us": time_us(lambda: run(), hint / 2),
-                 "plan": capi.FAMILY_NAMES.get(plan.family, str(plan.family)) + f"/{max(plan.split_k, 1)}" +
-                         ("+peel" if plan.peeled_columns else "")}
+                 "plan": _plan_label(plan) + ("+peel" if plan.peeled_columns else "")}
         try:
             entry["vendor_us"] = time_us(lambda: torch._int_mm(ai, bi.t(), out=ci), hint / 2)
         except RuntimeError:

@@ -39,3 +39,14 @@ def test_every_workload_of_only_is_dispatched():
     for name in bench.ONLY:
         assert f'"{name}": lambda' in source or name == "bf16", name
     assert len(bench.RULE_CHECK_SHAPES) >= 27 and len(bench.VENDOR_GRID) >= 27
+
+
+def test_labels_name_the_slim_tile():
+    from vecops_amd import capi
+    from test_capi_cpu import _operand, _plan
+    bench = _bench()
+    rc, plan = _plan(_operand(capi.BF16, (128, 4096)), _operand(capi.BF16, (11008, 4096)), _operand(capi.BF16, (128, 11008)))
+    assert rc == 0 and bench._kernel_label(plan, "bf16") == "vecops_hip tile_gemm_slim_kernel<bf16, 128, 48>, 16-byte loads, B K-contiguous"
+    assert bench._plan_label(plan) == "slim_128x48"
+    plan.slim_tile = 0
+    assert "family tile_128" in bench._kernel_label(plan, "bf16") and bench._plan_label(plan) == "tile_128/2"
