@@ -122,3 +122,72 @@ def test_registered_operator_forms(device):
     fused(a, b, None, None, None, 1, 0.5, 0.25, 0.0, 0.0, c)
     # (the same entry of the library: a product without a transform takes another kernel at these extents)
     assert torch.equal(c, capi.matmul_fused(a, b, torch.empty_like(c), capi.epilogue(activation="relu", scale=0.5, shift=0.25)))
+
+
+@pytest.mark.gpu
+def test_the_interpreter_lock_is_given_up_during_a_call(device):
+    """With threads switched only where one gives up the lock, another thread gets to run while this one does nothing but
+    calls."""
+    import sys
+    import threading
+    a, b, c = _bf16(device, 33, 512), _bf16(device, 260, 512), torch.empty(33, 260, device=device)
+    scales = torch.rand(33, device=device), torch.rand(260, device=device)
+    ia, ib = (torch.randint(-9, 9, (r, 512), device=device, dtype=torch.int8) for r in (33, 260))
+    ep, packed, x = capi.epilogue(activation="relu"), capi.pack_b(b), torch.randn(33, 512, device=device)
+    ipacked, w_scales, y = capi.pack_b(ib), torch.rand(260, 4, device=device), _bf16(device, 5, 260)
+    calls = [lambda: capi.matmul(a, b, c), lambda: capi.matmul_fused(a, b, c, ep), lambda: capi.matmul_packed_b(a, packed, c),
+             lambda: capi.matmul_i8_dequant(ia, ib, *scales, c), lambda: capi.matmul_w8a16_group(a[:5], ib, w_scales, y, 128),
+             lambda: capi.matmul_runtime_quant(x, scales[0], 128, ib, *scales, c),
+             lambda: capi.matmul_runtime_quant_packed_b(x, scales[0], 128, ipacked, *scales, c)]
+    interval = sys.getswitchinterval()
+    for call in calls:
+        call()
+        torch.cuda.synchronize()
+        go, ran = threading.Lock(), []
+        go.acquire()
+        thread = threading.Thread(target=lambda: (go.acquire(), ran.append(1)))  # noqa: B023
+        thread.start()
+        sys.setswitchinterval(1000.0)
+        try:
+            go.release()         # the thread may run from here on, once this one gives up the interpreter lock
+            for _ in range(5000):
+                if ran:
+                    break
+                call()
+            done = bool(ran)
+        finally:
+            sys.setswitchinterval(interval)
+        thread.join(60)
+        torch.cuda.synchronize()
+        assert done
+
+
+@pytest.mark.gpu
+def test_calls_from_several_threads(device):
+    """Each thread on a stream of its own, products that allocate a workspace among them."""
+    import threading
+    shapes = [(255, 63, 8191), (128, 11008, 512), (33, 260, 1000), (700, 900, 264)]
+    operands = [(_bf16(device, m, k), _bf16(device, n, k)) for m, n, k in shapes]
+    want = [capi.matmul(a, b, torch.empty(a.shape[0], b.shape[0], device=device)) for a, b in operands]
+    torch.cuda.synchronize()
+    results, errors = {}, []
+
+    def work(index):
+        try:
+            stream = torch.cuda.Stream()
+            with torch.cuda.stream(stream):
+                for turn in range(20):
+                    i = (index + turn) % len(shapes)
+                    a, b = operands[i]
+                    results[index, turn] = i, capi.matmul(a, b, torch.full_like(want[i], float("nan")))
+            stream.synchronize()
+        except Exception as e:  # noqa: BLE001
+            errors.append(e)
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    torch.cuda.synchronize()
+    assert not errors and len(results) == 80
+    assert all(torch.equal(got, want[i]) for i, got in results.values())

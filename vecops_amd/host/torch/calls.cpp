@@ -82,27 +82,46 @@ bool describe(PyObject* object, VecopsHipOperand* o) {
 
 void* current_stream() { return c10::hip::getCurrentHIPStream().stream(); }
 
+// The workspace a caller hands in, and the device of the output, where another one is allocated.
+struct Given {
+  void* data = nullptr;
+  uint64_t size = 0;
+  c10::Device device{c10::DeviceType::CPU};
+  bool describe(PyObject* given, const at::Tensor& output) {
+    device = output.device();
+    if (given == Py_None) return true;
+    const at::Tensor* t = plain_tensor(given);
+    if (t == nullptr) return false;
+    data = t->data_ptr();
+    size = static_cast<uint64_t>(t->numel()) * t->element_size();
+    return true;
+  }
+};
+
 // The caller's workspace if it is large enough, else one from torch's allocator, which lives as long as this object: its
 // reuse is ordered on the current stream, where the work goes.
 struct Workspace {
   at::Tensor own;
-  void* data = nullptr;
-  uint64_t size = 0;
-  bool usable = true;
-  Workspace(PyObject* given, uint64_t need, const at::Tensor& beside) {
-    if (given != Py_None) {
-      const at::Tensor* t = plain_tensor(given);
-      if (t == nullptr) { usable = false; return; }
-      data = t->data_ptr();
-      size = static_cast<uint64_t>(t->numel()) * t->element_size();
-    }
+  void* data;
+  uint64_t size;
+  Workspace(const Given& given, uint64_t need) : data(given.data), size(given.size) {
     if (need > 0 && (data == nullptr || size < need)) {
-      own = at::empty({static_cast<int64_t>(need)}, at::TensorOptions().dtype(at::kByte).device(beside.device()));
+      own = at::empty({static_cast<int64_t>(need)}, at::TensorOptions().dtype(at::kByte).device(given.device));
       data = own.data_ptr();
       size = need;
     }
   }
 };
+
+// The library's part of a call, without the interpreter lock: a launch may wait for room in the queue or load code, the
+// allocator may synchronise, and other threads' calls and host callbacks that need the lock must not wait for that (the lock
+// is given back and taken again in about 0.1 us).  Whatever it needs of the Python objects has been read before; they live
+// as long as the caller's references.
+template <class Call>
+int without_lock(Call&& call) {
+  const pybind11::gil_scoped_release released;
+  return call();
+}
 
 // An int argument that fits 64 bits; false (and no error set) otherwise.
 bool integer(PyObject* object, int64_t* out) {
@@ -125,15 +144,18 @@ int product(PyObject* const* args, uint64_t epilogue_address) {
     if (!describe(args[3], &cin)) return kNotPlain;
     ci = &cin;
   }
+  Given given;
+  if (!given.describe(args[5], *out)) return kNotPlain;
   const auto* epilogue = reinterpret_cast<const VecopsHipEpilogue*>(epilogue_address);
   const uint32_t how = static_cast<uint32_t>(compute);
-  VecopsHipPlan plan;
-  int32_t rc = epilogue ? vecops_hip_plan_matmul_fused(&a, &b, ci, &c, how, epilogue, &plan) : vecops_hip_plan_matmul(&a, &b, ci, &c, how, &plan);
-  if (rc != 0) return rc;
-  const Workspace workspace(args[5], plan.slim_tile != 0 ? 0 : plan.workspace_bytes, *out);
-  if (!workspace.usable) return kNotPlain;
-  return epilogue ? vecops_hip_matmul_fused(&a, &b, ci, &c, how, epilogue, workspace.data, workspace.size, current_stream())
-                  : vecops_hip_matmul(&a, &b, ci, &c, how, workspace.data, workspace.size, current_stream());
+  return without_lock([&]() -> int {
+    VecopsHipPlan plan;
+    int32_t rc = epilogue ? vecops_hip_plan_matmul_fused(&a, &b, ci, &c, how, epilogue, &plan) : vecops_hip_plan_matmul(&a, &b, ci, &c, how, &plan);
+    if (rc != 0) return rc;
+    const Workspace workspace(given, plan.slim_tile != 0 ? 0 : plan.workspace_bytes);
+    return epilogue ? vecops_hip_matmul_fused(&a, &b, ci, &c, how, epilogue, workspace.data, workspace.size, current_stream())
+                    : vecops_hip_matmul(&a, &b, ci, &c, how, workspace.data, workspace.size, current_stream());
+  });
 }
 
 int matmul(PyObject* const* args) { return product(args, 0); }
@@ -157,9 +179,12 @@ int matmul_w8a16_group(PyObject* const* args) {
   int64_t group = 0;
   if (x == nullptr || w == nullptr || scales == nullptr || y == nullptr || !scales->is_contiguous() || !integer(args[4], &group))
     return kNotPlain;
-  return vecops_hip_matmul_w8a16_group(x->data_ptr(), x->stride(0), static_cast<const int8_t*>(w->data_ptr()), w->stride(0),
-                                       static_cast<const float*>(scales->data_ptr()), y->data_ptr(), y->stride(0), x->size(0),
-                                       w->size(0), x->size(1), group, current_stream());
+  const void* xv = x->data_ptr();
+  const auto* wv = static_cast<const int8_t*>(w->data_ptr());
+  const auto* sv = static_cast<const float*>(scales->data_ptr());
+  void* yv = y->data_ptr();
+  const int64_t ldx = x->stride(0), ldw = w->stride(0), ldy = y->stride(0), m = x->size(0), n = w->size(0), k = x->size(1);
+  return without_lock([&] { return vecops_hip_matmul_w8a16_group(xv, ldx, wv, ldw, sv, yv, ldy, m, n, k, group, current_stream()); });
 }
 
 // matmul_i8_dequant(a, b or the packed storage, row_scales, column_scales, c, correction, workspace, n or -1): n < 0 says
@@ -172,18 +197,22 @@ int matmul_i8_dequant(PyObject* const* args) {
                    *columns = plain_tensor(args[3]), *c = matrix(args[4]), *correction = nullptr;
   if (a == nullptr || b == nullptr || rows == nullptr || columns == nullptr || c == nullptr) return kNotPlain;
   if (args[5] != Py_None && (correction = plain_tensor(args[5])) == nullptr) return kNotPlain;
-  const int64_t m = a->size(0), k = a->size(1);
+  const int64_t m = a->size(0), k = a->size(1), lda = a->stride(0), ldb = packed ? 0 : b->stride(0), ldc = c->stride(0);
   if (!packed) n = b->size(0);
-  const Workspace workspace(args[6], vecops_hip_matmul_i8_dequant_workspace(m, n, k), *c);
-  if (!workspace.usable) return kNotPlain;
+  Given given;
+  if (!given.describe(args[6], *c)) return kNotPlain;
   const auto* av = static_cast<const int8_t*>(a->data_ptr());
+  const void* bv = b->data_ptr();
   const auto *rv = static_cast<const float*>(rows->data_ptr()), *cv = static_cast<const float*>(columns->data_ptr());
   const auto* corr = correction ? static_cast<const int32_t*>(correction->data_ptr()) : nullptr;
   float* out = static_cast<float*>(c->data_ptr());
-  return packed ? vecops_hip_matmul_i8_dequant_packed_b(av, a->stride(0), b->data_ptr(), rv, cv, corr, out, c->stride(0), m, n, k,
-                                                        workspace.data, workspace.size, current_stream())
-                : vecops_hip_matmul_i8_dequant(av, a->stride(0), static_cast<const int8_t*>(b->data_ptr()), b->stride(0), rv, cv,
-                                               corr, out, c->stride(0), m, n, k, workspace.data, workspace.size, current_stream());
+  return without_lock([&]() -> int {
+    const Workspace workspace(given, vecops_hip_matmul_i8_dequant_workspace(m, n, k));
+    return packed ? vecops_hip_matmul_i8_dequant_packed_b(av, lda, bv, rv, cv, corr, out, ldc, m, n, k, workspace.data,
+                                                          workspace.size, current_stream())
+                  : vecops_hip_matmul_i8_dequant(av, lda, static_cast<const int8_t*>(bv), ldb, rv, cv, corr, out, ldc, m, n, k,
+                                                 workspace.data, workspace.size, current_stream());
+  });
 }
 
 // matmul_runtime_quant(a, multipliers, zero_point, b or the packed storage, row_scales, column_scales, c, correction,
@@ -199,16 +228,20 @@ int matmul_runtime_quant(PyObject* const* args) {
       !describe(args[0], &a) || !describe(*out, &c) || (!packed && !describe(*storage, &b)))
     return kNotPlain;
   if (args[7] != Py_None && (correction = plain_tensor(args[7])) == nullptr) return kNotPlain;
-  const Workspace workspace(args[8], packed ? vecops_hip_matmul_runtime_quant_packed_b_workspace(&a, n, &c)
-                                            : vecops_hip_matmul_runtime_quant_workspace(&a, &b, &c), *out);
-  if (!workspace.usable) return kNotPlain;
+  Given given;
+  if (!given.describe(args[8], *out)) return kNotPlain;
   const auto *mv = static_cast<const float*>(multipliers->data_ptr()), *rv = static_cast<const float*>(rows->data_ptr()),
              *cv = static_cast<const float*>(columns->data_ptr());
   const auto* corr = correction ? static_cast<const int32_t*>(correction->data_ptr()) : nullptr;
   const int32_t zp = static_cast<int32_t>(zero_point);
-  return packed ? vecops_hip_matmul_runtime_quant_packed_b(&a, mv, zp, storage->data_ptr(), n, corr, rv, cv, &c, workspace.data,
-                                                           workspace.size, current_stream())
-                : vecops_hip_matmul_runtime_quant(&a, mv, zp, &b, corr, rv, cv, &c, workspace.data, workspace.size, current_stream());
+  const void* weights = storage->data_ptr();
+  return without_lock([&]() -> int {
+    const Workspace workspace(given, packed ? vecops_hip_matmul_runtime_quant_packed_b_workspace(&a, n, &c)
+                                            : vecops_hip_matmul_runtime_quant_workspace(&a, &b, &c));
+    return packed ? vecops_hip_matmul_runtime_quant_packed_b(&a, mv, zp, weights, n, corr, rv, cv, &c, workspace.data,
+                                                             workspace.size, current_stream())
+                  : vecops_hip_matmul_runtime_quant(&a, mv, zp, &b, corr, rv, cv, &c, workspace.data, workspace.size, current_stream());
+  });
 }
 
 // matmul_packed_b(a, storage, c, c_in, dtype, workspace, n)
@@ -224,13 +257,17 @@ int matmul_packed_b(PyObject* const* args) {
     if (!describe(args[3], &cin)) return kNotPlain;
     ci = &cin;
   }
-  VecopsHipPlan plan;
-  int32_t rc = vecops_hip_plan_matmul_packed_b(&a, static_cast<uint32_t>(dtype), n, ci, &c, &plan);
-  if (rc != 0) return rc;
-  const Workspace workspace(args[5], plan.workspace_bytes, *out);
-  if (!workspace.usable) return kNotPlain;
-  return vecops_hip_matmul_packed_b(&a, storage->data_ptr(), static_cast<uint32_t>(dtype), n, ci, &c, workspace.data, workspace.size,
-                                    current_stream());
+  Given given;
+  if (!given.describe(args[5], *out)) return kNotPlain;
+  const void* packed = storage->data_ptr();
+  return without_lock([&]() -> int {
+    VecopsHipPlan plan;
+    int32_t rc = vecops_hip_plan_matmul_packed_b(&a, static_cast<uint32_t>(dtype), n, ci, &c, &plan);
+    if (rc != 0) return rc;
+    const Workspace workspace(given, plan.workspace_bytes);
+    return vecops_hip_matmul_packed_b(&a, packed, static_cast<uint32_t>(dtype), n, ci, &c, workspace.data, workspace.size,
+                                      current_stream());
+  });
 }
 
 // A Python function of COUNT positional arguments around one of the above: no C++ exception leaves it.
