@@ -191,3 +191,31 @@ def test_calls_from_several_threads(device):
     torch.cuda.synchronize()
     assert not errors and len(results) == 80
     assert all(torch.equal(got, want[i]) for i, got in results.values())
+
+
+def test_without_the_extension(monkeypatch):
+    """Not built (no torch headers where the library was made): a warning, and every call takes the Python form; operators are
+    registered as before."""
+    monkeypatch.setattr(capi, "CALLS_PATH", capi.CALLS_PATH + ".missing")
+    monkeypatch.setattr(capi, "_calls", None)
+    with pytest.warns(RuntimeWarning, match="missing"):
+        calls = capi.native_calls()
+    a, b, c = torch.zeros(4, 8), torch.zeros(5, 8), torch.zeros(4, 5)
+    assert calls.matmul(a, b, c, None, 0, None) == -1 and calls.matmul_w8a16_group(a, b, a, c, 8) == -1
+    assert capi.native_calls() is calls           # (one warning)
+    tb.register("vecops_hip_no_extension::matmul")
+    for key in ("CUDA", "CPU", "Meta"):
+        assert torch._C._dispatch_has_kernel_for_dispatch_key("vecops_hip_no_extension::matmul", key)
+
+
+@pytest.mark.gpu
+def test_products_without_the_extension(device, monkeypatch):
+    a, b = _bf16(device, 5, 4096), _bf16(device, 520, 4096)
+    want = capi.matmul(a, b, torch.empty(5, 520, device=device))
+    monkeypatch.setattr(capi, "CALLS_PATH", capi.CALLS_PATH + ".missing")
+    monkeypatch.setattr(capi, "_calls", None)
+    with pytest.warns(RuntimeWarning, match="missing"):
+        assert torch.equal(capi.matmul(a, b, torch.empty_like(want)), want)
+    plain = tb.register("vecops_hip_no_extension_g::matmul")
+    c = torch.empty_like(want)
+    assert plain(a, b, None, c) is c and torch.equal(c, want)

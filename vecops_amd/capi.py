@@ -175,6 +175,15 @@ CALLS_PATH = os.path.join(HERE, "lib", "vecops_torch_calls.so")
 _calls = None
 
 
+class _NoNativeCalls:
+    """In the module's place where it has not been built (it needs torch's C++ headers): leaves every call to the Python form."""
+
+    register_device_kernel = None
+
+    def __getattr__(self, name):
+        return lambda *args: -1
+
+
 def native_calls():
     """The per-call work of the functions below in native code (``host/torch/calls.cpp``): each of its functions answers
     with the library's status, or with -1 for a call it leaves to the Python form (tensors that are not plain device
@@ -183,9 +192,13 @@ def native_calls():
     if _calls is None:
         import importlib.util
         import torch  # noqa: F401  (the module links torch's libraries)
-        if not os.path.exists(CALLS_PATH):
-            raise RuntimeError(f"{CALLS_PATH} is missing: build it with vecops_amd.build.build_all()")
         lib()
+        if not os.path.exists(CALLS_PATH):
+            import warnings
+            warnings.warn(f"{CALLS_PATH} is missing: calls run the same kernels from Python, which costs several microseconds "
+                          "of host time each; build it with vecops_amd.build.build_all()", RuntimeWarning, stacklevel=3)
+            _calls = _NoNativeCalls()
+            return _calls
         spec = importlib.util.spec_from_file_location("vecops_torch_calls", CALLS_PATH)
         module = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(module)

@@ -167,10 +167,14 @@ class _Registration:
             return tuple(args[i] for i in outputs) if return_outputs else None
 
         # device tensors: native code from the dispatcher to the bridge entry, which hands calls it does not serve (host
-        # tensors among them, types outside the table) to ``invoke``
-        capi.native_calls().register_device_kernel(
-            self.library, self.name, self.operator.bridge_handle(), *self.operator.native_entries(),
-            [kind for _, kind in self.params], list(self.specs.items()), return_outputs, self.invoke, H.HostError)
+        # tensors among them, types outside the table) to ``invoke``; ``invoke`` itself where that code is not built
+        register_device_kernel = capi.native_calls().register_device_kernel
+        if register_device_kernel is not None:
+            register_device_kernel(
+                self.library, self.name, self.operator.bridge_handle(), *self.operator.native_entries(),
+                [kind for _, kind in self.params], list(self.specs.items()), return_outputs, self.invoke, H.HostError)
+        else:
+            lib.impl(self.name, self.invoke, "CUDA")
         lib.impl(self.name, self.invoke, "CPU")
         lib.impl(self.name, meta, "Meta")
         self._library = lib                                         # keeps the definitions alive
