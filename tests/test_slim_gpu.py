@@ -1,8 +1,9 @@
 """The slim tiles (tile_gemm_slim.hip): what the library runs in place of the rule table's own 64x64 or 128x128 tiles where
 few of them, or many K tiles for each, leave the chip waiting.  Each tile at the edges of its rows, columns and K - single
 elements past a tile, K shorter than a chunk, one K tile, a partial tile behind any number of whole ones, rings that wrap -
-with rows at any alignment, C inputs, output types, scales and transforms.  The forms are checked by their results, which
-differ in the last bits from the tile kernels' (K in four parts): a form that no longer takes a slim tile fails here."""
+with rows at any alignment, C inputs, output types, scales and transforms.  Results alone do not tell which kernel ran:
+test_slim_plan_cpu.py pins the tile of every entry of SHAPES, the tests below that need one ask the plan for it, and those
+that set `slim_tile` themselves run what they name."""
 import numpy as np
 import pytest
 
@@ -19,10 +20,13 @@ SHAPES = {
     "32x64": [(31, 14336, 640), (17, 12743, 512), (2, 14529, 769)],
     "64x48": [(33, 8209, 2560), (65, 5678, 1536), (129, 3338, 1344), (33, 8880, 2049), (100, 4224, 4672)],
     "64x64": [(127, 8001, 1023), (64, 14336, 768), (65, 7553, 1472), (65, 7754, 1217)],
-    "128x48": [(128, 11008, 4096), (129, 6083, 512), (65, 11787, 641), (513, 2401, 960)],
-    "128x64": [(128, 14336, 2048), (129, 8170, 239), (257, 5377, 190), (65, 13433, 512)],
+    "128x48": [(128, 11008, 4096), (149, 6050, 640), (68, 12193, 512)],
+    "128x64": [(128, 14336, 2048), (196, 7813, 904), (195, 8117, 961), (65, 16255, 1023)],
+    # beside them, where the table's own tiles are ahead
+    "none": [(129, 6083, 512), (65, 11787, 641), (513, 2401, 960), (129, 8170, 239), (257, 5377, 190), (65, 13433, 512)],
 }
 ALL = [s for shapes in SHAPES.values() for s in shapes]
+TILES = [(32, 16), (32, 32), (32, 48), (32, 64), (64, 48), (64, 64), (128, 48), (128, 64)]
 
 
 def _operands(device, dtype, m, n, k, seed=1, batch=(), pad=0):
@@ -233,3 +237,10 @@ def test_no_workspace(device):
         torch.cuda.synchronize()
         assert torch.cuda.max_memory_allocated() == before
     assert prepared._keep[4] is None
+
+
+# (m, n, k) on which the library's own plan takes each tile, for int8
+INT8 = {(32, 16): (45, 16, 511), (32, 32): (35, 2081, 648), (32, 48): (33, 4418, 1025), (32, 64): (33, 6146, 1800),
+        (64, 48): (65, 5442, 2624), (64, 64): (65, 8002, 1937), (128, 48): (132, 6095, 1408), (128, 64): (68, 16319, 1921)}
+BF16 = {(32, 16): (47, 15, 193), (32, 32): (38, 2162, 321), (32, 48): (34, 4162, 513), (32, 64): (34, 6239, 897),
+        (64, 48): (67, 5441, 1248), (64, 64): (65, 8159, 913), (128, 48): (149, 6050, 640), (128, 64): (195, 8117, 961)}

@@ -4,7 +4,10 @@ import ctypes as C
 
 from vecops_amd import capi
 
+import pytest
+
 from test_capi_cpu import _operand, _plan, _plan_family
+from test_slim_gpu import BF16, INT8, SHAPES
 
 
 def _product(dtype, m, n, k, out):
@@ -34,3 +37,37 @@ def test_own_plans_name_the_slim_tile_and_requested_families_do_not():
 
 def test_the_plan_record_kept_its_size():
     assert C.sizeof(capi.Plan) == 32 and capi.Plan.peeled_columns.offset == 20
+
+
+@pytest.mark.parametrize("tile", list(SHAPES))
+def test_the_tile_of_every_shape(tile):
+    want = 0 if tile == "none" else 256 * int(tile.split("x")[0]) + int(tile.split("x")[1])
+    for m, n, k in SHAPES[tile]:
+        for dtype in (capi.BF16, capi.F16):
+            for out in (dtype, capi.F32):        # (the result's type does not enter)
+                rc, p = _plan(*_product(dtype, m, n, k, out))
+                assert rc == 0 and p.slim_tile == want, (m, n, k, hex(p.slim_tile))
+    for (bm, bn), (m, n, k) in BF16.items():
+        assert _plan(*_product(capi.BF16, m, n, k, capi.F32))[1].slim_tile == 256 * bm + bn
+    for (bm, bn), (m, n, k) in INT8.items():
+        assert _plan(*_product(capi.I8, m, n, k, capi.I32))[1].slim_tile == 256 * bm + bn
+
+
+def test_one_round_and_what_it_replaces():
+    """More than one workgroup a compute unit: never (a second round's start and the first one's stores lie between).  128x128
+    tiles only in place of the four-stage kernel, whose short K is its own (4384 x 384 x 512: 7.4 us there, 9.0 on a slim tile)."""
+    for (m, n, k), dtype in (((4384, 384, 512), capi.BF16), ((736, 2048, 512), capi.BF16), ((2797, 608, 568), capi.BF16),
+                             ((5888, 512, 1000), capi.BF16), ((736, 3040, 6464), capi.I8), ((1152, 2040, 2080), capi.BF16),
+                             ((256, 7808, 397), capi.BF16)):
+        rc, p = _plan(*_product(dtype, m, n, k, capi.I32 if dtype == capi.I8 else capi.F32))
+        assert rc == 0 and p.slim_tile == 0, (m, n, k, hex(p.slim_tile))
+    batch, m, n, k = 13, 1, 3776, 1340
+    rc, p = _plan(_operand(capi.BF16, (batch, m, k)), _operand(capi.BF16, (batch, n, k)), _operand(capi.F32, (batch, m, n)))
+    assert rc == 0 and p.slim_tile == 0
+    # level or ahead where the vendor grid's and the table's own examples lie
+    for (m, n, k), dtype in (((512, 4096, 4096), capi.BF16), ((1024, 2048, 4096), capi.BF16), ((512, 4096, 4096), capi.I8),
+                             ((1024, 2048, 4096), capi.I8)):
+        rc, p = _plan(*_product(dtype, m, n, k, capi.I32 if dtype == capi.I8 else capi.BF16))
+        assert rc == 0 and p.slim_tile == 256 * 128 + 64, (m, n, k)
+    rc, p = _plan(*_product(capi.I8, 512, 4096, 11008, capi.I32))      # level: 37.4 us in two parts, 37.8 on a slim tile
+    assert rc == 0 and p.slim_tile == 0 and p.split_k == 2

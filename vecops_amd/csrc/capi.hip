@@ -311,17 +311,22 @@ struct RuleConstants {
   //    batch 8 of 3000 x 3000 x 17 to fp32 54 us against 69, to bf16 42 against 53; 8192 x 8192 x 32 43 against 57; with
   //    a second step along K - its loads are not overlapped - the two-stage kernel is ahead, 65 against 71 us at K = 64)
   int64_t short_k_direct_max_k = 32;
-  // -- the slim tiles (tile_gemm_slim.hip) in place of the table's own plan of 64x64 or 128x128 tiles: both sides in ns, the
-  //    constants fitted to 617 products of 16-bit operands (17 <= M <= 1024, 256 <= N, K <= 14336, half of them with rows at
-  //    any alignment; the mean of weights in a cache and not), the slim side to have a margin of 5 %: of the 617 calls 320 take
-  //    a slim tile, on average 0.75 of the time they took, the worst 1.1 (`tests/test_slim_gpu.py` names the forms).
-  //    slim: a launch, and for every round of workgroups its start and end and (BM + BN) rows of K at slim_bytes_per_ns;
-  //    own: a launch, K tiles of a part at own_*_tile_ns or, with more workgroups, own_*_ns_per_wg of a unit's each (rows
-  //    that are not 16-byte aligned: times own_*_staged per mille), a K split's second launch and its partial sums' way.
-  int64_t slim_launch_ns = 2000, slim_round_ns = 2000, slim_row_ns = 10, slim_bytes_per_ns = 65, slim_bytes_per_ns_unaligned = 40;
+  // -- the slim tiles (tile_gemm_slim.hip) in place of the table's own plan of 64x64 tiles, or of 128x128 tiles on the
+  //    four-stage kernel: both sides in ns, the mean of operands in a cache and not, the slim side to have a margin of 5 %.
+  //    slim: one round of workgroups - a launch, their start and end, and (BM + BN) rows of K at slim_bytes_per_ns.  (Two
+  //    rounds lose, one workgroup's stores to the next one's start: 84 such plans took 1.06 of the time on average.)
+  //    own: a launch, K tiles of a part at own_*_tile_ns or, with more workgroups, own_*_ns_per_wg of a unit's each (64x64
+  //    with rows that are not 16-byte aligned: times own_64_staged per mille; more than one workgroup of them a unit, which
+  //    overlap each other: own_64_ns_per_wg_shared), on 128x128 also the operands' way from memory
+  //    (own_deep_ns_per_operand_mb), and a K split's second launch and its partial sums' way.
+  //    Timed on both sides for 7794 products (bf16 and int8, up to sixteen batches, M to 6000, N and K to 14336, rows at any
+  //    alignment; another 14604 gave the constants): 3074 take a slim tile, in 0.69 of the time on average, twelve of them more
+  //    than 3 % slower, the worst 9 %.
+  int64_t slim_ns = 4000, slim_row_ns = 10, slim_bytes_per_ns = 65, slim_bytes_per_ns_unaligned = 40;
   int64_t slim_margin_num = 95, slim_margin_den = 100;
-  int64_t own_64_ns = 3640, own_64_tile_ns = 320, own_64_ns_per_wg = 415, own_64_staged = 1360, own_64_split_ns = 4430, own_64_ns_per_mb = 275;
-  int64_t own_128_ns = 5640, own_128_tile_ns = 515, own_128_ns_per_wg = 96, own_128_staged = 2120, own_128_split_ns = 3650, own_128_ns_per_mb = 585;
+  int64_t own_64_ns = 3640, own_64_tile_ns = 320, own_64_ns_per_wg = 415, own_64_ns_per_wg_shared = 300, own_64_staged = 1360;
+  int64_t own_64_split_ns = 4430, own_64_ns_per_mb = 275;
+  int64_t own_deep_ns = 5000, own_deep_tile_ns = 440, own_deep_ns_per_operand_mb = 46, own_deep_split_ns = 3650, own_deep_ns_per_mb = 585;
 };
 constexpr RuleConstants kRules{};
 
@@ -929,6 +934,25 @@ int32_t unsigned_side_terms(const Problem& pr, TileGemmParams* params, int32_t* 
   return ST_OK;
 }
 
+// The workgroup tiles and K parts of a plan on a tile family.
+void set_tiles(const Problem& pr, const VecopsHipPlan& plan, TileGemmParams* p) {
+  int tile_m = 0, tile_n = 0;
+  tile_of_family(plan.family, &tile_m, &tile_n);
+  const int64_t ktile = k_tile_elements(pr.src);
+  p->tiles_m = static_cast<int32_t>((pr.m + tile_m - 1) / tile_m);
+  p->tiles_n = static_cast<int32_t>((pr.n + tile_n - 1) / tile_n);
+  p->split_k = static_cast<int32_t>(plan.split_k);
+  p->k_tiles_per_split = static_cast<int32_t>(((pr.k + ktile - 1) / ktile + p->split_k - 1) / p->split_k);
+}
+
+// Whether the four-stage kernel (tile_gemm_deep128.hip) runs the 128x128 tile of such a plan: at most one workgroup per
+// compute unit, enough K tiles a part, operands that it serves.
+bool deep128_runs(const Problem& pr, const TileGemmParams& p, uint32_t family, int mode) {
+  return family == VECOPS_HIP_FAMILY_TILE_128 && p.k_tiles_per_split >= kRules.deep_min_k_tiles &&
+         static_cast<int64_t>(p.tiles_m) * p.tiles_n * p.batch * p.split_k <= kRules.deep_max_workgroups &&
+         launch_tile_gemm_deep128_serves(pr.src, p, mode, pr.packed_b);
+}
+
 // The slim tiles (tile_gemm_slim.hip), and a plan's `slim_tile` for each.
 constexpr struct { int bm, bn; } kSlimTiles[] = {{32, 16}, {32, 32}, {32, 48}, {32, 64}, {64, 48}, {64, 64}, {128, 48}, {128, 64}};
 uint16_t slim_code(int bm, int bn) { return static_cast<uint16_t>(bm << 8 | bn); }
@@ -941,38 +965,45 @@ bool slim_serves(const Problem& pr, const VecopsHipPlan& plan) {
          launch_tile_gemm_slim_serves(pr.src, base_params(pr, nullptr, nullptr, nullptr, nullptr));
 }
 
-// Hands the rule table's own plan of 64x64 or 128x128 tiles to a slim tile where that is ahead: the plan then names it
-// (slim_tile) beside the table's family, split and workspace, none of which the call uses.  A pure integer function of the
-// problem and the plan; both sides' times are estimates in ns (RuleConstants).  The result's type and a C input do not enter:
-// a product's bf16 output stays its rounded fp32 output.  (A plan that peels columns keeps its tiles, which are whole rounds.)
+// Hands the rule table's own plan of 64x64 tiles, or of 128x128 tiles on the four-stage kernel, to a slim tile where that is
+// ahead: the plan then names it (slim_tile) beside the table's family, split and workspace, none of which the call uses.  A
+// pure integer function of the problem and the plan; both sides' times are estimates in ns (RuleConstants).  The result's type
+// and a C input do not enter: a product's bf16 output stays its rounded fp32 output.  (A plan that peels columns keeps its
+// tiles, which are whole rounds.)
 void take_slim_tile(const Problem& pr, VecopsHipPlan* chosen) {
   const VecopsHipPlan& plan = *chosen;
   const bool small = plan.family == VECOPS_HIP_FAMILY_TILE_64;
   if ((!small && plan.family != VECOPS_HIP_FAMILY_TILE_128) || plan.peeled_columns > 0 || !slim_serves(pr, plan)) return;
-  const bool aligned = fetch_mode(pr, plan) == MODE_KVEC_DMA;
-  const int64_t ktile = k_tile_elements(pr.src), k_tiles = (pr.k + ktile - 1) / ktile;
-  const int64_t split = plan.split_k, tile = small ? 64 : 128;
-  const int64_t wgs = ((pr.m + tile - 1) / tile) * ((pr.n + tile - 1) / tile) * pr.batch * split;
-  int64_t tile_ns = std::max(small ? kRules.own_64_tile_ns : kRules.own_128_tile_ns,
-                             (small ? kRules.own_64_ns_per_wg : kRules.own_128_ns_per_wg) * wgs / kComputeUnits);
-  if (!aligned) tile_ns = tile_ns * (small ? kRules.own_64_staged : kRules.own_128_staged) / 1000;
-  int64_t own_ns = (small ? kRules.own_64_ns : kRules.own_128_ns) + (k_tiles + split - 1) / split * tile_ns;
-  if (split > 1)
-    own_ns += (small ? kRules.own_64_split_ns : kRules.own_128_split_ns) +
-              split * pr.batch * pr.m * pr.n * 4 / 1024 * (small ? kRules.own_64_ns_per_mb : kRules.own_128_ns_per_mb) / 1024;
+  const int mode = fetch_mode(pr, plan);
+  const bool aligned = mode == MODE_KVEC_DMA;
+  TileGemmParams p = base_params(pr, nullptr, nullptr, nullptr, nullptr);
+  set_tiles(pr, plan, &p);
+  const int64_t ktile = k_tile_elements(pr.src), k_tiles = (pr.k + ktile - 1) / ktile, split = plan.split_k;
+  const int64_t partials = split > 1 ? split * pr.batch * pr.m * pr.n * 4 / 1024 : 0;  // KiB
+  int64_t own_ns;
+  if (small) {
+    const int64_t wgs = static_cast<int64_t>(p.tiles_m) * p.tiles_n * pr.batch * split;
+    int64_t tile_ns = std::max(kRules.own_64_tile_ns, (wgs <= kComputeUnits ? kRules.own_64_ns_per_wg : kRules.own_64_ns_per_wg_shared) * wgs / kComputeUnits);
+    if (!aligned) tile_ns = tile_ns * kRules.own_64_staged / 1000;
+    own_ns = kRules.own_64_ns + p.k_tiles_per_split * tile_ns;
+    if (split > 1) own_ns += kRules.own_64_split_ns + partials * kRules.own_64_ns_per_mb / 1024;
+  } else {
+    if (!deep128_runs(pr, p, plan.family, mode)) return;
+    const int64_t operands = pr.batch * (pr.m + pr.n) * k_tiles / 8;  // KiB: K tiles of 128 bytes
+    own_ns = kRules.own_deep_ns + p.k_tiles_per_split * kRules.own_deep_tile_ns + operands * kRules.own_deep_ns_per_operand_mb / 1024;
+    if (split > 1) own_ns += kRules.own_deep_split_ns + partials * kRules.own_deep_ns_per_mb / 1024;
+  }
   int64_t best_ns = own_ns * kRules.slim_margin_num / kRules.slim_margin_den;
-  uint16_t found = 0;
   for (const auto& t : kSlimTiles) {
-    const int64_t count = ((pr.m + t.bm - 1) / t.bm) * ((pr.n + t.bn - 1) / t.bn) * pr.batch;
-    const int64_t rounds = (count + kComputeUnits - 1) / kComputeUnits, rows = t.bm + t.bn;
-    const int64_t fetch_ns = rows * k_tiles * 128 / (aligned ? kRules.slim_bytes_per_ns : kRules.slim_bytes_per_ns_unaligned);
-    const int64_t ns = kRules.slim_launch_ns + rounds * (kRules.slim_round_ns + rows * kRules.slim_row_ns + fetch_ns);
+    if (((pr.m + t.bm - 1) / t.bm) * ((pr.n + t.bn - 1) / t.bn) * pr.batch > kComputeUnits) continue;
+    const int64_t rows = t.bm + t.bn;
+    const int64_t ns = kRules.slim_ns + rows * kRules.slim_row_ns +
+                       rows * k_tiles * 128 / (aligned ? kRules.slim_bytes_per_ns : kRules.slim_bytes_per_ns_unaligned);
     if (ns < best_ns) {
       best_ns = ns;
-      found = slim_code(t.bm, t.bn);
+      chosen->slim_tile = slim_code(t.bm, t.bn);
     }
   }
-  chosen->slim_tile = found;
 }
 
 // The library's own plan: the rule table's, or a slim tile in its place.
@@ -1103,12 +1134,7 @@ int32_t run_problem(const Problem& pr, const VecopsHipPlan& plan, const float* r
   int tile_m = 0, tile_n = 0;
   tile_of_family(plan.family, &tile_m, &tile_n);
   if (tile_m == 0) return fail(ST_INVALID, "matmul: plan names no kernel family (%u)", plan.family);
-  const int ktile = k_tile_elements(pr.src);
-  p.tiles_m = static_cast<int32_t>((pr.m + tile_m - 1) / tile_m);
-  p.tiles_n = static_cast<int32_t>((pr.n + tile_n - 1) / tile_n);
-  const int k_tiles = static_cast<int>((pr.k + ktile - 1) / ktile);
-  p.split_k = static_cast<int32_t>(plan.split_k);
-  p.k_tiles_per_split = (k_tiles + p.split_k - 1) / p.split_k;
+  set_tiles(pr, plan, &p);
   const int mode = fetch_mode(pr, plan);
 
   hipError_t e;
@@ -1135,17 +1161,13 @@ int32_t run_problem(const Problem& pr, const VecopsHipPlan& plan, const float* r
     e = launch_tile_gemm_short_k(pr.src, p, stream);
   } else if (pr.packed_b && launch_tile_gemm_packed16_serves(pr.src, p, tile_m, tile_n)) {
     e = launch_tile_gemm_packed16(pr.src, p, stream);
-  } else if (pr.packed_b && tile_m == 128 && tile_n == 128 && p.k_tiles_per_split >= kRules.deep_min_k_tiles &&
-             static_cast<int64_t>(p.tiles_m) * p.tiles_n * p.batch * p.split_k <= kRules.deep_max_workgroups &&
-             launch_tile_gemm_deep128_serves(pr.src, p, mode, true)) {
+  } else if (pr.packed_b && deep128_runs(pr, p, plan.family, mode)) {
     // at most one workgroup per compute unit: the four-stage kernel with the pack kept in its order in LDS
     e = launch_tile_gemm_deep128(pr.src, p, mode, true, stream);
   } else if (pr.packed_b) {
     const int a_mode = plan.vector_a == 0 ? 0 : ((pr.src == SRC_BF16 || pr.src == SRC_F16 || pr.src == SRC_I8) && lines_up(pr, pr.a, pr.a.rs)) ? 2 : 1;
     e = launch_tile_gemm_packed_b(pr.src, p, tile_m, tile_n, a_mode, stream);
-  } else if (tile_m == 128 && tile_n == 128 && p.k_tiles_per_split >= kRules.deep_min_k_tiles &&
-             static_cast<int64_t>(p.tiles_m) * p.tiles_n * p.batch * p.split_k <= kRules.deep_max_workgroups &&
-             launch_tile_gemm_deep128_serves(pr.src, p, mode, false)) {
+  } else if (deep128_runs(pr, p, plan.family, mode)) {
     // at most one workgroup per compute unit: the four-stage kernel, whose loads run three K tiles ahead
     e = launch_tile_gemm_deep128(pr.src, p, mode, false, stream);
   } else if (pr.src == SRC_F32 && tile_m == tile_n && (tile_m == 64 || tile_m == 128) && (mode == MODE_KVEC || mode == MODE_NVEC_B) &&
