@@ -239,8 +239,131 @@ def test_no_workspace(device):
     assert prepared._keep[4] is None
 
 
+def _run_on(tile, a, b, c, c_in=None):
+    """The product on the named slim tile, whatever the library would choose."""
+    from vecops_amd import capi
+    plan = capi.plan_matmul_family(a, b, c, capi.family_request("tile_64", split_k=1), c_in=c_in)
+    plan.slim_tile = 256 * tile[0] + tile[1]
+    return capi.matmul_planned(a, b, c, plan, c_in=c_in)
+
+
+# (row tiles and rows past them, column tiles and columns past them, K): a K inside one chunk, inside one K tile, one element past
+# it, whole stages, and rings that wrap with a partial tile and without
+EDGES = [(1, -1, 1, 1, 9), (1, 1, 2, -1, 63), (0, 1, 3, 3, 65), (2, 0, 1, 0, 256), (1, 0, 2, 5, 1291), (1, 17, 1, 2, 2048)]
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("kind", ["bf16", "f16", "i8"])
+def test_every_instance(device, kind, tile):
+    """Against float64 (int8: exactly), and with C inputs, 16-bit results and strided C: added to or made from the same sums."""
+    import torch
+    dtype = {"bf16": torch.bfloat16, "f16": torch.float16, "i8": torch.int8}[kind]
+    for i, (mt, mr, nt, nr, k) in enumerate(EDGES):
+        m, n, pad = mt * tile[0] + mr, nt * tile[1] + nr, i % 3
+        a, b = _operands(device, dtype, m, n, k, seed=i, pad=pad)
+        g = torch.Generator(device=device).manual_seed(i)
+        if kind == "i8":
+            sums = _run_on(tile, a, b, torch.full((m, n), -1, dtype=torch.int32, device=device))
+            want = torch.from_numpy(_exact(a, b).astype(np.int64)).to(torch.int32).to(device)
+            assert torch.equal(sums, want), (i, "sums")
+            cin = torch.randint(-2 ** 31, 2 ** 31 - 1, (m, n), generator=g, device=device, dtype=torch.int32)
+            out, convert = torch.int32, lambda x: x
+        else:
+            sums = _run_on(tile, a, b, torch.full((m, n), float("nan"), device=device))
+            # (fp32_tol grows with K in tiles of 32 terms: at least one)
+            assert rel_err(sums.cpu().numpy(), _exact(a, b)) <= fp32_tol(max(k, 32)), (i, "sums")
+            cin = torch.randn((m, n), generator=g, device=device).to(dtype)
+            out, convert = dtype, lambda x: x.to(dtype)  # noqa: B023
+            assert torch.equal(_run_on(tile, a, b, torch.empty((m, n), device=device, dtype=dtype)), sums.to(dtype)), (i, "16 bits")
+        plus = lambda x: sums + (x if kind == "i8" else x.float())  # noqa: B023,E731
+        wide = torch.empty((m, 2 * n), device=device, dtype=out).copy_(torch.cat([cin, cin], 1))
+        for name, c, ci in (("full", torch.empty((m, n), device=device, dtype=out), cin),
+                            ("bias", torch.empty((m, n), device=device, dtype=out), cin[:1].expand(m, n)),
+                            ("column bias", torch.empty((m, n), device=device, dtype=out), cin[:, :1].expand(m, n)),
+                            ("strided input", torch.empty((m, n), device=device, dtype=out), wide[:, ::2]),
+                            ("transposed C", torch.empty((n, m), device=device, dtype=out).t(), cin),
+                            ("padded C", torch.empty((m, n + 3), device=device, dtype=out)[:, :n], cin),
+                            ("strided C", torch.empty((m, 2 * n), device=device, dtype=out)[:, ::2], cin)):
+            c.fill_(7)
+            assert torch.equal(_run_on(tile, a, b, c, c_in=ci), convert(plus(ci))), (i, name)
+        c = cin.clone()                                    # the C input in place
+        assert torch.equal(_run_on(tile, a, b, c, c_in=c), convert(plus(cin))), (i, "in place")
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("kind", ["bf16", "i8"])
+def test_batches_with_c_inputs_and_padded_rows(device, kind, tile):
+    import torch
+    dtype = torch.bfloat16 if kind == "bf16" else torch.int8
+    batch, m, n, k = 3, tile[0] + 1, 2 * tile[1] + 1, 197
+    a, b = _operands(device, dtype, m, n, k, batch=(batch,), pad=3)
+    out = torch.float32 if kind == "bf16" else torch.int32
+    cin = torch.arange(batch * m * n, device=device, dtype=torch.int32).view(batch, m, n).to(out)
+    one = torch.stack([_run_on(tile, a[i], b[i], torch.empty((m, n), dtype=out, device=device)) for i in range(batch)])
+    empty = lambda: torch.full((batch, m, n), 7, dtype=out, device=device)  # noqa: E731
+    assert torch.equal(_run_on(tile, a, b, empty()), one)
+    assert torch.equal(_run_on(tile, a, b, empty(), c_in=cin), one + cin)
+    bias = cin[:1, :1].expand(batch, m, n)
+    assert torch.equal(_run_on(tile, a, b, empty(), c_in=bias), one + bias)
+    shared = b[:1].expand(batch, n, k)                     # one B for every batch
+    want = torch.stack([_run_on(tile, a[i], b[0], torch.empty((m, n), dtype=out, device=device)) for i in range(batch)])
+    assert torch.equal(_run_on(tile, a, shared, empty()), want)
+
+
 # (m, n, k) on which the library's own plan takes each tile, for int8
 INT8 = {(32, 16): (45, 16, 511), (32, 32): (35, 2081, 648), (32, 48): (33, 4418, 1025), (32, 64): (33, 6146, 1800),
         (64, 48): (65, 5442, 2624), (64, 64): (65, 8002, 1937), (128, 48): (132, 6095, 1408), (128, 64): (68, 16319, 1921)}
 BF16 = {(32, 16): (47, 15, 193), (32, 32): (38, 2162, 321), (32, 48): (34, 4162, 513), (32, 64): (34, 6239, 897),
         (64, 48): (67, 5441, 1248), (64, 64): (65, 8159, 913), (128, 48): (149, 6050, 640), (128, 64): (195, 8117, 961)}
+
+
+@pytest.mark.parametrize("tile", TILES)
+def test_int8_dequantised_on_every_tile(device, tile):
+    import torch
+    from vecops_amd import capi
+    m, n, k = INT8[tile]
+    a, b = _operands(device, torch.int8, m, n, k, seed=3)
+    c = torch.full((m, n), -1, dtype=torch.int32, device=device)
+    assert capi.plan_matmul(a, b, c).slim_tile == 256 * tile[0] + tile[1]
+    capi.matmul(a, b, c)
+    rows, columns = torch.rand(m, device=device) + 0.5, torch.rand(n, device=device) + 0.5
+    correction = torch.randint(-100000, 100000, (n,), device=device, dtype=torch.int32)
+    plain, corrected = (torch.full((m, n), float("nan"), device=device) for _ in range(2))
+    capi.matmul_i8_dequant(a, b, rows, columns, plain)
+    capi.matmul_i8_dequant(a, b, rows, columns, corrected, correction=correction)
+    want = torch.from_numpy(_exact(a, b).astype(np.int64)).to(torch.int32).to(device)
+    assert torch.equal(c, want)
+    assert torch.equal(plain, (want.float() * rows[:, None]) * columns)
+    assert torch.equal(corrected, ((want + correction).float() * rows[:, None]) * columns)
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("activation", ["none", "relu", "sigmoid", "silu"])
+def test_transforms_on_every_tile(device, tile, activation):
+    """The transform of the same sums: bit for bit, but for the two activations on the hardware's exponential."""
+    import torch
+    from vecops_amd import capi
+    m, n, k = BF16[tile]
+    a, b = _operands(device, torch.bfloat16, m, n, k, seed=4)
+    a = (a.float() * 0.05).bfloat16()
+    sums = torch.empty((m, n), device=device)
+    assert capi.plan_matmul(a, b, sums).slim_tile == 256 * tile[0] + tile[1]
+    capi.matmul(a, b, sums)
+    g = torch.Generator(device=device).manual_seed(7)
+    rows, columns = torch.rand(m, generator=g, device=device) + 0.5, torch.rand(n, generator=g, device=device) + 0.5
+    cin = torch.randn((m, n), generator=g, device=device)
+    for ci in (None, cin, cin[:1].expand(m, n)):
+        ep = capi.epilogue(activation=activation, row_scales=rows, column_scales=columns, scale=0.5, shift=0.25)
+        c = torch.full((m, n), float("nan"), device=device)
+        assert capi.plan_matmul_fused(a, b, c, ep, c_in=ci).slim_tile == 256 * tile[0] + tile[1]
+        capi.matmul_fused(a, b, c, ep, c_in=ci)
+        v = (((sums if ci is None else sums + ci) * rows[:, None]) * columns) * 0.5 + 0.25
+        if activation in ("none", "relu"):
+            assert torch.equal(c, torch.relu(v) if activation == "relu" else v)
+        else:
+            want = torch.sigmoid(v.double()) * (v.double() if activation == "silu" else 1.0)
+            # (the library states 1e-6 relative for the exponential; the sums and quotients around it are fp32)
+            assert bool(((c.double() - want).abs() <= 2e-6 * want.abs() + 1e-30).all())
+            half = torch.empty((m, n), device=device, dtype=torch.bfloat16)
+            assert torch.equal(capi.matmul_fused(a, b, half, ep, c_in=None if ci is None else ci.bfloat16()),
+                               capi.matmul_fused(a, b, torch.empty_like(c), ep, c_in=None if ci is None else ci.bfloat16().float()).bfloat16())
