@@ -1,5 +1,6 @@
 """The weight-only ring kernel (w8a16_ring.hip): every count of weight rows a workgroup takes, single rows past it, K of one
-stage, of part of one, of rings that wrap and of an odd multiple of 64, every group size, padded rows."""
+stage, of part of one, of rings that wrap and of an odd multiple of 64, every group size, padded rows - and products beside the
+rule's lines (K below a stage, three or four rows), which the other kernels of the family run."""
 import pytest
 
 pytestmark = pytest.mark.gpu
@@ -9,7 +10,9 @@ pytestmark = pytest.mark.gpu
     (5, 17, 64, 64, 0), (16, 16, 512, 128, 0), (7, 257, 576, 64, 16), (16, 1000, 1216, 64, 0), (9, 4096, 1024, 256, 0),     # 16 rows
     (3, 2048, 4096, 128, 0), (4, 333, 6400, 256, 32), (16, 1089, 12672, 128, 0), (15, 4097, 640, 128, 0),                     # 16 and 32
     (5, 8191, 1152, 128, 0), (12, 9408, 1088, 64, 0), (16, 12288, 2048, 128, 16), (8, 12289, 2176, 128, 0),                   # 32, 48, 64
-    (14, 16384, 1024, 64, 0), (6, 16385, 1024, 128, 0), (10, 9378, 14208, 64, 0), (5, 700, 128, 128, 0)])
+    (14, 16384, 1024, 64, 0), (6, 16385, 1024, 128, 0), (10, 9378, 14208, 64, 0), (5, 700, 128, 128, 0),
+    (9, 8193, 320, 64, 0), (6, 16383, 256, 128, 16), (7, 16385, 1152, 128, 0), (5, 8192, 448, 64, 0), (7, 20000, 64, 64, 0),   # the lines of K
+    (3, 4097, 2112, 64, 0), (4, 1025, 8448, 256, 32), (3, 16385, 5120, 128, 0), (4, 1024, 8448, 64, 0)])
 def test_against_float64(device, m, n, k, group, pad):
     import torch
     from vecops_amd import capi

@@ -2261,12 +2261,20 @@ namespace {
 // kernels of the skinny family are ahead.  By estimated ns, `rounds * (start and end + what a workgroup fetches)`: the fewest
 // rows that fit one round, mostly - 16 x 8352 x 6272 in groups of 128 16.5 us on 48 rows (26.4 on 16, 25.3 on 32, 19.9 on 64;
 // 33.3 before), 14 x 1848 x 5376 7.5 on 16 (13.0), 16 x 4096 x 4096 8.5 on 16 (10.5), 16 x 8192 x 4096 11.9 on 32 (14.5).
-//   * From five rows of activations on; with three or four (the other kernels' share of activation loads is smaller) from K =
-//     2048 on: 4 x 15616 x 3840 14.7 against 19.6, 4 x 5760 x 2048 6.4 against 6.5, 4 x 6400 x 1664 6.1 against 6.0.
+//   * From a whole stage of K on (512); from half a stage on with 8192 to 16384 weight rows, which are one round of workgroups
+//     here and two of the others (9 x 10906 x 256 in 0.76 of the time); from the third stage on with more than 16384, whose
+//     workgroups' start-ups follow one another on a unit (8 x 49227 x 64 13.0 against 8.7, 5 x 82354 x 128 19.2 against 13.5,
+//     15 x 16513 x 576 8.7 against 7.8, 9 x 36875 x 1088 20.5 against 18.3).
+//   * With three or four rows of activations (the other kernels' share of activation loads is smaller) where the weight rows
+//     fill the units and K is long: 4 x 15616 x 3840 14.7 against 19.6, but 3 x 67374 x 2688 51 against 45, 4 x 19823 x 2688
+//     17.9 against 16.5, 3 x 3568 x 3648 6.6 against 6.0.
+//   * 15114 products of both kinds timed against the other kernels, weights in a cache and not: where the rule takes this kernel
+//     0.73 of the time on average.
 //   * At K = 4096 with more than 8192 weight rows the kernel whose activations are resident is level or ahead (16 x 14336 in
 //     a cache 13.1 against 13.9, not in one 17.0 both).
 int ring_weight_rows(const SkinnyW8A16Params& p) {
-  if (p.m < 3 || (p.m < 5 && p.k < 2048)) return 0;
+  if (p.m < 3 || p.k < (p.n <= 8192 ? 512 : p.n <= 16384 ? 256 : 1152)) return 0;
+  if (p.m < 5 && (p.n <= 1024 || p.k < (p.n <= 4096 ? 8192 : p.n <= 16384 ? 2048 : 5120))) return 0;
   if (p.k == 4096 && p.n > 8192 && (p.group == 128 || p.group == 256) && p.ldx < (int64_t{1} << 26)) return 0;
   int best = 0;
   int64_t best_ns = INT64_MAX;
