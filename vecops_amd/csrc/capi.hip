@@ -1819,7 +1819,7 @@ int32_t describe_grouped(uint32_t count, const VecopsHipOperand* a, const Vecops
     // the groups are independent problems: nothing folds across them, each may fold its own batches
     int32_t rc = describe(&a[i], &b[i], cin, &c[i], compute, &g->problems[i]);
     if (rc != ST_OK) return rc;
-    choose(g->problems[i], &g->plans[i]);
+    choose_table(g->problems[i], &g->plans[i]);
     const VecopsHipPlan& plan = g->plans[i];
     if (plan.family == VECOPS_HIP_FAMILY_NONE) continue;
     if (plan.workspace_bytes > g->loop_workspace) g->loop_workspace = plan.workspace_bytes;
@@ -1830,7 +1830,12 @@ int32_t describe_grouped(uint32_t count, const VecopsHipOperand* a, const Vecops
     else g->table_groups.push_back(static_cast<int>(i));
   }
   g->one_launch = same_class && g->src != kSrcF64 && g->table_groups.size() > 1;
-  if (!g->one_launch) return ST_OK;
+  // (groups that are launches of their own run the single call's plan)
+  for (int i : g->split_groups) take_slim_tile(g->problems[i], &g->plans[i]);
+  if (!g->one_launch) {
+    for (int i : g->table_groups) take_slim_tile(g->problems[i], &g->plans[i]);
+    return ST_OK;
+  }
   // One workgroup tile for every group: the biggest square tile that still yields two rounds' worth of
   // workgroups over all groups together (priced like the rule table's candidates), else 64 x 64.
   auto tiles = [&](int64_t t) {
