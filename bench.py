@@ -192,7 +192,7 @@ def bench_bf16_gemm(dev, steps, warmup):
 
 
 def bench_fp32_gemm(dev, steps, warmup, compute, n=1024):
-    """BASELINE configs[0]: fp32 1024^3, A[M,K] and B[K,N] row-major, U[-1,1); multiplied as bf16 (vecops' x86
+    """fp32 1024^3, A[M,K] and B[K,N] row-major, U[-1,1); multiplied as bf16 (vecops' x86
     behaviour) or in fp32 (its SME_F32F32 atom)."""
     import torch
     from vecops_amd import capi, synth
@@ -214,7 +214,7 @@ def bench_fp32_gemm(dev, steps, warmup, compute, n=1024):
         label = label.replace("tile_gemm_kernel<f32>", "tile_gemm_deep_f32_kernel")   # what run_problem launches for such a plan
     return {"metric": f"fp32_gemm_{n}_{compute}_compute_tflops", "workload": f"fp32 GEMM M=N=K={n}, A[M,K] and B[K,N] "
             f"row-major, uniform[-1,1), multiplied in {'fp32' if compute == 'f32' else 'bf16 (rounded on load)'}, fp32 "
-            "accumulate and output (BASELINE configs[0])", "value": tflops, "unit": "TFLOP/s",
+            "accumulate and output", "value": tflops, "unit": "TFLOP/s",
             "us_per_step": t["wall_ms"] * 1e3, "dtype": "f32" if compute == "f32" else "f32 memory, bf16 compute",
             "roofline": _roofline("mfma", tflops, peak, "TFLOP/s", kernel=label,
                                   algorithmic_flops_per_launch=flops, algorithmic_bytes_per_launch=3 * 4 * n * n,
@@ -252,7 +252,7 @@ def bench_bf16_mid(dev, steps, warmup, m, n, k, b_as_kn):
 
 
 def bench_batched(dev, steps, warmup, m, n, k):
-    """batch 8, bf16 operands uniform[-1,1), fp32 accumulate and output."""
+    """Batch 8, bf16 operands uniform[-1,1), fp32 accumulate and output."""
     import numpy as np
     import torch
     from vecops_amd import capi, synth
@@ -280,7 +280,7 @@ def bench_batched(dev, steps, warmup, m, n, k):
     roof.update(kernel=label, algorithmic_flops_per_launch=flops, algorithmic_bytes_per_launch=nbytes,
                 **_traffic(f"batched_{m}x{n}x{k}"), **_timing_fields(t))
     return {"metric": f"bf16_batched_{m}x{n}x{k}_tflops", "workload": f"batch 8 x bf16 ({m},{n},{k}), A[8,M,K] and "
-            "B[8,N,K], uniform[-1,1), fp32 accumulate and output (BASELINE configs[2])", "value": tflops,
+            "B[8,N,K], uniform[-1,1), fp32 accumulate and output", "value": tflops,
             "unit": "TFLOP/s", "hbm_gbps": gbps, "us_per_step": t["wall_ms"] * 1e3, "dtype": "bf16", "roofline": roof}
 
 
@@ -289,7 +289,7 @@ GROUPED_SHAPES = [(777, 1000, 3001), (1, 4097, 129), (255, 63, 8191), (3000, 300
 
 
 def bench_grouped(dev, steps, warmup):
-    """Irregular batches: eight bf16 products of unlike shapes (BASELINE configs[2]'s four among them, unbatched) as one
+    """Irregular batches: eight bf16 products of unlike shapes (the four irregular batched ones among them, unbatched) as one
     vecops_hip_matmul_grouped call, and the same eight as separate vecops_hip_matmul calls."""
     import numpy as np
     import torch
@@ -342,7 +342,7 @@ def bench_int8_dequant(dev, steps, warmup, ceiling=None):
     if ceiling:
         roof.update(measured_ceiling=ceiling, frac_of_ceiling=tops / ceiling)
     return {"metric": "int8_quantized_matmul_tops", "workload": "int8 2048x4096x11008, per-token x per-channel "
-            "dequant fused, fp32 out (BASELINE configs[3])", "value": tops, "unit": "TOP/s", "ms_per_step": t["wall_ms"],
+            "dequant fused, fp32 out", "value": tops, "unit": "TOP/s", "ms_per_step": t["wall_ms"],
             "dtype": "int8", "roofline": roof}
 
 
@@ -474,7 +474,7 @@ def bench_gemv(dev, steps, warmup, m=1):
     kernel = ("vecops_hip skinny_w8a16_stream_kernel" if m == 1 else "vecops_hip skinny_w8a16_stream_rows_kernel"
               if m == 2 else "vecops_hip skinny_w8a16_mfma_resident_kernel")
     return {"metric": f"w8a16_gemv_m{m}_hbm_gbps", "workload": f"weight-only int8 GEMV M={m} K=4096 N=14336 group 128, "
-            "bf16 activations, bf16 out, weights rotated through 8 buffers (BASELINE configs[4])", "value": gbps,
+            "bf16 activations, bf16 out, weights rotated through 8 buffers", "value": gbps,
             "unit": "GB/s", "us_per_step": t["wall_ms"] * 1e3, "dtype": "int8 x bf16 -> f32",
             "roofline": _roofline("hbm", gbps, PEAK_HBM_GBPS, "GB/s", kernel=kernel, algorithmic_bytes_per_launch=nbytes,
                                   **_traffic(f"gemv_m{m}"), **_timing_fields(t))}
@@ -748,7 +748,7 @@ def main() -> int:
     ap.add_argument("--gemv-m", type=int, default=1, help="activation rows of the --only gemv workload (1..16)")
     ap.add_argument("--ceiling-dtype", choices=["bf16", "int8"], default="bf16", help="operands of --only mfma_ceiling")
     ap.add_argument("--fp32-compute", choices=["bf16", "f32"], default="bf16", help="compute type of --only fp32")
-    ap.add_argument("--fp32-size", type=int, default=1024, help="M = N = K of --only fp32 (1024: BASELINE configs[0])")
+    ap.add_argument("--fp32-size", type=int, default=1024, help="M = N = K of --only fp32")
     ap.add_argument("--batched-shape", default="777,1000,3001", help="M,N,K of --only batched")
     ap.add_argument("--mid-shape", default="1024,4096,4096", help="M,N,K of --only bf16_mid")
     ap.add_argument("--mid-layout", choices=["kn", "nk"], default="kn", help="how B is stored for --only bf16_mid")
@@ -797,7 +797,7 @@ def main() -> int:
         "steps": K, "warmup": W, "ms_per_step": main_res["wall_ms"], "higher_is_better": True,
         "scaling": "weak", "vs_baseline": None, "dtype": "bf16", "data": "synthetic",
         "config": {"workload": "bf16 GEMM M=N=K=4096, A[M,K] and B[K,N] row-major, normal(0,0.02), fp32 accumulate, "
-                               "bf16 output (BASELINE configs[1])", "M": 4096, "N": 4096, "K": 4096},
+                               "bf16 output", "M": 4096, "N": 4096, "K": 4096},
     }
     roofline = main_res["roofline"]
     secondary = None

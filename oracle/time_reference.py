@@ -85,7 +85,7 @@ def main() -> int:
             raise RuntimeError("reference matmul unavailable")
 
     for lanes in (1, 8):
-        # configs[0]: fp32 1024^3, A[M,K] and B[K,N] row-major, U[-1,1): fp32 memory, bf16 compute, fp32 out
+        # fp32 1024^3, A[M,K] and B[K,N] row-major, U[-1,1): fp32 memory, bf16 compute, fp32 out
         n = 1024
         a, b_kn = synth.uniform_pm1(1, (n, n)), synth.uniform_pm1(2, (n, n))
         c = np.zeros((n, n), np.float32)
@@ -97,7 +97,7 @@ def main() -> int:
         record("fp32 1024^3 (fp32 memory, bf16 compute, fp32 out)", lanes, s, reps, 2.0 * n ** 3, "GFLOP/s",
                "ops::matmul<AMX_BF16F32>, dense tensors, B as the transposed view of [K,N]")
 
-        # bf16 4096^3, bf16 out, B[K,N] row-major (BASELINE) and B[N,K]
+        # bf16 4096^3, bf16 out, B[K,N] row-major and B[N,K]
         n = 4096
         a16 = synth.bf16_round(synth.normal(1, (n, n), 0.02))
         b16 = synth.bf16_round(synth.normal(2, (n, n), 0.02))
@@ -110,7 +110,7 @@ def main() -> int:
             record(f"bf16 4096^3 (B as {label}, bf16 out)", lanes, s, reps, 2.0 * n ** 3, "GFLOP/s",
                    "ops::matmul<AMX_BF16F32>, dense tensors")
 
-        # configs[2]: batch 8 of four irregular shapes, bf16 in, fp32 out (lanes split the batch)
+        # batch 8 of four irregular shapes, bf16 in, fp32 out (lanes split the batch)
         for (m, nn, k) in [(777, 1000, 3001), (1, 4097, 129), (255, 63, 8191), (3000, 3000, 17)]:
             a3 = synth.bf16_round(synth.uniform_pm1(1, (8, m, k)))
             b3 = synth.bf16_round(synth.uniform_pm1(2, (8, nn, k)))
@@ -124,7 +124,7 @@ def main() -> int:
             record(f"bf16 batch 8 x ({m},{nn},{k}), fp32 out", lanes, s, reps, 8 * 2.0 * m * nn * k, "GFLOP/s",
                    "rank-3 ops::matmul<AMX_BF16F32>, dense tensors; lanes split the batch")
 
-        # configs[3]: int8 2048 x 4096 x 11008 with per-token x per-channel dequantisation, fp32 out
+        # int8 2048 x 4096 x 11008 with per-token x per-channel dequantisation, fp32 out
         m, k, nn = 2048, 4096, 11008
         ai, bi = synth.int8_sym(1, (m, k)), synth.int8_sym(2, (nn, k))
         rs = synth.scales(3, m)
@@ -139,7 +139,7 @@ def main() -> int:
         record("int8 2048x4096x11008 + dequant, fp32 out", lanes, s, reps, 2.0 * m * nn * k, "GOP/s",
                "ops::matmul<AMX_I8I32<int8,int8>> with RuntimePerRowColumnDequantizeTransform, dense tensors; every lane packs all of B")
 
-        # configs[4] has no vecops counterpart (no weight-only group-scaled matmul): the nearest form it can express,
+        # the weight-only group-scaled product has no vecops counterpart: the nearest form it can express,
         # bf16 x bf16 with the weights dequantised to bf16 beforehand
         k, nn = 4096, 14336
         wq = synth.bf16_round((synth.int8_sym(2, (nn, k)).astype(np.float32) * np.float32(0.01)))
