@@ -476,7 +476,7 @@ struct Accumulators {
   // and stay there until the epilogue takes them one by one: left to itself the compiler copies all 256 values into
   // vector registers ahead of the branch between the epilogue's paths, spills what does not fit, and reloaded one
   // spilled value wrongly (ROCm 7.2).  The empty statement pins a quad to its accumulation registers at its use.
-  static constexpr bool kPinned = M16 && WM * WN > 8;
+  static constexpr bool kPinned = WM * WN > 8;
   template <int I, int J, int Q>
   __device__ __forceinline__ Quad quad() const {
     if constexpr (M16) {
@@ -485,6 +485,9 @@ struct Accumulators {
 #endif
       return t[2 * I + (Q >> 1)][2 * J + (Q & 1)];
     } else {
+#if defined(__HIP_DEVICE_COMPILE__)
+      if constexpr (kPinned) asm volatile("" : "+a"(const_cast<Frag&>(t[I][J])));
+#endif
       return __builtin_shufflevector(t[I][J], t[I][J], 4 * Q, 4 * Q + 1, 4 * Q + 2, 4 * Q + 3);
     }
   }
@@ -602,16 +605,24 @@ __device__ __forceinline__ bool c_takes_quads(const TileGemmParams& p) {
   return p.c_cs == 1 && (p.c_rs & 3) == 0 && (p.c_bs & 3) == 0 && (reinterpret_cast<uintptr_t>(p.c) & (quad_bytes - 1)) == 0;
 }
 
+// Four or eight consecutive elements of a row of C (or of a C input) as one access at element alignment: rows of an odd
+// number of elements begin anywhere, and the memory system takes 16-byte accesses at any byte address.  (Through global
+// pointers: of a generic pointer the compiler makes one access per element at such an alignment.)
+typedef uint32_t u32x4_align4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x2_align2 __attribute__((ext_vector_type(2), aligned(2)));
+typedef uint32_t u32x4_align2 __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u32_align1 __attribute__((aligned(1)));
+
 __device__ __forceinline__ void store_quad_bits(const TileGemmParams& p, int64_t c_off, const uint32_t (&bits)[4]) {
   switch (output_element_bytes(p.out_kind)) {
     case 2:
-      *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(p.c) + c_off) = u32x2{bits[0] | (bits[1] << 16), bits[2] | (bits[3] << 16)};
+      *reinterpret_cast<VECOPS_GLOBAL u32x2_align2*>((VECOPS_GLOBAL uint16_t*)p.c + c_off) = u32x2{bits[0] | (bits[1] << 16), bits[2] | (bits[3] << 16)};
       break;
     case 1:
-      *reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(p.c) + c_off) = bits[0] | (bits[1] << 8) | (bits[2] << 16) | (bits[3] << 24);
+      *reinterpret_cast<VECOPS_GLOBAL u32_align1*>((VECOPS_GLOBAL uint8_t*)p.c + c_off) = bits[0] | (bits[1] << 8) | (bits[2] << 16) | (bits[3] << 24);
       break;
     default:
-      *reinterpret_cast<u32x4*>(static_cast<uint32_t*>(p.c) + c_off) = u32x4{bits[0], bits[1], bits[2], bits[3]};
+      *reinterpret_cast<VECOPS_GLOBAL u32x4_align4*>((VECOPS_GLOBAL uint32_t*)p.c + c_off) = u32x4{bits[0], bits[1], bits[2], bits[3]};
   }
 }
 
@@ -647,8 +658,6 @@ __device__ __forceinline__ Finisher make_finisher(const TileGemmParams& p, bool 
 // Four consecutive columns of one output row from their staged 32-bit values (int32 sums with the
 // correction added, dequantised fp32, or fp32 sums) to the bits of C.  C-input rows are contiguous and
 // need no alignment; `ecs` are the lane's four fused column scales (ones when there are none).
-typedef uint32_t u32x4_align4 __attribute__((ext_vector_type(4), aligned(4)));
-typedef uint32_t u32x2_align2 __attribute__((ext_vector_type(2), aligned(2)));
 __device__ __forceinline__ void finish_quad(const TileGemmParams& p, const Finisher& fin, const u32x4& v, int batch,
                                             int row, int col0, int cols_left, const f32x4& ecs, uint32_t (&bits)[4]) {
   const uint32_t none = fin.int_sums ? 0u : 0x80000000u;  // adding int 0 or fp32 -0.0 changes nothing
@@ -1489,6 +1498,226 @@ constexpr int kTileLdsBytes() {
   return stages > epilogue ? stages : epilogue;
 }
 
+// Two fp32 as the packed 16-bit pair of a floating output type; a bf16 NaN leaves as 0x7fc0 (bf16_bits_rne).
+template <bool BF16>
+__device__ __forceinline__ uint32_t narrow_pair(float lo, float hi) {
+  if constexpr (BF16) {
+    uint32_t w = cvt_pk_bf16(lo, hi);
+    if (__builtin_isunordered(lo, hi)) w = pack_bf16x2(lo, hi);
+    return w;
+  } else {
+    return f16_bits_rne(lo) | (f16_bits_rne(hi) << 16);
+  }
+}
+
+// One block of 32 rows of fp32 sums, row-major in LDS, on its way out (store_rows): a lane keeps the same U columns through all
+// of the block's rows.
+template <int WN, int U>
+struct RowWalk {
+  static constexpr int COLS = WN * 32, PITCH = COLS + 4;                                           // 32-bit words
+  static constexpr int LANES = COLS / U, ROWS = 64 / LANES, STEPS = (32 + ROWS - 1) / ROWS;        // of a row; a step's rows; steps
+};
+
+// fp32 sums to C through whole rows of the wavefront's tile: everything that is not a plain 16-bit result - C inputs, bias
+// rows, the fused transform, fp32 results - of unsplit products with contiguous columns, rows at any alignment.  One
+// block of 32 rows at a time goes through LDS in 32 bits (sums are rounded once, after the C input) and is walked with a lane on
+// the same output columns in every row (eight of 16 bits, four of 32), so that
+//   * C is written and a C input read in runs of a whole tile row (256 bytes of a 16-bit row of the 256x256 tile);
+//   * a bias row and column scales are loaded once per lane, and row scales once per block (into the rows' LDS pad);
+//   * a block's C input is requested a block ahead of its use (more than eight steps: in front of the block), the first in front
+//     of the barrier - where it is all there is to do besides the conversion, and no lane holds fewer columns than its share.
+//     Other C inputs are added to the sums in LDS first.
+// What it replaced walked blocks of 32 columns and loaded each C input quad where it added it, behind the stores before it:
+// 64 memory round trips one after the other in a 256x256 tile.  Measured (us, before -> now; without a C input 21 and 94):
+// f16 4096 x 4096 x 512 with a C input 68 -> 29, with a bias row 54 -> 28; f16 4096^3 160 -> 119 and 140 -> 103; fp32 results with
+// an fp32 C input 85 -> 42 and 166 -> 127; f16 results without one, which went the same way, 43 -> 22.6 and 129 -> 97; rows of
+// 4097 elements, which were stored one by one, bf16 4096 x 4097 x 1024 82 -> 46.
+// PLAIN: fp32 sums as they are (an instance of its own: what the others prepare delays a short product's only round of tiles).
+template <int WAVES_M, int WAVES_N, int WM, int WN, int LDS_BYTES, bool PLAIN, typename ACC>
+__device__ __forceinline__ void store_rows(const TileGemmParams& p, char* lds, const ACC& acc, int batch, int m0, int n0, int wm,
+                                           int wn, int wave, int lane) {
+  constexpr int COLS = WN * 32, PITCH = COLS + 4;  // 32-bit words; the pad staggers rows across banks
+  constexpr int BN = COLS * WAVES_N;
+  static_assert(32 * PITCH * 4 * WAVES_M * WAVES_N <= LDS_BYTES, "the blocks must fit the launch's LDS");
+  uint32_t* mine = reinterpret_cast<uint32_t*>(lds) + wave * (32 * PITCH);
+  const int first_row = m0 + wm * (WM * 32), first_col = n0 + wn * COLS;
+  const bool wide_out = PLAIN || p.out_kind == OUT_F32;  // else bf16 or f16
+  const bool cin16 = p.cin_kind != OUT_F32;
+  const bool full = (p.cin != nullptr) & (p.cin_rs != 0);  // a C input with a row for every row of C
+  const int share = wide_out ? 4 : 8;                   // columns of a lane
+  const bool whole_shares = (n0 + BN <= p.n) | (p.n % share == 0);
+  const bool ahead = full & (p.fused == 0) & whole_shares & (cin16 != wide_out);
+  const int cin_bytes = cin16 ? 2 : 4;
+  const VECOPS_GLOBAL char* cin = (const VECOPS_GLOBAL char*)p.cin + batch * p.cin_bs * cin_bytes;
+  auto widen = [&](uint32_t half) __attribute__((always_inline)) { return p.cin_kind == OUT_BF16 ? __uint_as_float(half << 16) : f16_bits_to_f32(half); };
+  auto cin_at = [&](int64_t at) __attribute__((always_inline)) {
+    return cin16 ? widen(reinterpret_cast<const VECOPS_GLOBAL uint16_t*>(cin)[at]) : reinterpret_cast<const VECOPS_GLOBAL float*>(cin)[at];
+  };
+  using W4 = RowWalk<WN, 4>;
+  using W8 = RowWalk<WN, 8>;
+  using U4 = std::integral_constant<int, 4>;
+  using U8 = std::integral_constant<int, 8>;
+  using I0 = std::integral_constant<int, 0>;
+  using I1 = std::integral_constant<int, 1>;
+  using I2 = std::integral_constant<int, 2>;
+  static_assert(W4::STEPS <= 16 && W8::STEPS <= 8, "the requested C input's registers");
+  u32x4 coming[16] = {};  // two blocks' worth, or one of more than eight steps
+  // the C input of block i, at addresses inside it whatever the lane (lanes past an edge drop what they get)
+  auto request = [&](auto u_tag, auto i_tag) __attribute__((always_inline)) {
+    constexpr int U = decltype(u_tag)::value, i = decltype(i_tag)::value;
+    using W = RowWalk<WN, U>;
+    if constexpr (i < WM) {
+      const int col = min(first_col + lane % W::LANES * U, p.n - U);
+#pragma unroll
+      for (int s = 0; s < W::STEPS; ++s) {
+        const int row = min(first_row + i * 32 + min(s * W::ROWS + lane / W::LANES, 31), p.m - 1);
+        const VECOPS_GLOBAL char* at = cin + (static_cast<int64_t>(row) * p.cin_rs + col) * (U == 8 ? 2 : 4);
+        coming[(W::STEPS <= 8 ? (i & 1) * 8 : 0) + s] = *reinterpret_cast<const VECOPS_GLOBAL u32x4_align2*>(at);
+      }
+    }
+  };
+  if (!PLAIN && ahead && !wide_out) request(U8{}, I0{});
+  if (!PLAIN && ahead && wide_out) request(U4{}, I0{});
+  const int out_bytes = wide_out ? 4 : 2;
+  const int lane_col = wide_out ? lane % W4::LANES * 4 : lane % W8::LANES * 8, cols_left = p.n - (first_col + lane_col);
+  // FORM 0: the lane's bias and column scales, and the transform
+  Finisher fin;
+  bool scaled = false;
+  float bias[8], column_scales[8];
+  VECOPS_GLOBAL char* c = (VECOPS_GLOBAL char*)p.c + (batch * p.c_bs + static_cast<int64_t>(first_row) * p.c_rs + first_col + lane_col) * out_bytes;
+  // One step of a block: U columns of the lane's row.  FORM 0: any; 1: `given` is that row's part of the C input, and nothing
+  // but the conversion follows; 2: fp32 sums as they are.  INSIDE: the tile lies wholly inside C (no branch stands between the
+  // steps, which then overlap).
+  auto step = [&](auto u_tag, auto form_tag, auto inside_tag, int i, int s, const u32x4& given) __attribute__((always_inline)) {
+    constexpr int U = decltype(u_tag)::value, FORM = decltype(form_tag)::value;
+    constexpr bool AHEAD = FORM == 1, INSIDE = decltype(inside_tag)::value;
+    using W = RowWalk<WN, U>;
+    const int r = s * W::ROWS + lane / W::LANES, row = first_row + i * 32 + r;
+    if ((W::ROWS * W::LANES != 64 && lane >= W::ROWS * W::LANES) || (32 % W::ROWS != 0 && r > 31) || (!INSIDE && (row >= p.m || cols_left <= 0))) return;
+    const uint32_t* sums = mine + r * PITCH + lane % W::LANES * U;
+    float f[U];
+#pragma unroll
+    for (int e = 0; e < U; e += 4) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(sums + e);
+      f[e] = v.x; f[e + 1] = v.y; f[e + 2] = v.z; f[e + 3] = v.w;
+    }
+    if constexpr (AHEAD) {
+#pragma unroll
+      for (int e = 0; e < U; ++e)
+        f[e] += U == 4 ? __uint_as_float(given[e & 3]) : widen((given[e >> 1] >> ((e & 1) * 16)) & 0xffffu);
+    } else if constexpr (FORM == 0) {
+#pragma unroll
+      for (int e = 0; e < U; ++e) f[e] += bias[e];
+      if (scaled) {
+        const float row_scale = fin.row_scaled ? __uint_as_float(mine[r * PITCH + COLS]) : 1.0f;
+#pragma unroll
+        for (int e = 0; e < U; ++e) f[e] = ((f[e] * row_scale) * column_scales[e]) * fin.scale + fin.shift;
+      }
+      if (fin.clamps) {
+#pragma unroll
+        for (int e = 0; e < U; ++e) {  // x86 max_ps(a, b) = a > b ? a : b, min_ps(a, b) = a < b ? a : b
+          const float t = f[e] > fin.lo ? f[e] : fin.lo;
+          f[e] = t < fin.hi ? t : fin.hi;
+        }
+      }
+      if (fin.smooth) {
+#pragma unroll
+        for (int e = 0; e < U; ++e) {
+          const float sg = __builtin_amdgcn_rcpf(1.0f + __expf(-f[e]));
+          f[e] = fin.silu ? f[e] * sg : sg;
+        }
+      }
+    }
+    u32x4 out = {0u, 0u, 0u, 0u};
+    if constexpr (U == 4) {
+      out = u32x4{__float_as_uint(f[0]), __float_as_uint(f[1]), __float_as_uint(f[2]), __float_as_uint(f[3])};
+    } else if (p.out_kind == OUT_BF16) {
+#pragma unroll
+      for (int w = 0; w < 4; ++w) out[w] = narrow_pair<true>(f[2 * w], f[2 * w + 1]);
+    } else {
+#pragma unroll
+      for (int w = 0; w < 4; ++w) out[w] = narrow_pair<false>(f[2 * w], f[2 * w + 1]);
+    }
+    VECOPS_GLOBAL char* to = c + static_cast<int64_t>(i * 32 + r) * p.c_rs * out_bytes;
+    if (INSIDE || AHEAD || cols_left >= U) {
+      *reinterpret_cast<VECOPS_GLOBAL u32x4_align2*>(to) = out;
+    } else {  // the last, fewer columns of a row
+#pragma unroll
+      for (int e = 0; e < U - 1; ++e)
+        if (e < cols_left) {
+          if constexpr (U == 4) reinterpret_cast<VECOPS_GLOBAL uint32_t*>(to)[e] = out[e];
+          else reinterpret_cast<VECOPS_GLOBAL uint16_t*>(to)[e] = static_cast<uint16_t>(out[e >> 1] >> ((e & 1) * 16));
+        }
+    }
+  };
+  // (each form has its own walk over the blocks, and the forms part on a scalar: where their paths meet between blocks, the
+  // compiler lets every form wait for the loads and stores of the others)
+  auto blocks = [&](auto u_tag, auto form_tag, auto inside_tag) __attribute__((always_inline)) {
+    constexpr int U = decltype(u_tag)::value, FORM = decltype(form_tag)::value, STEPS = RowWalk<WN, U>::STEPS;
+    constexpr bool EARLY = STEPS <= 8;
+    if constexpr (FORM == 0) {
+      fin = make_finisher<false>(p, false);
+      scaled = p.fused != 0 && (p.ep_row_scales != nullptr || p.ep_column_scales != nullptr || (p.ep_flags & 3u) != 0u);
+#pragma unroll
+      for (int e = 0; e < U; ++e) {
+        const int col = min(first_col + lane_col + e, p.n - 1);
+        bias[e] = p.cin && !full ? cin_at(col) : -0.0f;  // (adding -0 changes nothing)
+        column_scales[e] = scaled && p.ep_column_scales ? p.ep_column_scales[col] : 1.0f;
+      }
+    }
+    __syncthreads();  // every wavefront is done reading fragments
+    static_for<WM>([&](auto ci) {
+      constexpr int i = decltype(ci)::value;
+      using Next = std::integral_constant<int, i + 1>;
+      static_for<WN>([&](auto cj) {
+        constexpr int j = decltype(cj)::value;
+        static_for<4>([&](auto cq) {
+          constexpr int q = decltype(cq)::value;
+          const auto v = acc.template quad<i, j, q>();
+          *reinterpret_cast<u32x4*>(mine + ACC::row(lane, q) * PITCH + j * 32 + ACC::col(lane, q)) = __builtin_bit_cast(u32x4, v);
+        });
+      });
+      // (the wavefront reads back only what it wrote itself: its own LDS traffic is ordered)
+      if constexpr (FORM == 0) {
+        if (full) {  // (clamped like a request: what lies past an edge is never stored)
+#pragma unroll 8
+          for (int idx = lane; idx < 32 * COLS; idx += 64) {
+            const int r = idx / COLS, col = idx % COLS;
+            float* sum = reinterpret_cast<float*>(mine + r * PITCH + col);
+            *sum += cin_at(static_cast<int64_t>(min(first_row + i * 32 + r, p.m - 1)) * p.cin_rs + min(first_col + col, p.n - 1));
+          }
+        }
+        if (fin.row_scaled && lane < 32)
+          mine[lane * PITCH + COLS] = __float_as_uint(p.ep_row_scales[static_cast<int64_t>(batch) * p.m + min(first_row + i * 32 + lane, p.m - 1)]);
+#pragma unroll 2
+        for (int s = 0; s < STEPS; ++s) step(u_tag, form_tag, inside_tag, i, s, u32x4{});
+      } else {
+        if constexpr (FORM == 1 && EARLY) request(u_tag, Next{});
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) step(u_tag, form_tag, inside_tag, i, s, coming[(EARLY ? (i & 1) * 8 : 0) + s]);
+        if constexpr (FORM == 1 && !EARLY) request(u_tag, Next{});
+      }
+    });
+  };
+  const bool inside = m0 + 32 * WAVES_M * WM <= p.m && n0 + BN <= p.n;
+  using Yes = std::true_type;
+  using No = std::false_type;
+  if constexpr (PLAIN) {
+    if (__builtin_amdgcn_readfirstlane(inside)) blocks(U4{}, I2{}, Yes{});
+    else blocks(U4{}, I2{}, No{});
+    return;
+  } else {
+    switch (__builtin_amdgcn_readfirstlane(ahead ? (wide_out ? 4 : 2) + inside : wide_out ? 1 : 0)) {
+      case 0: blocks(U8{}, I0{}, No{}); break;
+      case 1: blocks(U4{}, I0{}, No{}); break;
+      case 2: blocks(U8{}, I1{}, No{}); break;
+      case 3: blocks(U8{}, I1{}, Yes{}); break;
+      case 4: blocks(U4{}, I1{}, No{}); break;
+      default: blocks(U4{}, I1{}, Yes{}); break;
+    }
+  }
+}
+
 // Epilogue of the tile kernels: the accumulators of one wavefront to C.
 template <int SRC, int WAVES_M, int WAVES_N, int WM, int WN, int LDS_BYTES, bool M16>
 __device__ __forceinline__ void store_accumulators(const TileGemmParams& p, char* lds,
@@ -1500,13 +1729,11 @@ __device__ __forceinline__ void store_accumulators(const TileGemmParams& p, char
   // Epilogue.  The MFMAs were issued with the B tile as first operand, so the
   // accumulators hold C transposed: a lane holds quads of four consecutive columns
   // of one row of C (Accumulators::row / col), which
-  // become one 8-byte (bf16) or 16-byte (fp32 / int32) store.  Tiles that lie
-  // wholly inside C, need no C-input or split-K and have 16-byte aligned rows take
-  // one of three inline store loops; everything else goes through the general
-  // out-of-line routine.
+  // become one 8-byte (bf16) or 16-byte (fp32 / int32) store.  Products without split-K
+  // whose C (and C-input) has contiguous columns take one of the inline store loops, at any
+  // alignment of its rows; everything else goes through the general routine.
   const bool interior = m0 + BM <= p.m && n0 + BN <= p.n;
-  const bool aligned = (p.c_rs & 3) == 0 && (p.c_bs & 3) == 0 && (reinterpret_cast<uintptr_t>(p.c) & 15) == 0;
-  // the two fast paths take edge tiles too: their stores (and scale loads) are guarded per row and per run
+  // the fast paths take edge tiles too: their stores (and scale loads) are guarded per row and per run
   // of columns, which costs an interior tile a few compares
   const bool dequant = INT && p.row_scales != nullptr;
   // work that happens on the row-major side of the 32-bit staging: C-input, int32 sums leaving as floats,
@@ -1515,11 +1742,18 @@ __device__ __forceinline__ void store_accumulators(const TileGemmParams& p, char
   // (an unsigned operand's terms go through the general path, unless the launcher has folded them into the
   // per-column correction: unsigned A, one batch)
   const bool flip_terms = SRC == SRC_I8_FLIP && (p.row_term != nullptr || p.col_term != nullptr || p.const_term != 0u);
-  const bool simple = aligned && p.split_k == 1 && p.c_cs == 1 && !flip_terms &&
-                      (p.cin == nullptr || (p.cin_cs == 1 && !dequant));
+  const bool simple = p.split_k == 1 && p.c_cs == 1 && !flip_terms && (p.cin == nullptr || (p.cin_cs == 1 && !dequant));
   char* c_base = static_cast<char*>(p.c);
-  if (simple && !INT && p.out_kind == OUT_BF16 && p.cin == nullptr && p.fused == 0) {
-    // bf16: 8-byte pieces scattered over 32 rows would waste most of every memory
+  const bool out16 = p.out_kind == OUT_BF16 || p.out_kind == OUT_F16;
+  // (a scalar switch: where the paths part on conditions of their own, the compiler lays them behind one another and lets
+  // each wait for the loads and stores of those before it)
+  enum { PATH_PLAIN_16, PATH_PLAIN_32, PATH_SIMPLE, PATH_PARTIALS, PATH_GENERAL };
+  const bool raw_partials = interior && p.split_k > 1 && (p.n & 3) == 0 && (reinterpret_cast<uintptr_t>(p.partial) & 15) == 0;
+  const int part = simple ? (INT || p.cin != nullptr || p.fused != 0 ? PATH_SIMPLE : out16 ? PATH_PLAIN_16 : PATH_PLAIN_32)
+                          : (raw_partials ? PATH_PARTIALS : PATH_GENERAL);
+  const int path = INT ? part : __builtin_amdgcn_readfirstlane(part);
+  if (path == PATH_PLAIN_16) {
+    // bf16 / f16: 8-byte pieces scattered over 32 rows would waste most of every memory
     // transaction, so each wavefront first lays its tile out row-major in LDS (the
     // staging buffers are dead by now) and then stores whole 16-byte row segments.
     constexpr int TILE_COLS = WN * 32, TILE_ROWS = WM * 32;
@@ -1528,28 +1762,46 @@ __device__ __forceinline__ void store_accumulators(const TileGemmParams& p, char
                   "epilogue staging must fit the launch's LDS");
     __syncthreads();  // every wavefront is done reading fragments
     char* mine = lds + wave * (PITCH * TILE_ROWS);
-    static_for<WM>([&](auto ci) {
-      constexpr int i = decltype(ci)::value;
-      static_for<WN>([&](auto cj) {
-        constexpr int j = decltype(cj)::value;
-        static_for<4>([&](auto cq) {
-          constexpr int q = decltype(cq)::value;
-          if constexpr (!INT) {
-            const auto a4 = acc.template quad<i, j, q>();
-            u32x2 v;
-            v.x = cvt_pk_bf16(a4[0], a4[1]);
-            v.y = cvt_pk_bf16(a4[2], a4[3]);
-            *reinterpret_cast<u32x2*>(mine + (i * 32 + ACC::row(lane, q)) * PITCH + (j * 32 + ACC::col(lane, q)) * 2) = v;
-          }
+    auto lay_out = [&](auto bf16_tag) {
+      static_for<WM>([&](auto ci) {
+        constexpr int i = decltype(ci)::value;
+        static_for<WN>([&](auto cj) {
+          constexpr int j = decltype(cj)::value;
+          static_for<4>([&](auto cq) {
+            constexpr int q = decltype(cq)::value;
+            if constexpr (!INT) {
+              const auto a4 = acc.template quad<i, j, q>();
+              u32x2 v;
+              if constexpr (decltype(bf16_tag)::value) {
+                v.x = cvt_pk_bf16(a4[0], a4[1]);
+                v.y = cvt_pk_bf16(a4[2], a4[3]);
+              } else {
+                v.x = narrow_pair<false>(a4[0], a4[1]);
+                v.y = narrow_pair<false>(a4[2], a4[3]);
+              }
+              *reinterpret_cast<u32x2*>(mine + (i * 32 + ACC::row(lane, q)) * PITCH + (j * 32 + ACC::col(lane, q)) * 2) = v;
+            }
+          });
         });
       });
-    });
+    };
+    if (p.out_kind == OUT_BF16) lay_out(std::true_type{});
+    else lay_out(std::false_type{});
     // the wavefront reads back only what it wrote itself: its own LDS traffic is ordered
     constexpr int SEGS = TILE_COLS / 8;        // 16-byte segments per row
     constexpr int TOTAL = TILE_ROWS * SEGS;    // 16-byte segments of this wavefront's tile
     static_assert(TOTAL % 64 == 0, "whole store instructions");
     uint16_t* out = reinterpret_cast<uint16_t*>(c_base) + batch * p.c_bs +
                     static_cast<int64_t>(m0 + wm * TILE_ROWS) * p.c_rs + n0 + wn * TILE_COLS;
+    if (interior) {  // (no branch between the segments, which then overlap)
+#pragma unroll
+      for (int base = 0; base < TOTAL; base += 64) {
+        const int idx = base + lane, r = idx / SEGS, seg = idx % SEGS;
+        const u32x4 v = *reinterpret_cast<const u32x4*>(mine + r * PITCH + seg * 16);
+        *reinterpret_cast<VECOPS_GLOBAL u32x4_align2*>((VECOPS_GLOBAL uint16_t*)out + static_cast<int64_t>(r) * p.c_rs + seg * 8) = v;
+      }
+      return;
+    }
 #pragma unroll
     for (int base = 0; base < TOTAL; base += 64) {
       const int idx = base + lane, r = idx / SEGS, seg = idx % SEGS;
@@ -1560,15 +1812,20 @@ __device__ __forceinline__ void store_accumulators(const TileGemmParams& p, char
       const int cols_left = p.n - (n0 + wn * TILE_COLS + seg * 8);
       if (m0 + wm * TILE_ROWS + r < p.m) {
         if (cols_left >= 8) {
-          *reinterpret_cast<u32x4*>(dst) = v;
+          *reinterpret_cast<VECOPS_GLOBAL u32x4_align2*>((VECOPS_GLOBAL uint16_t*)dst) = v;
         } else {
 #pragma unroll
-          for (int e = 0; e < 8; ++e)
+          for (int e = 0; e < 7; ++e)
             if (e < cols_left) dst[e] = static_cast<uint16_t>(v[e >> 1] >> ((e & 1) * 16));
         }
       }
     }
-  } else if (simple) {
+  } else if (!INT && path == PATH_PLAIN_32) {
+    if constexpr (!INT) store_rows<WAVES_M, WAVES_N, WM, WN, LDS_BYTES, true>(p, lds, acc, batch, m0, n0, wm, wn, wave, lane);
+  } else if (!INT && path == PATH_SIMPLE) {
+    if constexpr (!INT) store_rows<WAVES_M, WAVES_N, WM, WN, LDS_BYTES, false>(p, lds, acc, batch, m0, n0, wm, wn, wave, lane);
+  } else if (INT && path == PATH_SIMPLE) {
+   if constexpr (INT) {
     // 32-bit outputs: one 32-column block of the wavefront's tile at a time goes row-major through LDS
     // (128 rows x 128 bytes) and leaves as whole cache lines (16-byte pieces scattered over 32 rows, straight
     // from the accumulator layout, wrote 8192 x 8192 fp32 at 3.9 TB/s; whole lines at 4.9 TB/s).
@@ -1641,7 +1898,7 @@ __device__ __forceinline__ void store_accumulators(const TileGemmParams& p, char
           const int cols_left = p.n - (col_block + cq * 4);
           if (m0 + wm * ROWS + r < p.m) {
             if (cols_left >= 4) {
-              *reinterpret_cast<u32x4*>(dst) = v;
+              *reinterpret_cast<VECOPS_GLOBAL u32x4_align4*>((VECOPS_GLOBAL uint32_t*)dst) = v;
             } else {
 #pragma unroll
               for (int e = 0; e < 4; ++e)
@@ -1682,7 +1939,8 @@ __device__ __forceinline__ void store_accumulators(const TileGemmParams& p, char
         }
       }
     });
-  } else if (interior && p.split_k > 1 && (p.n & 3) == 0 && (reinterpret_cast<uintptr_t>(p.partial) & 15) == 0) {
+   }
+  } else if (path == PATH_PARTIALS) {
     // split-K partial sums of an interior tile: raw accumulators, 16 bytes per store
     uint32_t* partial = static_cast<uint32_t*>(p.partial) + (static_cast<int64_t>(split) * p.batch + batch) * p.m * p.n;
     static_for<WM>([&](auto ci) {
