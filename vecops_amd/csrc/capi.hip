@@ -81,11 +81,14 @@ bool k_vector_ok(const View& v) {
   return v.cs == 1 && v.rs >= 0 && (v.rs * 256 + v.cols + 256) * eb < (int64_t{1} << 31);
 }
 
-// B stored [K,N] row-major: unit stride along N and N a multiple of 8 elements (the loader has no
-// N tail), 16-bit or 32-bit source elements.
+// B stored [K,N] row-major: unit stride along N, 16-bit or 32-bit source elements, rows at any alignment.  The last chunk of
+// a row whose N is no multiple of 8 reaches into the next row (kn_reaches_past in tile_gemm.h), so that one must lie behind it.
+// (Element by element, which such an N took before: bf16 1000 x 4001 x 4000 298 us where this takes 41, 4096 x 4097 x 4096 981
+// where this takes 173, fp32 memory 356 and 67; through loads that write LDS, as aligned rows, 56 and 193: these rows stay on
+// the staging registers.)
 bool n_vector_ok(const View& v) {
   const int64_t eb = dtype_bytes(v.dtype);
-  return v.rs == 1 && v.rows % 8 == 0 && v.rows >= 8 && v.cs > 0 &&
+  return v.rs == 1 && v.rows >= 8 && v.cs > 0 && (v.rows % 8 == 0 || v.cs >= v.rows) &&
          (v.cs * 64 + 512) * eb < (int64_t{1} << 31);  // 32-bit offsets inside a K tile
 }
 

@@ -937,6 +937,30 @@ struct Stager {
   }
 };
 
+// Four 32-bit (ELEM_BYTES 4) or eight 16-bit elements n .. of k row `k` of an operand stored [k][n], every access inside it:
+// one load and no branch.  A run that reaches past `extent` loads the row's last elements instead and shifts them down; a row
+// past k_end reads as zero.  (extent is at least a run long.)
+template <int ELEM_BYTES>
+__device__ __forceinline__ u32x4 load_kn_words(const void* base, int64_t ks, int k, int k_end, int n, int extent) {
+  constexpr int RUN = 16 / ELEM_BYTES;
+  const int start = min(n, extent - RUN), row = min(k, k_end - 1);
+  const VECOPS_GLOBAL char* at = (const VECOPS_GLOBAL char*)base + (row * ks + start) * ELEM_BYTES;
+  const u32x4 v = *reinterpret_cast<const VECOPS_GLOBAL u32x4_align2*>(at);
+  const uint32_t bits = static_cast<uint32_t>(k < k_end ? min(n - start, RUN) : RUN) * (8 * ELEM_BYTES);  // 0 .. 128
+  const uint64_t lo = (static_cast<uint64_t>(v.y) << 32) | v.x, hi = (static_cast<uint64_t>(v.w) << 32) | v.z;
+  const uint32_t b = bits & 63u;
+  const uint64_t carry = b ? hi << (64u - b) : 0;
+  const uint64_t out_lo = bits >= 128u ? 0 : bits >= 64u ? hi >> b : (lo >> b) | carry;
+  const uint64_t out_hi = bits >= 64u ? 0 : hi >> b;
+  return u32x4{static_cast<uint32_t>(out_lo), static_cast<uint32_t>(out_lo >> 32), static_cast<uint32_t>(out_hi),
+               static_cast<uint32_t>(out_hi >> 32)};
+}
+
+// Whether a tile of an operand stored [k][n] has chunks that reach past the operand's extent.  They read the next row's first
+// elements into columns that are never stored; in the last row there is none, so such a tile's last K tile is walked as a
+// partial one, through checked loads.
+__device__ __forceinline__ bool kn_reaches_past(int first_n, int cols, int extent) { return extent % 8 != 0 && first_n + cols > extent; }
+
 // LOAD_NTR: the operand is stored with its spatial index contiguous (B handed over
 // as [K,N] row-major) and goes into LDS untransposed: row k of the K tile holds the
 // tile's ROWS spatial positions, kPitch bytes apart.  Thread t stages 16-byte chunk
@@ -987,8 +1011,8 @@ struct Stager<SRC, LOAD_NTR, ROWS, THREADS> {
     k_end = k_end_;
     tid_ = tid;
     tile_base = uniform_ptr((const VECOPS_GLOBAL char*)(base + static_cast<int64_t>(first_row) * T::kSrcBytes));
-    // extent is a multiple of 8 on this path: a chunk past it is clamped onto the last one
-    const int n = min(first_row + chunk(0, tid) * 8, extent - 8) - first_row;
+    // a chunk past the extent is clamped onto the last one (which may itself reach past it: kn_reaches_past)
+    const int n = min(first_row + chunk(0, tid) * 8, (extent - 1) & ~7) - first_row;
     // the launcher admits this path only when a K tile's 64 rows span less than 2 GiB
     chunk_bytes = static_cast<uint32_t>((static_cast<int64_t>(k_row(0, tid)) * ks + n) * T::kSrcBytes);
   }
@@ -1022,31 +1046,16 @@ struct Stager<SRC, LOAD_NTR, ROWS, THREADS> {
     }
   }
 
-  // Whole tile with bounds checks (the partial last K tile): rows k >= K read as
-  // zero, columns n >= N as zero.
+  // Whole tile with bounds checks (the partial last K tile, or the last one where chunks reach past N): rows k >= K read
+  // as zero, what columns n >= N read as is never stored.
   __device__ __forceinline__ void fetch_checked(int kt) {
 #pragma unroll
     for (int i = 0; i < CHUNKS; ++i) {
-      const int k = kt * 64 + k_row(i, tid_);
-      if constexpr (SRC == SRC_BF16 || SRC == SRC_F16) {
-        uint32_t w[4] = {0u, 0u, 0u, 0u};
-        if (k < k_end) {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const int n = first_row + chunk(i, tid_) * 8 + e;
-            if (n < extent) w[e >> 1] |= static_cast<uint32_t>(reinterpret_cast<const uint16_t*>(base)[k * ks + n]) << ((e & 1) * 16);
-          }
-        }
-        regs[i] = Staged<SRC>{u32x4{w[0], w[1], w[2], w[3]}};
-      } else {
-        uint32_t w[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int n = first_row + chunk(i, tid_) * 8 + e;
-          w[e] = (k < k_end && n < extent) ? __float_as_uint(reinterpret_cast<const float*>(base)[k * ks + n]) : 0u;
-        }
-        regs[i] = Staged<SRC>{u32x4{w[0], w[1], w[2], w[3]}, u32x4{w[4], w[5], w[6], w[7]}};
-      }
+      const int k = kt * 64 + k_row(i, tid_), n = first_row + chunk(i, tid_) * 8;
+      if constexpr (SRC == SRC_F32_AS_BF16)
+        regs[i] = Staged<SRC>{load_kn_words<4>(base, ks, k, k_end, n, extent), load_kn_words<4>(base, ks, k, k_end, n + 4, extent)};
+      else
+        regs[i] = Staged<SRC>{load_kn_words<2>(base, ks, k, k_end, n, extent)};
     }
   }
 
@@ -1068,7 +1077,7 @@ struct Stager<SRC, LOAD_NTR, ROWS, THREADS> {
 };
 
 // The partial last K tile of an operand stored [k][n] (bf16), bounds-checked, straight into the packed and
-// swizzled LDS tile of the LOAD_NTR_DMA stager: rows k >= K and columns n >= N read as zero.
+// swizzled LDS tile of the LOAD_NTR_DMA stager: rows k >= K read as zero.
 // Where chunk `chunk` (16 bytes, 8 columns) of k row `krow` lies in its row of a [k][n] tile filled by loads that
 // write LDS (rows packed, cols * 2 bytes apart): the four rows a transposing read touches must lie in different
 // 64-byte groups of the bank period.  A power-of-two count of chunk slots: bits 2-3 of the slot xored with the row's
@@ -1084,21 +1093,20 @@ __device__ __forceinline__ int ntr_dma_slot(int cols, int krow, int chunk) {
 
 __device__ __noinline__ void stage_kn_checked(const void* base, int64_t ks, int first_n, int extent, int cols,
                                               int k0_tile, int k_end, char* lds_tile, int tid, int threads) {
-  const int chunks_per_row = cols / 8;
-#pragma unroll 2
-  for (int idx = tid; idx < 64 * chunks_per_row; idx += threads) {
-    const int krow = idx / chunks_per_row, chunk = idx % chunks_per_row;
-    const int k = k0_tile + krow;
-    uint32_t w[4] = {0u, 0u, 0u, 0u};
-    if (k < k_end) {
+  const int chunks_per_row = cols / 8, chunks = 64 * chunks_per_row;
+  constexpr int BATCH = 4;  // loads in flight before the first is stored
+  for (int idx0 = tid; idx0 < chunks; idx0 += threads * BATCH) {
+    u32x4 v[BATCH];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int n = first_n + chunk * 8 + e;
-        if (n < extent)
-          w[e >> 1] |= static_cast<uint32_t>(static_cast<const uint16_t*>(base)[k * ks + n]) << ((e & 1) * 16);
-      }
+    for (int j = 0; j < BATCH; ++j) {
+      const int idx = min(idx0 + j * threads, chunks - 1);
+      v[j] = load_kn_words<2>(base, ks, k0_tile + idx / chunks_per_row, k_end, first_n + idx % chunks_per_row * 8, extent);
     }
-    *reinterpret_cast<u32x4*>(lds_tile + krow * (cols * 2) + (ntr_dma_slot(cols, krow, chunk) << 4)) = u32x4{w[0], w[1], w[2], w[3]};
+#pragma unroll
+    for (int j = 0; j < BATCH; ++j) {
+      const int idx = idx0 + j * threads, krow = idx / chunks_per_row, chunk = idx % chunks_per_row;
+      if (idx < chunks) *reinterpret_cast<u32x4*>(lds_tile + krow * (cols * 2) + (ntr_dma_slot(cols, krow, chunk) << 4)) = v[j];
+    }
   }
 }
 
@@ -1265,8 +1273,8 @@ struct Stager<SRC, LOAD_NTR_DMA, ROWS, THREADS> {
     } else {
       chunk = slot ^ ((krow & 3) << 2);
     }
-    // extent is a multiple of 8 on this path: a chunk past it is clamped onto the last one
-    const int n = min(first_row + chunk * 8, extent - 8) - first_row;
+    // a chunk past the extent is clamped onto the last one (which may itself reach past it: kn_reaches_past)
+    const int n = min(first_row + chunk * 8, (extent - 1) & ~7) - first_row;
     return static_cast<uint32_t>((static_cast<int64_t>(krow) * ks + n) * T::kSrcBytes);
   }
   __device__ __forceinline__ void init(const void* base_, int64_t /*rs*/, int64_t ks_, int first_row_, int extent_,
@@ -1359,8 +1367,8 @@ struct Stager<SRC_F32, LOAD_KN32, ROWS, THREADS> {
     k_end = k_end_;
     tid_ = tid;
     tile_base = uniform_ptr((const VECOPS_GLOBAL char*)(base + static_cast<int64_t>(first_row) * 4));
-    // extent is a multiple of 8 on this path: a chunk past it is clamped onto the last one
-    const int n = min(first_row + chunk(0, tid) * 4, extent - 4) - first_row;
+    // a chunk past the extent is clamped onto the last one (which may itself reach past it: kn_reaches_past)
+    const int n = min(first_row + chunk(0, tid) * 4, (extent - 1) & ~3) - first_row;
     chunk_bytes = static_cast<uint32_t>((static_cast<int64_t>(k_row(0, tid)) * ks + n) * 4);
   }
   __device__ __forceinline__ uint32_t part_offset(int part) const {
@@ -1378,19 +1386,11 @@ struct Stager<SRC_F32, LOAD_KN32, ROWS, THREADS> {
   }
   __device__ __forceinline__ void fetch_full_spare(Spare&, int) {}
   __device__ __forceinline__ void take_spare(const Spare&) {}
-  // Whole tile with bounds checks (the partial last K tile): rows k >= K and columns n >= N read as zero.
+  // Whole tile with bounds checks, as the 16-bit stager's.
   __device__ __forceinline__ void fetch_checked(int kt) {
 #pragma unroll
-    for (int i = 0; i < CHUNKS; ++i) {
-      const int k = kt * 32 + k_row(i, tid_);
-      uint32_t w[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int n = first_row + chunk(i, tid_) * 4 + e;
-        w[e] = (k < k_end && n < extent) ? __float_as_uint(reinterpret_cast<const float*>(base)[k * ks + n]) : 0u;
-      }
-      regs[i] = u32x4{w[0], w[1], w[2], w[3]};
-    }
+    for (int i = 0; i < CHUNKS; ++i)
+      regs[i] = load_kn_words<4>(base, ks, kt * 32 + k_row(i, tid_), k_end, first_row + chunk(i, tid_) * 4, extent);
   }
   template <int PART>
   __device__ __forceinline__ void commit_part(char* lds_tile) const {
@@ -2109,7 +2109,9 @@ __device__ __forceinline__ void tile_gemm_workgroup(const TileGemmParams& p, int
   const int m0 = tm * BM, n0 = tn * BN;
 
   const int total_k_tiles = (p.k + KTILE - 1) / KTILE;
-  const int full_k_tiles = p.k / KTILE;
+  // (an operand stored [k][n]: see kn_reaches_past)
+  const bool past_n = (load_is_ntr(LOAD_B) || LOAD_B == LOAD_KN32) && kn_reaches_past(n0, BN, p.n);
+  const int full_k_tiles = (p.k - (past_n ? 1 : 0)) / KTILE;
   const int kt_begin = split * p.k_tiles_per_split;
   const int kt_end = min(total_k_tiles, kt_begin + p.k_tiles_per_split);
 
