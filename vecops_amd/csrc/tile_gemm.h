@@ -956,10 +956,12 @@ __device__ __forceinline__ u32x4 load_kn_words(const void* base, int64_t ks, int
                static_cast<uint32_t>(out_hi >> 32)};
 }
 
-// Whether a tile of an operand stored [k][n] has chunks that reach past the operand's extent.  They read the next row's first
+// Whether a tile of an operand stored [k][n] has chunks (of `chunk` elements) that reach past the operand's extent.  They read the next row's first
 // elements into columns that are never stored; in the last row there is none, so such a tile's last K tile is walked as a
 // partial one, through checked loads.
-__device__ __forceinline__ bool kn_reaches_past(int first_n, int cols, int extent) { return extent % 8 != 0 && first_n + cols > extent; }
+__device__ __forceinline__ bool kn_reaches_past(int first_n, int cols, int extent, int chunk) {
+  return extent % chunk != 0 && first_n + cols > extent;
+}
 
 // LOAD_NTR: the operand is stored with its spatial index contiguous (B handed over
 // as [K,N] row-major) and goes into LDS untransposed: row k of the K tile holds the
@@ -2110,7 +2112,7 @@ __device__ __forceinline__ void tile_gemm_workgroup(const TileGemmParams& p, int
 
   const int total_k_tiles = (p.k + KTILE - 1) / KTILE;
   // (an operand stored [k][n]: see kn_reaches_past)
-  const bool past_n = (load_is_ntr(LOAD_B) || LOAD_B == LOAD_KN32) && kn_reaches_past(n0, BN, p.n);
+  const bool past_n = (load_is_ntr(LOAD_B) || LOAD_B == LOAD_KN32) && kn_reaches_past(n0, BN, p.n, LOAD_B == LOAD_KN32 ? 4 : 8);
   const int full_k_tiles = (p.k - (past_n ? 1 : 0)) / KTILE;
   const int kt_begin = split * p.k_tiles_per_split;
   const int kt_end = min(total_k_tiles, kt_begin + p.k_tiles_per_split);
