@@ -215,15 +215,16 @@ VECOPS_HIP_EXPORT int32_t vecops_hip_matmul_static_workspace(const VecopsHipOper
  * their shapes.  a, b, c (and c_in, which may be null; an entry of rank 0 means "no C input for this group") are
  * arrays of count descriptors obeying the rules of vecops_hip_matmul group by group.  Groups of one operand
  * class - bf16, f16, int8 x int8, 8-bit integers with an unsigned side, or fp32 in either compute type - run as ONE
- * launch over a table of problem records (written into the workspace by small kernels fed through their arguments: no
- * host buffer has to outlive the call, nothing is allocated; the row-sum terms of unsigned sides are computed group by
- * group into the workspace first); fp64 operands, a mix of classes (signed x signed bytes beside groups with an
- * unsigned side count as a mix), groups with K = 0 and groups whose K vecops_hip_matmul would split (few output tiles,
- * long K: they run that call's plan, partial sums behind the table) run as launches of their own on the same stream.
- * Results
- * are those of vecops_hip_matmul on each group (bit-equal when that call runs the same tile shape without splitting K and
- * its plan names no slim tile - except 16-bit products with K <= 256 on 128 x 128 tiles, where the single call takes the
- * other MFMA shape; otherwise equal up to the order of the fp32 sums - integer results are always the same bits).  workspace: vecops_hip_matmul_grouped_workspace bytes, 16-byte aligned.
+ * launch: up to 24 groups in that launch's own arguments, more through a table of problem records (written into the workspace by
+ * small kernels fed through their arguments: no host buffer has to outlive the call, nothing is allocated; so do groups with an
+ * unsigned side, whose row-sum terms are computed group by group into the workspace first).  Groups whose K vecops_hip_matmul
+ * would split (few output tiles, long K) run that call's plan as launches of their own or, several of them, together: on slim
+ * tiles, or in the one launch with the others, where that is estimated well ahead.  fp64 operands, a mix of classes (signed x
+ * signed bytes beside groups with an unsigned side count as a mix) and groups with K = 0 run as launches of their own on the
+ * same stream.  Results are those of vecops_hip_matmul on each group (bit-equal when that call runs the same tile shape without
+ * splitting K and its plan names no slim tile - except 16-bit products with K <= 256 on 128 x 128 tiles, where the single call
+ * takes the other MFMA shape; otherwise equal up to the order of the fp32 sums - integer results are always the same bits).
+ * workspace: vecops_hip_matmul_grouped_workspace bytes, 16-byte aligned.
  */
 VECOPS_HIP_EXPORT uint64_t vecops_hip_matmul_grouped_workspace(uint32_t count, const VecopsHipOperand* a,
                                                                const VecopsHipOperand* b, const VecopsHipOperand* c_in,

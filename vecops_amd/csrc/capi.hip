@@ -968,17 +968,12 @@ bool slim_serves(const Problem& pr, const VecopsHipPlan& plan) {
          launch_tile_gemm_slim_serves(pr.src, base_params(pr, nullptr, nullptr, nullptr, nullptr));
 }
 
-// Hands the rule table's own plan of 64x64 tiles, or of 128x128 tiles on the four-stage kernel, to a slim tile where that is
-// ahead: the plan then names it (slim_tile) beside the table's family, split and workspace, none of which the call uses.  A
-// pure integer function of the problem and the plan; both sides' times are estimates in ns (RuleConstants).  The result's type
-// and a C input do not enter: a product's bf16 output stays its rounded fp32 output.  (A plan that peels columns keeps its
-// tiles, which are whole rounds.)
-void take_slim_tile(const Problem& pr, VecopsHipPlan* chosen) {
-  const VecopsHipPlan& plan = *chosen;
+// What the rule table's plan of 64x64 tiles, or of 128x128 tiles on the four-stage kernel, takes in ns (RuleConstants); -1 for
+// any other.
+int64_t own_plan_ns(const Problem& pr, const VecopsHipPlan& plan) {
   const bool small = plan.family == VECOPS_HIP_FAMILY_TILE_64;
-  if ((!small && plan.family != VECOPS_HIP_FAMILY_TILE_128) || plan.peeled_columns > 0 || !slim_serves(pr, plan)) return;
+  if (!small && plan.family != VECOPS_HIP_FAMILY_TILE_128) return -1;
   const int mode = fetch_mode(pr, plan);
-  const bool aligned = mode == MODE_KVEC_DMA;
   TileGemmParams p = base_params(pr, nullptr, nullptr, nullptr, nullptr);
   set_tiles(pr, plan, &p);
   const int64_t ktile = k_tile_elements(pr.src), k_tiles = (pr.k + ktile - 1) / ktile, split = plan.split_k;
@@ -987,21 +982,41 @@ void take_slim_tile(const Problem& pr, VecopsHipPlan* chosen) {
   if (small) {
     const int64_t wgs = static_cast<int64_t>(p.tiles_m) * p.tiles_n * pr.batch * split;
     int64_t tile_ns = std::max(kRules.own_64_tile_ns, (wgs <= kComputeUnits ? kRules.own_64_ns_per_wg : kRules.own_64_ns_per_wg_shared) * wgs / kComputeUnits);
-    if (!aligned) tile_ns = tile_ns * kRules.own_64_staged / 1000;
+    if (mode != MODE_KVEC_DMA) tile_ns = tile_ns * kRules.own_64_staged / 1000;
     own_ns = kRules.own_64_ns + p.k_tiles_per_split * tile_ns;
     if (split > 1) own_ns += kRules.own_64_split_ns + partials * kRules.own_64_ns_per_mb / 1024;
   } else {
-    if (!deep128_runs(pr, p, plan.family, mode)) return;
+    if (!deep128_runs(pr, p, plan.family, mode)) return -1;
     const int64_t operands = pr.batch * (pr.m + pr.n) * k_tiles / 8;  // KiB: K tiles of 128 bytes
     own_ns = kRules.own_deep_ns + p.k_tiles_per_split * kRules.own_deep_tile_ns + operands * kRules.own_deep_ns_per_operand_mb / 1024;
     if (split > 1) own_ns += kRules.own_deep_split_ns + partials * kRules.own_deep_ns_per_mb / 1024;
   }
+  return own_ns;
+}
+
+// What one workgroup of a slim tile takes on K tiles of 128 bytes, in ns.
+int64_t slim_workgroup_ns(int bm, int bn, int64_t k_tiles, bool aligned) {
+  const int64_t rows = bm + bn;
+  return kRules.slim_ns + rows * kRules.slim_row_ns +
+         rows * k_tiles * 128 / (aligned ? kRules.slim_bytes_per_ns : kRules.slim_bytes_per_ns_unaligned);
+}
+
+// Hands the rule table's own plan of 64x64 tiles, or of 128x128 tiles on the four-stage kernel, to a slim tile where that is
+// ahead: the plan then names it (slim_tile) beside the table's family, split and workspace, none of which the call uses.  A
+// pure integer function of the problem and the plan; both sides' times are estimates in ns (RuleConstants).  The result's type
+// and a C input do not enter: a product's bf16 output stays its rounded fp32 output.  (A plan that peels columns keeps its
+// tiles, which are whole rounds.)
+void take_slim_tile(const Problem& pr, VecopsHipPlan* chosen) {
+  const VecopsHipPlan& plan = *chosen;
+  if (plan.peeled_columns > 0 || !slim_serves(pr, plan)) return;
+  const int64_t own_ns = own_plan_ns(pr, plan);
+  if (own_ns < 0) return;
+  const bool aligned = fetch_mode(pr, plan) == MODE_KVEC_DMA;
+  const int64_t ktile = k_tile_elements(pr.src), k_tiles = (pr.k + ktile - 1) / ktile;
   int64_t best_ns = own_ns * kRules.slim_margin_num / kRules.slim_margin_den;
   for (const auto& t : kSlimTiles) {
     if (((pr.m + t.bm - 1) / t.bm) * ((pr.n + t.bn - 1) / t.bn) * pr.batch > kComputeUnits) continue;
-    const int64_t rows = t.bm + t.bn;
-    const int64_t ns = kRules.slim_ns + rows * kRules.slim_row_ns +
-                       rows * k_tiles * 128 / (aligned ? kRules.slim_bytes_per_ns : kRules.slim_bytes_per_ns_unaligned);
+    const int64_t ns = slim_workgroup_ns(t.bm, t.bn, k_tiles, aligned);
     if (ns < best_ns) {
       best_ns = ns;
       chosen->slim_tile = slim_code(t.bm, t.bn);
@@ -1773,10 +1788,11 @@ namespace vecops_hip {
 // them back, and no group waits for the one before it: what bounds it is the launch.  Eight bf16 groups of
 // 2048 rows in all, 4096 x 2048 each: the call 67.3 -> 61.1 us (before: one wavefront wrote the records one after the
 // other, 6.3 us, and a second launch searched the runs for every entry, 4.6 us).
-__global__ __launch_bounds__(256) void write_groups_kernel(const GroupChunk chunk, int32_t* __restrict__ first,
-                                                           TileGemmParams* __restrict__ groups, int32_t* __restrict__ group_of) {
+template <typename RECORD>
+__global__ __launch_bounds__(256) void write_groups_kernel(const GroupChunk<RECORD> chunk, int32_t* __restrict__ first,
+                                                           RECORD* __restrict__ groups, int32_t* __restrict__ group_of) {
   const int g = blockIdx.x;
-  constexpr int kWords = sizeof(TileGemmParams) / 4;
+  constexpr int kWords = sizeof(RECORD) / 4;
   static_assert(kWords <= 256, "a thread copies at most one word of a record");
   if (blockIdx.y == 0) {
     const uint32_t* src = reinterpret_cast<const uint32_t*>(&chunk.params[g]);
@@ -1792,23 +1808,122 @@ __global__ __launch_bounds__(256) void write_groups_kernel(const GroupChunk chun
 
 namespace {
 // A grouped call: several independent products (irregular batches - every group with its own extents, strides and
-// pointers).  bf16 and int8 groups that all multiply run as ONE launch of tile_gemm_grouped_kernel over a table of
-// problem records in the workspace (so do f16 groups and fp32 groups, in either compute type, and groups with an
-// unsigned 8-bit side, whose row-sum terms are computed group by group into the workspace first); fp64 operands,
-// groups of mixed classes, and groups with K = 0, run as launches of their own on the same stream.  So do groups whose K the rule table splits (few output tiles, long K):
-// the grouped kernel walks a group's whole K in every workgroup, and two workgroups with 128 K tiles each would
-// be what the whole launch waits for (eight products, 255 x 63 x 8191 among them: 99 us in one launch).
+// pointers).  Groups of one class that all multiply run as ONE launch of tile_gemm_grouped_kernel (groups with an unsigned 8-bit
+// side too, whose row-sum terms are computed group by group into the workspace first); fp64 operands, groups of mixed
+// classes, and groups with K = 0, run as launches of their own on the same stream.  Groups whose K the rule table splits (few
+// output tiles, long K) would be what that launch waits for - the grouped kernel walks a group's whole K in every workgroup:
+// eight products, 255 x 63 x 8191 among them, 99 us in one launch.  They run their own plan, or, two or more of them, together on
+// slim tiles, or with all others on the one tile, whichever is estimated ahead (plan_split_groups).
 struct Grouped {
   std::vector<Problem> problems;
   std::vector<VecopsHipPlan> plans;
   std::vector<int> table_groups;  // indices of the groups served by the one grouped launch
-  std::vector<int> split_groups;  // ... and of those that split K: launches of their own
-  bool one_launch = false;
+  std::vector<int> split_groups;  // ... of those that split K: launches of their own
+  std::vector<int> slim_groups;   // ... and of those that run on slim tiles together
+  int slim_bm = 0, slim_bn = 0;
+  bool one_launch = false, inline_groups = false;
   int src = -1, tile = 0, mode = 0;
   std::vector<int32_t> first;     // first workgroup of each table group, and the end
   uint64_t first_bytes = 0, record_bytes = 0, map_bytes = 0, term_bytes = 0, loop_workspace = 0;
   std::vector<uint64_t> term_offset;  // unsigned 8-bit sides: where a table group's row and column terms lie
 };
+
+// What a grouped launch on one square tile takes in ns: the longest workgroup alone, or all of them on the units' slots.  (Two
+// 128x128 workgroups share a unit, three or four of 64x64; bf16 256x256 tiles walk a K tile in 1.3 us, 128x128 ones alone in 0.67
+// and in pairs in 0.78, 64x64 ones as in RuleConstants; rows that are not 16-byte aligned 1.36 of that.)
+int64_t grouped_tiles_ns(const Grouped& g, const std::vector<int>& groups, int tile) {
+  const int64_t alone = tile == 256 ? 1300 : tile == 128 ? 670 : 320, shared = tile == 256 ? 1300 : tile == 128 ? 390 : 300;
+  const int64_t fixed = tile == 256 ? 12000 : tile == 128 ? 5000 : 3600;
+  int64_t longest = 0, sum = 0;
+  for (int i : groups) {
+    const Problem& pr = g.problems[i];
+    const int64_t ktile = k_tile_elements(pr.src), k_tiles = (pr.k + ktile - 1) / ktile;
+    const int64_t wgs = ((pr.m + tile - 1) / tile) * ((pr.n + tile - 1) / tile) * pr.batch;
+    const int64_t slow = fetch_mode(pr, g.plans[i]) == MODE_KVEC_DMA ? 1000 : kRules.own_64_staged;
+    longest = std::max(longest, fixed + k_tiles * alone * slow / 1000);
+    sum += wgs * (fixed * shared / alone + k_tiles * shared * slow / 1000);
+  }
+  if (groups.empty()) return 0;
+  const int64_t table = static_cast<int>(groups.size()) > kGroupsInline ? 4500 : 0;
+  return table + std::max(longest, sum / kComputeUnits);
+}
+
+// Where the groups run that split K on their own, and with them those of at most sixteen rows or columns and a long K (16-bit and
+// signed 8-bit classes, K-contiguous operands): the former in a launch or two each and the latter in the grouped launch, or all
+// of them together on slim tiles, or every group in one launch on one tile.  A pure integer function of the problems; the other
+// ways have to be estimated a third ahead.  Measured (us, before -> together; f16 but for the third, bf16): 18 groups of 768 rows in
+// all, 409 x 1985 155 -> 15, 18 of 592, 896 x 4760 237-262 -> 63, 8 of 174, 768 x 8183 113 -> 37, 24 of 770, 1085 x 1536 112 -> 25;
+// 12 of 2193, 1890 x 6144 on 128x128 tiles 255 -> 122.
+void plan_split_groups(Grouped* g, bool same_class) {
+  if (!same_class || g->split_groups.empty() || g->split_groups.size() + g->table_groups.size() < 2) return;
+  auto long_k = [&](int i) {
+    const int64_t ktile = k_tile_elements(g->problems[i].src);
+    return (g->problems[i].k + ktile - 1) / ktile;
+  };
+  auto aligned = [&](int i) { return fetch_mode(g->problems[i], g->plans[i]) == MODE_KVEC_DMA; };
+  std::vector<int> slim, others, all = g->table_groups;
+  int64_t own = 0;
+  for (int i : g->split_groups) {
+    const Problem& pr = g->problems[i];
+    if (!slim_serves(pr, g->plans[i])) return;  // (of another class, or B as [K,N]: as they are)
+    int64_t ns = own_plan_ns(pr, g->plans[i]);
+    if (ns < 0) ns = 15000 + long_k(i) / g->plans[i].split_k * 700;
+    VecopsHipPlan single = g->plans[i];
+    take_slim_tile(pr, &single);
+    if (single.slim_tile != 0) ns = slim_workgroup_ns(single.slim_tile >> 8, single.slim_tile & 255, long_k(i), aligned(i));
+    own += ns;
+    slim.push_back(i);
+    all.push_back(i);
+  }
+  for (int i : g->table_groups) {
+    const bool narrow = g->plans[i].family == VECOPS_HIP_FAMILY_SKINNY && long_k(i) >= kRules.split_min_k_tiles && slim_serves(g->problems[i], g->plans[i]);
+    (narrow ? slim : others).push_back(i);
+  }
+  if (slim.size() < 2) return;
+  auto table_ns = [&](const std::vector<int>& groups) {
+    return std::min(grouped_tiles_ns(*g, groups, 64), std::min(grouped_tiles_ns(*g, groups, 128), grouped_tiles_ns(*g, groups, 256)));
+  };
+  int64_t best = (own + table_ns(g->table_groups)) * 2 / 3;
+  const int64_t others_ns = table_ns(others);
+  const struct { int bm, bn; } tiles[] = {{32, 32}, {32, 64}, {64, 64}, {128, 64}};
+  for (const auto& t : tiles) {
+    int64_t longest = 0, sum = 0, most = 0;
+    for (int i : slim) {
+      const Problem& pr = g->problems[i];
+      const int64_t wgs = ((pr.m + t.bm - 1) / t.bm) * ((pr.n + t.bn - 1) / t.bn) * pr.batch;
+      const int64_t ns = slim_workgroup_ns(t.bm, t.bn, long_k(i), aligned(i));
+      longest = std::max(longest, ns);
+      sum += wgs * ns;
+      most = std::max(most, wgs);
+    }
+    if (most > kMostBlocks / (2 * kGroupsInline)) continue;  // (keeps a launch's workgroups in bounds)
+    const int64_t launches = (static_cast<int64_t>(slim.size()) + kGroupsInline - 1) / kGroupsInline;
+    const int64_t ns = others_ns + std::max(longest, sum / kComputeUnits) + (launches - 1) * kRules.slim_ns;
+    if (ns < best) {
+      best = ns;
+      g->slim_bm = t.bm;
+      g->slim_bn = t.bn;
+    }
+  }
+  std::sort(all.begin(), all.end());
+  for (int tile : {256, 128, 64}) {
+    const int64_t ns = grouped_tiles_ns(*g, all, tile);
+    if (ns < best * 9 / 10) {
+      best = ns * 10 / 9;
+      g->tile = tile;
+    }
+  }
+  if (g->tile != 0) {
+    g->table_groups = all;
+    g->split_groups.clear();
+  } else if (g->slim_bm != 0) {
+    std::sort(slim.begin(), slim.end());
+    g->slim_groups = slim;
+    g->table_groups.clear();
+    g->split_groups.clear();
+    (others.size() == 1 ? g->split_groups : g->table_groups) = others;  // (one group left: a launch of its own plan)
+  }
+}
 
 int32_t describe_grouped(uint32_t count, const VecopsHipOperand* a, const VecopsHipOperand* b, const VecopsHipOperand* c_in,
                          const VecopsHipOperand* c, uint32_t compute, Grouped* g) {
@@ -1832,7 +1947,8 @@ int32_t describe_grouped(uint32_t count, const VecopsHipOperand* a, const Vecops
     if (plan.split_k > 1) g->split_groups.push_back(static_cast<int>(i));
     else g->table_groups.push_back(static_cast<int>(i));
   }
-  g->one_launch = same_class && g->src != kSrcF64 && g->table_groups.size() > 1;
+  plan_split_groups(g, same_class);
+  g->one_launch = same_class && g->src != kSrcF64 && (g->table_groups.size() > 1 || !g->slim_groups.empty());
   // (groups that are launches of their own run the single call's plan)
   for (int i : g->split_groups) take_slim_tile(g->problems[i], &g->plans[i]);
   if (!g->one_launch) {
@@ -1849,10 +1965,12 @@ int32_t describe_grouped(uint32_t count, const VecopsHipOperand* a, const Vecops
     }
     return total;
   };
-  g->tile = 64;
   int64_t best = INT64_MAX;
+  const bool tile_chosen = g->tile != 0;  // (with the groups that split K on their own)
+  if (!tile_chosen) g->tile = 64;
   const struct { int tile; int64_t quality; } candidates[] = {{256, 1000}, {128, kQuality128}};
   for (const auto& cand : candidates) {
+    if (tile_chosen) break;
     const int64_t n_tiles = tiles(cand.tile);
     if (n_tiles < kComputeUnits / 2) continue;
     const int64_t rounds = (n_tiles + kComputeUnits - 1) / kComputeUnits;
@@ -1884,9 +2002,12 @@ int32_t describe_grouped(uint32_t count, const VecopsHipOperand* a, const Vecops
     if (next > kMostBlocks) return fail(ST_INVALID, "matmul_grouped: too many workgroups");
   }
   g->first.push_back(static_cast<int32_t>(next));
-  g->first_bytes = round_up_256(g->first.size() * 4u);
-  g->record_bytes = round_up_256(g->table_groups.size() * sizeof(TileGemmParams));
-  g->map_bytes = round_up_256(static_cast<uint64_t>(next) * 4u);
+  g->inline_groups = g->src != SRC_I8_FLIP && static_cast<int>(g->table_groups.size()) <= kGroupsInline;
+  if (!g->inline_groups) {
+    g->first_bytes = round_up_256(g->first.size() * 4u);
+    g->record_bytes = round_up_256(g->table_groups.size() * (g->src == SRC_I8_FLIP ? sizeof(TileGemmParams) : sizeof(GroupRecord)));
+    g->map_bytes = round_up_256(static_cast<uint64_t>(next) * 4u);
+  }
   if (g->src == SRC_I8_FLIP) {
     for (int i : g->table_groups) {
       const Problem& pr = g->problems[i];
@@ -1897,13 +2018,36 @@ int32_t describe_grouped(uint32_t count, const VecopsHipOperand* a, const Vecops
   return ST_OK;
 }
 
+// A group's record, and the end of a part's groups.
+int32_t group_record(const Problem& pr, int number, GroupRecord* r) {
+  if (pr.a.data == nullptr || pr.b.data == nullptr || pr.c.data == nullptr)
+    return fail(ST_INVALID, "matmul_grouped: group %d has an operand without storage", number);
+  const TileGemmParams p = base_params(pr, nullptr, nullptr, nullptr, nullptr);
+  r->a = p.a; r->b = p.b; r->cin = p.cin; r->c = p.c;
+  r->a_rs = p.a_rs; r->a_ks = p.a_ks; r->a_bs = p.a_bs;
+  r->b_rs = p.b_rs; r->b_ks = p.b_ks; r->b_bs = p.b_bs;
+  r->c_rs = p.c_rs; r->c_cs = p.c_cs; r->c_bs = p.c_bs;
+  r->cin_rs = p.cin_rs; r->cin_cs = p.cin_cs; r->cin_bs = p.cin_bs;
+  r->m = p.m; r->n = p.n; r->k = p.k; r->batch = p.batch;
+  r->out_kind = static_cast<int16_t>(p.out_kind);
+  r->cin_kind = static_cast<int16_t>(p.cin_kind);
+  r->unused = 0;
+  return ST_OK;
+}
+void end_of_groups(GroupChunk<GroupRecord>* chunk, int count, int64_t workgroups) {
+  chunk->count = count;
+  chunk->first[count] = static_cast<int32_t>(workgroups);
+  for (int j = count + 1; j <= GroupChunk<GroupRecord>::kMost; ++j) chunk->first[j] = INT32_MAX;
+}
+
+// (at least 256 of a grouped launch: 0 is what a refused call answers)
 uint64_t grouped_table_bytes(const Grouped& g) {
-  return g.one_launch ? g.first_bytes + g.record_bytes + g.map_bytes + g.term_bytes : 0;
+  return g.one_launch ? std::max<uint64_t>(g.first_bytes + g.record_bytes + g.map_bytes + g.term_bytes, 256) : 0;
 }
 
 uint64_t grouped_workspace(const Grouped& g) {
-  // the table, and behind it the scratch of the groups that run as launches of their own (one launch at a time, so
-  // the largest need serves them all: with a table these are the groups that split K - K = 0 groups need none)
+  // the table, if there is one, and behind it the scratch of the groups that run as launches of their own (one launch at a
+  // time, so the largest need serves them all: these are the groups that split K - K = 0 groups need none)
   if (!g.one_launch) return g.loop_workspace;
   uint64_t most = 0;
   for (int i : g.split_groups) most = g.plans[i].workspace_bytes > most ? g.plans[i].workspace_bytes : most;
@@ -1952,50 +2096,83 @@ int32_t vecops_hip_matmul_grouped(uint32_t count, const VecopsHipOperand* a, con
     rc = run_problem(g.problems[i], g.plans[i], nullptr, nullptr, nullptr, base + table, workspace_size - table, s);
     if (rc != ST_OK) return rc;
   }
-  int32_t* first = reinterpret_cast<int32_t*>(base);
-  TileGemmParams* records = reinterpret_cast<TileGemmParams*>(base + g.first_bytes);
-  int32_t* group_of = reinterpret_cast<int32_t*>(base + g.first_bytes + g.record_bytes);
-  const int groups = static_cast<int>(g.table_groups.size());
-  const int ktile = k_tile_elements(g.src);
-  for (int offset = 0; offset < groups; offset += kGroupChunk) {
-    GroupChunk chunk;
-    memset(&chunk, 0, sizeof(chunk));
-    chunk.offset = offset;
-    chunk.count = groups - offset < kGroupChunk ? groups - offset : kGroupChunk;
-    for (int j = 0; j < chunk.count; ++j) {
-      const Problem& pr = g.problems[g.table_groups[offset + j]];
-      if (pr.a.data == nullptr || pr.b.data == nullptr || pr.c.data == nullptr)
-        return fail(ST_INVALID, "matmul_grouped: group %d has an operand without storage", g.table_groups[offset + j]);
-      TileGemmParams& p = chunk.params[j];
-      p = base_params(pr, nullptr, nullptr, nullptr, nullptr);
-      if (g.src == SRC_I8_FLIP) {
-        char* terms = base + g.first_bytes + g.record_bytes + g.map_bytes + g.term_offset[offset + j];
-        rc = unsigned_side_terms(pr, &p, reinterpret_cast<int32_t*>(terms), s);
-        if (rc != ST_OK) return rc;
-      }
-      p.tiles_m = static_cast<int32_t>((pr.m + g.tile - 1) / g.tile);
-      p.tiles_n = static_cast<int32_t>((pr.n + g.tile - 1) / g.tile);
-      p.split_k = 1;
-      p.k_tiles_per_split = static_cast<int32_t>((pr.k + ktile - 1) / ktile);
+  // groups on slim tiles
+  for (size_t offset = 0; offset < g.slim_groups.size(); offset += kGroupsInline) {
+    GroupLaunch t;
+    memset(&t, 0, sizeof(t));
+    int64_t next = 0;
+    const int part = static_cast<int>(std::min<size_t>(g.slim_groups.size() - offset, kGroupsInline));
+    for (int j = 0; j < part; ++j) {
+      const Problem& pr = g.problems[g.slim_groups[offset + j]];
+      if (rc = group_record(pr, g.slim_groups[offset + j], &t.groups.params[j]); rc != ST_OK) return rc;
+      t.groups.first[j] = static_cast<int32_t>(next);
+      const int64_t wgs = ((pr.m + g.slim_bm - 1) / g.slim_bm) * ((pr.n + g.slim_bn - 1) / g.slim_bn) * pr.batch;
+      next += (wgs + 7) & ~int64_t{7};
     }
-    for (int j = 0; j <= chunk.count; ++j) chunk.first[j] = g.first[offset + j];
-    int longest = 0;  // workgroups of the chunk's longest run
-    for (int j = 0; j < chunk.count; ++j) longest = std::max(longest, chunk.first[j + 1] - chunk.first[j]);
-    const int shares = std::min(std::max((longest + 255) / 256, 1), 64);
-    hipLaunchKernelGGL(write_groups_kernel, dim3(chunk.count, shares), dim3(256), 0, s, chunk, first, records, group_of);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return fail(ST_EXEC, "group table launch: %s", hipGetErrorString(e));
+    end_of_groups(&t.groups, part, next);
+    hipError_t e = launch_tile_gemm_slim_grouped(g.src, t, static_cast<int32_t>(next), g.slim_bm, g.slim_bn, s);
+    if (e != hipSuccess) return fail(ST_EXEC, "grouped slim kernel launch: %s", hipGetErrorString(e));
+  }
+  const int groups = static_cast<int>(g.table_groups.size());
+  if (groups == 0) return ST_OK;
+  GroupLaunch t;
+  memset(&t, 0, sizeof(t));
+  if (g.inline_groups) {
+    for (int j = 0; j < groups; ++j) {
+      if (rc = group_record(g.problems[g.table_groups[j]], g.table_groups[j], &t.groups.params[j]); rc != ST_OK) return rc;
+      t.groups.first[j] = g.first[j];
+    }
+    end_of_groups(&t.groups, groups, g.first[groups]);
+  } else {
+    int32_t* first = reinterpret_cast<int32_t*>(base);
+    int32_t* group_of = reinterpret_cast<int32_t*>(base + g.first_bytes + g.record_bytes);
+    auto write_table = [&](auto record_tag) -> int32_t {
+      using Record = decltype(record_tag);
+      Record* records = reinterpret_cast<Record*>(base + g.first_bytes);
+      constexpr int kMost = GroupChunk<Record>::kMost;
+      for (int offset = 0; offset < groups; offset += kMost) {
+        GroupChunk<Record> chunk;
+        memset(&chunk, 0, sizeof(chunk));
+        chunk.offset = offset;
+        chunk.count = groups - offset < kMost ? groups - offset : kMost;
+        for (int j = 0; j < chunk.count; ++j) {
+          const int number = g.table_groups[offset + j];
+          const Problem& pr = g.problems[number];
+          if constexpr (std::is_same<Record, GroupRecord>::value) {
+            if (int32_t one = group_record(pr, number, &chunk.params[j]); one != ST_OK) return one;
+          } else {
+            if (pr.a.data == nullptr || pr.b.data == nullptr || pr.c.data == nullptr)
+              return fail(ST_INVALID, "matmul_grouped: group %d has an operand without storage", number);
+            chunk.params[j] = base_params(pr, nullptr, nullptr, nullptr, nullptr);
+            char* terms = base + g.first_bytes + g.record_bytes + g.map_bytes + g.term_offset[offset + j];
+            if (int32_t one = unsigned_side_terms(pr, &chunk.params[j], reinterpret_cast<int32_t*>(terms), s); one != ST_OK) return one;
+          }
+        }
+        for (int j = 0; j <= chunk.count; ++j) chunk.first[j] = g.first[offset + j];
+        int longest = 0;  // workgroups of the chunk's longest run
+        for (int j = 0; j < chunk.count; ++j) longest = std::max(longest, chunk.first[j + 1] - chunk.first[j]);
+        const int shares = std::min(std::max((longest + 255) / 256, 1), 64);
+        hipLaunchKernelGGL(write_groups_kernel<Record>, dim3(chunk.count, shares), dim3(256), 0, s, chunk, first, records, group_of);
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return fail(ST_EXEC, "group table launch: %s", hipGetErrorString(e));
+      }
+      t.table = records;
+      return ST_OK;
+    };
+    rc = g.src == SRC_I8_FLIP ? write_table(TileGemmParams{}) : write_table(GroupRecord{});
+    if (rc != ST_OK) return rc;
+    t.group_of = group_of;
+    t.first = first;
   }
   const int32_t workgroups = g.first.back();
   hipError_t e = hipSuccess;
-  GroupedTables t{group_of, first, records, workgroups};
   switch (g.src) {
-    case SRC_BF16: e = launch_tile_gemm_grouped_bf16(t, g.tile, g.mode, s); break;
-    case SRC_F16: e = launch_tile_gemm_grouped_f16(t, g.tile, g.mode, s); break;
-    case SRC_F32_AS_BF16: e = launch_tile_gemm_grouped_f32_as_bf16(t, g.tile, g.mode, s); break;
-    case SRC_F32: e = launch_tile_gemm_grouped_f32(t, g.tile, g.mode, s); break;
-    case SRC_I8_FLIP: e = launch_tile_gemm_grouped_i8_flip(t, g.tile, g.mode, s); break;
-    default: e = launch_tile_gemm_grouped_i8(t, g.tile, g.mode, s); break;
+    case SRC_BF16: e = launch_tile_gemm_grouped_bf16(t, workgroups, g.tile, g.mode, s); break;
+    case SRC_F16: e = launch_tile_gemm_grouped_f16(t, workgroups, g.tile, g.mode, s); break;
+    case SRC_F32_AS_BF16: e = launch_tile_gemm_grouped_f32_as_bf16(t, workgroups, g.tile, g.mode, s); break;
+    case SRC_F32: e = launch_tile_gemm_grouped_f32(t, workgroups, g.tile, g.mode, s); break;
+    case SRC_I8_FLIP: e = launch_tile_gemm_grouped_i8_flip(t, workgroups, g.tile, g.mode, s); break;
+    default: e = launch_tile_gemm_grouped_i8(t, workgroups, g.tile, g.mode, s); break;
   }
   if (e != hipSuccess) return fail(ST_EXEC, "grouped tile kernel launch: %s", hipGetErrorString(e));
   return ST_OK;

@@ -1,7 +1,7 @@
 // f16 x f16: tile GEMM instances of the grouped launch.
 #include "tile_gemm_launch.h"
 namespace vecops_hip {
-hipError_t launch_tile_gemm_grouped_f16(const GroupedTables& t, int tile, int mode, hipStream_t stream) {
-  return launch_grouped_class<SRC_F16>(t, tile, mode, stream);
+hipError_t launch_tile_gemm_grouped_f16(const GroupLaunch& t, int32_t workgroups, int tile, int mode, hipStream_t stream) {
+  return launch_grouped_class<SRC_F16>(t, workgroups, tile, mode, stream);
 }
 }  // namespace vecops_hip

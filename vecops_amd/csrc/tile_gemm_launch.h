@@ -163,16 +163,8 @@ hipError_t launch_tile_class(const TileGemmParams& p, int tile_m, int tile_n, in
   return launch_tile_mode<SRC, 2, 2, 1, 1>(p, mode, stream);
 }
 
-// A grouped launch: the device tables written by launch_group_tables, `workgroups` = first[groups].
-struct GroupedTables {
-  const int32_t* group_of;
-  const int32_t* first;
-  const TileGemmParams* groups;
-  int32_t workgroups;
-};
-
 template <int SRC, int WAVES_M, int WAVES_N, int WM, int WN, int LA, int LB, bool M16 = kShortMfma<SRC, WM, WN>>
-hipError_t launch_grouped_instance(const GroupedTables& t, hipStream_t stream) {
+hipError_t launch_grouped_instance(const GroupLaunch& t, int32_t workgroups, hipStream_t stream) {
   constexpr int kLds = kTileLdsBytes<WAVES_M, WAVES_N, WM, WN, LB>();
   constexpr int kThreads = 64 * WAVES_M * WAVES_N;
   auto kernel = tile_gemm_grouped_kernel<SRC, WAVES_M, WAVES_N, WM, WN, LA, LB, M16>;
@@ -185,28 +177,27 @@ hipError_t launch_grouped_instance(const GroupedTables& t, hipStream_t stream) {
     if (e != hipSuccess) return e;
     configured_device = device;
   }
-  if (t.workgroups <= 0) return hipErrorInvalidConfiguration;
-  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(t.workgroups)), dim3(kThreads), kLds, stream, t.group_of, t.first,
-                     t.groups);
+  if (workgroups <= 0) return hipErrorInvalidConfiguration;
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(workgroups)), dim3(kThreads), kLds, stream, t);
   return hipGetLastError();
 }
 
 // Square tiles of 256, 128 or 64.
 template <int SRC>
-hipError_t launch_grouped_class(const GroupedTables& t, int tile, int mode, hipStream_t stream) {
+hipError_t launch_grouped_class(const GroupLaunch& t, int32_t workgroups, int tile, int mode, hipStream_t stream) {
   auto go = [&](auto wm_tag) {
     constexpr int W = decltype(wm_tag)::value;
     return with_loaders<SRC, 2, 2, W, W>(mode, [&](auto la, auto lb) {
-      return launch_grouped_instance<SRC, 2, 2, W, W, decltype(la)::value, decltype(lb)::value>(t, stream);
+      return launch_grouped_instance<SRC, 2, 2, W, W, decltype(la)::value, decltype(lb)::value>(t, workgroups, stream);
     });
   };
   if (tile == 256) {
     // as a single product's 256 x 256 tiles: the written-out K loop where the loads write LDS themselves (the table's
     // mode is that of its weakest group, and none of them then needs more than 32-bit K offsets)
     if constexpr (SRC == SRC_BF16 || SRC == SRC_F16 || SRC == SRC_I8) {
-      if (mode == MODE_KVEC_DMA) return launch_grouped_instance<SRC, 2, 2, 4, 4, LOAD_KDMA, LOAD_KDMA, true>(t, stream);
+      if (mode == MODE_KVEC_DMA) return launch_grouped_instance<SRC, 2, 2, 4, 4, LOAD_KDMA, LOAD_KDMA, true>(t, workgroups, stream);
       if constexpr (SRC != SRC_I8) {
-        if (mode == MODE_NVEC_B_DMA) return launch_grouped_instance<SRC, 2, 2, 4, 4, LOAD_KDMA, LOAD_NTR_DMA, true>(t, stream);
+        if (mode == MODE_NVEC_B_DMA) return launch_grouped_instance<SRC, 2, 2, 4, 4, LOAD_KDMA, LOAD_NTR_DMA, true>(t, workgroups, stream);
       }
     }
     return go(std::integral_constant<int, 4>{});
@@ -230,6 +221,8 @@ hipError_t launch_tile_gemm_deep_f32(const TileGemmParams& p, int tile, bool b_a
 // operands, both K-contiguous at any alignment; bm x bn one of 32 x {16, 32, 48, 64}, 64 x {48, 64}, 128 x {48, 64}.
 bool launch_tile_gemm_slim_serves(int src, const TileGemmParams& p);
 hipError_t launch_tile_gemm_slim(int src, const TileGemmParams& p, int bm, int bn, hipStream_t stream);
+// the same for the groups in the launch's own arguments; bm x bn one of 32 x {32, 64}, 64 x 64, 128 x 64
+hipError_t launch_tile_gemm_slim_grouped(int src, const GroupLaunch& t, int32_t workgroups, int bm, int bn, hipStream_t stream);
 // The 128 x 256 tile for K-contiguous bf16, f16 or signed 8-bit operands with rows at any alignment (tile_gemm_rows.hip).
 bool launch_tile_gemm_rows_serves(int src, const TileGemmParams& p);
 hipError_t launch_tile_gemm_rows(int src, const TileGemmParams& p, hipStream_t stream);
@@ -237,12 +230,12 @@ hipError_t launch_tile_gemm_rows(int src, const TileGemmParams& p, hipStream_t s
 // (tile_gemm_short_k.hip).
 bool launch_tile_gemm_short_k_serves(int src, const TileGemmParams& p);
 hipError_t launch_tile_gemm_short_k(int src, TileGemmParams p, hipStream_t stream);
-hipError_t launch_tile_gemm_grouped_bf16(const GroupedTables& t, int tile, int mode, hipStream_t stream);
-hipError_t launch_tile_gemm_grouped_i8(const GroupedTables& t, int tile, int mode, hipStream_t stream);
-hipError_t launch_tile_gemm_grouped_i8_flip(const GroupedTables& t, int tile, int mode, hipStream_t stream);
-hipError_t launch_tile_gemm_grouped_f16(const GroupedTables& t, int tile, int mode, hipStream_t stream);
-hipError_t launch_tile_gemm_grouped_f32_as_bf16(const GroupedTables& t, int tile, int mode, hipStream_t stream);
-hipError_t launch_tile_gemm_grouped_f32(const GroupedTables& t, int tile, int mode, hipStream_t stream);
+hipError_t launch_tile_gemm_grouped_bf16(const GroupLaunch& t, int32_t workgroups, int tile, int mode, hipStream_t stream);
+hipError_t launch_tile_gemm_grouped_i8(const GroupLaunch& t, int32_t workgroups, int tile, int mode, hipStream_t stream);
+hipError_t launch_tile_gemm_grouped_i8_flip(const GroupLaunch& t, int32_t workgroups, int tile, int mode, hipStream_t stream);
+hipError_t launch_tile_gemm_grouped_f16(const GroupLaunch& t, int32_t workgroups, int tile, int mode, hipStream_t stream);
+hipError_t launch_tile_gemm_grouped_f32_as_bf16(const GroupLaunch& t, int32_t workgroups, int tile, int mode, hipStream_t stream);
+hipError_t launch_tile_gemm_grouped_f32(const GroupLaunch& t, int32_t workgroups, int tile, int mode, hipStream_t stream);
 
 }  // namespace vecops_hip
 #endif

@@ -47,8 +47,9 @@ struct SlimTile {
   static_assert(kLds <= 160 * 1024, "LDS of a compute unit");
 };
 
+// The work of one workgroup: number `pid` of the `total` that serve the problem `p`.
 template <int SRC, int BM, int BN>
-__global__ __launch_bounds__(kThreads, 2) void tile_gemm_slim_kernel(const TileGemmParams p) {
+__device__ __forceinline__ void slim_workgroup(const TileGemmParams& p, int pid, int total) {
   using T = SrcTraits<SRC>;
   using L = SlimTile<BM, BN>;
   using Quad = typename AccQuad<T::kInt>::type;
@@ -59,8 +60,9 @@ __global__ __launch_bounds__(kThreads, 2) void tile_gemm_slim_kernel(const TileG
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave & 1, wk = wave >> 1;  // half of the rows, quarter of a stage's K
   int batch, split, tm, tn;
-  map_workgroup(p, blockIdx.x, gridDim.x, batch, split, tm, tn);
+  map_workgroup(p, pid, total, batch, split, tm, tn);
   batch = __builtin_amdgcn_readfirstlane(batch);
+  if (batch >= p.batch) return;  // a grouped launch rounds each group's run of workgroups up to a multiple of eight
   tm = __builtin_amdgcn_readfirstlane(tm);
   tn = __builtin_amdgcn_readfirstlane(tn);
   const int m0 = tm * BM, n0 = tn * BN;
@@ -258,18 +260,60 @@ __global__ __launch_bounds__(kThreads, 2) void tile_gemm_slim_kernel(const TileG
 }
 
 template <int SRC, int BM, int BN>
-hipError_t launch(TileGemmParams p, hipStream_t stream) {
-  auto kernel = tile_gemm_slim_kernel<SRC, BM, BN>;
-  constexpr int kLds = SlimTile<BM, BN>::kLds;
+__global__ __launch_bounds__(kThreads, 2) void tile_gemm_slim_kernel(const TileGemmParams p) {
+  slim_workgroup<SRC, BM, BN>(p, blockIdx.x, gridDim.x);
+}
+
+// Several problems in one launch: the groups of a grouped call that split K on their own.  Each of them a launch (and mostly
+// two) of its own, a call over eighteen groups of 43 x 409 x 1985 took 155 us; together 15.
+template <int SRC, int BM, int BN>
+__global__ __launch_bounds__(kThreads, 2) void tile_gemm_slim_grouped_kernel(const GroupLaunch) {
+  int begin = 0, end = 0;
+  const TileGemmParams p = group_problem<SRC>(BM, BN, blockIdx.x, begin, end);
+  slim_workgroup<SRC, BM, BN>(p, static_cast<int>(blockIdx.x) - begin, end - begin);
+}
+
+// > 64 KiB of dynamic LDS has to be enabled once per kernel and device; cheap enough to repeat per thread.
+template <auto KERNEL, int LDS>
+hipError_t allow_lds() {
   static thread_local int configured_device = -1;
   int device = 0;
   hipError_t e = hipGetDevice(&device);
   if (e != hipSuccess) return e;
   if (configured_device != device) {
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(KERNEL), hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
     if (e != hipSuccess) return e;
     configured_device = device;
   }
+  return hipSuccess;
+}
+
+template <int SRC, int BM, int BN>
+hipError_t launch_grouped(const GroupLaunch& t, int32_t workgroups, hipStream_t stream) {
+  constexpr auto kernel = tile_gemm_slim_grouped_kernel<SRC, BM, BN>;
+  constexpr int kLds = SlimTile<BM, BN>::kLds;
+  if (hipError_t e = allow_lds<kernel, kLds>(); e != hipSuccess) return e;
+  if (workgroups <= 0) return hipErrorInvalidConfiguration;
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(workgroups)), dim3(kThreads), kLds, stream, t);
+  return hipGetLastError();
+}
+
+template <int SRC>
+hipError_t launch_grouped_tile(const GroupLaunch& t, int32_t workgroups, int bm, int bn, hipStream_t stream) {
+  switch (bm * 1000 + bn) {
+    case 32032: return launch_grouped<SRC, 32, 32>(t, workgroups, stream);
+    case 32064: return launch_grouped<SRC, 32, 64>(t, workgroups, stream);
+    case 64064: return launch_grouped<SRC, 64, 64>(t, workgroups, stream);
+    case 128064: return launch_grouped<SRC, 128, 64>(t, workgroups, stream);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+template <int SRC, int BM, int BN>
+hipError_t launch(TileGemmParams p, hipStream_t stream) {
+  constexpr auto kernel = tile_gemm_slim_kernel<SRC, BM, BN>;
+  constexpr int kLds = SlimTile<BM, BN>::kLds;
+  if (hipError_t e = allow_lds<kernel, kLds>(); e != hipSuccess) return e;
   p.tiles_m = (p.m + BM - 1) / BM;
   p.tiles_n = (p.n + BN - 1) / BN;
   p.split_k = 1;
@@ -310,6 +354,15 @@ hipError_t launch_tile_gemm_slim(int src, const TileGemmParams& p, int bm, int b
     case SRC_BF16: return launch_class<SRC_BF16>(p, bm, bn, stream);
     case SRC_F16: return launch_class<SRC_F16>(p, bm, bn, stream);
     case SRC_I8: return launch_class<SRC_I8>(p, bm, bn, stream);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+hipError_t launch_tile_gemm_slim_grouped(int src, const GroupLaunch& t, int32_t workgroups, int bm, int bn, hipStream_t stream) {
+  switch (src) {
+    case SRC_BF16: return launch_grouped_tile<SRC_BF16>(t, workgroups, bm, bn, stream);
+    case SRC_F16: return launch_grouped_tile<SRC_F16>(t, workgroups, bm, bn, stream);
+    case SRC_I8: return launch_grouped_tile<SRC_I8>(t, workgroups, bm, bn, stream);
     default: return hipErrorInvalidValue;
   }
 }
