@@ -298,6 +298,8 @@ struct RuleConstants {
   // -- 128x128 tiles that leave a compute unit at most one workgroup run the four-stage kernel (tile_gemm_deep128.hip),
   //    from this many K tiles per workgroup on (rule_check, 1024 x 4096 x 4096)
   int64_t deep_max_workgroups = 256, deep_min_k_tiles = 8;
+  //    and with rows that are not 16-byte aligned from this many on (deep128_fits)
+  int64_t deep_unaligned_k_tiles = 48;
   // -- planning for that kernel (operands it serves): from deep_alone_from_tiles tiles of 128x128 on (three eighths of the
   //    units) the tiles stay whole or split in two, whichever the split rule's costs favour, with deep_k_tile_ns per K
   //    tile (a lone workgroup of this kernel walks a K tile in 0.3 us) and deep_fixed_ns per launch; between
@@ -329,7 +331,7 @@ struct RuleConstants {
   int64_t slim_margin_num = 95, slim_margin_den = 100;
   int64_t own_64_ns = 3640, own_64_tile_ns = 320, own_64_ns_per_wg = 415, own_64_ns_per_wg_shared = 300, own_64_staged = 1360;
   int64_t own_64_split_ns = 4430, own_64_ns_per_mb = 275;
-  int64_t own_deep_ns = 5000, own_deep_tile_ns = 440, own_deep_ns_per_operand_mb = 46, own_deep_split_ns = 3650, own_deep_ns_per_mb = 585;
+  int64_t own_deep_ns = 5000, own_deep_tile_ns = 440, own_deep_unaligned_tile_ns = 660, own_deep_ns_per_operand_mb = 46, own_deep_split_ns = 3650, own_deep_ns_per_mb = 585;
 };
 constexpr RuleConstants kRules{};
 
@@ -404,6 +406,19 @@ void finish_tile_plan(const Problem& pr, VecopsHipPlan* plan, uint32_t forced_sp
 
 int fetch_mode(const Problem& pr, const VecopsHipPlan& plan);
 bool lines_up(const Problem& pr, const View& v, int64_t line_stride);
+
+// Whether the four-stage 128x128 kernel is the one for `tiles` such tiles and operands fetched like that (not prepacked).  Its
+// loads take rows at any alignment and it walks a partial K tile; where it replaces what the table took before (us, before -> now,
+// bf16): 1000 x 4000 x 4008 57 -> 50, 768 x 3000 x 2008 30.6 -> 24.8, 2000 x 2000 x 1000 19.7 -> 17.7, but 700 x 2048 x 1096, 96
+// tiles, 14.8 on 64x64 tiles -> 15.9: a partial K tile's checked start wants more than half the units in use.  Rows that are
+// not 16-byte aligned: with a long K and up to three quarters of the units in use 1728 x 1280 x 7853 122 -> 89, 186 x 3712 x 11835 73 -> 58,
+// 300 x 4000 x 4001 44 -> 37 (64x64 tiles before); beyond, the two-stage kernel is level or ahead (int8 2000 x 2000 x 2001 23.5
+// against 24.8).  B as [K,N] at any alignment: 300 x 4001 x 4000 37 -> 34, 512 x 4097 x 1000 18.9 -> 16.7.
+bool deep128_fits(const Problem& pr, int mode, int64_t tiles) {
+  const int64_t ktile = k_tile_elements(pr.src), k_tiles = (pr.k + ktile - 1) / ktile;
+  if (mode == MODE_KVEC) return k_tiles >= kRules.deep_unaligned_k_tiles && tiles <= kRules.lonely_tiles_num * kComputeUnits / kRules.lonely_tiles_den;
+  return mode == MODE_NVEC_B || pr.k % ktile == 0 || tiles > kComputeUnits / 2;
+}
 
 // The two halves of a problem cut between columns n_main - 1 and n_main of C: rows of B, columns of C and C_in.
 void cut_columns(const Problem& pr, int64_t n_main, Problem* main, Problem* rest) {
@@ -582,16 +597,16 @@ void choose_table(const Problem& pr, VecopsHipPlan* plan, uint64_t scratch_limit
   }
   const int64_t ktile = k_tile_elements(pr.src);
   const int64_t k_tiles = (pr.k + ktile - 1) / ktile;
-  // operands the four-stage 128x128 kernel (tile_gemm_deep128.hip) serves: fetched by loads that write LDS (both
-  // K-contiguous, or 16-bit operands with B as [K,N]), K in whole K tiles
-  const bool deep_tr = mode == MODE_NVEC_B_DMA && (pr.src == SRC_BF16 || pr.src == SRC_F16) && pr.n % 8 == 0 &&
+  // operands the four-stage 128x128 kernel (tile_gemm_deep128.hip) serves: both K-contiguous, or 16-bit operands with B as
+  // [K,N]; a prepacked B with K in whole K tiles
+  const bool deep_tr = (mode == MODE_NVEC_B_DMA || mode == MODE_NVEC_B) && (pr.src == SRC_BF16 || pr.src == SRC_F16) &&
                        pr.k * pr.b.cs * 2 + 256 < (int64_t{1} << 31);   // B as [K,N]: 16-bit operands, 32-bit K offsets
   // (a prepacked B keeps its pack order in LDS there: A's alignment decides)
   const bool deep_pk = pr.packed_b && (pr.src == SRC_BF16 || pr.src == SRC_F16 || pr.src == SRC_I8) && plan->vector_a != 0 &&
                        lines_up(pr, pr.a, pr.a.rs);
   const bool deep_ok = (pr.packed_b ? deep_pk
-                                    : (mode == MODE_KVEC_DMA && (pr.src == SRC_BF16 || pr.src == SRC_F16 || pr.src == SRC_I8)) || deep_tr) &&
-                       pr.k % ktile == 0 && k_tiles >= kRules.deep_min_k_tiles;
+                                    : ((mode == MODE_KVEC_DMA || mode == MODE_KVEC) && (pr.src == SRC_BF16 || pr.src == SRC_F16 || pr.src == SRC_I8)) || deep_tr) &&
+                       (pr.packed_b ? pr.k % ktile == 0 : deep128_fits(pr, mode, tiles(128))) && k_tiles >= kRules.deep_min_k_tiles;
   // At most four K tiles of 16-bit or 8-bit operands: the tile's life is its start-up and its stores, and
   // two or three 128x128 workgroups on a compute unit overlap one's stores with another's loads, which a
   // single big tile cannot (batch 8 of 3000x3000x17 to fp32: 93 us against 111; 8 x 1000x1000x100: 17.7
@@ -633,7 +648,7 @@ void choose_table(const Problem& pr, VecopsHipPlan* plan, uint64_t scratch_limit
   // with thirty-two per part - bf16 1024 x 4096 x 4096, int8 ... x 8192 - the unsplit tiles are level or ahead).
   uint32_t band_split = 0;
   bool deep_planned = false;
-  if (((direct && !pr.packed_b) || (deep_pk && deep_ok)) && (family == VECOPS_HIP_FAMILY_TILE_64 || family == VECOPS_HIP_FAMILY_TILE_128) &&
+  if (((direct && !pr.packed_b) || deep_ok) && (family == VECOPS_HIP_FAMILY_TILE_64 || family == VECOPS_HIP_FAMILY_TILE_128) &&
       tiles(128) >= kComputeUnits / 8 && tiles(128) <= kComputeUnits) {
     const int64_t count = tiles(128);
     int64_t parts = kRules.small_tile_workgroups_per_unit * kComputeUnits / count;
@@ -645,9 +660,11 @@ void choose_table(const Problem& pr, VecopsHipPlan* plan, uint64_t scratch_limit
     // unsplit 31-34 us against 43 on the two-stage kernel, 768 x 4096 x 4096 27 against 38 in two parts, 512 x 4096 x
     // 4096 25 against 28 on 64x64 tiles, 1024 x 4096 x 11008 79 against 84 on the big tile in four parts; int8
     // 1024 x 4096 x 4096 21 against 28): at most one workgroup per unit, K split only to fill the units.
-    const bool idle_units_long_k = count > kComputeUnits / 2 && count <= kRules.deep_idle_tiles &&
+    const bool idle_units_long_k = direct && count > kComputeUnits / 2 && count <= kRules.deep_idle_tiles &&
                                    k_tiles / parts >= kRules.deep_idle_k_tiles_per_part && fits;
-    if (deep_ok && count >= kRules.deep_alone_from_tiles && !idle_units_long_k) {
+    // (with a partial last K tile the two-stage kernel's split stays as well where its parts are long enough)
+    const bool ragged_long_k = direct && !pr.packed_b && pr.k % ktile != 0 && k_tiles / parts >= least && fits;
+    if (deep_ok && count >= kRules.deep_alone_from_tiles && !idle_units_long_k && !ragged_long_k) {
       // whole, or in two parts where the units allow and the split rule's costs favour it
       int64_t best_parts = 1;
       if (2 * count <= kRules.deep_max_workgroups && k_tiles / 2 >= kRules.deep_min_k_tiles &&
@@ -671,7 +688,7 @@ void choose_table(const Problem& pr, VecopsHipPlan* plan, uint64_t scratch_limit
       family = VECOPS_HIP_FAMILY_TILE_128;
       band_split = static_cast<uint32_t>(kRules.deep_max_workgroups / count);
       deep_planned = true;
-    } else if (!pr.packed_b && k_tiles / parts >= least && fits) {
+    } else if (direct && !pr.packed_b && k_tiles / parts >= least && fits) {
       family = VECOPS_HIP_FAMILY_TILE_128;
       band_split = static_cast<uint32_t>(parts);
     }
@@ -953,6 +970,7 @@ void set_tiles(const Problem& pr, const VecopsHipPlan& plan, TileGemmParams* p) 
 bool deep128_runs(const Problem& pr, const TileGemmParams& p, uint32_t family, int mode) {
   return family == VECOPS_HIP_FAMILY_TILE_128 && p.k_tiles_per_split >= kRules.deep_min_k_tiles &&
          static_cast<int64_t>(p.tiles_m) * p.tiles_n * p.batch * p.split_k <= kRules.deep_max_workgroups &&
+         (pr.packed_b || deep128_fits(pr, mode, static_cast<int64_t>(p.tiles_m) * p.tiles_n * p.batch)) &&
          launch_tile_gemm_deep128_serves(pr.src, p, mode, pr.packed_b);
 }
 
@@ -988,7 +1006,8 @@ int64_t own_plan_ns(const Problem& pr, const VecopsHipPlan& plan) {
   } else {
     if (!deep128_runs(pr, p, plan.family, mode)) return -1;
     const int64_t operands = pr.batch * (pr.m + pr.n) * k_tiles / 8;  // KiB: K tiles of 128 bytes
-    own_ns = kRules.own_deep_ns + p.k_tiles_per_split * kRules.own_deep_tile_ns + operands * kRules.own_deep_ns_per_operand_mb / 1024;
+    const int64_t tile_ns = mode == MODE_KVEC ? kRules.own_deep_unaligned_tile_ns : kRules.own_deep_tile_ns;
+    own_ns = kRules.own_deep_ns + p.k_tiles_per_split * tile_ns + operands * kRules.own_deep_ns_per_operand_mb / 1024;
     if (split > 1) own_ns += kRules.own_deep_split_ns + partials * kRules.own_deep_ns_per_mb / 1024;
   }
   return own_ns;

@@ -4,11 +4,12 @@
 // instance is built for two workgroups per unit, each hiding the other's waits; alone on a unit it waits out every K
 // tile's loads (0.67 us per K tile of 0.25 us of matrix instructions at 1024 x 4096 x 4096).
 //
-// What it serves (launch_tile_gemm_deep128_serves): bf16, f16 or signed 8-bit operands, both K-contiguous with 16-byte
-// aligned bases, rows and batches (the loads write LDS themselves), or - 16-bit operands - B handed over as [K,N]
-// (TR: the tile lies [k][n] in LDS, 64 rows of 256 bytes, swizzled as tile_gemm_kernel's, and the fragment reads
-// transpose); K a whole number of K tiles.  Any M, N, batch count, K split, C input and output type of the class: the
-// epilogue is tile_gemm_kernel's.  PK: B prepacked by vecops_hip_pack_b and kept in its pack order in LDS - a load
+// What it serves (launch_tile_gemm_deep128_serves): bf16, f16 or signed 8-bit operands, both K-contiguous, or - 16-bit
+// operands - B handed over as [K,N] (TR: the tile lies [k][n] in LDS, 64 rows of 256 bytes, swizzled as tile_gemm_kernel's,
+// and the fragment reads transpose); rows at any alignment.  A partial last K tile is walked first, through checked stores
+// into stage 0, while the loads of the next two are under way (1000 x 4000 x 4008: 57 us on the two-stage kernel, 50 here).
+// Any M, N, batch count, K split, C input and output type of the class: the epilogue is tile_gemm_kernel's.  PK (16-byte
+// aligned A, K in whole K tiles): B prepacked by vecops_hip_pack_b and kept in its pack order in LDS - a load
 // instruction of a wavefront moves one whole (panel of 32 rows, k-step of two chunks) block, 1 KiB contiguous on both
 // sides, and a fragment read is the stage pair's one per-lane base plus a constant (as in tile_gemm_packed16.hip).
 #include "tile_gemm_launch.h"
@@ -40,10 +41,14 @@ __global__ __launch_bounds__(256, 1) void tile_gemm_deep128_kernel(const TileGem
   tm = __builtin_amdgcn_readfirstlane(tm);
   tn = __builtin_amdgcn_readfirstlane(tn);
   const int m0 = tm * 128, n0 = tn * 128;
-  const int total_k_tiles = p.k / KTILE;
+  // the walk over K as in tile_gemm_workgroup: a partial last K tile (and, B as [K,N], one whose chunks reach past N) comes
+  // first, through checked stores
+  const int total_k_tiles = (p.k + KTILE - 1) / KTILE;
+  const int full_k_tiles = PK ? total_k_tiles : (p.k - (TR && kn_reaches_past(n0, 128, p.n, 8) ? 1 : 0)) / KTILE;
   const int kt_begin = split * p.k_tiles_per_split;
   const int kt_end = min(total_k_tiles, kt_begin + p.k_tiles_per_split);
   const int nk = __builtin_amdgcn_readfirstlane(max(kt_end - kt_begin, 0));
+  const int has_tail = __builtin_amdgcn_readfirstlane(nk > 0 && kt_end > full_k_tiles ? 1 : 0);
 
   // Loads: instruction i of an operand's K tile fills its rows 32 i .. 32 i + 31, this wavefront eight of them; lane l
   // fetches the chunk of row l / 8 whose swizzled slot is l % 8.  Rows past the operand's extent are clamped onto its
@@ -61,11 +66,10 @@ __global__ __launch_bounds__(256, 1) void tile_gemm_deep128_kernel(const TileGem
     if constexpr (TR) {
       // B as [K,N]: a load instruction of the workgroup fills sixteen k rows of 256 bytes; lane t fetches, of k row
       // t / 16, the chunk of eight columns whose swizzled slot is t % 16 (slot = chunk xor 4 * (k row % 4): the four
-      // rows a transposing read touches lie in different bank groups).  N is a multiple of eight on this path: a chunk
-      // past it is clamped onto the last one.
+      // rows a transposing read touches lie in different bank groups).  A chunk past N is clamped onto the last one.
       const int krow = tid >> 4, slot = tid & 15;
       const int chunk = slot ^ ((krow & 3) << 2);
-      const int col = min(n0 + chunk * 8, p.n - 8) - n0;
+      const int col = min(n0 + chunk * 8, (p.n - 1) & ~7) - n0;
       rows_b[0] = static_cast<uint32_t>((static_cast<int64_t>(krow) * p.b_ks + col) * T::kSrcBytes);
     }
     if constexpr (PK) {
@@ -98,7 +102,7 @@ __global__ __launch_bounds__(256, 1) void tile_gemm_deep128_kernel(const TileGem
     if (t >= nk) da[2] = db[2] = 0u;
     // (wavefront-uniform by construction; said so, or the compiler may carry them in vector registers, which the
     //  load's scalar offset does not take)
-    const uint32_t k_tile = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(kt_begin + t));
+    const uint32_t k_tile = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(max(kt_begin + t - has_tail, 0)));
     const uint32_t k_bytes = k_tile * 128u;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -108,9 +112,18 @@ __global__ __launch_bounds__(256, 1) void tile_gemm_deep128_kernel(const TileGem
       load_16_bytes_into_lds(db, m0_wave, static_cast<uint32_t>(t * kDeepStage + 16384 + i * 4096), rows_b[TR ? 0 : i],
                              TR ? k_tile * step_b + static_cast<uint32_t>(i) * part_b : PK ? k_tile * step_b : k_bytes);
   };
-  fill(0);
+  if (!has_tail) fill(0);
   fill(1);
   fill(2);
+  if constexpr (!PK) {
+    if (has_tail) {
+      const char* a = static_cast<const char*>(p.a) + batch * p.a_bs * T::kSrcBytes;
+      const char* b = static_cast<const char*>(p.b) + batch * p.b_bs * T::kSrcBytes;
+      stage_rows_checked<SRC>(a, p.a_rs, 1, m0, p.m, 128, (kt_end - 1) * KTILE, p.k, lds, tid, 256, 0u);
+      if constexpr (TR) stage_kn_checked(b, p.b_ks, n0, p.n, 128, (kt_end - 1) * KTILE, p.k, lds + 16384, tid, 256);
+      else stage_rows_checked<SRC>(b, p.b_rs, 1, n0, p.n, 128, (kt_end - 1) * KTILE, p.k, lds + 16384, tid, 256, 0u);
+    }
+  }
 
   // Fragment reads: lane l supplies row l % 16 of a block and one of the four chunks of the matrix k-step (the 16-lane
   // groups in the order 0, 2, 1, 3, as in tile_gemm_kernel).  [stage pair][q]: the odd stage lies 32 KiB up.
@@ -144,13 +157,13 @@ __global__ __launch_bounds__(256, 1) void tile_gemm_deep128_kernel(const TileGem
   Accumulators<INT, 2, 2, true> acc;
   acc.clear();
   if (nk > 0) {
-    asm volatile("s_waitcnt vmcnt(16)" ::: "memory");   // tile 0 has landed
+    asm volatile("s_waitcnt vmcnt(16) lgkmcnt(0)" ::: "memory");   // tile 0 has landed
     __builtin_amdgcn_s_barrier();
 #if defined(__HIP_DEVICE_COMPILE__)
     auto uniform = [](uint32_t v) { return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(v)); };
     int left = nk - 3, n = nk;
-    uint32_t k_a = uniform(static_cast<uint32_t>(kt_begin + 3) * 128u);   // the loop fetches tile 3 of the range first
-    uint32_t k_b = uniform(static_cast<uint32_t>(kt_begin + 3) * step_b);
+    uint32_t k_a = uniform(static_cast<uint32_t>(kt_begin + 3 - has_tail) * 128u);   // the loop fetches tile 3 of the range first
+    uint32_t k_b = uniform(static_cast<uint32_t>(kt_begin + 3 - has_tail) * step_b);
     const uint32_t sb = uniform(step_b), pb = uniform(part_b);
     const uint32_t da[4] = {uniform(desc_a[0]), uniform(desc_a[1]), uniform(desc_a[2]), uniform(desc_a[3])};
     const uint32_t db[4] = {uniform(desc_b[0]), uniform(desc_b[1]), uniform(desc_b[2]), uniform(desc_b[3])};
@@ -212,10 +225,10 @@ hipError_t launch(const TileGemmParams& p, hipStream_t stream) {
 
 bool launch_tile_gemm_deep128_serves(int src, const TileGemmParams& p, int mode, bool packed_b) {
   if (src != SRC_BF16 && src != SRC_F16 && src != SRC_I8) return false;
-  const bool tr = !packed_b && mode == MODE_NVEC_B_DMA;
+  const bool tr = !packed_b && (mode == MODE_NVEC_B_DMA || mode == MODE_NVEC_B);
   if (p.m <= 0 || p.n <= 0 || p.split_k < 1) return false;
   const int elem = src == SRC_I8 ? 1 : 2, ktile = 128 / elem;
-  if (p.k < ktile || p.k % ktile != 0) return false;
+  if (p.k < ktile || (packed_b && p.k % ktile != 0)) return false;
   // 32-bit byte offsets inside a tile's 128 rows
   if (128 * p.a_rs * elem + static_cast<int64_t>(p.k) * elem >= (int64_t{1} << 31)) return false;
   if (packed_b) {
@@ -223,13 +236,12 @@ bool launch_tile_gemm_deep128_serves(int src, const TileGemmParams& p, int mode,
     if (p.a_ks != 1 || (reinterpret_cast<uintptr_t>(p.a) & 15u) != 0 || (p.a_rs * elem) % 16 != 0 || (p.a_bs * elem) % 16 != 0) return false;
     return (reinterpret_cast<uintptr_t>(p.b) & 15u) == 0 && 4 * static_cast<int64_t>(p.k / ktile) * 4096 < (int64_t{1} << 31);
   }
-  if ((mode != MODE_KVEC_DMA && !tr) || (tr && src == SRC_I8)) return false;
-  if (tr) return p.n % 8 == 0 && p.n >= 8 && p.b_rs == 1 && static_cast<int64_t>(p.k) * p.b_ks * elem + 256 < (int64_t{1} << 31);
-  return 128 * p.b_rs * elem + static_cast<int64_t>(p.k) * elem < (int64_t{1} << 31);
+  if (tr) return src != SRC_I8 && p.n >= 8 && (p.n % 8 == 0 || p.b_ks >= p.n) && p.b_rs == 1 && static_cast<int64_t>(p.k) * p.b_ks * elem + 256 < (int64_t{1} << 31);
+  return (mode == MODE_KVEC_DMA || mode == MODE_KVEC) && 128 * p.b_rs * elem + static_cast<int64_t>(p.k) * elem < (int64_t{1} << 31);
 }
 
 hipError_t launch_tile_gemm_deep128(int src, const TileGemmParams& p, int mode, bool packed_b, hipStream_t stream) {
-  const bool tr = !packed_b && mode == MODE_NVEC_B_DMA;
+  const bool tr = !packed_b && (mode == MODE_NVEC_B_DMA || mode == MODE_NVEC_B);
   if (packed_b) {
     switch (src) {
       case SRC_BF16: return launch<SRC_BF16, false, true>(p, stream);
