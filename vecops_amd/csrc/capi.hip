@@ -298,8 +298,8 @@ struct RuleConstants {
   // -- 128x128 tiles that leave a compute unit at most one workgroup run the four-stage kernel (tile_gemm_deep128.hip),
   //    from this many K tiles per workgroup on (rule_check, 1024 x 4096 x 4096)
   int64_t deep_max_workgroups = 256, deep_min_k_tiles = 8;
-  //    and with rows that are not 16-byte aligned from this many on (deep128_fits)
-  int64_t deep_unaligned_k_tiles = 48;
+  //    and with rows that are not 16-byte aligned from this many K tiles and a fifth of the units on (deep128_fits)
+  int64_t deep_unaligned_k_tiles = 48, deep_unaligned_units_den = 5;
   // -- planning for that kernel (operands it serves): from deep_alone_from_tiles tiles of 128x128 on (three eighths of the
   //    units) the tiles stay whole or split in two, whichever the split rule's costs favour, with deep_k_tile_ns per K
   //    tile (a lone workgroup of this kernel walks a K tile in 0.3 us) and deep_fixed_ns per launch; between
@@ -412,11 +412,14 @@ bool lines_up(const Problem& pr, const View& v, int64_t line_stride);
 // bf16): 1000 x 4000 x 4008 57 -> 50, 768 x 3000 x 2008 30.6 -> 24.8, 2000 x 2000 x 1000 19.7 -> 17.7, but 700 x 2048 x 1096, 96
 // tiles, 14.8 on 64x64 tiles -> 15.9: a partial K tile's checked start wants more than half the units in use.  Rows that are
 // not 16-byte aligned: with a long K and up to three quarters of the units in use 1728 x 1280 x 7853 122 -> 89, 186 x 3712 x 11835 73 -> 58,
-// 300 x 4000 x 4001 44 -> 37 (64x64 tiles before); beyond, the two-stage kernel is level or ahead (int8 2000 x 2000 x 2001 23.5
+// 300 x 4000 x 4001 44 -> 37 (64x64 and slim tiles before; on less than a fifth slim tiles are ahead, 150 x 3000 x 5001 23.4
+// against 24.9); beyond, the two-stage kernel is level or ahead (int8 2000 x 2000 x 2001 23.5
 // against 24.8).  B as [K,N] at any alignment: 300 x 4001 x 4000 37 -> 34, 512 x 4097 x 1000 18.9 -> 16.7.
 bool deep128_fits(const Problem& pr, int mode, int64_t tiles) {
   const int64_t ktile = k_tile_elements(pr.src), k_tiles = (pr.k + ktile - 1) / ktile;
-  if (mode == MODE_KVEC) return k_tiles >= kRules.deep_unaligned_k_tiles && tiles <= kRules.lonely_tiles_num * kComputeUnits / kRules.lonely_tiles_den;
+  if (mode == MODE_KVEC)
+    return k_tiles >= kRules.deep_unaligned_k_tiles && tiles * kRules.deep_unaligned_units_den >= kComputeUnits &&
+           tiles <= kRules.lonely_tiles_num * kComputeUnits / kRules.lonely_tiles_den;
   return mode == MODE_NVEC_B || pr.k % ktile == 0 || tiles > kComputeUnits / 2;
 }
 
