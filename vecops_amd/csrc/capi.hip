@@ -247,6 +247,12 @@ constexpr int kStreamGroupsPerUnit = 2;  // workgroups of 4 wavefronts per compu
 // rectangles on the 16x16 shapes; 133 / 130 before), int8 4096^3 58 / 75 / 77 / 70 (`bench.py --only families`,
 // `--only rule_check`).
 constexpr int64_t kQuality256x128 = 800, kQuality128 = 900, kQuality128Int8 = 970, kQuality128Staged = 850;
+// K-contiguous 16-bit and 8-bit rows at any alignment: the 128x256 tile has a kernel of its own for them (tile_gemm_rows.hip),
+// and more 128x128 tiles than units run in pairs there as well (bf16, us on 256x256 / 256x128 / 128x256 / 128x128 tiles: 5000 x
+// 4000 x 2001 126 / 134 / 115 / 132, 2500 x 2500 x 2501 81 / 55 / 49 / 62, 2048 x 4096 x 4097 93 / 82 / 78 / 90, 1536 x 4096 x 4097
+// 91 / 74 / 69 / 84, 4096 x 4096 x 4097 129 / 162 / 151 / 180; of fifteen such shapes 512 x 9600 x 4359, 130 / 93 / 100 / 114, is
+// the one that loses; bytes keep their 128x128 pricing, with which 5000 x 4000 x 2001 is level).
+constexpr int64_t kQuality128x256Rows = 820, kQuality128RowPairs = 716;
 constexpr int64_t kQuality256x128Direct = 780, kQuality128Direct = 830, kQuality128Int8Direct = 850, kQuality192 = 850;
 
 // Every other number the rule table and the split rule compare against, in one place, each with the mechanism it
@@ -533,9 +539,11 @@ void choose_table(const Problem& pr, VecopsHipPlan* plan, uint64_t scratch_limit
   const bool bytes = pr.src == SRC_I8 || pr.src == SRC_I8_FLIP;
   const int mode = fetch_mode(pr, *plan);
   const bool direct = mode == MODE_KVEC_DMA || mode == MODE_NVEC_B_DMA;  // loads that write LDS themselves
+  const bool any_rows = mode == MODE_KVEC && (pr.src == SRC_BF16 || pr.src == SRC_F16 || pr.src == SRC_I8);
   const Candidate candidates[] = {{VECOPS_HIP_FAMILY_TILE_256, 256, 256, 1000},
                                   {VECOPS_HIP_FAMILY_TILE_256X128, 256, 128, direct ? kQuality256x128Direct : kQuality256x128},
-                                  {VECOPS_HIP_FAMILY_TILE_128X256, 128, 256, direct ? kQuality256x128Direct : kQuality256x128},
+                                  {VECOPS_HIP_FAMILY_TILE_128X256, 128, 256,
+                                   direct ? kQuality256x128Direct : any_rows ? kQuality128x256Rows : kQuality256x128},
                                   // (256 tiles of 192 x 192 cover 3072 x 3072: one round where 144 big tiles leave 112
                                   //  units idle - bf16 3000^3 71 us against 81, 768 x 11008 x 4096 64 against 80)
                                   {VECOPS_HIP_FAMILY_TILE_192, 192, 192, kQuality192},
@@ -552,10 +560,11 @@ void choose_table(const Problem& pr, VecopsHipPlan* plan, uint64_t scratch_limit
     if (count * kRules.min_busy_den < kComputeUnits * kRules.min_busy_num) continue;
     // two 128x128 workgroups live on a compute unit at a time (64 KiB of LDS and at most 256 registers each): a
     // round of them is 512 tiles
-    const int64_t per_unit = c.family == VECOPS_HIP_FAMILY_TILE_128 && direct ? kRules.small_tile_workgroups_per_unit : 1;
+    const bool row_pairs = any_rows && !bytes && c.family == VECOPS_HIP_FAMILY_TILE_128 && count > kComputeUnits;
+    const int64_t per_unit = row_pairs || (c.family == VECOPS_HIP_FAMILY_TILE_128 && direct) ? kRules.small_tile_workgroups_per_unit : 1;
     const int64_t slots = per_unit * kComputeUnits;
     const int64_t rounds = (count + slots - 1) / slots;
-    int64_t cost = rounds * per_unit * c.tm * c.tn * 1000 / c.quality;
+    int64_t cost = rounds * per_unit * c.tm * c.tn * 1000 / (row_pairs ? kQuality128RowPairs : c.quality);
     // a single part-filled round runs faster than a full one (the chip is power-limited: fewer busy compute units
     // clock higher): half full costs three quarters (3000^3 as 144 big tiles 87 us against 105 for 576 small ones;
     // 8 x 777 x 1000 x 3001 as 224 tiles of 128x256 65 us, as 256 of 256x128 73, as 128 of 256x256 86)
@@ -565,8 +574,12 @@ void choose_table(const Problem& pr, VecopsHipPlan* plan, uint64_t scratch_limit
     // 49 us against 60 for the rectangles, 2048 x 4096 x 4096 58 against 67; int8 31 against 38 and 36 against 42).
     const bool smaller = best_cost != INT64_MAX && c.tm * c.tn < tile_m * tile_n &&
                          !(c.family == VECOPS_HIP_FAMILY_TILE_128 && direct);
+    // (the rows kernel on 16-bit operands: 5 %)
+    const bool rows_kernel = any_rows && !bytes && c.family == VECOPS_HIP_FAMILY_TILE_128X256;
     if (best_cost == INT64_MAX ||
-        (smaller ? cost * kRules.rectangle_margin_num < best_cost * kRules.rectangle_margin_den : cost < best_cost)) {
+        (rows_kernel ? cost * 21 < best_cost * (smaller ? 20 : 21)
+         : smaller   ? cost * kRules.rectangle_margin_num < best_cost * kRules.rectangle_margin_den
+                     : cost < best_cost)) {
       best_cost = cost;
       family = c.family;
       tile_m = c.tm;
