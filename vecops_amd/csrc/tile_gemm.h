@@ -475,7 +475,8 @@ struct Accumulators {
   // The 64 quads of the 256x256 tile's 16x16 form come out of its written-out K loop in the accumulation registers
   // and stay there until the epilogue takes them one by one: left to itself the compiler copies all 256 values into
   // vector registers ahead of the branch between the epilogue's paths, spills what does not fit, and reloaded one
-  // spilled value wrongly (ROCm 7.2).  The empty statement pins a quad to its accumulation registers at its use.
+  // spilled value wrongly (ROCm 7.2).  The empty statement pins a quad to its accumulation registers at its use.  (The 32x32
+  // form likewise, a block at a time: 209 spilled registers without it.)
   static constexpr bool kPinned = WM * WN > 8;
   template <int I, int J, int Q>
   __device__ __forceinline__ Quad quad() const {
