@@ -87,3 +87,50 @@ def test_repeated_and_captured(device):
         graph.replay()
         torch.cuda.synchronize()
         assert all(torch.equal(x, y) for x, y in zip(c, want))
+
+
+SRC = {"bf16": 0, "f16": 5, "i8": 2}
+
+
+def _kernels_and_values(device, shapes, kind):
+    """(m, n, k, layout of b) of each group: the kernels of the call; its values checked."""
+    import torch
+    from conftest import launched_kernels
+    from vecops_amd import capi
+    dtype = {"bf16": torch.bfloat16, "f16": torch.float16, "i8": torch.int8}[kind]
+    gen = torch.Generator().manual_seed(len(shapes))
+    a, b, c = [], [], []
+    for m, n, k, layout in shapes:
+        a.append(torch.randint(-3, 4, (m, k), generator=gen).to(dtype).to(device))
+        y = torch.randint(-3, 4, (n, k), generator=gen).to(dtype).to(device)
+        b.append(y if layout == "nk" else y.t().contiguous().t())
+        c.append(torch.empty((m, n), dtype=torch.int32 if kind == "i8" else torch.float32, device=device))
+    names = launched_kernels(lambda: capi.matmul_grouped(a, b, c))
+    for t in c:
+        t.fill_(77)
+    capi.matmul_grouped(a, b, c)
+    torch.cuda.synchronize()
+    for x, y, out in zip(a, b, c):
+        assert torch.equal(out, (x.double() @ y.t().contiguous().double()).to(out.dtype))
+    return names
+
+
+# groups with B as [K,N] beside long K-contiguous ones: they would turn the loads of a launch together into element loads
+# (tile_gemm_grouped_kernel<..., 1, 1, ...>)
+LONG = [(150 + 10 * i, 1890, 6144, "nk") for i in range(12)]
+
+
+@pytest.mark.parametrize("shapes,together,others", [
+    ([(256, 2048, 8192, "nk")] * 8 + [(64, 256, 256, "kn")], "tile_gemm_grouped_kernel<5,2,2,2,2,4,4,", "tile_gemm_kernel<5,2,2,1,1,0,3,"),
+    (LONG + [(300, 700, 264, "kn")], "tile_gemm_grouped_kernel<5,2,2,2,2,4,4,", "tile_gemm_kernel<5,2,2,1,1,0,3,"),
+    ([(42, 409, 1985, "nk")] * 18 + [(64, 256, 256, "kn")] * 2, "tile_gemm_slim_grouped_kernel<5,32,64>", "tile_gemm_grouped_kernel<5,2,2,1,1,0,3,"),
+    (LONG + [(700, 900, 264, "kn")] * 14, "tile_gemm_slim_grouped_kernel<5,128,64>", "tile_gemm_grouped_kernel<5,2,2,4,4,0,3,")])
+def test_other_layouts_stay_apart(device, shapes, together, others):
+    names = _kernels_and_values(device, shapes, "f16")
+    assert len(names) == 2 and sorted(name.startswith(together) for name in names) == [False, True]
+    assert sorted(name.startswith(others) for name in names) == [False, True]
+
+
+def test_an_unaligned_group_among_aligned_ones(device):
+    names = _kernels_and_values(device, LONG + [(700, 904, 264, "nk")] * 6 + [(300, 640, 333, "nk")], "f16")
+    assert len(names) == 1 and names[0].startswith("tile_gemm_grouped_kernel<5,2,2,2,2,0,0,")

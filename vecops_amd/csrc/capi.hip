@@ -1863,18 +1863,42 @@ struct Grouped {
   std::vector<uint64_t> term_offset;  // unsigned 8-bit sides: where a table group's row and column terms lie
 };
 
+// The loaders that serve all of `groups`: the weakest fetch mode that any of them needs.
+int common_mode(const Grouped& g, const std::vector<int>& groups) {
+  bool all_k = true, all_n = true, all_dma = true;
+  for (int i : groups) {
+    const int mode = fetch_mode(g.problems[i], g.plans[i]);
+    all_k = all_k && (mode == MODE_KVEC || mode == MODE_KVEC_DMA);
+    all_n = all_n && (mode == MODE_NVEC_B || mode == MODE_NVEC_B_DMA);
+    all_dma = all_dma && (mode == MODE_KVEC_DMA || mode == MODE_NVEC_B_DMA);
+    // (the 256 x 256 tile's written-out K loop walks a [K,N] operand with 32-bit byte offsets)
+    if (mode == MODE_NVEC_B_DMA && g.problems[i].k * g.problems[i].b.cs * 2 >= (int64_t{1} << 31)) all_dma = false;
+  }
+  return all_k ? (all_dma ? MODE_KVEC_DMA : MODE_KVEC) : all_n ? (all_dma ? MODE_NVEC_B_DMA : MODE_NVEC_B) : MODE_GENERIC;
+}
+
 // What a grouped launch on one square tile takes in ns: the longest workgroup alone, or all of them on the units' slots.  (Two
 // 128x128 workgroups share a unit, three or four of 64x64; bf16 256x256 tiles walk a K tile in 1.3 us, 128x128 ones alone in 0.67
-// and in pairs in 0.78, 64x64 ones as in RuleConstants; rows that are not 16-byte aligned 1.36 of that.)
+// and in pairs in 0.78, 64x64 ones as in RuleConstants; groups whose rows are not 16-byte aligned 1.36 of that.)  All groups
+// load as the weakest of them has to: through staging registers, aligned ones as well, on 64x64 tiles 1.12 of the time (40 groups
+// 100 x 400 x 512, one of them K = 511, 23.3 -> 26.2 us), on 128x128 ones next to nothing (12 of 205 x 1890 x 6144 and a small
+// one level at 121), on 256x256 ones 1.3 (8 of 1024 x 2048 x 2048 68 -> 86); element by element 3 (23.3 -> 60; 30 of 250 x 900 x 512
+// on 128x128 tiles 25.7 -> 62) and 6 (68 -> 351).
 int64_t grouped_tiles_ns(const Grouped& g, const std::vector<int>& groups, int tile) {
   const int64_t alone = tile == 256 ? 1300 : tile == 128 ? 670 : 320, shared = tile == 256 ? 1300 : tile == 128 ? 390 : 300;
   const int64_t fixed = tile == 256 ? 12000 : tile == 128 ? 5000 : 3600;
+  const int mode = common_mode(g, groups);
+  const int64_t staged = tile == 256 ? 1300 : tile == 128 ? 1000 : 1120, generic = tile == 256 ? 6000 : 3000;
   int64_t longest = 0, sum = 0;
   for (int i : groups) {
     const Problem& pr = g.problems[i];
     const int64_t ktile = k_tile_elements(pr.src), k_tiles = (pr.k + ktile - 1) / ktile;
     const int64_t wgs = ((pr.m + tile - 1) / tile) * ((pr.n + tile - 1) / tile) * pr.batch;
-    const int64_t slow = fetch_mode(pr, g.plans[i]) == MODE_KVEC_DMA ? 1000 : kRules.own_64_staged;
+    const int own_mode = fetch_mode(pr, g.plans[i]);
+    const int64_t slow = mode == MODE_GENERIC                                                                       ? generic
+                         : own_mode != MODE_KVEC_DMA && own_mode != MODE_NVEC_B_DMA                                 ? kRules.own_64_staged
+                         : mode == MODE_KVEC_DMA || mode == MODE_NVEC_B_DMA                                         ? 1000
+                                                                                                                    : staged;
     longest = std::max(longest, fixed + k_tiles * alone * slow / 1000);
     sum += wgs * (fixed * shared / alone + k_tiles * shared * slow / 1000);
   }
@@ -1885,7 +1909,7 @@ int64_t grouped_tiles_ns(const Grouped& g, const std::vector<int>& groups, int t
 
 // Where the groups run that split K on their own, and with them those of at most sixteen rows or columns and a long K (16-bit and
 // signed 8-bit classes, K-contiguous operands): the former in a launch or two each and the latter in the grouped launch, or all
-// of them together on slim tiles, or every group in one launch on one tile.  A pure integer function of the problems; the other
+// of them together on slim tiles, or all groups with K-contiguous operands in one launch on one tile.  A pure integer function of the problems; the other
 // ways have to be estimated a third ahead.  Measured (us, before -> together; f16 but for the third, bf16): 18 groups of 768 rows in
 // all, 409 x 1985 155 -> 15, 18 of 592, 896 x 4760 237-262 -> 63, 8 of 174, 768 x 8183 113 -> 37, 24 of 770, 1085 x 1536 112 -> 25;
 // 12 of 2193, 1890 x 6144 on 128x128 tiles 255 -> 122.
@@ -1896,7 +1920,9 @@ void plan_split_groups(Grouped* g, bool same_class) {
     return (g->problems[i].k + ktile - 1) / ktile;
   };
   auto aligned = [&](int i) { return fetch_mode(g->problems[i], g->plans[i]) == MODE_KVEC_DMA; };
-  std::vector<int> slim, others, all = g->table_groups;
+  // `all`: the groups that one tile's launch takes together; `apart`: those whose layout of B would turn that launch's loads
+  // into element loads
+  std::vector<int> slim, others, all, apart;
   int64_t own = 0;
   for (int i : g->split_groups) {
     const Problem& pr = g->problems[i];
@@ -1913,6 +1939,8 @@ void plan_split_groups(Grouped* g, bool same_class) {
   for (int i : g->table_groups) {
     const bool narrow = g->plans[i].family == VECOPS_HIP_FAMILY_SKINNY && long_k(i) >= kRules.split_min_k_tiles && slim_serves(g->problems[i], g->plans[i]);
     (narrow ? slim : others).push_back(i);
+    const int mode = fetch_mode(g->problems[i], g->plans[i]);
+    (mode == MODE_KVEC || mode == MODE_KVEC_DMA ? all : apart).push_back(i);
   }
   if (slim.size() < 2) return;
   auto table_ns = [&](const std::vector<int>& groups) {
@@ -1941,8 +1969,12 @@ void plan_split_groups(Grouped* g, bool same_class) {
     }
   }
   std::sort(all.begin(), all.end());
+  // (one group apart keeps the launch that it would be without the others; several are one launch as long as the others run
+  // their own plans)
+  const int64_t apart_ns = table_ns(apart);
   for (int tile : {256, 128, 64}) {
-    const int64_t ns = grouped_tiles_ns(*g, all, tile);
+    if (apart.size() > 1) break;
+    const int64_t ns = apart_ns + grouped_tiles_ns(*g, all, tile);
     if (ns < best * 9 / 10) {
       best = ns * 10 / 9;
       g->tile = tile;
@@ -1950,7 +1982,7 @@ void plan_split_groups(Grouped* g, bool same_class) {
   }
   if (g->tile != 0) {
     g->table_groups = all;
-    g->split_groups.clear();
+    g->split_groups = apart;
   } else if (g->slim_bm != 0) {
     std::sort(slim.begin(), slim.end());
     g->slim_groups = slim;
@@ -2016,17 +2048,7 @@ int32_t describe_grouped(uint32_t count, const VecopsHipOperand* a, const Vecops
       g->tile = cand.tile;
     }
   }
-  // the weakest fetch mode any group needs serves them all
-  bool all_k = true, all_n = true, all_dma = true;
-  for (int i : g->table_groups) {
-    const int mode = fetch_mode(g->problems[i], g->plans[i]);
-    all_k = all_k && (mode == MODE_KVEC || mode == MODE_KVEC_DMA);
-    all_n = all_n && (mode == MODE_NVEC_B || mode == MODE_NVEC_B_DMA);
-    all_dma = all_dma && (mode == MODE_KVEC_DMA || mode == MODE_NVEC_B_DMA);
-    // (the 256 x 256 tile's written-out K loop walks a [K,N] operand with 32-bit byte offsets)
-    if (mode == MODE_NVEC_B_DMA && g->problems[i].k * g->problems[i].b.cs * 2 >= (int64_t{1} << 31)) all_dma = false;
-  }
-  g->mode = all_k ? (all_dma ? MODE_KVEC_DMA : MODE_KVEC) : all_n ? (all_dma ? MODE_NVEC_B_DMA : MODE_NVEC_B) : MODE_GENERIC;
+  g->mode = common_mode(*g, g->table_groups);
   int64_t next = 0;
   for (int i : g->table_groups) {
     const Problem& pr = g->problems[i];
