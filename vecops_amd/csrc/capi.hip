@@ -306,6 +306,8 @@ struct RuleConstants {
   int64_t deep_max_workgroups = 256, deep_min_k_tiles = 8;
   //    and with rows that are not 16-byte aligned from this many K tiles and a fifth of the units on (deep128_fits)
   int64_t deep_unaligned_k_tiles = 48, deep_unaligned_units_den = 5;
+  // -- a pack whose rows of A are not 16-byte aligned is priced like such rows without one from this many K tiles on
+  int64_t pack_rows_k_tiles = 29;
   // -- planning for that kernel (operands it serves): from deep_alone_from_tiles tiles of 128x128 on (three eighths of the
   //    units) the tiles stay whole or split in two, whichever the split rule's costs favour, with deep_k_tile_ns per K
   //    tile (a lone workgroup of this kernel walks a K tile in 0.3 us) and deep_fixed_ns per launch; between
@@ -539,7 +541,13 @@ void choose_table(const Problem& pr, VecopsHipPlan* plan, uint64_t scratch_limit
   const bool bytes = pr.src == SRC_I8 || pr.src == SRC_I8_FLIP;
   const int mode = fetch_mode(pr, *plan);
   const bool direct = mode == MODE_KVEC_DMA || mode == MODE_NVEC_B_DMA;  // loads that write LDS themselves
-  const bool any_rows = mode == MODE_KVEC && (pr.src == SRC_BF16 || pr.src == SRC_F16 || pr.src == SRC_I8);
+  // (a prepacked B runs other kernels, which read A through staging registers: with a long K they rank the same - 3975 x 6055 x
+  // 6105 390 us on 128x128 tiles, 318 on 128x256 ones, 3822 x 5307 x 2023 112 and 110, 4394 x 7607 x 3533 366 and on 256x256 ones
+  // 306, 51 such shapes from K = 1665 on - with a short one 128x128 pairs stay ahead, 2577 x 6815 x 475 36.4 against 44.0, 2869 x
+  // 5728 x 740 40 against 49, 3115 x 5506 x 1265 71 against 76; of the two rectangles 128x256 is ahead at any K, bf16 1489 x
+  // 3724 x 751 21.0 against 19.9, 54 shapes 6 % on average)
+  const bool odd_rows = mode == MODE_KVEC && (pr.src == SRC_BF16 || pr.src == SRC_F16 || pr.src == SRC_I8);
+  const bool any_rows = odd_rows && (!pr.packed_b || (pr.k + k_tile_elements(pr.src) - 1) / k_tile_elements(pr.src) >= kRules.pack_rows_k_tiles);
   const Candidate candidates[] = {{VECOPS_HIP_FAMILY_TILE_256, 256, 256, 1000},
                                   {VECOPS_HIP_FAMILY_TILE_256X128, 256, 128, direct ? kQuality256x128Direct : kQuality256x128},
                                   {VECOPS_HIP_FAMILY_TILE_128X256, 128, 256,
@@ -576,6 +584,14 @@ void choose_table(const Problem& pr, VecopsHipPlan* plan, uint64_t scratch_limit
                          !(c.family == VECOPS_HIP_FAMILY_TILE_128 && direct);
     // (the rows kernel on 16-bit operands: 5 %)
     const bool rows_kernel = any_rows && !bytes && c.family == VECOPS_HIP_FAMILY_TILE_128X256;
+    if (odd_rows && !any_rows && c.family == VECOPS_HIP_FAMILY_TILE_128X256 && family == VECOPS_HIP_FAMILY_TILE_256X128 &&
+        cost * kQuality256x128 < best_cost * kQuality128x256Rows) {
+      best_cost = std::min(best_cost, cost);
+      family = c.family;
+      tile_m = c.tm;
+      tile_n = c.tn;
+      continue;
+    }
     if (best_cost == INT64_MAX ||
         (rows_kernel ? cost * 21 < best_cost * (smaller ? 20 : 21)
          : smaller   ? cost * kRules.rectangle_margin_num < best_cost * kRules.rectangle_margin_den
