@@ -1,8 +1,13 @@
-"""The four-stage 128x128 kernel with a partial last K tile, rows at any alignment, and B as [K,N] with any N.  Operands are small
-integers: sums are exact and compared bit for bit; what lies around the operands' rows is NaN and must reach no element of C."""
+"""The four-stage 128x128 kernel with a partial last K tile, rows at any alignment, and B as [K,N] with any N: extents that its
+rule gives it (asserted from the launched kernel's name).  Operands are small integers: sums are exact and compared bit for bit;
+what lies around the operands' rows is NaN and must reach no element of C."""
 import pytest
 
+from conftest import launched_kernels
+
 pytestmark = pytest.mark.gpu
+
+SRC = {"bf16": 0, "f16": 5, "i8": 2}
 
 
 def _inside_nan(values, pad, offset):
@@ -15,11 +20,7 @@ def _inside_nan(values, pad, offset):
     return view
 
 
-# (m, n): more than half the units, few tiles; K: one element past a K tile, one short of it, a single whole one among few
-@pytest.mark.parametrize("m,n", [(1400, 1300), (1000, 1793), (257, 513), (100, 129)])
-@pytest.mark.parametrize("k,split", [(513, 1), (575, 1), (1025, 2), (2600, 3), (520, 1), (4001, 4), (3072, 1)])
-@pytest.mark.parametrize("kind,layout,pad,offset", [("bf16", "nk", 0, 0), ("f16", "nk", 1, 1), ("i8", "nk", 3, 5), ("bf16", "kn", 0, 0), ("f16", "kn", 3, 1)])
-def test_against_exact_sums(device, m, n, k, split, kind, layout, pad, offset):
+def _check(device, kind, layout, pad, offset, m, n, k, split):
     import torch
     from vecops_amd import capi
     dtype = {"bf16": torch.bfloat16, "f16": torch.float16, "i8": torch.int8}[kind]
@@ -30,7 +31,12 @@ def test_against_exact_sums(device, m, n, k, split, kind, layout, pad, offset):
     a = _inside_nan(x, pad, offset)
     b = _inside_nan(y, pad, offset) if layout == "nk" else _inside_nan(y.t().contiguous(), pad, offset).t()
     c = torch.full((m, n), 77, dtype=torch.int32 if kind == "i8" else torch.float32, device=device)
-    capi.matmul_family(a, b, c, capi.family_request("tile_128", capi.SELECT_REQUIRE, split_k=split))
+    request = capi.family_request("tile_128", capi.SELECT_REQUIRE, split_k=split)
+    kernels = launched_kernels(lambda: capi.matmul_family(a, b, c, request))
+    partial = k % (128 if kind == "i8" else 64) != 0 or (layout == "kn" and n % 8 != 0)
+    assert kernels[0] == f"tile_gemm_deep128_kernel<{SRC[kind]},{int(layout == 'kn')},0,{int(partial)}>" and len(kernels) == (2 if split > 1 else 1)
+    c.fill_(77)
+    capi.matmul_family(a, b, c, request)
     torch.cuda.synchronize()
     assert torch.equal(c, sums.to(c.dtype))
     capi.matmul(a, b, c.fill_(77))           # the library's own plan
@@ -38,13 +44,52 @@ def test_against_exact_sums(device, m, n, k, split, kind, layout, pad, offset):
     assert torch.equal(c, sums.to(c.dtype))
 
 
-def test_batches(device):
+# 16-byte aligned rows: more than 128 tiles (132, 156, 180, 256); K one chunk past a K tile, one short of it, and between
+@pytest.mark.parametrize("kind,m,n,k", [("bf16", 1400, 1500, 968), ("f16", 1400, 1500, 1016), ("bf16", 1531, 1663, 2600),
+                                        ("f16", 1793, 1500, 520), ("bf16", 1999, 2048, 1000), ("f16", 2048, 1930, 2104),
+                                        ("i8", 1400, 1500, 3472), ("i8", 1531, 1663, 3568), ("i8", 1793, 1500, 2704), ("i8", 2048, 1930, 2160)])
+def test_partial_k_tile(device, kind, m, n, k):
+    _check(device, kind, "nk", 0, 0, m, n, k, 1)
+
+
+# rows at any alignment: 52 to 192 tiles, 48 K tiles or more; K in whole tiles, one element past one, one short of one
+@pytest.mark.parametrize("kind,k,split", [("bf16", 3073, 1), ("bf16", 3135, 1), ("f16", 4001, 1), ("f16", 3136, 1), ("bf16", 4001, 2), ("f16", 3201, 4),
+                                          ("i8", 6145, 1), ("i8", 6271, 1), ("i8", 6272, 1), ("i8", 7001, 2), ("i8", 8001, 4)])
+@pytest.mark.parametrize("pad,offset", [(0, 0), (1, 1), (3, 5)])
+def test_rows_at_any_alignment(device, kind, k, split, pad, offset):
+    m, n = {1: (1200, 2200), 2: (1000, 1793), 4: (600, 1300)}[split]
+    if k % 64 == 0 and pad == 0:
+        pad = 1                                # (aligned rows without it)
+    _check(device, kind, "nk", pad, offset, m, n, k, split)
+
+
+# B as [K,N]: any count of tiles; N of every kind
+@pytest.mark.parametrize("m,n", [(1400, 1300), (1000, 1793), (257, 513), (100, 129)])
+@pytest.mark.parametrize("k,split", [(513, 1), (575, 1), (1025, 2), (520, 1), (3072, 1)])
+@pytest.mark.parametrize("kind,pad,offset", [("bf16", 0, 0), ("f16", 3, 1)])
+def test_b_as_kn(device, kind, pad, offset, m, n, k, split):
+    _check(device, kind, "kn", pad, offset, m, n + (3 if n % 8 == 4 else 0), k, split)
+
+
+@pytest.mark.parametrize("kind,batch,m,n,k", [("bf16", 3, 768, 896, 3201), ("f16", 2, 900, 1000, 3075), ("i8", 3, 768, 1000, 6150), ("bf16", 5, 777, 801, 968)])
+def test_batches(device, kind, batch, m, n, k):
     import torch
     from vecops_amd import capi
+    dtype = {"bf16": torch.bfloat16, "f16": torch.float16, "i8": torch.int8}[kind]
     gen = torch.Generator().manual_seed(4)
-    a = torch.randint(-3, 4, (5, 777, 3001), generator=gen).bfloat16().to(device)
-    b = torch.randint(-3, 4, (5, 801, 3001), generator=gen).bfloat16().to(device)
-    c = torch.empty((5, 777, 801), dtype=torch.float32, device=device)
-    capi.matmul_family(a, b, c, capi.family_request("tile_128", capi.SELECT_REQUIRE, split_k=1))
+    a = torch.randint(-3, 4, (batch, m, k), generator=gen).to(dtype).to(device)
+    b = torch.randint(-3, 4, (batch, n, k), generator=gen).to(dtype).to(device)
+    c = torch.full((batch, m, n), 77, dtype=torch.int32 if kind == "i8" else torch.float32, device=device)
+    request = capi.family_request("tile_128", capi.SELECT_REQUIRE, split_k=1)
+    assert launched_kernels(lambda: capi.matmul_family(a, b, c, request)) == [f"tile_gemm_deep128_kernel<{SRC[kind]},0,0,1>"]
+    c.fill_(77)
+    capi.matmul_family(a, b, c, request)
     torch.cuda.synchronize()
-    assert torch.equal(c, torch.matmul(a.double(), b.double().transpose(1, 2).contiguous()).float())
+    assert torch.equal(c, torch.matmul(a.double(), b.double().transpose(1, 2).contiguous()).to(c.dtype))
+
+
+def test_whole_k_tiles_run_without_the_partial_ones_code(device):
+    for kind, k in (("bf16", 1024), ("f16", 1024), ("i8", 2048)):
+        _check(device, kind, "nk", 0, 0, 1400, 1500, k, 1)
+    for kind in ("bf16", "f16"):
+        _check(device, kind, "kn", 0, 0, 1000, 1496, 1024, 1)

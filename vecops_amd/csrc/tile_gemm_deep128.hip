@@ -8,6 +8,8 @@
 // operands - B handed over as [K,N] (TR: the tile lies [k][n] in LDS, 64 rows of 256 bytes, swizzled as tile_gemm_kernel's,
 // and the fragment reads transpose); rows at any alignment.  A partial last K tile is walked first, through checked stores
 // into stage 0, while the loads of the next two are under way (1000 x 4000 x 4008: 57 us on the two-stage kernel, 50 here).
+// (TAIL: an instance of its own - the out-of-line routines that stage it leave the epilogue's scalars spilled, which costs an
+// int8 product without one 10 %: 1000 x 2000 x 2048 12.8 us, 14.5 with that code in, with a C input 21.9 and 26.2.)
 // Any M, N, batch count, K split, C input and output type of the class: the epilogue is tile_gemm_kernel's.  PK (16-byte
 // aligned A, K in whole K tiles): B prepacked by vecops_hip_pack_b and kept in its pack order in LDS - a load
 // instruction of a wavefront moves one whole (panel of 32 rows, k-step of two chunks) block, 1 KiB contiguous on both
@@ -21,9 +23,9 @@ namespace {
 constexpr int kDeepStage = 32768;  // 128 rows of A, then 128 of B, 128 bytes of K each
 constexpr int kDeepStages = 4;
 
-template <int SRC, bool TR, bool PK>
+template <int SRC, bool TR, bool PK, bool TAIL>
 __global__ __launch_bounds__(256, 1) void tile_gemm_deep128_kernel(const TileGemmParams p) {
-  static_assert(!(TR && PK), "one layout of B");
+  static_assert(!(TR && PK) && !(PK && TAIL), "one layout of B; a pack has whole K tiles");
   using T = SrcTraits<SRC>;
   constexpr bool INT = T::kInt;
   constexpr int KTILE = 8 * T::kElemsPerChunk;
@@ -44,11 +46,11 @@ __global__ __launch_bounds__(256, 1) void tile_gemm_deep128_kernel(const TileGem
   // the walk over K as in tile_gemm_workgroup: a partial last K tile (and, B as [K,N], one whose chunks reach past N) comes
   // first, through checked stores
   const int total_k_tiles = (p.k + KTILE - 1) / KTILE;
-  const int full_k_tiles = PK ? total_k_tiles : (p.k - (TR && kn_reaches_past(n0, 128, p.n, 8) ? 1 : 0)) / KTILE;
+  const int full_k_tiles = !TAIL ? total_k_tiles : (p.k - (TR && kn_reaches_past(n0, 128, p.n, 8) ? 1 : 0)) / KTILE;
   const int kt_begin = split * p.k_tiles_per_split;
   const int kt_end = min(total_k_tiles, kt_begin + p.k_tiles_per_split);
   const int nk = __builtin_amdgcn_readfirstlane(max(kt_end - kt_begin, 0));
-  const int has_tail = __builtin_amdgcn_readfirstlane(nk > 0 && kt_end > full_k_tiles ? 1 : 0);
+  const int has_tail = TAIL ? __builtin_amdgcn_readfirstlane(nk > 0 && kt_end > full_k_tiles ? 1 : 0) : 0;
 
   // Loads: instruction i of an operand's K tile fills its rows 32 i .. 32 i + 31, this wavefront eight of them; lane l
   // fetches the chunk of row l / 8 whose swizzled slot is l % 8.  Rows past the operand's extent are clamped onto its
@@ -115,7 +117,7 @@ __global__ __launch_bounds__(256, 1) void tile_gemm_deep128_kernel(const TileGem
   if (!has_tail) fill(0);
   fill(1);
   fill(2);
-  if constexpr (!PK) {
+  if constexpr (TAIL) {
     if (has_tail) {
       const char* a = static_cast<const char*>(p.a) + batch * p.a_bs * T::kSrcBytes;
       const char* b = static_cast<const char*>(p.b) + batch * p.b_bs * T::kSrcBytes;
@@ -201,11 +203,11 @@ __global__ __launch_bounds__(256, 1) void tile_gemm_deep128_kernel(const TileGem
   store_accumulators<SRC, 2, 2, 2, 2, kLdsBytes, true>(p, lds, acc, batch, split, m0, n0, wm, wn, wave, lane);
 }
 
-template <int SRC, bool TR, bool PK>
+template <int SRC, bool TR, bool PK, bool TAIL>
 hipError_t launch(const TileGemmParams& p, hipStream_t stream) {
   constexpr int kEpilogue = kEpilogueLdsBytes<2, 2, 2, 2>();
   constexpr int kLds = kDeepStages * kDeepStage > kEpilogue ? kDeepStages * kDeepStage : kEpilogue;
-  auto kernel = tile_gemm_deep128_kernel<SRC, TR, PK>;
+  auto kernel = tile_gemm_deep128_kernel<SRC, TR, PK, TAIL>;
   static thread_local int configured_device = -1;
   int device = 0;
   hipError_t e = hipGetDevice(&device);
@@ -232,7 +234,8 @@ bool launch_tile_gemm_deep128_serves(int src, const TileGemmParams& p, int mode,
   // 32-bit byte offsets inside a tile's 128 rows
   if (128 * p.a_rs * elem + static_cast<int64_t>(p.k) * elem >= (int64_t{1} << 31)) return false;
   if (packed_b) {
-    // A: loads that write LDS need 16-byte aligned addresses; B: 32-bit byte offsets inside the tile's four panels
+    // A: where its rows are not 16-byte aligned, the packed tile kernels run (its loads here would take them); B: 32-bit byte
+    // offsets inside the tile's four panels
     if (p.a_ks != 1 || (reinterpret_cast<uintptr_t>(p.a) & 15u) != 0 || (p.a_rs * elem) % 16 != 0 || (p.a_bs * elem) % 16 != 0) return false;
     return (reinterpret_cast<uintptr_t>(p.b) & 15u) == 0 && 4 * static_cast<int64_t>(p.k / ktile) * 4096 < (int64_t{1} << 31);
   }
@@ -242,18 +245,19 @@ bool launch_tile_gemm_deep128_serves(int src, const TileGemmParams& p, int mode,
 
 hipError_t launch_tile_gemm_deep128(int src, const TileGemmParams& p, int mode, bool packed_b, hipStream_t stream) {
   const bool tr = !packed_b && (mode == MODE_NVEC_B_DMA || mode == MODE_NVEC_B);
-  if (packed_b) {
-    switch (src) {
-      case SRC_BF16: return launch<SRC_BF16, false, true>(p, stream);
-      case SRC_F16: return launch<SRC_F16, false, true>(p, stream);
-      case SRC_I8: return launch<SRC_I8, false, true>(p, stream);
-      default: return hipErrorInvalidValue;
+  auto layout = [&](auto src_tag) {
+    constexpr int SRC = decltype(src_tag)::value;
+    if (packed_b) return launch<SRC, false, true, false>(p, stream);
+    const bool tail = p.k % (8 * SrcTraits<SRC>::kElemsPerChunk) != 0 || (tr && p.n % 8 != 0);
+    if constexpr (SRC != SRC_I8) {
+      if (tr) return tail ? launch<SRC, true, false, true>(p, stream) : launch<SRC, true, false, false>(p, stream);
     }
-  }
+    return tail ? launch<SRC, false, false, true>(p, stream) : launch<SRC, false, false, false>(p, stream);
+  };
   switch (src) {
-    case SRC_BF16: return tr ? launch<SRC_BF16, true, false>(p, stream) : launch<SRC_BF16, false, false>(p, stream);
-    case SRC_F16: return tr ? launch<SRC_F16, true, false>(p, stream) : launch<SRC_F16, false, false>(p, stream);
-    case SRC_I8: return launch<SRC_I8, false, false>(p, stream);
+    case SRC_BF16: return layout(std::integral_constant<int, SRC_BF16>{});
+    case SRC_F16: return layout(std::integral_constant<int, SRC_F16>{});
+    case SRC_I8: return layout(std::integral_constant<int, SRC_I8>{});
     default: return hipErrorInvalidValue;
   }
 }
