@@ -169,3 +169,41 @@ def test_dequantised_rows_that_line_up_with_nothing(device, m, n, k):
     capi.matmul_i8_dequant(a, b, rows, cols, c)
     torch.cuda.synchronize()
     assert torch.equal(c, ((a.double() @ b.double().t()).float() * rows[:, None]) * cols)
+
+
+# C inputs that go into the sums in LDS (of another width than C's, before a transform, past a lane's whole share): every
+# remainder of four columns, fewer than four in all, tiles of every shape cut off anywhere
+@pytest.mark.parametrize("family", FAMILIES)
+@pytest.mark.parametrize("m,n", [(257, 388), (300, 389), (200, 390), (129, 391), (520, 513), (70, 1), (40, 2), (33, 3), (65, 5)])
+@pytest.mark.parametrize("src,out,cin", [("bf16", "bf16", "f32"), ("f16", "f32", "f16"), ("bf16", "f32", "f32"), ("f16", "f16", "f16")])
+def test_c_inputs_of_any_width_and_extent(device, family, m, n, src, out, cin):
+    import torch
+    from vecops_amd import capi
+    t, gen, k = _dtypes(), torch.Generator().manual_seed(m * n), 96
+    a, b = _ints(gen, (m, k), -3, 3, t[src], device), _ints(gen, (n, k), -3, 3, t[src], device)
+    c_in = _ints(gen, (m, n), -9, 9, t[cin], device)
+    want = (a.float() @ b.float().t() + c_in.float()).to(t[out])
+    request = capi.family_request(family, capi.SELECT_REQUIRE, split_k=1)
+    for pad, offset in ((0, 0), (3, 1)):
+        c = _strided(torch.full((m, n), 77.0, dtype=t[out], device=device), pad, offset)
+        capi.matmul_family(a, b, c, request, c_in=_strided(c_in, pad + 2, offset))
+        torch.cuda.synchronize()
+        assert torch.equal(c, want), (pad, offset)
+
+
+@pytest.mark.parametrize("m,n,k", [(70, 3, 640), (1000, 4002, 512), (4096, 4095, 512), (300, 391, 640), (3000, 2999, 256)])
+@pytest.mark.parametrize("src,out,cin", [("bf16", "bf16", "bf16"), ("f16", "f32", "f32"), ("f16", "f16", "f32"), ("bf16", "f32", "bf16")])
+def test_c_inputs_before_a_transform(device, m, n, k, src, out, cin):
+    import torch
+    from vecops_amd import capi
+    t, gen = _dtypes(), torch.Generator().manual_seed(m + 5 * n + k)
+    a, b = _ints(gen, (m, k), -2, 2, t[src], device), _ints(gen, (n, k), -2, 2, t[src], device)
+    c_in = _ints(gen, (m, n), -9, 9, t[cin], device)
+    rows, cols = 2.0 ** _ints(gen, (m,), -2, 1, torch.float32, device), 2.0 ** _ints(gen, (n,), -1, 2, torch.float32, device)
+    want = ((((a.float() @ b.float().t() + c_in.float()) * rows[:, None]) * cols) * 0.5 + 3.0).clamp_min(0.0).to(t[out])
+    for pad, offset in ((0, 0), (5, 1)):
+        c = _strided(torch.full((m, n), 77.0, device=device).to(t[out]), pad, offset)
+        capi.matmul_fused(a, b, c, capi.epilogue(activation="relu", scale=0.5, shift=3.0, row_scales=rows, column_scales=cols),
+                          c_in=_strided(c_in, pad + 1, offset))
+        torch.cuda.synchronize()
+        assert torch.equal(c, want), (pad, offset)

@@ -1529,7 +1529,10 @@ struct RowWalk {
 //   * a bias row and column scales are loaded once per lane, and row scales once per block (into the rows' LDS pad);
 //   * a block's C input is requested a block ahead of its use (more than eight steps: in front of the block), the first in front
 //     of the barrier - where it is all there is to do besides the conversion, and no lane holds fewer columns than its share.
-//     Other C inputs are added to the sums in LDS first.
+//     Other C inputs (of another width than C's, in front of a transform, past a lane's whole share) are added to the sums in LDS
+//     first, in runs of four columns requested a block ahead (one element a lane and step, as they were at first: bf16 4096 x
+//     4096 x 512 with an fp32 C input 144 -> 40, fp32 results with a bf16 one 151 -> 47, silu behind a full one 110 -> 43; 84, 70
+//     and 73 before any of this; 1000 x 4001 x 1024 30 -> 18.6).
 // What it replaced walked blocks of 32 columns and loaded each C input quad where it added it, behind the stores before it:
 // 64 memory round trips one after the other in a 256x256 tile.  Measured (us, before -> now; without a C input 21 and 94):
 // f16 4096 x 4096 x 512 with a C input 68 -> 29, with a bias row 54 -> 28; f16 4096^3 160 -> 119 and 140 -> 103; fp32 results with
@@ -1563,6 +1566,7 @@ __device__ __forceinline__ void store_rows(const TileGemmParams& p, char* lds, c
   using I0 = std::integral_constant<int, 0>;
   using I1 = std::integral_constant<int, 1>;
   using I2 = std::integral_constant<int, 2>;
+  using I3 = std::integral_constant<int, 3>;
   static_assert(W4::STEPS <= 16 && W8::STEPS <= 8, "the requested C input's registers");
   u32x4 coming[16] = {};  // two blocks' worth, or one of more than eight steps
   // the C input of block i, at addresses inside it whatever the lane (lanes past an edge drop what they get)
@@ -1583,12 +1587,13 @@ __device__ __forceinline__ void store_rows(const TileGemmParams& p, char* lds, c
   if (!PLAIN && ahead && wide_out) request(U4{}, I0{});
   const int out_bytes = wide_out ? 4 : 2;
   const int lane_col = wide_out ? lane % W4::LANES * 4 : lane % W8::LANES * 8, cols_left = p.n - (first_col + lane_col);
-  // FORM 0: the lane's bias and column scales, and the transform
+  // FORMs 0 and 3: the lane's bias and column scales, and the transform
   Finisher fin;
   bool scaled = false;
   float bias[8], column_scales[8];
   VECOPS_GLOBAL char* c = (VECOPS_GLOBAL char*)p.c + (batch * p.c_bs + static_cast<int64_t>(first_row) * p.c_rs + first_col + lane_col) * out_bytes;
-  // One step of a block: U columns of the lane's row.  FORM 0: any; 1: `given` is that row's part of the C input, and nothing
+  // One step of a block: U columns of the lane's row.  FORM 0: any without a C input for every row, 3: with one, in the
+  // sums already; 1: `given` is that row's part of the C input, and nothing
   // but the conversion follows; 2: fp32 sums as they are.  INSIDE: the tile lies wholly inside C (no branch stands between the
   // steps, which then overlap).
   auto step = [&](auto u_tag, auto form_tag, auto inside_tag, int i, int s, const u32x4& given) __attribute__((always_inline)) {
@@ -1608,9 +1613,11 @@ __device__ __forceinline__ void store_rows(const TileGemmParams& p, char* lds, c
 #pragma unroll
       for (int e = 0; e < U; ++e)
         f[e] += U == 4 ? __uint_as_float(given[e & 3]) : widen((given[e >> 1] >> ((e & 1) * 16)) & 0xffffu);
-    } else if constexpr (FORM == 0) {
+    } else if constexpr (FORM == 0 || FORM == 3) {
+      if constexpr (FORM == 0) {
 #pragma unroll
-      for (int e = 0; e < U; ++e) f[e] += bias[e];
+        for (int e = 0; e < U; ++e) f[e] += bias[e];
+      }
       if (scaled) {
         const float row_scale = fin.row_scaled ? __uint_as_float(mine[r * PITCH + COLS]) : 1.0f;
 #pragma unroll
@@ -1658,15 +1665,70 @@ __device__ __forceinline__ void store_rows(const TileGemmParams& p, char* lds, c
   auto blocks = [&](auto u_tag, auto form_tag, auto inside_tag) __attribute__((always_inline)) {
     constexpr int U = decltype(u_tag)::value, FORM = decltype(form_tag)::value, STEPS = RowWalk<WN, U>::STEPS;
     constexpr bool EARLY = STEPS <= 8;
-    if constexpr (FORM == 0) {
+    // FORM 3: the same in runs of four elements of either width, and the runs' way into the block's sums in LDS.  (A run that
+    // would reach past N begins earlier, inside the row, and is shifted back.)
+    // (Requested a block ahead on the tiles that are alone on their unit.  On the small ones several workgroups overlap each other,
+    // and the registers for that, or for all of a block's runs at a time, would leave them a wavefront a SIMD less: 128x128 tiles
+    // on the 32x32 shape 260 of them for 216, 3072 x 4800 x 128 13.5 -> 19.8 us; 64x64 ones 100 for 96.)
+    constexpr bool RUNS_AHEAD = WM * WN > 4;
+    const bool runs = p.n >= 4, whole_runs = (n0 + BN <= p.n) | (p.n % 4 == 0);
+    const int run_col = first_col + lane % W4::LANES * 4, run_early = max(run_col - (p.n - 4), 0);
+    constexpr int RUNS = RUNS_AHEAD ? W4::STEPS : W4::STEPS / 2;  // at a time
+    auto request_runs = [&](auto i_tag, int first) __attribute__((always_inline)) {
+      constexpr int i = decltype(i_tag)::value;
+      if constexpr (i < WM) {
+        auto from = [&](int s) __attribute__((always_inline)) {
+          const int row = min(first_row + i * 32 + min((first + s) * W4::ROWS + lane / W4::LANES, 31), p.m - 1);
+          return cin + (static_cast<int64_t>(row) * p.cin_rs + (run_col - run_early)) * cin_bytes;
+        };
+        if (cin16) {
+#pragma unroll
+          for (int s = 0; s < RUNS; ++s) {
+            const u32x2 v = *reinterpret_cast<const VECOPS_GLOBAL u32x2_align2*>(from(s));
+            coming[s].x = v.x;
+            coming[s].y = v.y;
+          }
+        } else {
+#pragma unroll
+          for (int s = 0; s < RUNS; ++s) coming[s] = *reinterpret_cast<const VECOPS_GLOBAL u32x4_align4*>(from(s));
+        }
+      }
+    };
+    auto add_runs = [&](int first) __attribute__((always_inline)) {
+      auto add = [&](int s, f32x4 v) __attribute__((always_inline)) {
+        if (!whole_runs) {
+          if (run_early & 1) v = f32x4{v.y, v.z, v.w, v.w};
+          if (run_early & 2) v = f32x4{v.z, v.w, v.w, v.w};
+        }
+        const int r = (first + s) * W4::ROWS + lane / W4::LANES;
+        if ((W4::ROWS * W4::LANES != 64 && lane >= W4::ROWS * W4::LANES) || (32 % W4::ROWS != 0 && r > 31)) return;
+        f32x4* sums = reinterpret_cast<f32x4*>(mine + r * PITCH + lane % W4::LANES * 4);
+        *sums += v;
+      };
+      if (cin16) {
+#pragma unroll
+        for (int s = 0; s < RUNS; ++s)
+          add(s, f32x4{widen(coming[s].x & 0xffffu), widen(coming[s].x >> 16), widen(coming[s].y & 0xffffu), widen(coming[s].y >> 16)});
+      } else {
+#pragma unroll
+        for (int s = 0; s < RUNS; ++s) add(s, __builtin_bit_cast(f32x4, coming[s]));
+      }
+    };
+    // (Nothing is under way here.  Said to the compiler, which otherwise carries loads of the other forms' paths along and waits for
+    // them, and with them for this form's own stores, at each use of one of their registers: fp32 results of 2000 x 2000 x 128 8.8
+    // us for 7.5.)
+    if constexpr (FORM != 1) __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+    if constexpr (FORM == 0 || FORM == 3) {
       fin = make_finisher<false>(p, false);
       scaled = p.fused != 0 && (p.ep_row_scales != nullptr || p.ep_column_scales != nullptr || (p.ep_flags & 3u) != 0u);
 #pragma unroll
       for (int e = 0; e < U; ++e) {
         const int col = min(first_col + lane_col + e, p.n - 1);
-        bias[e] = p.cin && !full ? cin_at(col) : -0.0f;  // (adding -0 changes nothing)
+        if constexpr (FORM == 0) bias[e] = p.cin ? cin_at(col) : -0.0f;  // (adding -0 changes nothing)
         column_scales[e] = scaled && p.ep_column_scales ? p.ep_column_scales[col] : 1.0f;
       }
+      if constexpr (FORM == 3 && RUNS_AHEAD)
+        if (runs) request_runs(I0{}, 0);
     }
     __syncthreads();  // every wavefront is done reading fragments
     static_for<WM>([&](auto ci) {
@@ -1681,9 +1743,23 @@ __device__ __forceinline__ void store_rows(const TileGemmParams& p, char* lds, c
         });
       });
       // (the wavefront reads back only what it wrote itself: its own LDS traffic is ordered)
-      if constexpr (FORM == 0) {
-        if (full) {  // (clamped like a request: what lies past an edge is never stored)
-#pragma unroll 8
+      if constexpr (FORM == 0 || FORM == 3) {
+        if constexpr (FORM == 3) {
+#pragma unroll
+          for (int first = 0; first < W4::STEPS; first += RUNS) {
+            if constexpr (!RUNS_AHEAD)
+              if (runs) request_runs(ci, first);
+            // (the runs' registers are waited for here, whatever their width: where one of the paths below leaves some of them
+            // unread, the compiler waits for them again at every later use of a register)
+#pragma unroll
+            for (int s = 0; s < RUNS; ++s) asm volatile("" : "+v"(coming[s]));
+            if (runs) add_runs(first);
+          }
+          if constexpr (RUNS_AHEAD)
+            if (runs) request_runs(Next{}, 0);
+        }
+        if (FORM == 3 && !runs) {  // fewer than four columns (clamped like a request: what lies past an edge is never stored)
+#pragma unroll 1
           for (int idx = lane; idx < 32 * COLS; idx += 64) {
             const int r = idx / COLS, col = idx % COLS;
             float* sum = reinterpret_cast<float*>(mine + r * PITCH + col);
@@ -1710,13 +1786,15 @@ __device__ __forceinline__ void store_rows(const TileGemmParams& p, char* lds, c
     else blocks(U4{}, I2{}, No{});
     return;
   } else {
-    switch (__builtin_amdgcn_readfirstlane(ahead ? (wide_out ? 4 : 2) + inside : wide_out ? 1 : 0)) {
+    switch (__builtin_amdgcn_readfirstlane(ahead ? (wide_out ? 4 : 2) + inside : (full ? 6 : 0) + wide_out)) {
       case 0: blocks(U8{}, I0{}, No{}); break;
       case 1: blocks(U4{}, I0{}, No{}); break;
       case 2: blocks(U8{}, I1{}, No{}); break;
       case 3: blocks(U8{}, I1{}, Yes{}); break;
       case 4: blocks(U4{}, I1{}, No{}); break;
-      default: blocks(U4{}, I1{}, Yes{}); break;
+      case 5: blocks(U4{}, I1{}, Yes{}); break;
+      case 6: blocks(U8{}, I3{}, No{}); break;
+      default: blocks(U4{}, I3{}, No{}); break;
     }
   }
 }
