@@ -93,3 +93,18 @@ def test_whole_k_tiles_run_without_the_partial_ones_code(device):
         _check(device, kind, "nk", 0, 0, 1400, 1500, k, 1)
     for kind in ("bf16", "f16"):
         _check(device, kind, "kn", 0, 0, 1000, 1496, 1024, 1)
+
+
+# past the rule: the two-stage kernel (more than 192 tiles) and 64x64 tiles, in the library's own plans
+@pytest.mark.parametrize("m,n,k,kernel", [(2000, 2000, 1040, "tile_gemm_kernel<2,2,2,2,2,4,4,1>"), (1256, 1752, 3088, "tile_gemm_kernel<2,2,2,1,1,0,0,1>")])
+def test_bytes_with_a_short_partial_k(device, m, n, k, kernel):
+    import torch
+    from vecops_amd import capi
+    gen = torch.Generator().manual_seed(k)
+    a, b = (torch.randint(-127, 128, (rows, k), generator=gen).to(torch.int8).to(device) for rows in (m, n))
+    c = torch.full((m, n), 77, dtype=torch.int32, device=device)
+    assert launched_kernels(lambda: capi.matmul(a, b, c)) == [kernel]
+    c.fill_(77)
+    capi.matmul(a, b, c)
+    torch.cuda.synchronize()
+    assert torch.equal(c, (a.double() @ b.double().t()).to(torch.int32))

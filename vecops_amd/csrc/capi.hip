@@ -306,6 +306,10 @@ struct RuleConstants {
   int64_t deep_max_workgroups = 256, deep_min_k_tiles = 8;
   //    and with rows that are not 16-byte aligned from this many K tiles and a fifth of the units on (deep128_fits)
   int64_t deep_unaligned_k_tiles = 48, deep_unaligned_units_den = 5;
+  //    and with a partial last K tile from these many K tiles on (deep128_fits: 16-bit operands, bytes up to deep_idle_tiles
+  //    tiles, up to three quarters of the units, and beyond)
+  int64_t deep_ragged_k_tiles = 15, deep_ragged_k_tiles_8bit = 28, deep_ragged_k_tiles_8bit_idle = 20, deep_ragged_k_tiles_8bit_busy = 16;
+  int64_t deep_least_64_tiles_per_unit = 2;
   // -- a pack whose rows of A are not 16-byte aligned is priced like such rows without one from this many K tiles on
   int64_t pack_rows_k_tiles = 29;
   // -- planning for that kernel (operands it serves): from deep_alone_from_tiles tiles of 128x128 on (three eighths of the
@@ -416,19 +420,37 @@ int fetch_mode(const Problem& pr, const VecopsHipPlan& plan);
 bool lines_up(const Problem& pr, const View& v, int64_t line_stride);
 
 // Whether the four-stage 128x128 kernel is the one for `tiles` such tiles and operands fetched like that (not prepacked).  Its
-// loads take rows at any alignment and it walks a partial K tile; where it replaces what the table took before (us, before -> now,
-// bf16): 1000 x 4000 x 4008 57 -> 50, 768 x 3000 x 2008 30.6 -> 24.8, 2000 x 2000 x 1000 19.7 -> 17.7, but 700 x 2048 x 1096, 96
-// tiles, 14.8 on 64x64 tiles -> 15.9: a partial K tile's checked start wants more than half the units in use.  Rows that are
-// not 16-byte aligned: with a long K and up to three quarters of the units in use 1728 x 1280 x 7853 122 -> 89, 186 x 3712 x 11835 73 -> 58,
-// 300 x 4000 x 4001 44 -> 37 (64x64 and slim tiles before; on less than a fifth slim tiles are ahead, 150 x 3000 x 5001 23.4
-// against 24.9); beyond, the two-stage kernel is level or ahead (int8 2000 x 2000 x 2001 23.5
-// against 24.8).  B as [K,N] at any alignment: 300 x 4001 x 4000 37 -> 34, 512 x 4097 x 1000 18.9 -> 16.7.
+// loads take rows at any alignment and it walks a partial K tile; where it replaces what the table took before (us, before -> now):
+//   * a partial K tile's checked start wants more than half the units in use (bf16 700 x 2048 x 1096, 96 tiles, 14.8 on 64x64
+//     tiles, 15.9 here) and a K that outweighs it.  bf16 of 140 tiles, 1256 x 1752, K = 520 11.8 -> 12.4, 1000 17.5 -> 16.1, 2008
+//     28.9 -> 25.2; of 176, 1384 x 2008, K = 520 12.7 -> 12.3; of 252, 1512 x 2648, K = 520 13.9 -> 13.2, 4008 57.6 -> 43.9.  int8,
+//     whose 64x64 tiles are better, of 140 tiles K = 2064 19.3 -> 20.6, 3088 24.7 -> 25.1, 4112 30.1 -> 29.1, 6160 42.3 -> 38.5; of
+//     176 K = 2064 19.9 -> 20.8, 3088 26.3 -> 25.3; of 252 K = 1040 16.9 -> 17.4, 2064 23.8 -> 21.9, 8208 60.5 -> 48.1; with a C
+//     input, which leaves 64x64 tiles sooner, of 140 tiles K = 6160 45.0 -> 52.0, of 252 K = 3088 39.1 -> 39.5, 4112 45.0 -> 43.6;
+//   * rows that are not 16-byte aligned, on a fifth (below, slim tiles are ahead, 150 x 3000 x 5001 23.4 and 24.9) to three quarters
+//     of the units (beyond, the two-stage kernel is level or ahead, int8 2000 x 2000 x 2001 23.5 and 24.8) with a long K: bf16 1728 x
+//     1280 x 7853 125 -> 92, 300 x 4000 x 4001 45.4 -> 37.2, 1512 x 1624 x 3074 43.4 -> 34.7, int8 1728 x 1280 x 7853 74 -> 57, 640 x
+//     2000 x 6405 43 -> 30.6, 1512 x 1624 x 6148 44.6 -> 38.9;
+//   * neither where so much of the 128x128 tiles is padding that 64x64 ones are at most two to a unit: int8 288 x 5624 x 4016, 132
+//     and 440 tiles, 21.2 -> 27.4, x 8004 36.8 -> 44.8, bf16 x 4001 43.6 -> 50.0, 513 x 3300 x 2008 23.0 -> 23.8;
+//   * B as [K,N] at any alignment: 300 x 4001 x 4000 37 -> 34, 512 x 4097 x 1000 18.9 -> 16.7.
 bool deep128_fits(const Problem& pr, int mode, int64_t tiles) {
   const int64_t ktile = k_tile_elements(pr.src), k_tiles = (pr.k + ktile - 1) / ktile;
+  if (mode == MODE_NVEC_B || (mode != MODE_KVEC && pr.k % ktile == 0)) return true;
+  // (more tiles than can be split in two, padded so much that 64x64 ones are no more than two a unit: those)
+  const int64_t tiles_64 = ((pr.m + 63) / 64) * ((pr.n + 63) / 64) * pr.batch;
+  if (tiles > kComputeUnits / 2 && tiles_64 <= kRules.deep_least_64_tiles_per_unit * kComputeUnits) return false;
   if (mode == MODE_KVEC)
     return k_tiles >= kRules.deep_unaligned_k_tiles && tiles * kRules.deep_unaligned_units_den >= kComputeUnits &&
            tiles <= kRules.lonely_tiles_num * kComputeUnits / kRules.lonely_tiles_den;
-  return mode == MODE_NVEC_B || pr.k % ktile == 0 || tiles > kComputeUnits / 2;
+  if (tiles <= kComputeUnits / 2) return false;
+  // (up to three quarters of the units the other way is 64x64 tiles, beyond the two-stage kernel)
+  const bool busy = tiles * kRules.lonely_tiles_den > kRules.lonely_tiles_num * kComputeUnits;
+  if (pr.src != SRC_I8) return k_tiles >= (tiles <= kRules.deep_idle_tiles ? kRules.deep_ragged_k_tiles : kRules.deep_min_k_tiles);
+  if (pr.has_cin) return busy && k_tiles >= kRules.deep_ragged_k_tiles_8bit;
+  return k_tiles >= (tiles <= kRules.deep_idle_tiles ? kRules.deep_ragged_k_tiles_8bit
+                     : !busy                         ? kRules.deep_ragged_k_tiles_8bit_idle
+                                                     : kRules.deep_ragged_k_tiles_8bit_busy);
 }
 
 // The two halves of a problem cut between columns n_main - 1 and n_main of C: rows of B, columns of C and C_in.
