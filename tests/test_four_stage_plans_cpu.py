@@ -39,3 +39,18 @@ def test_a_partial_k_tile(dtype, m, n, k, cin, family):
                                          (capi.I8, 513, 3300, 8001)])      # 51.7, 56.0
 def test_padded_tiles(dtype, m, n, k):
     assert _plan(dtype, m, n, k)[0] == "tile_64"
+
+
+# rows of whole words, which slim tiles load faster than rows at odd addresses
+@pytest.mark.parametrize("dtype,m,n,k,slim", [(capi.BF16, 744, 1112, 3074, 0x4040),     # 20.1, 21.0
+                                              (capi.BF16, 744, 1112, 3073, 0),          # 21.4, 23.4
+                                              (capi.BF16, 744, 1112, 6002, 0),          # 27.0, 32.2
+                                              (capi.I8, 744, 1112, 6152, 0x4040),       # 19.4, 21.8
+                                              (capi.I8, 744, 1112, 12008, 0),           # 28.4, 31.5
+                                              (capi.BF16, 488, 4056, 8004, 0x8040),     # 57.4, 65.1
+                                              (capi.BF16, 488, 4056, 6001, 0),          # 47.1, 53.8
+                                              (capi.I8, 488, 4056, 12008, 0x8040),      # 45.1, 53.8
+                                              (capi.I8, 488, 4056, 12001, 0)])          # 53.1, 60.1
+def test_rows_of_words(dtype, m, n, k, slim):
+    family, split, tile = _plan(dtype, m, n, k)
+    assert family == "tile_128" and split > 1 and tile == slim

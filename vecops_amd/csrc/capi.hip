@@ -339,11 +339,15 @@ struct RuleConstants {
   //    Timed on both sides for 7794 products (bf16 and int8, up to sixteen batches, M to 6000, N and K to 14336, rows at any
   //    alignment; another 14604 gave the constants): 3074 take a slim tile, in 0.69 of the time on average, twelve of them more
   //    than 3 % slower, the worst 9 %.
-  int64_t slim_ns = 4000, slim_row_ns = 10, slim_bytes_per_ns = 65, slim_bytes_per_ns_unaligned = 40;
+  //    Against the four-stage kernel on rows that are not 16-byte aligned, rows of whole words have rates of their own (bf16 488 x
+  //    4056 on a slim tile and in two parts: K = 6004 45.3 and 45.7 us, out of the caches 45.8 and 52.5, 7004 50.8 and 49.2, 60.6
+  //    and 61.5, odd 8001 68.7 and 58.0, 79.8 and 75.1; 744 x 1112 in four parts: K = 3074 20.1 and 21.0, 5004 27.5 and 26.3; int8
+  //    488 x 4056 x 12008 45.0 and 46.6, 47.7 and 55.4).
+  int64_t slim_ns = 4000, slim_row_ns = 10, slim_bytes_per_ns = 65, slim_bytes_per_ns_unaligned = 40, slim_bytes_per_ns_words = 57;
   int64_t slim_margin_num = 95, slim_margin_den = 100;
   int64_t own_64_ns = 3640, own_64_tile_ns = 320, own_64_ns_per_wg = 415, own_64_ns_per_wg_shared = 300, own_64_staged = 1360;
   int64_t own_64_split_ns = 4430, own_64_ns_per_mb = 275;
-  int64_t own_deep_ns = 5000, own_deep_tile_ns = 440, own_deep_unaligned_tile_ns = 660, own_deep_ns_per_operand_mb = 46, own_deep_split_ns = 3650, own_deep_ns_per_mb = 585;
+  int64_t own_deep_ns = 5000, own_deep_tile_ns = 440, own_deep_unaligned_tile_ns = 660, own_deep_words_tile_ns = 620, own_deep_words_tile_ns_busy = 700, own_deep_ns_per_operand_mb = 46, own_deep_split_ns = 3650, own_deep_ns_per_mb = 585;
 };
 constexpr RuleConstants kRules{};
 
@@ -1040,6 +1044,15 @@ bool slim_serves(const Problem& pr, const VecopsHipPlan& plan) {
          launch_tile_gemm_slim_serves(pr.src, base_params(pr, nullptr, nullptr, nullptr, nullptr));
 }
 
+// Whether every row of A and B begins at a multiple of four bytes.
+bool rows_of_words(const Problem& pr) {
+  auto words = [&](const View& v) {
+    const int64_t eb = dtype_bytes(v.dtype);
+    return (reinterpret_cast<uintptr_t>(v.data) & 3u) == 0 && (v.rs * eb) % 4 == 0 && (pr.batch == 1 || (v.bs * eb) % 4 == 0);
+  };
+  return words(pr.a) && words(pr.b);
+}
+
 // What the rule table's plan of 64x64 tiles, or of 128x128 tiles on the four-stage kernel, takes in ns (RuleConstants); -1 for
 // any other.
 int64_t own_plan_ns(const Problem& pr, const VecopsHipPlan& plan) {
@@ -1060,7 +1073,11 @@ int64_t own_plan_ns(const Problem& pr, const VecopsHipPlan& plan) {
   } else {
     if (!deep128_runs(pr, p, plan.family, mode)) return -1;
     const int64_t operands = pr.batch * (pr.m + pr.n) * k_tiles / 8;  // KiB: K tiles of 128 bytes
-    const int64_t tile_ns = mode == MODE_KVEC ? kRules.own_deep_unaligned_tile_ns : kRules.own_deep_tile_ns;
+    const int64_t wgs = static_cast<int64_t>(p.tiles_m) * p.tiles_n * pr.batch * split;
+    const int64_t tile_ns = mode != MODE_KVEC      ? kRules.own_deep_tile_ns
+                            : !rows_of_words(pr)   ? kRules.own_deep_unaligned_tile_ns
+                            : wgs * 16 > kComputeUnits * 15 ? kRules.own_deep_words_tile_ns_busy
+                                                   : kRules.own_deep_words_tile_ns;
     own_ns = kRules.own_deep_ns + p.k_tiles_per_split * tile_ns + operands * kRules.own_deep_ns_per_operand_mb / 1024;
     if (split > 1) own_ns += kRules.own_deep_split_ns + partials * kRules.own_deep_ns_per_mb / 1024;
   }
@@ -1068,10 +1085,9 @@ int64_t own_plan_ns(const Problem& pr, const VecopsHipPlan& plan) {
 }
 
 // What one workgroup of a slim tile takes on K tiles of 128 bytes, in ns.
-int64_t slim_workgroup_ns(int bm, int bn, int64_t k_tiles, bool aligned) {
+int64_t slim_workgroup_ns(int bm, int bn, int64_t k_tiles, int64_t bytes_per_ns) {
   const int64_t rows = bm + bn;
-  return kRules.slim_ns + rows * kRules.slim_row_ns +
-         rows * k_tiles * 128 / (aligned ? kRules.slim_bytes_per_ns : kRules.slim_bytes_per_ns_unaligned);
+  return kRules.slim_ns + rows * kRules.slim_row_ns + rows * k_tiles * 128 / bytes_per_ns;
 }
 
 // Hands the rule table's own plan of 64x64 tiles, or of 128x128 tiles on the four-stage kernel, to a slim tile where that is
@@ -1084,12 +1100,14 @@ void take_slim_tile(const Problem& pr, VecopsHipPlan* chosen) {
   if (plan.peeled_columns > 0 || !slim_serves(pr, plan)) return;
   const int64_t own_ns = own_plan_ns(pr, plan);
   if (own_ns < 0) return;
-  const bool aligned = fetch_mode(pr, plan) == MODE_KVEC_DMA;
+  const int64_t bytes_per_ns = fetch_mode(pr, plan) == MODE_KVEC_DMA                             ? kRules.slim_bytes_per_ns
+                               : plan.family == VECOPS_HIP_FAMILY_TILE_128 && rows_of_words(pr) ? kRules.slim_bytes_per_ns_words
+                                                                                                : kRules.slim_bytes_per_ns_unaligned;
   const int64_t ktile = k_tile_elements(pr.src), k_tiles = (pr.k + ktile - 1) / ktile;
   int64_t best_ns = own_ns * kRules.slim_margin_num / kRules.slim_margin_den;
   for (const auto& t : kSlimTiles) {
     if (((pr.m + t.bm - 1) / t.bm) * ((pr.n + t.bn - 1) / t.bn) * pr.batch > kComputeUnits) continue;
-    const int64_t ns = slim_workgroup_ns(t.bm, t.bn, k_tiles, aligned);
+    const int64_t ns = slim_workgroup_ns(t.bm, t.bn, k_tiles, bytes_per_ns);
     if (ns < best_ns) {
       best_ns = ns;
       chosen->slim_tile = slim_code(t.bm, t.bn);
@@ -1957,7 +1975,9 @@ void plan_split_groups(Grouped* g, bool same_class) {
     const int64_t ktile = k_tile_elements(g->problems[i].src);
     return (g->problems[i].k + ktile - 1) / ktile;
   };
-  auto aligned = [&](int i) { return fetch_mode(g->problems[i], g->plans[i]) == MODE_KVEC_DMA; };
+  auto bytes_per_ns = [&](int i) {
+    return fetch_mode(g->problems[i], g->plans[i]) == MODE_KVEC_DMA ? kRules.slim_bytes_per_ns : kRules.slim_bytes_per_ns_unaligned;
+  };
   // `all`: the groups that one tile's launch takes together; `apart`: those whose layout of B would turn that launch's loads
   // into element loads
   std::vector<int> slim, others, all, apart;
@@ -1969,7 +1989,7 @@ void plan_split_groups(Grouped* g, bool same_class) {
     if (ns < 0) ns = 15000 + long_k(i) / g->plans[i].split_k * 700;
     VecopsHipPlan single = g->plans[i];
     take_slim_tile(pr, &single);
-    if (single.slim_tile != 0) ns = slim_workgroup_ns(single.slim_tile >> 8, single.slim_tile & 255, long_k(i), aligned(i));
+    if (single.slim_tile != 0) ns = slim_workgroup_ns(single.slim_tile >> 8, single.slim_tile & 255, long_k(i), bytes_per_ns(i));
     own += ns;
     slim.push_back(i);
     all.push_back(i);
@@ -1992,7 +2012,7 @@ void plan_split_groups(Grouped* g, bool same_class) {
     for (int i : slim) {
       const Problem& pr = g->problems[i];
       const int64_t wgs = ((pr.m + t.bm - 1) / t.bm) * ((pr.n + t.bn - 1) / t.bn) * pr.batch;
-      const int64_t ns = slim_workgroup_ns(t.bm, t.bn, long_k(i), aligned(i));
+      const int64_t ns = slim_workgroup_ns(t.bm, t.bn, long_k(i), bytes_per_ns(i));
       longest = std::max(longest, ns);
       sum += wgs * ns;
       most = std::max(most, wgs);
