@@ -43,7 +43,7 @@ def test_groups_in_the_launchs_arguments(device, count, table, kind, out):
     assert (need > 256) == table
 
 
-# rows per group, N, K: on slim tiles of each size; a row alone and sixteen (the skinny family's), rows at any alignment, K ragged
+# rows per group, N, K: a row alone and sixteen (the skinny family's) among others, rows at any alignment, K ragged
 @pytest.mark.parametrize("rows,n,k", [([42, 7, 100, 33, 16, 1, 64, 30], 409, 1985), ([33, 40, 20, 5, 1, 16, 60, 17, 33, 30, 29, 31], 896, 2048),
                                       ([22, 30, 19, 3], 768, 8183), ([183, 150, 200, 170, 129], 640, 3080), ([300, 1], 70, 8192)])
 @pytest.mark.parametrize("kind,out,cin,offset", [("bf16", "bf16", False, 0), ("bf16", "f32", True, 0), ("f16", "f16", True, 1), ("i8", "i32", True, 3)])
@@ -113,6 +113,15 @@ def _kernels_and_values(device, shapes, kind):
     for x, y, out in zip(a, b, c):
         assert torch.equal(out, (x.double() @ y.t().contiguous().double()).to(out.dtype))
     return names
+
+
+@pytest.mark.parametrize("tile,rows,n,k", [((32, 32), [22, 30, 19, 3], 768, 8183), ((32, 64), [60, 59, 60, 57, 60, 60, 58, 60], 700, 4096),
+                                           ((64, 64), [128, 127, 126, 128, 120, 128, 128, 125, 128], 700, 4090), ((64, 64), [120, 119] * 6, 600, 4096),
+                                           ((128, 64), [128, 127] * 6, 1000, 4096)])
+@pytest.mark.parametrize("kind", ["bf16", "f16", "i8"])
+def test_each_slim_tile(device, kind, tile, rows, n, k):
+    names = _kernels_and_values(device, [(m, n, k, "nk") for m in rows], kind)
+    assert names == [f"tile_gemm_slim_grouped_kernel<{SRC[kind]},{tile[0]},{tile[1]}>"]
 
 
 # groups with B as [K,N] beside long K-contiguous ones: they would turn the loads of a launch together into element loads

@@ -54,6 +54,37 @@ def test_families(device, family, src, m, n, k, pad, offset):
     _check(device, capi, dtype, compute, m, n, k, pad, offset, capi.family_request(family, capi.SELECT_REQUIRE, split_k=1))
 
 
+# (N odd, the rows of B padded to a multiple of eight elements: loads that write LDS, as aligned rows take)
+@pytest.mark.parametrize("family", FAMILIES + ["tile_192"])
+@pytest.mark.parametrize("src", ["bf16", "f16", "f32", "f32c"])
+@pytest.mark.parametrize("m,n,k", [(300, 391, 128), (257, 255, 320), (130, 513, 77), (64, 9, 64), (520, 777, 648), (70, 63, 1)])
+def test_odd_n_in_rows_that_line_up(device, family, src, m, n, k):
+    import torch
+    from conftest import launched_kernels
+    from vecops_amd import capi
+    dtype = {"bf16": torch.bfloat16, "f16": torch.float16}.get(src, torch.float32)
+    if family == "tile_192" and dtype == torch.float32:
+        pytest.skip("the 192 x 192 tile takes 16-bit and 8-bit operands")
+    compute = capi.COMPUTE_F32 if src == "f32c" else capi.COMPUTE_BF16
+    gen = torch.Generator().manual_seed(m + 7 * n + k)
+    store = torch.randint(-3, 4, (m, (k + 7) // 8 * 8), generator=gen).to(dtype).to(device)
+    a, values = store[:, :k], torch.randint(-3, 4, (k, n), generator=gen).to(dtype).to(device)
+    b = _b_as_kn(values, -n % 8, 0)
+    c = torch.full((m, n), 77.0, dtype=torch.float32, device=device)
+    request = capi.family_request(family, capi.SELECT_REQUIRE, split_k=1)
+    plan = capi.plan_matmul_family(a, b, c, request, compute=compute)
+    assert capi.FAMILY_NAMES[plan.family] == family and plan.b_layout == 1 and plan.vector_b == 1
+    kernels = launched_kernels(lambda: capi.matmul_family(a, b, c, request, compute=compute))
+    if dtype != torch.float32 and family != "tile_64" and kernels[0].startswith("tile_gemm_kernel"):
+        assert kernels[0].split(",")[5:7] == ["4", "5"]      # LOAD_KDMA and LOAD_NTR_DMA
+    if (family, k) in (("tile_256", 648), ("tile_192", 648), ("tile_128x256", 648)) and dtype != torch.float32:
+        assert kernels[0].startswith("tile_gemm_kernel")
+    c.fill_(77)
+    capi.matmul_family(a, b, c, request, compute=compute)
+    torch.cuda.synchronize()
+    assert torch.equal(c, torch.matmul(a.double(), values.double()).float())
+
+
 @pytest.mark.parametrize("n", [1001, 1002, 1004, 1007, 4097])
 @pytest.mark.parametrize("m,k", [(1000, 1024), (333, 4001), (17, 640)])
 def test_the_librarys_own_plans(device, m, n, k):
