@@ -348,6 +348,24 @@ struct RuleConstants {
   int64_t own_64_ns = 3640, own_64_tile_ns = 320, own_64_ns_per_wg = 415, own_64_ns_per_wg_shared = 300, own_64_staged = 1360;
   int64_t own_64_split_ns = 4430, own_64_ns_per_mb = 275;
   int64_t own_deep_ns = 5000, own_deep_tile_ns = 440, own_deep_unaligned_tile_ns = 660, own_deep_words_tile_ns = 620, own_deep_words_tile_ns_busy = 700, own_deep_ns_per_operand_mb = 46, own_deep_split_ns = 3650, own_deep_ns_per_mb = 585;
+  //    (the four-stage kernel on rows of whole words: with this share of the units or more at work its parts' loads are in each
+  //    other's way)
+  int64_t own_deep_busy_num = 15, own_deep_busy_den = 16;
+  // -- the any-alignment 128x256 kernel on 16-bit operands against the tiles before it in the table (kQuality128x256Rows)
+  int64_t rows_margin_num = 21, rows_margin_den = 20;
+  // -- grouped launches on one square tile, in ns: what a workgroup takes beside its K tiles, and per K tile alone on its unit and
+  //    as its share of a full one (two 128x128 workgroups a unit, three or four of 64x64); per mille of that, through staging
+  //    registers, and element by element (grouped_tiles_ns says what was measured)
+  int64_t grouped_256_ns = 12000, grouped_256_tile_ns = 1300, grouped_256_staged = 1300, grouped_256_generic = 6000;
+  int64_t grouped_128_ns = 5000, grouped_128_tile_ns = 670, grouped_128_tile_ns_shared = 390, grouped_128_staged = 1000;
+  int64_t grouped_64_ns = 3600, grouped_64_tile_ns = 320, grouped_64_tile_ns_shared = 300, grouped_64_staged = 1120;
+  int64_t grouped_small_generic = 3000;
+  //    the launch that writes more groups' records than one launch's arguments carry
+  int64_t grouped_table_ns = 4500;
+  // -- groups that split K on their own (plan_split_groups): such a group's launches where own_plan_ns has no estimate; how
+  //    far ahead the groups together have to be estimated, and one tile for all of them ahead of slim tiles
+  int64_t group_launches_ns = 15000, group_k_tile_ns = 700;
+  int64_t groups_margin_num = 2, groups_margin_den = 3, groups_one_tile_num = 9, groups_one_tile_den = 10;
 };
 constexpr RuleConstants kRules{};
 
@@ -619,7 +637,7 @@ void choose_table(const Problem& pr, VecopsHipPlan* plan, uint64_t scratch_limit
       continue;
     }
     if (best_cost == INT64_MAX ||
-        (rows_kernel ? cost * 21 < best_cost * (smaller ? 20 : 21)
+        (rows_kernel ? cost * kRules.rows_margin_num < best_cost * (smaller ? kRules.rows_margin_den : kRules.rows_margin_num)
          : smaller   ? cost * kRules.rectangle_margin_num < best_cost * kRules.rectangle_margin_den
                      : cost < best_cost)) {
       best_cost = cost;
@@ -1074,10 +1092,11 @@ int64_t own_plan_ns(const Problem& pr, const VecopsHipPlan& plan) {
     if (!deep128_runs(pr, p, plan.family, mode)) return -1;
     const int64_t operands = pr.batch * (pr.m + pr.n) * k_tiles / 8;  // KiB: K tiles of 128 bytes
     const int64_t wgs = static_cast<int64_t>(p.tiles_m) * p.tiles_n * pr.batch * split;
-    const int64_t tile_ns = mode != MODE_KVEC      ? kRules.own_deep_tile_ns
-                            : !rows_of_words(pr)   ? kRules.own_deep_unaligned_tile_ns
-                            : wgs * 16 > kComputeUnits * 15 ? kRules.own_deep_words_tile_ns_busy
-                                                   : kRules.own_deep_words_tile_ns;
+    const bool busy = wgs * kRules.own_deep_busy_den > kComputeUnits * kRules.own_deep_busy_num;
+    const int64_t tile_ns = mode != MODE_KVEC    ? kRules.own_deep_tile_ns
+                            : !rows_of_words(pr) ? kRules.own_deep_unaligned_tile_ns
+                            : busy               ? kRules.own_deep_words_tile_ns_busy
+                                                 : kRules.own_deep_words_tile_ns;
     own_ns = kRules.own_deep_ns + p.k_tiles_per_split * tile_ns + operands * kRules.own_deep_ns_per_operand_mb / 1024;
     if (split > 1) own_ns += kRules.own_deep_split_ns + partials * kRules.own_deep_ns_per_mb / 1024;
   }
@@ -1933,42 +1952,45 @@ int common_mode(const Grouped& g, const std::vector<int>& groups) {
   return all_k ? (all_dma ? MODE_KVEC_DMA : MODE_KVEC) : all_n ? (all_dma ? MODE_NVEC_B_DMA : MODE_NVEC_B) : MODE_GENERIC;
 }
 
-// What a grouped launch on one square tile takes in ns: the longest workgroup alone, or all of them on the units' slots.  (Two
-// 128x128 workgroups share a unit, three or four of 64x64; bf16 256x256 tiles walk a K tile in 1.3 us, 128x128 ones alone in 0.67
-// and in pairs in 0.78, 64x64 ones as in RuleConstants; groups whose rows are not 16-byte aligned 1.36 of that.)  All groups
-// load as the weakest of them has to: through staging registers, aligned ones as well, on 64x64 tiles 1.12 of the time (40 groups
+// What a grouped launch on one square tile takes in ns: the longest workgroup alone, or all of them on the units' slots.  (bf16
+// 256x256 tiles walk a K tile in 1.3 us, 128x128 ones alone in 0.67 and in pairs in 0.78; groups whose rows are not 16-byte
+// aligned 1.36 of that.)  All groups load as the weakest of them has to: through staging registers, aligned ones as well, on 64x64 tiles 1.12 of the time (40 groups
 // 100 x 400 x 512, one of them K = 511, 23.3 -> 26.2 us), on 128x128 ones next to nothing (12 of 205 x 1890 x 6144 and a small
 // one level at 121), on 256x256 ones 1.3 (8 of 1024 x 2048 x 2048 68 -> 86); element by element 3 (23.3 -> 60; 30 of 250 x 900 x 512
 // on 128x128 tiles 25.7 -> 62) and 6 (68 -> 351).
 int64_t grouped_tiles_ns(const Grouped& g, const std::vector<int>& groups, int tile) {
-  const int64_t alone = tile == 256 ? 1300 : tile == 128 ? 670 : 320, shared = tile == 256 ? 1300 : tile == 128 ? 390 : 300;
-  const int64_t fixed = tile == 256 ? 12000 : tile == 128 ? 5000 : 3600;
+  auto of_tile = [&](int64_t big, int64_t middle, int64_t small) { return tile == 256 ? big : tile == 128 ? middle : small; };
+  const int64_t alone = of_tile(kRules.grouped_256_tile_ns, kRules.grouped_128_tile_ns, kRules.grouped_64_tile_ns);
+  const int64_t shared = of_tile(kRules.grouped_256_tile_ns, kRules.grouped_128_tile_ns_shared, kRules.grouped_64_tile_ns_shared);
+  const int64_t fixed = of_tile(kRules.grouped_256_ns, kRules.grouped_128_ns, kRules.grouped_64_ns);
+  const int64_t staged = of_tile(kRules.grouped_256_staged, kRules.grouped_128_staged, kRules.grouped_64_staged);
+  const int64_t generic = of_tile(kRules.grouped_256_generic, kRules.grouped_small_generic, kRules.grouped_small_generic);
   const int mode = common_mode(g, groups);
-  const int64_t staged = tile == 256 ? 1300 : tile == 128 ? 1000 : 1120, generic = tile == 256 ? 6000 : 3000;
   int64_t longest = 0, sum = 0;
   for (int i : groups) {
     const Problem& pr = g.problems[i];
     const int64_t ktile = k_tile_elements(pr.src), k_tiles = (pr.k + ktile - 1) / ktile;
     const int64_t wgs = ((pr.m + tile - 1) / tile) * ((pr.n + tile - 1) / tile) * pr.batch;
     const int own_mode = fetch_mode(pr, g.plans[i]);
-    const int64_t slow = mode == MODE_GENERIC                                                                       ? generic
-                         : own_mode != MODE_KVEC_DMA && own_mode != MODE_NVEC_B_DMA                                 ? kRules.own_64_staged
-                         : mode == MODE_KVEC_DMA || mode == MODE_NVEC_B_DMA                                         ? 1000
-                                                                                                                    : staged;
+    const int64_t slow = mode == MODE_GENERIC                                        ? generic
+                         : own_mode != MODE_KVEC_DMA && own_mode != MODE_NVEC_B_DMA ? kRules.own_64_staged
+                         : mode == MODE_KVEC_DMA || mode == MODE_NVEC_B_DMA         ? 1000
+                                                                                    : staged;
     longest = std::max(longest, fixed + k_tiles * alone * slow / 1000);
     sum += wgs * (fixed * shared / alone + k_tiles * shared * slow / 1000);
   }
   if (groups.empty()) return 0;
-  const int64_t table = static_cast<int>(groups.size()) > kGroupsInline ? 4500 : 0;
+  const int64_t table = static_cast<int>(groups.size()) > kGroupsInline ? kRules.grouped_table_ns : 0;
   return table + std::max(longest, sum / kComputeUnits);
 }
 
 // Where the groups run that split K on their own, and with them those of at most sixteen rows or columns and a long K (16-bit and
 // signed 8-bit classes, K-contiguous operands): the former in a launch or two each and the latter in the grouped launch, or all
-// of them together on slim tiles, or all groups with K-contiguous operands in one launch on one tile.  A pure integer function of the problems; the other
-// ways have to be estimated a third ahead.  Measured (us, before -> together; f16 but for the third, bf16): 18 groups of 768 rows in
-// all, 409 x 1985 155 -> 15, 18 of 592, 896 x 4760 237-262 -> 63, 8 of 174, 768 x 8183 113 -> 37, 24 of 770, 1085 x 1536 112 -> 25;
-// 12 of 2193, 1890 x 6144 on 128x128 tiles 255 -> 122.
+// of them together on slim tiles, or all groups with K-contiguous operands in one launch on one tile.  A pure integer function of the
+// problems; the other ways have to be estimated a third ahead.  Measured (us, before -> together; f16 but for the third, bf16): 18
+// groups of 768 rows in all, 409 x 1985 155 -> 15, 18 of 592, 896 x 4760 237-262 -> 63, 8 of 174, 768 x 8183 113 -> 37, 24 of 770,
+// 1085 x 1536 112 -> 25; 12 of 2193, 1890 x 6144 on 128x128 tiles 255 -> 122, with a group of 300 x 700 x 264, B as [K,N], beside them
+// 294 -> 129 (469 in one launch with it).
 void plan_split_groups(Grouped* g, bool same_class) {
   if (!same_class || g->split_groups.empty() || g->split_groups.size() + g->table_groups.size() < 2) return;
   auto long_k = [&](int i) {
@@ -1986,7 +2008,7 @@ void plan_split_groups(Grouped* g, bool same_class) {
     const Problem& pr = g->problems[i];
     if (!slim_serves(pr, g->plans[i])) return;  // (of another class, or B as [K,N]: as they are)
     int64_t ns = own_plan_ns(pr, g->plans[i]);
-    if (ns < 0) ns = 15000 + long_k(i) / g->plans[i].split_k * 700;
+    if (ns < 0) ns = kRules.group_launches_ns + long_k(i) / g->plans[i].split_k * kRules.group_k_tile_ns;
     VecopsHipPlan single = g->plans[i];
     take_slim_tile(pr, &single);
     if (single.slim_tile != 0) ns = slim_workgroup_ns(single.slim_tile >> 8, single.slim_tile & 255, long_k(i), bytes_per_ns(i));
@@ -2004,7 +2026,7 @@ void plan_split_groups(Grouped* g, bool same_class) {
   auto table_ns = [&](const std::vector<int>& groups) {
     return std::min(grouped_tiles_ns(*g, groups, 64), std::min(grouped_tiles_ns(*g, groups, 128), grouped_tiles_ns(*g, groups, 256)));
   };
-  int64_t best = (own + table_ns(g->table_groups)) * 2 / 3;
+  int64_t best = (own + table_ns(g->table_groups)) * kRules.groups_margin_num / kRules.groups_margin_den;
   const int64_t others_ns = table_ns(others);
   const struct { int bm, bn; } tiles[] = {{32, 32}, {32, 64}, {64, 64}, {128, 64}};
   for (const auto& t : tiles) {
@@ -2027,14 +2049,14 @@ void plan_split_groups(Grouped* g, bool same_class) {
     }
   }
   std::sort(all.begin(), all.end());
-  // (one group apart keeps the launch that it would be without the others; several are one launch as long as the others run
-  // their own plans)
+  // (one group apart keeps the launch that it would be without the others; several of them are a launch of their own, beside which
+  // there is none for the others)
   const int64_t apart_ns = table_ns(apart);
   for (int tile : {256, 128, 64}) {
     if (apart.size() > 1) break;
     const int64_t ns = apart_ns + grouped_tiles_ns(*g, all, tile);
-    if (ns < best * 9 / 10) {
-      best = ns * 10 / 9;
+    if (ns < best * kRules.groups_one_tile_num / kRules.groups_one_tile_den) {
+      best = ns * kRules.groups_one_tile_den / kRules.groups_one_tile_num;
       g->tile = tile;
     }
   }
