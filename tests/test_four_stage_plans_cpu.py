@@ -48,6 +48,11 @@ def test_padded_tiles(dtype, m, n, k):
                                               (capi.I8, 744, 1112, 6152, 0x4040),       # 19.4, 21.8
                                               (capi.I8, 744, 1112, 12008, 0),           # 28.4, 31.5
                                               (capi.BF16, 488, 4056, 8004, 0x8040),     # 57.4, 65.1
+                                              (capi.BF16, 150, 8000, 6004, 0),          # 47.3, 60.3
+                                              (capi.I8, 150, 8000, 16004, 0),           # 60.8, 81.4
+                                              (capi.BF16, 1000, 1000, 6004, 0),         # 28.1, 30.9
+                                              (capi.BF16, 200, 7000, 5004, 0x8040),     # 37.8, 42.9
+                                              (capi.I8, 1000, 1300, 6148, 0x8030),      # 26.0, 29.0
                                               (capi.BF16, 488, 4056, 6001, 0),          # 47.1, 53.8
                                               (capi.I8, 488, 4056, 12008, 0x8040),      # 45.1, 53.8
                                               (capi.I8, 488, 4056, 12001, 0)])          # 53.1, 60.1

@@ -344,12 +344,11 @@ struct RuleConstants {
   //    and 61.5, odd 8001 68.7 and 58.0, 79.8 and 75.1; 744 x 1112 in four parts: K = 3074 20.1 and 21.0, 5004 27.5 and 26.3; int8
   //    488 x 4056 x 12008 45.0 and 46.6, 47.7 and 55.4).
   int64_t slim_ns = 4000, slim_row_ns = 10, slim_bytes_per_ns = 65, slim_bytes_per_ns_unaligned = 40, slim_bytes_per_ns_words = 57;
-  int64_t slim_margin_num = 95, slim_margin_den = 100;
+  int64_t slim_margin_num = 95, slim_words_margin_num = 85, slim_margin_den = 100;
   int64_t own_64_ns = 3640, own_64_tile_ns = 320, own_64_ns_per_wg = 415, own_64_ns_per_wg_shared = 300, own_64_staged = 1360;
   int64_t own_64_split_ns = 4430, own_64_ns_per_mb = 275;
   int64_t own_deep_ns = 5000, own_deep_tile_ns = 440, own_deep_unaligned_tile_ns = 660, own_deep_words_tile_ns = 620, own_deep_words_tile_ns_busy = 700, own_deep_ns_per_operand_mb = 46, own_deep_split_ns = 3650, own_deep_ns_per_mb = 585;
-  //    (the four-stage kernel on rows of whole words: with this share of the units or more at work its parts' loads are in each
-  //    other's way)
+  //    (the four-stage kernel on rows of whole words: whole or in halves, with this share of the units at work)
   int64_t own_deep_busy_num = 15, own_deep_busy_den = 16;
   // -- the any-alignment 128x256 kernel on 16-bit operands against the tiles before it in the table (kQuality128x256Rows)
   int64_t rows_margin_num = 21, rows_margin_den = 20;
@@ -1092,7 +1091,7 @@ int64_t own_plan_ns(const Problem& pr, const VecopsHipPlan& plan) {
     if (!deep128_runs(pr, p, plan.family, mode)) return -1;
     const int64_t operands = pr.batch * (pr.m + pr.n) * k_tiles / 8;  // KiB: K tiles of 128 bytes
     const int64_t wgs = static_cast<int64_t>(p.tiles_m) * p.tiles_n * pr.batch * split;
-    const bool busy = wgs * kRules.own_deep_busy_den > kComputeUnits * kRules.own_deep_busy_num;
+    const bool busy = split <= 2 && wgs * kRules.own_deep_busy_den > kComputeUnits * kRules.own_deep_busy_num;
     const int64_t tile_ns = mode != MODE_KVEC    ? kRules.own_deep_tile_ns
                             : !rows_of_words(pr) ? kRules.own_deep_unaligned_tile_ns
                             : busy               ? kRules.own_deep_words_tile_ns_busy
@@ -1119,19 +1118,34 @@ void take_slim_tile(const Problem& pr, VecopsHipPlan* chosen) {
   if (plan.peeled_columns > 0 || !slim_serves(pr, plan)) return;
   const int64_t own_ns = own_plan_ns(pr, plan);
   if (own_ns < 0) return;
-  const int64_t bytes_per_ns = fetch_mode(pr, plan) == MODE_KVEC_DMA                             ? kRules.slim_bytes_per_ns
-                               : plan.family == VECOPS_HIP_FAMILY_TILE_128 && rows_of_words(pr) ? kRules.slim_bytes_per_ns_words
-                                                                                                : kRules.slim_bytes_per_ns_unaligned;
   const int64_t ktile = k_tile_elements(pr.src), k_tiles = (pr.k + ktile - 1) / ktile;
-  int64_t best_ns = own_ns * kRules.slim_margin_num / kRules.slim_margin_den;
-  for (const auto& t : kSlimTiles) {
-    if (((pr.m + t.bm - 1) / t.bm) * ((pr.n + t.bn - 1) / t.bn) * pr.batch > kComputeUnits) continue;
-    const int64_t ns = slim_workgroup_ns(t.bm, t.bn, k_tiles, bytes_per_ns);
-    if (ns < best_ns) {
-      best_ns = ns;
-      chosen->slim_tile = slim_code(t.bm, t.bn);
+  // the slim tile ahead of `limit` ns, if one is
+  auto fastest = [&](int64_t limit, int64_t bytes_per_ns) {
+    uint16_t code = 0;
+    for (const auto& t : kSlimTiles) {
+      if (((pr.m + t.bm - 1) / t.bm) * ((pr.n + t.bn - 1) / t.bn) * pr.batch > kComputeUnits) continue;
+      const int64_t ns = slim_workgroup_ns(t.bm, t.bn, k_tiles, bytes_per_ns);
+      if (ns < limit) {
+        limit = ns;
+        code = slim_code(t.bm, t.bn);
+      }
+    }
+    return code;
+  };
+  int64_t margin_num = kRules.slim_margin_num, bytes_per_ns = kRules.slim_bytes_per_ns;
+  if (fetch_mode(pr, plan) != MODE_KVEC_DMA) {
+    bytes_per_ns = kRules.slim_bytes_per_ns_unaligned;
+    if (plan.family == VECOPS_HIP_FAMILY_TILE_128 && rows_of_words(pr)) {
+      // (a margin of its own where 64x64 tiles would keep the product without the four-stage kernel: there are many slim workgroups
+      // to little work each, 150 x 8000 x 6004 47 us on the four-stage kernel, 60 on slim tiles, 69 on 64x64 ones)
+      VecopsHipPlan small = plan;
+      small.family = VECOPS_HIP_FAMILY_TILE_64;
+      finish_tile_plan(pr, &small, 0);
+      if (fastest(own_plan_ns(pr, small) * margin_num / kRules.slim_margin_den, bytes_per_ns) == 0) margin_num = kRules.slim_words_margin_num;
+      bytes_per_ns = kRules.slim_bytes_per_ns_words;
     }
   }
+  chosen->slim_tile = fastest(own_ns * margin_num / kRules.slim_margin_den, bytes_per_ns);
 }
 
 // The library's own plan: the rule table's, or a slim tile in its place.
