@@ -300,7 +300,7 @@ def bench_grouped(dev, steps, warmup):
         b_list.append(torch.from_numpy(synth.bf16_round(synth.uniform_pm1(40 + i, (n, k))).view(np.int16)).to(dev).view(torch.bfloat16))
         c_list.append(torch.empty((m, n), dtype=torch.float32, device=dev))
     ws = torch.empty(64 << 20, dtype=torch.uint8, device=dev)
-    # (a call is seven launches - two groups split K - and a separate-calls step ten: at most 100 steps between
+    # (a call is five launches - two groups split K - and a separate-calls step ten: at most 100 steps between
     # synchronisations, because with thousands of launches queued the HIP runtime's own bookkeeping stalls the host
     # in the first such loop of a process, 160-200 us per step of wall time where the GPU needs 76)
     count = min(max(steps, 50), 100)

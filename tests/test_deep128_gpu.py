@@ -1,8 +1,7 @@
 """The four-stage 128 x 128 kernel (tile_gemm_deep128.hip): what the library runs when a product gives a compute unit at
-most one 128 x 128 workgroup (256 workgroups or fewer, operands aligned and K-contiguous - or, 16-bit ones, B handed
-over as [K,N] -, K in whole K tiles).
-Checked against the oracle, against exact integer sums, and against the two-stage kernel of the same tile - which a
-K that is no whole number of K tiles, or more than 256 workgroups, still selects - on ragged extents, batches, K
+most one 128 x 128 workgroup (256 workgroups or fewer) and has K in whole K tiles, both operands K-contiguous and aligned or B
+handed over as [K,N].  (Partial K tiles, rows at any alignment and any N of a [K,N] operand: test_deep128_any_rows_gpu.py.)
+Checked against the oracle, against exact integer sums and against other tiles' results on ragged extents, batches, K
 splits, C inputs, bf16 outputs and a transposed C."""
 import numpy as np
 import pytest
@@ -137,8 +136,8 @@ def test_deep_kernel_batches_cin_bf16_out_transposed_c(device, oracle):
 
 
 def test_the_table_plans_one_workgroup_per_unit(device):
-    """1024 x 4096 x 4096 and its neighbours: the plan is the unsplit 128 x 128 tile, and it equals the two-stage kernel's
-    result (which a K of one element more, padded operands apart, selects) up to the order of the fp32 sums."""
+    """1024 x 4096 x 4096 and its neighbours: the plan is the unsplit 128 x 128 tile, and its result equals the 256 x 256 tile's
+    up to the order of the fp32 sums."""
     import torch
     from vecops_amd import capi
     for (m, n, k), b_as_kn in (((1024, 4096, 4096), False), ((768, 4096, 4096), False), ((512, 4096, 4096), False),

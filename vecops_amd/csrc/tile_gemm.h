@@ -1817,9 +1817,6 @@ __device__ __forceinline__ void store_accumulators(const TileGemmParams& p, char
   // the fast paths take edge tiles too: their stores (and scale loads) are guarded per row and per run
   // of columns, which costs an interior tile a few compares
   const bool dequant = INT && p.row_scales != nullptr;
-  // work that happens on the row-major side of the 32-bit staging: C-input, int32 sums leaving as floats,
-  // the fused output transform, outputs narrower than 32 bits
-  const bool finishing = p.cin != nullptr || p.fused != 0 || (INT ? (!dequant && p.out_kind != OUT_I32) : p.out_kind != OUT_F32);
   // (an unsigned operand's terms go through the general path, unless the launcher has folded them into the
   // per-column correction: unsigned A, one batch)
   const bool flip_terms = SRC == SRC_I8_FLIP && (p.row_term != nullptr || p.col_term != nullptr || p.const_term != 0u);
@@ -1924,6 +1921,9 @@ __device__ __forceinline__ void store_accumulators(const TileGemmParams& p, char
     });
     uint32_t* out = reinterpret_cast<uint32_t*>(c_base) + batch * p.c_bs + static_cast<int64_t>(m0 + wm * ROWS) * p.c_rs;
     const int out_bytes = output_element_bytes(p.out_kind);
+    // work that happens on the row-major side of the staging: a C input, int32 sums leaving as floats or 8-bit values, the fused
+    // transform
+    const bool finishing = p.cin != nullptr || p.fused != 0 || (!dequant && p.out_kind != OUT_I32);
     const Finisher fin = make_finisher<INT>(p, dequant);
     static_for<WN>([&](auto cj) {
       constexpr int j = decltype(cj)::value;
@@ -2038,8 +2038,8 @@ __device__ __forceinline__ void store_accumulators(const TileGemmParams& p, char
       });
     });
   } else {
-    // Everything else (edge tiles, C-input, split-K partials, strided or unaligned C, unsigned-operand
-    // terms): each wavefront lays one 32-row block of its accumulators out row-major in LDS and walks it
+    // Everything else (split-K partials of edge tiles, strided columns of C or of a C input, unsigned-operand terms, a C
+    // input beside dequantisation): each wavefront lays one 32-row block of its accumulators out row-major in LDS and walks it
     // in a rolled loop, a lane taking four consecutive columns of one row per step - one copy of the
     // general store code, and stores that run along rows.
     constexpr int COLS = WN * 32, QUADS = COLS / 4;

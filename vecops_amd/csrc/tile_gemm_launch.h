@@ -14,7 +14,7 @@ namespace vecops_hip {
 // How the operand pair is fetched.
 enum LoadMode : int {
   MODE_GENERIC = 0,  // element loads, any strides
-  MODE_KVEC = 1,     // A and B K-contiguous and 16-byte aligned
+  MODE_KVEC = 1,     // A and B K-contiguous, rows at any alignment
   MODE_NVEC_B = 2,   // A K-contiguous; B stored [K,N] row-major, any N and alignment (16- and 32-bit compute types)
   MODE_KVEC_DMA = 3,   // MODE_KVEC with 16-byte aligned rows and bases: loads that write LDS themselves
   MODE_NVEC_B_DMA = 4  // MODE_NVEC_B likewise
