@@ -219,7 +219,8 @@ VECOPS_HIP_EXPORT int32_t vecops_hip_matmul_static_workspace(const VecopsHipOper
  * small kernels fed through their arguments: no host buffer has to outlive the call, nothing is allocated; so do groups with an
  * unsigned side, whose row-sum terms are computed group by group into the workspace first).  Groups whose K vecops_hip_matmul
  * would split (few output tiles, long K) run that call's plan as launches of their own or, several of them, together: on slim
- * tiles, or in the one launch with the others, where that is estimated well ahead.  fp64 operands, a mix of classes (signed x
+ * tiles, or in the one launch with the others, where that is estimated well ahead (beside it one group whose layout of B would
+ * turn the others' loads into element loads keeps a launch of its own).  fp64 operands, a mix of classes (signed x
  * signed bytes beside groups with an unsigned side count as a mix) and groups with K = 0 run as launches of their own on the
  * same stream.  Results are those of vecops_hip_matmul on each group (bit-equal when that call runs the same tile shape without
  * splitting K and its plan names no slim tile - except 16-bit products with K <= 256 on 128 x 128 tiles, where the single call
